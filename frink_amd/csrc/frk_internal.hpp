@@ -218,21 +218,14 @@ int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTile
 // max_rows rows whose first entry is not negative
 int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, size_t max_rows, Q8KTiled out,
                                 hipStream_t s);
-// batched GEMM on the int8 matrix cores (Q4_K, and Q5_K with q5 set: its fifth bits are a third plane of
-// the same kernel); ws must hold gemm_q4_k_workspace_bytes(M, cols, rows, kind is Q5_K)
-size_t gemm_q4_k_workspace_bytes(size_t M, size_t cols, size_t rows, bool q5 = false);
-int launch_gemm_q4_k(const frk_weights *w, const float *x, size_t M, float *y, void *ws, hipStream_t s);
-// the same over activations already quantized into the tiled form; `partial` holds the parts' sums of a split
-int launch_gemm_q4_k_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, float *partial, hipStream_t s);
-// the same for Q6_K (frk_gemm_q6.hip)
-size_t gemm_q6_k_workspace_bytes(size_t M, size_t cols, size_t rows);
-int launch_gemm_q6_k(const frk_weights *w, const float *x, size_t M, float *y, void *ws, hipStream_t s);
-int launch_gemm_q6_k_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, float *partial, hipStream_t s);
-// its grouped (per-expert) form: tile t = rows [64*t, 64*t+64) of the activations and of y, tiles[t] =
-// {expert, 64*t, rows in use, 0}, tiles past *n_tiles idle; expert e owns rows [e*rows_e, (e+1)*rows_e) of w
-int launch_gemm_q6_k_grouped(const frk_weights *w, size_t rows_e, Q8KTiled a, const int4 *tiles, const int *n_tiles,
-                             int max_tiles, float *y, hipStream_t s);
-// and for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time
+// batched GEMM of the K-quants on the int8 matrix cores; ws must hold pipe_gemm_workspace_bytes(...): the tiled
+// activations, then room for the parts' sums where the blocks are split between workgroups.  With a limit on the memory
+// the blocks are split no further than it allows.
+size_t pipe_gemm_workspace_bytes(int kind, size_t M, size_t cols, size_t rows, size_t limit = SIZE_MAX);
+int launch_pipe_gemm(const frk_weights *w, const float *x, size_t M, float *y, void *ws, size_t ws_bytes, hipStream_t s);
+// the same over activations already quantized into the tiled form; `parts` holds the parts' sums of a split
+int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, size_t parts_bytes, hipStream_t s);
+// the same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time
 size_t gemm_q8_0_workspace_bytes(size_t M, size_t cols, size_t rows);
 // y[n] = partial[0][n] + partial[1][n] + ... in that order (the split GEMMs' second step; frk_gemm_q6.hip)
 int launch_sum_parts(const float *partial, int parts, size_t n, float *y, hipStream_t s);
@@ -281,11 +274,11 @@ constexpr size_t MOE_PER_TOKEN_MAX_BATCH = 16;
 // add up in ascending expert id; smaller batches run per position and add up in routing order.
 constexpr size_t MOE_BUCKET_ORDER_FROM = 32;
 bool moe_takes_per_token_path(size_t batch, size_t hidden, size_t ffn, int down_kind);
-// The grouped Q4_K GEMM over the tile list (one matrix, or two that share the activations).  The activations
-// are `a`, quantized in the grouped order, or -- with `src` -- the source rows' Q8_K and `gather`, the source
+// The grouped Q4_K or Q6_K GEMM over the tile list (one matrix, or two that share the activations).  The activations
+// are `a`, quantized in the grouped order, or -- Q4_K only, with `src` -- the source rows' Q8_K and `gather`, the source
 // row of every row of the grouped order (gemm_q4_k_stream_gathers tells whether the kernel can address them).
 bool gemm_q4_k_stream_gathers(size_t src_rows, size_t cols);
-int launch_gemm_q4_k_stream(const frk_weights *w0, const frk_weights *w1, size_t rows_e, Q8KTiled a,
+int launch_gemm_k_stream(const frk_weights *w0, const frk_weights *w1, size_t rows_e, Q8KTiled a,
                             const Q8KRows *src, const int *gather, const int4 *tiles, const int *n_tiles,
                             int max_tiles, float *y0, float *y1, hipStream_t s);
 // The grouped GEMM over groups the caller lists (Q4_K or Q6_K weights stacked group by group): y[p] = W[group of

@@ -608,7 +608,7 @@ int launch_moe_ffn(const frk_weights *gate, const frk_weights *up, const frk_wei
         hipLaunchKernelGGL(moe_group_quantize_kernel, dim3(1 + quantizers), dim3(1024), sizeof(GroupLds), s, ga, x,
                            (int)n_blocks, m.xr);
         FRK_LAUNCH_CHECK("moe_group_quantize");
-        rc = launch_gemm_q4_k_stream(gate, up, (size_t)ffn, m.xa, &m.xr, m.gather, m.tiles, m.n_tiles, max_tiles, m.gate_out,
+        rc = launch_gemm_k_stream(gate, up, (size_t)ffn, m.xa, &m.xr, m.gather, m.tiles, m.n_tiles, max_tiles, m.gate_out,
                                      m.up_out, s);
     } else {
         hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), sizeof(GroupLds), s, ga);
@@ -616,18 +616,15 @@ int launch_moe_ffn(const frk_weights *gate, const frk_weights *up, const frk_wei
         // the token rows, gathered into the grouped order and quantized; gate and up share them
         rc = launch_quantize_q8_k_gather(x, (size_t)hidden, m.gather, rows, m.xa, s);
         if (rc) return rc;
-        rc = launch_gemm_q4_k_stream(gate, up, (size_t)ffn, m.xa, nullptr, nullptr, m.tiles, m.n_tiles, max_tiles, m.gate_out,
+        rc = launch_gemm_k_stream(gate, up, (size_t)ffn, m.xa, nullptr, nullptr, m.tiles, m.n_tiles, max_tiles, m.gate_out,
                                      m.up_out, s);
     }
     if (rc) return rc;
     hipLaunchKernelGGL(swiglu_quantize_kernel, dim3((unsigned)(rows / 32 * (ffn / QK_K))), dim3(64 * SWIGLU_WAVES), 0, s,
                        m.gate_out, m.up_out, ffn / QK_K, m.tiles, m.n_tiles, m.act);
     FRK_LAUNCH_CHECK("swiglu_quantize");
-    // (a Q4_K_M checkpoint keeps some layers' down experts in Q6_K: the matrix-core Q6_K kernel, by tile)
-    rc = down->kind == FRK_KIND_Q6_K
-             ? launch_gemm_q6_k_grouped(down, (size_t)hidden, m.act, m.tiles, m.n_tiles, max_tiles, m.down_out, s)
-             : launch_gemm_q4_k_stream(down, nullptr, (size_t)hidden, m.act, nullptr, nullptr, m.tiles, m.n_tiles, max_tiles,
-                                       m.down_out, nullptr, s);
+    // (a Q4_K_M checkpoint keeps some layers' down experts in Q6_K)
+    rc = launch_gemm_k_stream(down, nullptr, (size_t)hidden, m.act, nullptr, nullptr, m.tiles, m.n_tiles, max_tiles, m.down_out, nullptr, s);
     if (rc) return rc;
     hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)batch, (unsigned)((hidden + 1023) / 1024)), dim3(256), 0, s, m.down_out, ids, weights, m.pos_of, k,
                        hidden, n_experts, (int)(batch >= MOE_BUCKET_ORDER_FROM), out);
@@ -681,15 +678,13 @@ int launch_gemm_grouped(const frk_weights *w, size_t n_groups, const int32_t *gr
         const unsigned quantizers = (unsigned)std::min<size_t>((n_blocks + 15) / 16, 512);
         hipLaunchKernelGGL(grouped_tiles_quantize_kernel, dim3(1 + quantizers), dim3(1024), 0, s, ta, x, (int)n_blocks, m.xr);
         FRK_LAUNCH_CHECK("grouped_tiles_quantize");
-        return launch_gemm_q4_k_stream(w, nullptr, rows_g, m.xa, &m.xr, m.src_rows, m.tiles, m.n_tiles, max_tiles, y, nullptr, s);
+        return launch_gemm_k_stream(w, nullptr, rows_g, m.xa, &m.xr, m.src_rows, m.tiles, m.n_tiles, max_tiles, y, nullptr, s);
     }
     hipLaunchKernelGGL(grouped_tiles_kernel, dim3(1), dim3(1024), 0, s, ta);
     FRK_LAUNCH_CHECK("grouped_tiles");
     int rc = launch_quantize_q8_k_gather(x, cols, m.src_rows, rows, m.xa, s);
     if (rc) return rc;
-    return w->kind == FRK_KIND_Q6_K
-               ? launch_gemm_q6_k_grouped(w, rows_g, m.xa, m.tiles, m.n_tiles, max_tiles, y, s)
-               : launch_gemm_q4_k_stream(w, nullptr, rows_g, m.xa, nullptr, nullptr, m.tiles, m.n_tiles, max_tiles, y, nullptr, s);
+    return launch_gemm_k_stream(w, nullptr, rows_g, m.xa, nullptr, nullptr, m.tiles, m.n_tiles, max_tiles, y, nullptr, s);
 }
 
 // Experts in Q5_0 / IQ4_XS / MXFP4 (run_expert takes any WeightMatrix, crates/frink-moe/src/lib.rs:1068-1165; gpt-oss

@@ -483,6 +483,7 @@ struct Scratch {
         *out = lease.ptr;
         return rc;
     }
+    size_t limit() const { return fixed ? fixed_bytes : SIZE_MAX; }
 };
 
 // Quantizes `batch` activation rows of w->cols values to Q8_K in the call's scratch memory.
@@ -631,12 +632,14 @@ static bool q6_k_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     const size_t q6k_gemm_from = w->rows * w->cols > (size_t)2 * 4096 * 4096 ? 25 : 41;
     return w->kind == FRK_KIND_Q6_K && batch >= q6k_gemm_from;
 }
+static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
+    return q4_k_takes_the_matrix_cores(w, batch) || q5_k_takes_the_matrix_cores(w, batch) || q6_k_takes_the_matrix_cores(w, batch);
+}
 // whether a batch of this matrix multiplies on the thin kernels (over plain Q8_K rows)
 static bool batch_takes_the_thin_kernels(const frk_weights *w, size_t batch) {
     const bool k_quant = w->kind == FRK_KIND_Q4_K || w->kind == FRK_KIND_Q5_K || w->kind == FRK_KIND_Q6_K;
     if (!k_quant || batch < 2) return false;
-    if (q4_k_takes_the_matrix_cores(w, batch) || q5_k_takes_the_matrix_cores(w, batch) || q6_k_takes_the_matrix_cores(w, batch))
-        return false;
+    if (k_quant_takes_the_matrix_cores(w, batch)) return false;
     return thin_gemm_max_batch(w) >= 2;
 }
 
@@ -728,18 +731,12 @@ static int gemm_units_int(const frk_weights *w, const float *x, size_t batch, fl
 static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *y, void *stream, Scratch &scratch) {
     // one row is the decode path, whatever the kind
     if (batch == 1) return gemv_impl(w, x, y, FRK_ACT_F32, (hipStream_t)stream, scratch);
-    if (q4_k_takes_the_matrix_cores(w, batch) || q5_k_takes_the_matrix_cores(w, batch)) {  // (frk_hip_gemm_pair_dev: the same test)
+    if (k_quant_takes_the_matrix_cores(w, batch)) {  // (frk_hip_gemm_pair_dev: the same test)
         void *ws = nullptr;
-        int rc = scratch.get(gemm_q4_k_workspace_bytes(batch, w->cols, w->rows, w->kind == FRK_KIND_Q5_K),
-                             (hipStream_t)stream, &ws);
+        const size_t bytes = pipe_gemm_workspace_bytes(w->kind, batch, w->cols, w->rows, scratch.limit());
+        int rc = scratch.get(bytes, (hipStream_t)stream, &ws);
         if (rc) return rc;
-        return launch_gemm_q4_k(w, x, batch, y, ws, (hipStream_t)stream);
-    }
-    if (q6_k_takes_the_matrix_cores(w, batch)) {
-        void *ws = nullptr;
-        int rc = scratch.get(gemm_q6_k_workspace_bytes(batch, w->cols, w->rows), (hipStream_t)stream, &ws);
-        if (rc) return rc;
-        return launch_gemm_q6_k(w, x, batch, y, ws, (hipStream_t)stream);
+        return launch_pipe_gemm(w, x, batch, y, ws, bytes, (hipStream_t)stream);
     }
     // Q8_0: a batch is the integer path, as in the reference (Q8_0 activation blocks and dot_q8_0_q8,
     // crates/frink-core/src/weight_matrix.rs:2701-2829); a single row keeps the f32 dot of its decode path
@@ -816,21 +813,20 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
         return set_error(FRK_ERR_SHAPE, "the matrices have %zu and %zu columns: they share one batch of activations", w0->cols, w1->cols);
     hipStream_t s = (hipStream_t)stream;
     Scratch scratch;
-    auto tiled = [&](const frk_weights *w) { return q4_k_takes_the_matrix_cores(w, batch) || q5_k_takes_the_matrix_cores(w, batch); };
-    if (tiled(w0) && tiled(w1)) {
+    if (k_quant_takes_the_matrix_cores(w0, batch) && k_quant_takes_the_matrix_cores(w1, batch)) {
         // one quantization into the tiled form, then the two GEMMs (each with its own room for a split's parts)
         const size_t acts_bytes = round_up(q8k_tiled_bytes(batch, w0->cols), 256);
-        const size_t part0 = gemm_q4_k_workspace_bytes(batch, w0->cols, w0->rows, w0->kind == FRK_KIND_Q5_K) - acts_bytes;
-        const size_t part1 = gemm_q4_k_workspace_bytes(batch, w1->cols, w1->rows, w1->kind == FRK_KIND_Q5_K) - acts_bytes;
+        const size_t part0 = pipe_gemm_workspace_bytes(w0->kind, batch, w0->cols, w0->rows) - acts_bytes;
+        const size_t part1 = pipe_gemm_workspace_bytes(w1->kind, batch, w1->cols, w1->rows) - acts_bytes;
         void *ws = nullptr;
         int rc = scratch.get(acts_bytes + round_up(part0, 256) + part1, s, &ws);
         if (rc) return rc;
         const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
         rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
         if (rc) return rc;
-        rc = launch_gemm_q4_k_acts(w0, acts, batch, y0, reinterpret_cast<float *>((char *)ws + acts_bytes), s);
+        rc = launch_pipe_gemm_acts(w0, acts, batch, y0, (char *)ws + acts_bytes, part0, s);
         if (rc) return rc;
-        return launch_gemm_q4_k_acts(w1, acts, batch, y1, reinterpret_cast<float *>((char *)ws + acts_bytes + round_up(part0, 256)), s);
+        return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)ws + acts_bytes + round_up(part0, 256), part1, s);
     }
     // otherwise each matrix takes the path frk_hip_gemm_dev gives it (the same results, two quantizations)
     int rc = gemm_impl(w0, x, batch, y0, stream, scratch);
@@ -929,21 +925,17 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *a, float *
         return set_error(FRK_ERR_UNSUPPORTED, "Q8_K activations feed Q4_K, Q5_K and Q6_K weights only (kind %d): frk_hip_gemm_dev", w->kind);
     const size_t batch = a->batch;
     hipStream_t s = (hipStream_t)stream;
-    const bool q45 = q4_k_takes_the_matrix_cores(w, batch) || q5_k_takes_the_matrix_cores(w, batch);
-    if (q45 || q6_k_takes_the_matrix_cores(w, batch)) {
+    if (k_quant_takes_the_matrix_cores(w, batch)) {
         const Q8KTiled acts = q8k_tiled_carve((char *)a->base + a->tiled_off, batch, a->cols);
         const size_t acts_bytes = round_up(q8k_tiled_bytes(batch, w->cols), 256);
-        const size_t need = q45 ? gemm_q4_k_workspace_bytes(batch, w->cols, w->rows, w->kind == FRK_KIND_Q5_K)
-                                : gemm_q6_k_workspace_bytes(batch, w->cols, w->rows);
-        float *partial = nullptr;
+        const size_t need = pipe_gemm_workspace_bytes(w->kind, batch, w->cols, w->rows);
+        void *parts = nullptr;
         Scratch scratch;
         if (need > acts_bytes) {  // a split of the blocks between workgroups: room for the parts' sums
-            void *ws = nullptr;
-            int rc = scratch.get(need - acts_bytes, s, &ws);
+            int rc = scratch.get(need - acts_bytes, s, &parts);
             if (rc) return rc;
-            partial = (float *)ws;
         }
-        return q45 ? launch_gemm_q4_k_acts(w, acts, batch, y, partial, s) : launch_gemm_q6_k_acts(w, acts, batch, y, partial, s);
+        return launch_pipe_gemm_acts(w, acts, batch, y, parts, need - acts_bytes, s);
     }
     // (below the matrix-core GEMMs' batches the plain rows are there: ACTS_PLAIN_MAX_BATCH covers every such batch)
     if (batch > ACTS_PLAIN_MAX_BATCH)

@@ -250,7 +250,8 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *acts, floa
 
 /* frk_hip_gemm_dev for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same arguments, same
- * kernels and bit for bit the same y, but the scratch memory (quantized activations, the parts of a
+ * kernels and bit for bit the same y (where the parts of a split GEMM fit; where they do not the blocks of a
+ * row are split less and add up in another order), but the scratch memory (quantized activations, the parts of a
  * split GEMM) is a fixed array of FRK_NOALLOC_SCRATCH_MIB MiB inside the library's device image, looked
  * up on the first call on a device; the call never allocates or frees.  A shape whose scratch does not
  * fit returns FRK_ERR_SHAPE and launches nothing (it fits every batch of up to 64 rows of matrices up to

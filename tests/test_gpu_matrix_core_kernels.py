@@ -1,0 +1,35 @@
+"""The matrix-core kernels at the edges of their tiles and splits, on arbitrary block bytes (every scale and code)."""
+import numpy as np
+import pytest
+
+import oracle as fo
+from test_gpu_parity import fa, to_dev  # noqa: F401 (fa: the module's fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols,batch", [
+    (33, 512, 65),        # one row group and one token past a tile, two blocks a row
+    (257, 2816, 130),     # a row past a large tile, eleven blocks: splits of unequal length
+    (129, 16384, 70),     # 64 blocks split over eight workgroups
+    (4130, 1024, 700),    # large tiles, the last of both kinds partly filled
+    (1, 768, 97),
+])
+@pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K, fo.Q6_K])
+def test_pipelined_gemm_at_the_edges_of_its_tiles(fa, kind, rows, cols, batch):
+    from bench import random_blocks
+    from frink_amd import synth
+    data = random_blocks(kind, rows, cols, seed=rows + kind)
+    x = synth.activations(31 + batch, batch, cols, outlier_frac=0.01)
+    w = fa.Weights.from_host(kind, data, rows, cols)
+    got = w.gemm(to_dev(x)).cpu().numpy().astype(np.float64)
+    q, d, _ = fo.quantize_q8_k(x.reshape(-1))
+    a = (q.reshape(-1, 256).astype(np.float64) * d.reshape(-1, 1).astype(np.float64)).reshape(batch, cols)
+    wd = fo.dequant(kind, data).reshape(rows, cols).astype(np.float64)
+    # Per block an output gains d_a * (d * S1 - dmin * S2): integers exact (S1 rounded once to f32), up to eight f32
+    # roundings, then one per block in the sum; every rounding is of a number no larger than |W| |x| with the two terms
+    # of Q4_K and Q5_K, whose difference the weight is, taken apart.  |d * sc * q| and |dmin * m| are each below the sum
+    # of the largest weight of their row and twice its largest offset, hence the row's largest |w| times sum |x|.
+    room = np.abs(a).sum(axis=1)[:, None] * (3.0 * np.abs(wd).max(axis=1))[None, :]
+    assert (np.abs(got - a @ wd.T) <= (cols // 256 + 9) * 2.0 ** -24 * room).all()
+    w.release()
