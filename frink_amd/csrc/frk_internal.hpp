@@ -53,10 +53,11 @@ inline int block_elems(int kind) {
 //   Q6_K row of nb blocks: ql[nb][128] | qh[nb][64] | sc[nb][16] | d[nb] f16, padded to 16
 //   Q8_0 row of nb blocks: qs[nb][32] | d[nb] f16, padded to 16
 //   Q4_0 row of nb blocks (18-byte blocks): qs[nb][16] | d[nb] f16, padded to 16
+//   MXFP4 row of nb blocks (17-byte blocks): qs[nb][16] | e[nb] (E8M0), padded to 16
 // Same bytes, same count per block; only their order changes.
 struct Layout {
     size_t row_stride = 0;  // bytes between resident rows
-    size_t off_a = 0;       // Q6_K: qh plane offset in a row; Q8_0, Q4_0: d plane offset
+    size_t off_a = 0;       // Q6_K: qh plane offset in a row; Q8_0, Q4_0: d plane offset; MXFP4: e plane offset
     size_t off_b = 0;       // Q6_K: sc plane offset
     size_t off_c = 0;       // Q6_K: d plane offset
 };
@@ -84,7 +85,10 @@ inline Layout layout_for(int kind, size_t cols) {
     } else if (kind == FRK_KIND_Q4_0) {
         l.off_a = nb * 16;
         l.row_stride = round_up(l.off_a + nb * 2, 16);
-    } else {  // Q5_0, IQ4_XS, MXFP4: the GGUF bytes in place, rows 16-byte aligned
+    } else if (kind == FRK_KIND_MXFP4) {
+        l.off_a = nb * 16;
+        l.row_stride = round_up(nb * MXFP4_BYTES, 16);
+    } else {  // Q5_0, IQ4_XS: the GGUF bytes in place, rows 16-byte aligned
         l.row_stride = round_up(nb * (size_t)block_bytes(kind), 16);
     }
     return l;
@@ -242,6 +246,19 @@ int launch_gemm_planar_grouped(const uint8_t *W, size_t row_stride, size_t off_d
                                size_t max_tiles, float *y, hipStream_t s);
 size_t q8_0_gemm_acts_bytes(size_t rows, size_t cols);
 int launch_quantize_q8_0_gemm(const float *x, const float *up, size_t rows, size_t cols, int8_t *q, uint16_t *d, hipStream_t s);
+// the grouped form over MXFP4 matrices as they are (frk_gemm_mx.hip): activation rows as planes of digits, and the
+// GEMM; with `up` y = silu(w x) * (up x)
+struct MxActs {
+    uint8_t *digits;   // [rows][blocks of 32, padded to a multiple of 8][96]
+    uint32_t *scales;  // [rows][blocks]: a byte per plane
+    float *factor;     // [rows]: 1, or infinity where a block's scale is
+};
+MxActs mx_acts_carve(void *base, size_t rows, size_t cols);
+size_t mx_acts_bytes(size_t rows, size_t cols);
+int launch_quantize_mx(const float *x, size_t rows, size_t cols, const int *used, const MxActs &out, hipStream_t s);
+bool mx_gemm_fits(size_t act_rows, size_t rows_g, size_t cols);
+int launch_gemm_mx_grouped(const frk_weights *w, const frk_weights *up, size_t rows_g, const MxActs &acts, const int *src_rows,
+                           const int4 *tiles, const int *n_tiles, size_t max_tiles, float *y, hipStream_t s);
 // the grouped GEMM over groups of Q5_0 / IQ4_XS / MXFP4 matrices that have a decoded form for the matrix cores
 bool units_have_planar_form(const frk_weights *w);
 // that form: rows of layout_for(FRK_KIND_Q8_0, cols) -- signed bytes, then f16 scales per 32 (IQ4_XS: per block of
@@ -249,12 +266,12 @@ bool units_have_planar_form(const frk_weights *w);
 size_t units_planar_bytes(size_t rows, size_t cols);
 int launch_units_decode(const frk_weights *w, uint8_t *dst, hipStream_t s);
 int units_decoded(const frk_weights *w, uint8_t *room, hipStream_t s, const uint8_t **out);
-size_t grouped_units_workspace_bytes(size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs, size_t cols);
+size_t grouped_units_workspace_bytes(int kind, size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs, size_t cols);
 int launch_gemm_grouped_units(const frk_weights *w, size_t n_groups, const int32_t *group_off, const int32_t *gather, const float *x,
                               size_t x_rows, size_t pairs, float *y, void *ws, hipStream_t s);
 // MoE layer over Q5_0 / IQ4_XS / MXFP4 experts by bucket, on the matrix cores (32 tokens and more)
 bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, size_t batch);
-size_t moe_units_grouped_workspace_bytes(size_t batch, int k, int n_experts, int hidden, int ffn);
+size_t moe_units_grouped_workspace_bytes(int gate_kind, int down_kind, size_t batch, int k, int n_experts, int hidden, int ffn);
 int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts,
                                  const float *x, size_t batch, const int32_t *ids, const float *weights, int k, float *out,
                                  void *ws, hipStream_t s);

@@ -3,7 +3,8 @@
 // (crates/frink-cuda/src/mul_mm.rs:146-205; CPU forms dequant_q5_0 / dot_q5_0_f32,
 // crates/frink-quant/src/lib.rs:4356-4418, dequant_iq4_xs / dot_iq4_xs_f32 :4860-4934, the E8M0 x E2M1
 // arithmetic of dequant_mxfp4_row / dot_mxfp4_row_f32 :4947-5040 over 17-byte GGUF blocks :5560-5570).
-// The resident copy keeps the GGUF bytes of a row in place (rows start 16-byte aligned); a weight is the
+// The resident copy keeps the GGUF bytes of a row in place (rows start 16-byte aligned; MXFP4: codes [units][16], then
+// scale bytes [units]); a weight is the
 // dequantizer's value bit for bit.  The GEMV is the f32 dot of the reference's decode path: a wavefront
 // per row, a lane per unit of 32 weights, the activation staged in LDS; the integer tier of these kinds
 // (Q8_0 / Q8_K activations, crates/frink-quant/src/legacy_q8.rs, iq4_xs_q8.rs) is the second half of this file.
@@ -50,9 +51,9 @@ __device__ __forceinline__ float e2m1_value(const E2M1x4 &v, int k) {
 }
 __device__ __forceinline__ uint32_t load_u16(const uint8_t *p) { return *reinterpret_cast<const uint16_t *>(p); }
 
-// the 32 weights of unit u of a row (a block of Q5_0 / MXFP4, a sub-block of IQ4_XS), in element order
+// the 32 weights of unit u of a row of `units` (a block of Q5_0 / MXFP4, a sub-block of IQ4_XS), in element order
 template <int KIND>
-__device__ __forceinline__ void unit_weights(const uint8_t *__restrict__ row, int u, float (&w)[32]) {
+__device__ __forceinline__ void unit_weights(const uint8_t *__restrict__ row, int u, int units, float (&w)[32]) {
     if (KIND == FRK_KIND_Q5_0) {
         const uint8_t *blk = row + (size_t)u * Q5_0_BYTES;  // 2-byte aligned
         const float d = h2f(load_u16(blk));
@@ -89,13 +90,13 @@ __device__ __forceinline__ void unit_weights(const uint8_t *__restrict__ row, in
                 w[4 * i + k + 16] = __fmul_rn(dl, signed_byte(hi, k));
             }
         }
-    } else {  // MXFP4: 17-byte blocks, no alignment
-        const uint8_t *blk = row + (size_t)u * MXFP4_BYTES;
-        const float d = e8m0_scale(blk[0]);
+    } else {
+        const float d = e8m0_scale(row[units * 16 + u]);
+        const uint4 codes = *reinterpret_cast<const uint4 *>(row + u * 16);
+        const uint32_t qs[4] = {codes.x, codes.y, codes.z, codes.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const uint32_t q = (uint32_t)blk[1 + 4 * i] | ((uint32_t)blk[2 + 4 * i] << 8) | ((uint32_t)blk[3 + 4 * i] << 16) |
-                               ((uint32_t)blk[4 + 4 * i] << 24);
+            const uint32_t q = qs[i];
             const E2M1x4 lo = e2m1_lookup4(q & 0x0f0f0f0fu), hi = e2m1_lookup4((q >> 4) & 0x0f0f0f0fu);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(256) void dequant_units_kernel(const uint8_t *__res
         r = id < 0 ? 0 : (size_t)id >= table_rows ? table_rows - 1 : (size_t)id;
     }
     float w[32];
-    unit_weights<KIND>(W + r * row_stride, (int)u, w);
+    unit_weights<KIND>(W + r * row_stride, (int)u, (int)units, w);
     float4 *dst = reinterpret_cast<float4 *>(out + r_out * cols + u * 32);
 #pragma unroll
     for (int k = 0; k < 8; k++) dst[k] = make_float4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(512) void gemv_units_f32_kernel(const uint8_t *__re
         float acc = 0.0f;
         for (int u = lane; u < units; u += 64) {
             float w[32];
-            unit_weights<KIND>(row, u, w);
+            unit_weights<KIND>(row, u, units, w);
             const float4 *x4 = reinterpret_cast<const float4 *>(xs + (size_t)u * 32);
 #pragma unroll
             for (int k = 0; k < 8; k++) {
@@ -179,11 +180,11 @@ __device__ __forceinline__ uint32_t mxfp4_x2_lookup4(uint32_t n) {
 // ggml_e8m0_to_fp32_half (legacy_q8.rs:154-161): 2^(e - 128), the two subnormal patterns for e < 2
 __device__ __forceinline__ float e8m0_half_scale(uint32_t e) { return __uint_as_float(e < 2 ? 0x00200000u << e : (e - 1) << 23); }
 
-// The 32 codes of unit u of a row held in LDS, as eight registers of four signed bytes: c[0..3] = elements 0..15,
+// The 32 codes of unit u of a row of `units`, as eight registers of four signed bytes: c[0..3] = elements 0..15,
 // c[4..7] = elements 16..31; `scale` = the unit's multiplier (Q5_0: d; MXFP4: the halved E8M0 scale; IQ4_XS: ls - 32
 // as an integer in scale_i, the block's d in scale).
 template <int KIND>
-__device__ __forceinline__ void unit_codes(const uint8_t *row, int u, uint32_t (&c)[8], float &scale, int &scale_i) {
+__device__ __forceinline__ void unit_codes(const uint8_t *row, int u, int units, uint32_t (&c)[8], float &scale, int &scale_i) {
     scale_i = 1;
     if (KIND == FRK_KIND_Q5_0) {
         const uint8_t *blk = row + u * Q5_0_BYTES;  // 2-byte aligned
@@ -209,14 +210,10 @@ __device__ __forceinline__ void unit_codes(const uint8_t *row, int u, uint32_t (
             c[i] = iq4nl_lookup4(q[i] & 0x0f0f0f0fu);
             c[4 + i] = iq4nl_lookup4((q[i] >> 4) & 0x0f0f0f0fu);
         }
-    } else {  // MXFP4: 17-byte blocks, no alignment -- the sixteen code bytes out of five aligned words
-        const uint32_t at = (uint32_t)u * MXFP4_BYTES;
-        scale = e8m0_half_scale(row[at]);
-        const uint32_t *words = reinterpret_cast<const uint32_t *>(row) + ((at + 1) >> 2);
-        const uint32_t shift = (at + 1) & 3;  // (0: the fifth word is read and not used; the slot ends in slack for it)
-        const uint32_t g0 = words[0], g1 = words[1], g2 = words[2], g3 = words[3], g4 = words[4];
-        const uint32_t q[4] = {__builtin_amdgcn_alignbyte(g1, g0, shift), __builtin_amdgcn_alignbyte(g2, g1, shift),
-                               __builtin_amdgcn_alignbyte(g3, g2, shift), __builtin_amdgcn_alignbyte(g4, g3, shift)};
+    } else {
+        scale = e8m0_half_scale(row[units * 16 + u]);
+        const uint4 codes = *reinterpret_cast<const uint4 *>(row + u * 16);
+        const uint32_t q[4] = {codes.x, codes.y, codes.z, codes.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             c[i] = mxfp4_x2_lookup4(q[i] & 0x0f0f0f0fu);
@@ -227,7 +224,7 @@ __device__ __forceinline__ void unit_codes(const uint8_t *row, int u, uint32_t (
 
 // A wavefront per row, a lane per unit.  The quantized activation sits in LDS for the whole launch; a row's bytes go
 // global -> registers (whole 16-byte pieces, the next row's while this one is multiplied) -> the wavefront's own
-// LDS slot, from where the lanes pick their blocks apart (22- and 17-byte blocks have no alignment to load by).
+// LDS slot, from where the lanes pick their blocks apart (a 22-byte block has no alignment to load by).
 // JOBS: a grid of expert-indexed jobs (run_expert's projections, crates/frink-moe/src/lib.rs:1068-1165): job
 // blockIdx.y multiplies the rows of expert ids[job] (a slice of `rows` rows of the stacked matrix) with activation
 // row job / act_div and writes output row job; a job whose id is outside the experts does nothing.
@@ -299,7 +296,7 @@ __global__ __launch_bounds__(512) void gemv_units_int_kernel(const uint8_t *__re
             uint32_t c[8];
             float scale;
             int scale_i;
-            unit_codes<KIND>(row, u, c, scale, scale_i);
+            unit_codes<KIND>(row, u, units, c, scale, scale_i);
             const uint4 a0 = *reinterpret_cast<const uint4 *>(sq + u * 32), a1 = *reinterpret_cast<const uint4 *>(sq + u * 32 + 16);
             int isum = 0;
             isum = dot4(c[0], a0.x, isum);
@@ -469,7 +466,7 @@ __global__ __launch_bounds__(256) void units_to_q8_0_planar_kernel(const uint8_t
     uint32_t c[8];
     float scale;
     int scale_i;
-    unit_codes<KIND>(W + r * row_stride, (int)u, c, scale, scale_i);
+    unit_codes<KIND>(W + r * row_stride, (int)u, (int)units, c, scale, scale_i);
     uint4 *q = reinterpret_cast<uint4 *>(dst + r * dst_stride + u * 32);
     q[0] = make_uint4(c[0], c[1], c[2], c[3]);
     q[1] = make_uint4(c[4], c[5], c[6], c[7]);
@@ -501,7 +498,7 @@ __global__ __launch_bounds__(256) void iq4_xs_to_sub_planar_kernel(const uint8_t
     uint32_t c[8];
     float scale;
     int scale_i;
-    unit_codes<FRK_KIND_IQ4_XS>(W + r * row_stride, (int)u, c, scale, scale_i);
+    unit_codes<FRK_KIND_IQ4_XS>(W + r * row_stride, (int)u, (int)units, c, scale, scale_i);
     uint4 *q = reinterpret_cast<uint4 *>(dst + r * dst_stride + u * 32);
     q[0] = make_uint4(c[0], c[1], c[2], c[3]);
     q[1] = make_uint4(c[4], c[5], c[6], c[7]);
@@ -527,7 +524,7 @@ __global__ __launch_bounds__(256) void mxfp4_scale_range_kernel(const uint8_t *_
                                                                int *__restrict__ range) {
     int lo = 255, hi = 0;
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < rows * units; i += (size_t)gridDim.x * 256) {
-        const int e = W[(i / units) * row_stride + (i % units) * MXFP4_BYTES];
+        const int e = W[(i / units) * row_stride + units * 16 + i % units];
         lo = min(lo, e);
         hi = max(hi, e);
     }

@@ -748,15 +748,16 @@ int launch_moe_ffn_units(const frk_weights *gate, const frk_weights *up, const f
 
 // The same layer from 32 tokens on, when every projection's kind has a decoded form the matrix cores read (Q5_0;
 // MXFP4 with scales that are f16 values; IQ4_XS): the reference's bucket path (crates/frink-models/src/decoder/
-// ffn_batch.rs:343-434) -- the pairs bucketed by expert, every expert's rows read once -- with the experts decoded
-// into signed bytes in the call's scratch memory and the grouped form of the Q8_0 matrix-core kernel.  The
+// ffn_batch.rs:343-434) -- the pairs bucketed by expert, every expert's rows read once.  MXFP4 experts go to the
+// block-scaled matrix cores as they are (frk_gemm_mx.hip); the others are decoded into signed bytes in the call's scratch
+// memory for the grouped form of the Q8_0 matrix-core kernel.  The
 // activations are quantized per token (gate and up) and per grouped row (down) exactly as the per-pair jobs
 // quantize them, and the integers are the same: the two paths differ in the order of the float additions only.
 bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, size_t batch) {
     return batch >= MOE_BUCKET_ORDER_FROM && units_have_planar_form(gate) && units_have_planar_form(up) && units_have_planar_form(down);
 }
 struct UnitsGroupedScratch {
-    uint8_t *gate_w, *up_w, *down_w;  // decoded experts
+    uint8_t *gate_w, *up_w, *down_w;  // decoded experts (not of projections in their own form)
     char *x_acts, *a_acts;            // quantized token rows; quantized intermediate rows (grouped order)
     float *gate_out, *up_out, *down_out;
     int *group_off, *gather, *pos_of, *cpos_of, *n_tiles;
@@ -767,7 +768,18 @@ static size_t units_grouped_acts_bytes(size_t rows, size_t cols) {
     const size_t q8k = round_up(rows * cols, 256) + round_up(rows * cols / QK_K * 4 + 4, 256) + round_up(rows * cols / 16 * 2 + 2, 256);
     return std::max(q8_0_gemm_acts_bytes(rows, cols), q8k);
 }
-static UnitsGroupedScratch units_grouped_carve(void *base, size_t batch, int k, int n_experts, int hidden, int ffn, size_t *end) {
+// which projections multiply MXFP4 experts as they are (frk_gemm_mx.hip): no decoded copy, gate and up in one launch
+struct UnitsNative {
+    bool gate_up, down;
+};
+static UnitsNative units_native(int gate_kind, int down_kind, size_t batch, size_t rows, size_t hidden, size_t ffn) {
+    UnitsNative n;
+    n.gate_up = gate_kind == FRK_KIND_MXFP4 && mx_gemm_fits(std::max(batch, rows), ffn, hidden);
+    n.down = n.gate_up && down_kind == FRK_KIND_MXFP4 && mx_gemm_fits(rows, hidden, ffn);
+    return n;
+}
+static UnitsGroupedScratch units_grouped_carve(void *base, UnitsNative native, size_t batch, int k, int n_experts, int hidden, int ffn,
+                                               size_t *end) {
     const size_t pairs = batch * (size_t)k, rows = moe_max_rows(pairs, n_experts);
     char *p = (char *)base;
     auto take = [&](size_t bytes) {
@@ -776,13 +788,13 @@ static UnitsGroupedScratch units_grouped_carve(void *base, size_t batch, int k, 
         return r;
     };
     UnitsGroupedScratch m;
-    m.gate_w = (uint8_t *)take(units_planar_bytes((size_t)n_experts * ffn, hidden));
-    m.up_w = (uint8_t *)take(units_planar_bytes((size_t)n_experts * ffn, hidden));
-    m.down_w = (uint8_t *)take(units_planar_bytes((size_t)n_experts * hidden, ffn));
-    m.x_acts = take(units_grouped_acts_bytes(batch, hidden));
-    m.a_acts = take(units_grouped_acts_bytes(rows, ffn));
-    m.gate_out = (float *)take(rows * ffn * 4);
-    m.up_out = (float *)take(rows * ffn * 4);
+    m.gate_w = (uint8_t *)take(native.gate_up ? 0 : units_planar_bytes((size_t)n_experts * ffn, hidden));
+    m.up_w = (uint8_t *)take(native.gate_up ? 0 : units_planar_bytes((size_t)n_experts * ffn, hidden));
+    m.down_w = (uint8_t *)take(native.down ? 0 : units_planar_bytes((size_t)n_experts * hidden, ffn));
+    m.x_acts = take(native.gate_up ? mx_acts_bytes(batch, hidden) : units_grouped_acts_bytes(batch, hidden));
+    m.a_acts = take(native.down ? mx_acts_bytes(rows, ffn) : units_grouped_acts_bytes(rows, ffn));
+    m.gate_out = (float *)take(rows * ffn * 4);  // (native: silu(gate) * up)
+    m.up_out = (float *)take(native.gate_up ? 0 : rows * ffn * 4);
     m.down_out = (float *)take(rows * hidden * 4);
     m.group_off = (int *)take((n_experts + 1) * 4);
     m.gather = (int *)take(rows * 4);
@@ -793,9 +805,10 @@ static UnitsGroupedScratch units_grouped_carve(void *base, size_t batch, int k, 
     if (end) *end = (size_t)(p - (char *)base);
     return m;
 }
-size_t moe_units_grouped_workspace_bytes(size_t batch, int k, int n_experts, int hidden, int ffn) {
+size_t moe_units_grouped_workspace_bytes(int gate_kind, int down_kind, size_t batch, int k, int n_experts, int hidden, int ffn) {
     size_t end = 0;
-    (void)units_grouped_carve(nullptr, batch, k, n_experts, hidden, ffn, &end);
+    const UnitsNative native = units_native(gate_kind, down_kind, batch, moe_max_rows(batch * (size_t)k, n_experts), hidden, ffn);
+    (void)units_grouped_carve(nullptr, native, batch, k, n_experts, hidden, ffn, &end);
     return end;
 }
 // rows x cols floats quantized into `room` for a projection of `kind`; the pointers the grouped GEMM takes
@@ -818,7 +831,7 @@ static int quantize_for_units_grouped(int kind, const float *x, const float *up,
     a->d = d;
     return launch_quantize_q8_0_gemm(x, up, rows, cols, q, d, s);
 }
-// The grouped GEMM as an entry of its own over groups of these kinds: the tile list, the stack decoded, the
+// The grouped GEMM as an entry of its own over groups of these kinds: the tile list, the stack decoded (MXFP4: as it is), the
 // activation rows quantized once (Q8_0 blocks, or Q8_K for IQ4_XS), the grouped kernel gathering through the list.
 struct GroupedUnitsScratch {
     uint8_t *decoded;
@@ -826,8 +839,11 @@ struct GroupedUnitsScratch {
     int *src_rows, *n_tiles;
     int4 *tiles;
 };
-static GroupedUnitsScratch grouped_units_carve(void *base, size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs, size_t cols,
-                                               size_t *end) {
+static bool grouped_units_native(int kind, size_t rows_g, size_t x_rows, size_t cols) {
+    return kind == FRK_KIND_MXFP4 && mx_gemm_fits(x_rows, rows_g, cols);
+}
+static GroupedUnitsScratch grouped_units_carve(void *base, bool native, size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs,
+                                               size_t cols, size_t *end) {
     const size_t rows = moe_max_rows(pairs, (int)n_groups);
     char *p = (char *)base;
     auto take = [&](size_t bytes) {
@@ -836,28 +852,36 @@ static GroupedUnitsScratch grouped_units_carve(void *base, size_t n_groups, size
         return r;
     };
     GroupedUnitsScratch m;
-    m.decoded = (uint8_t *)take(units_planar_bytes(w_rows, cols));
-    m.acts = take(units_grouped_acts_bytes(x_rows, cols));
+    m.decoded = (uint8_t *)take(native ? 0 : units_planar_bytes(w_rows, cols));
+    m.acts = take(native ? mx_acts_bytes(x_rows, cols) : units_grouped_acts_bytes(x_rows, cols));
     m.src_rows = (int *)take(rows * 4);
     m.n_tiles = (int *)take(256);
     m.tiles = (int4 *)take((rows / MOE_TILE + 1) * 16);
     if (end) *end = (size_t)(p - (char *)base);
     return m;
 }
-size_t grouped_units_workspace_bytes(size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs, size_t cols) {
+size_t grouped_units_workspace_bytes(int kind, size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs, size_t cols) {
     size_t end = 0;
-    (void)grouped_units_carve(nullptr, n_groups, w_rows, x_rows, pairs, cols, &end);
+    (void)grouped_units_carve(nullptr, grouped_units_native(kind, w_rows / n_groups, x_rows, cols), n_groups, w_rows, x_rows, pairs, cols, &end);
     return end;
 }
 int launch_gemm_grouped_units(const frk_weights *w, size_t n_groups, const int32_t *group_off, const int32_t *gather, const float *x,
                               size_t x_rows, size_t pairs, float *y, void *ws, hipStream_t s) {
     const size_t rows_g = w->rows / n_groups, cols = w->cols, rows = moe_max_rows(pairs, (int)n_groups);
-    const GroupedUnitsScratch m = grouped_units_carve(ws, n_groups, w->rows, x_rows, pairs, cols, nullptr);
+    const bool native = grouped_units_native(w->kind, rows_g, x_rows, cols);
+    const GroupedUnitsScratch m = grouped_units_carve(ws, native, n_groups, w->rows, x_rows, pairs, cols, nullptr);
     const GroupedTilesArgs ta{group_off, gather, (int)n_groups, (int)pairs, (int)x_rows, (int)rows, m.src_rows, m.tiles, m.n_tiles};
     hipLaunchKernelGGL(grouped_tiles_kernel, dim3(1), dim3(1024), 0, s, ta);
     FRK_LAUNCH_CHECK("grouped_tiles");
+    int rc;
+    if (native) {
+        const MxActs xa = mx_acts_carve(m.acts, x_rows, cols);
+        rc = launch_quantize_mx(x, x_rows, cols, nullptr, xa, s);
+        if (rc) return rc;
+        return launch_gemm_mx_grouped(w, nullptr, rows_g, xa, m.src_rows, m.tiles, m.n_tiles, rows / MOE_TILE, y, s);
+    }
     const uint8_t *decoded = nullptr;
-    int rc = units_decoded(w, m.decoded, s, &decoded);
+    rc = units_decoded(w, m.decoded, s, &decoded);
     if (rc) return rc;
     UnitsGroupedActs xa;
     rc = quantize_for_units_grouped(w->kind, x, nullptr, x_rows, cols, m.acts, &xa, s);
@@ -872,7 +896,8 @@ int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up,
                                  void *ws, hipStream_t s) {
     const int hidden = (int)gate->cols, ffn = (int)down->cols;
     const size_t pairs = batch * (size_t)k, rows = moe_max_rows(pairs, n_experts), max_tiles = rows / MOE_TILE;
-    const UnitsGroupedScratch m = units_grouped_carve(ws, batch, k, n_experts, hidden, ffn, nullptr);
+    const UnitsNative native = units_native(gate->kind, down->kind, batch, rows, hidden, ffn);
+    const UnitsGroupedScratch m = units_grouped_carve(ws, native, batch, k, n_experts, hidden, ffn, nullptr);
     static bool sized = false;  // a benign race: every thread sets the same attribute
     if (!sized) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_kernel),
@@ -883,29 +908,48 @@ int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up,
     const GroupArgs ga{ids, (int)pairs, k, n_experts, m.group_off, m.gather, m.pos_of, m.cpos_of, m.tiles, m.n_tiles, (int)rows};
     hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), sizeof(GroupLds), s, ga);
     FRK_LAUNCH_CHECK("moe_group");
-    const uint8_t *gate_w = nullptr, *up_w = nullptr, *down_w = nullptr;
-    int rc = units_decoded(gate, m.gate_w, s, &gate_w);
-    if (rc) return rc;
-    rc = units_decoded(up, m.up_w, s, &up_w);
-    if (rc) return rc;
-    rc = units_decoded(down, m.down_w, s, &down_w);
-    if (rc) return rc;
-    UnitsGroupedActs xa, aa;
-    rc = quantize_for_units_grouped(gate->kind, x, nullptr, batch, (size_t)hidden, m.x_acts, &xa, s);
-    if (rc) return rc;
-    const Layout lg = layout_for(FRK_KIND_Q8_0, (size_t)hidden), ld = layout_for(FRK_KIND_Q8_0, (size_t)ffn);
-    rc = launch_gemm_planar_grouped(gate_w, lg.row_stride, lg.off_a, (size_t)ffn, (size_t)hidden, gate->kind == FRK_KIND_IQ4_XS, xa.q,
-                                    xa.d, m.gather, m.tiles, m.n_tiles, max_tiles, m.gate_out, s);
-    if (rc) return rc;
-    rc = launch_gemm_planar_grouped(up_w, lg.row_stride, lg.off_a, (size_t)ffn, (size_t)hidden, up->kind == FRK_KIND_IQ4_XS, xa.q,
-                                    xa.d, m.gather, m.tiles, m.n_tiles, max_tiles, m.up_out, s);
-    if (rc) return rc;
-    // silu(gate) * up, quantized in the same launch (rows of the grouped order that no pair uses hold whatever the
-    // memory held: nothing reads their results)
-    rc = quantize_for_units_grouped(down->kind, m.gate_out, m.up_out, rows, (size_t)ffn, m.a_acts, &aa, s);
-    if (rc) return rc;
-    rc = launch_gemm_planar_grouped(down_w, ld.row_stride, ld.off_a, (size_t)hidden, (size_t)ffn, down->kind == FRK_KIND_IQ4_XS, aa.q,
-                                    aa.d, nullptr, m.tiles, m.n_tiles, max_tiles, m.down_out, s);
+    int rc;
+    if (native.gate_up) {
+        const MxActs xa = mx_acts_carve(m.x_acts, batch, hidden);
+        rc = launch_quantize_mx(x, batch, (size_t)hidden, nullptr, xa, s);
+        if (rc) return rc;
+        rc = launch_gemm_mx_grouped(gate, up, (size_t)ffn, xa, m.gather, m.tiles, m.n_tiles, max_tiles, m.gate_out, s);
+        if (rc) return rc;
+    } else {
+        const uint8_t *gate_w = nullptr, *up_w = nullptr;
+        rc = units_decoded(gate, m.gate_w, s, &gate_w);
+        if (rc) return rc;
+        rc = units_decoded(up, m.up_w, s, &up_w);
+        if (rc) return rc;
+        UnitsGroupedActs xa;
+        rc = quantize_for_units_grouped(gate->kind, x, nullptr, batch, (size_t)hidden, m.x_acts, &xa, s);
+        if (rc) return rc;
+        const Layout lg = layout_for(FRK_KIND_Q8_0, (size_t)hidden);
+        rc = launch_gemm_planar_grouped(gate_w, lg.row_stride, lg.off_a, (size_t)ffn, (size_t)hidden, gate->kind == FRK_KIND_IQ4_XS, xa.q,
+                                        xa.d, m.gather, m.tiles, m.n_tiles, max_tiles, m.gate_out, s);
+        if (rc) return rc;
+        rc = launch_gemm_planar_grouped(up_w, lg.row_stride, lg.off_a, (size_t)ffn, (size_t)hidden, up->kind == FRK_KIND_IQ4_XS, xa.q,
+                                        xa.d, m.gather, m.tiles, m.n_tiles, max_tiles, m.up_out, s);
+        if (rc) return rc;
+    }
+    // silu(gate) * up, quantized (rows of the grouped order that no pair uses hold whatever the memory held: nothing
+    // reads their results)
+    if (native.down) {
+        const MxActs aa = mx_acts_carve(m.a_acts, rows, ffn);
+        rc = launch_quantize_mx(m.gate_out, rows, (size_t)ffn, m.gather, aa, s);
+        if (rc) return rc;
+        rc = launch_gemm_mx_grouped(down, nullptr, (size_t)hidden, aa, nullptr, m.tiles, m.n_tiles, max_tiles, m.down_out, s);
+    } else {
+        const uint8_t *down_w = nullptr;
+        rc = units_decoded(down, m.down_w, s, &down_w);
+        if (rc) return rc;
+        UnitsGroupedActs aa;
+        rc = quantize_for_units_grouped(down->kind, m.gate_out, native.gate_up ? nullptr : m.up_out, rows, (size_t)ffn, m.a_acts, &aa, s);
+        if (rc) return rc;
+        const Layout ld = layout_for(FRK_KIND_Q8_0, (size_t)ffn);
+        rc = launch_gemm_planar_grouped(down_w, ld.row_stride, ld.off_a, (size_t)hidden, (size_t)ffn, down->kind == FRK_KIND_IQ4_XS, aa.q,
+                                        aa.d, nullptr, m.tiles, m.n_tiles, max_tiles, m.down_out, s);
+    }
     if (rc) return rc;
     hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)batch, (unsigned)((hidden + 1023) / 1024)), dim3(256), 0, s, m.down_out, ids,
                        weights, m.pos_of, k, hidden, n_experts, 1, out);

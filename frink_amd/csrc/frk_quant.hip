@@ -116,6 +116,9 @@ __global__ __launch_bounds__(256) void repack_kernel(int kind, const uint8_t *__
     } else if (kind == FRK_KIND_Q4_0) {
         const size_t blk = o / Q4_0_BYTES, w = o % Q4_0_BYTES;
         to = w < 2 ? l.off_a + blk * 2 + w : blk * 16 + (w - 2);
+    } else if (kind == FRK_KIND_MXFP4) {
+        const size_t blk = o / MXFP4_BYTES, w = o % MXFP4_BYTES;
+        to = w < 1 ? l.off_a + blk : blk * 16 + (w - 1);
     } else {
         to = o;
     }

@@ -1118,7 +1118,7 @@ int frk_hip_moe_ffn_dev(const frk_weights *gate, const frk_weights *up, const fr
     if (batch * k > (size_t)1 << 30) return set_error(FRK_ERR_SHAPE, "batch*k = %zu pairs is too many", batch * k);
     WorkspaceLease lease;
     if (unit_experts && moe_units_takes_grouped_path(gate, up, down, batch)) {
-        int rc = workspace(moe_units_grouped_workspace_bytes(batch, (int)k, (int)n_experts, (int)hidden, (int)ffn), (hipStream_t)stream, lease);
+        int rc = workspace(moe_units_grouped_workspace_bytes(gate->kind, down->kind, batch, (int)k, (int)n_experts, (int)hidden, (int)ffn), (hipStream_t)stream, lease);
         if (rc) return rc;
         return launch_moe_ffn_units_grouped(gate, up, down, (int)n_experts, x, batch, ids, weights, (int)k, out, lease.ptr,
                                             (hipStream_t)stream);
@@ -1154,7 +1154,7 @@ int frk_hip_gemm_grouped_dev(const frk_weights *stacked, size_t n_groups, const 
     if (x_rows == 0) return set_error(FRK_ERR_SHAPE, "%zu pairs over no activation rows", pairs);
     WorkspaceLease lease;
     if (units) {
-        int rc = workspace(grouped_units_workspace_bytes(n_groups, stacked->rows, x_rows, pairs, stacked->cols), (hipStream_t)stream, lease);
+        int rc = workspace(grouped_units_workspace_bytes(stacked->kind, n_groups, stacked->rows, x_rows, pairs, stacked->cols), (hipStream_t)stream, lease);
         if (rc) return rc;
         return launch_gemm_grouped_units(stacked, n_groups, group_off, gather, x, x_rows, pairs, y, lease.ptr, (hipStream_t)stream);
     }

@@ -1,0 +1,83 @@
+"""MXFP4 experts on the block-scaled matrix cores (frk_gemm_mx.hip), at the edges of its tiles: rows, blocks a row, rows in
+use of a tile, both workgroup sizes; and the activations whose Q8_0 scale leaves f16."""
+import numpy as np
+import pytest
+
+import oracle as fo
+from test_gpu_parity import _other_kind_blocks, fa, test_moe_ffn_with_experts_of_the_other_kinds, to_dev  # noqa: F401 (fa: a fixture)
+
+_moe_case = test_moe_ffn_with_experts_of_the_other_kinds
+del test_moe_ffn_with_experts_of_the_other_kinds  # (collected in its own file)
+
+
+def _case(fa, counts, rows_g, cols, x, seed):
+    n_groups = len(counts)
+    off = np.zeros(n_groups + 1, np.int32)
+    off[1:] = np.cumsum(counts)
+    data = _other_kind_blocks(fo.MXFP4, n_groups * rows_g, cols, seed=seed)
+    blk = data.reshape(-1, 17)
+    blk[:, 0] = 104 + blk[:, 0] % 40
+    w = fa.Weights.from_host(fo.MXFP4, data, n_groups * rows_g, cols)
+    got = fa.gemm_grouped(w, n_groups, to_dev(off), to_dev(x)).cpu().numpy()
+    w.release()
+    return off, data.reshape(n_groups, -1), got
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows_g,cols,counts", [
+    (1, 32, [1, 64]), (63, 96, [0, 33, 2]), (65, 128, [32, 31, 65]), (257, 160, [64, 5]), (72, 544, [97, 1]),
+    (512, 1056, [40]), (1100, 160, [3, 0, 34] * 30),  # (the last: eight wavefronts a workgroup, three workgroups a tile)
+])
+def test_grouped_gemm_at_the_edges_of_its_tiles(fa, rows_g, cols, counts):
+    from frink_amd import synth
+    print("mxfp4 experts", rows_g, cols, len(counts), flush=True)
+    pairs = sum(counts)
+    x = synth.activations(71, pairs, cols, outlier_frac=0.01)
+    off, per, got = _case(fa, counts, rows_g, cols, x, seed=rows_g + cols)
+    # Q8_0 activations in exact arithmetic.  A matrix-core step sums 64 exact products within 8 units in the last place
+    # of its largest (6.2 seen), eight steps in a row to a running sum of 128 columns, then one addition each.
+    xb = x.reshape(pairs, cols // 32, 32)
+    amax = np.abs(xb).max(axis=2)
+    inv = np.where(amax != 0, np.float32(127) / np.where(amax != 0, amax, 1), 0).astype(np.float32)
+    q = np.clip(np.rint(xb * inv[:, :, None]), -127, 127).astype(np.float64)
+    a = (q * (amax / np.float32(127)).astype(np.float16).astype(np.float64)[:, :, None]).reshape(pairs, cols)
+    for g in range(len(counts)):
+        s = slice(int(off[g]), int(off[g + 1]))
+        wd = fo.dequant(fo.MXFP4, per[g]).reshape(rows_g, cols).astype(np.float64)
+        room = (64 + cols // 128 + 1) * 2.0 ** -24 * (np.abs(a[s]) @ np.abs(wd).T)
+        assert (np.abs(got[s] - a[s] @ wd.T) <= room).all(), g
+
+
+@pytest.mark.gpu
+def test_activations_whose_scale_leaves_f16(fa):
+    """An infinite value empties its block (0 times an infinite scale: NaN), one above 8.3e6 makes the results infinite
+    with its block's sign, a NaN counts as zero; a tiny block's scale is an f16 subnormal; the other rows are untouched."""
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((40, 96)).astype(np.float32)
+    x[3, 40] = np.inf
+    x[7, 10] = 2.0e7
+    x[9, 50] = np.nan
+    x[11, :32] *= 1e-5
+    x[12] = 0.0
+    off, per, got = _case(fa, [40], 70, 96, x, seed=9)
+    want = fo.gemm(fo.MXFP4, per[0], 70, 96, x, fo.INT_DOT)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(got[3]).all()
+    assert np.isinf(got[7]).any() and np.array_equal(np.isinf(got), np.isinf(want))
+    inf = np.isinf(want)
+    assert np.array_equal(np.sign(got[inf]), np.sign(want[inf]))
+    fine = [r for r in range(40) if r not in (3, 7)]
+    assert (np.abs(got[fine] - want[fine]).max(axis=1) <= 1e-5 * np.abs(want[fine]).max(axis=1)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_experts,k,hidden,ffn,batch", [(64, 2, 160, 1056, 40), (3, 2, 544, 288, 33)])
+def test_moe_layer_at_the_edges_of_its_tiles(fa, n_experts, k, hidden, ffn, batch):
+    _moe_case(fa, fo.MXFP4, fo.MXFP4, n_experts, k, hidden, ffn, batch)
+
+
+def test_no_result_of_the_matrix_core_is_read_too_soon(tmp_path):
+    import isa_mfma_lint
+    from test_isa_waits import _assembly
+    asm = _assembly(tmp_path, "frk_gemm_mx.hip")
+    assert "v_mfma_scale_f32_32x32x64_f8f6f4" in asm
+    assert isa_mfma_lint.violations(asm) == []
