@@ -270,7 +270,8 @@ size_t grouped_units_workspace_bytes(int kind, size_t n_groups, size_t w_rows, s
 int launch_gemm_grouped_units(const frk_weights *w, size_t n_groups, const int32_t *group_off, const int32_t *gather, const float *x,
                               size_t x_rows, size_t pairs, float *y, void *ws, hipStream_t s);
 // MoE layer over Q5_0 / IQ4_XS / MXFP4 experts by bucket, on the matrix cores (32 tokens and more)
-bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, size_t batch);
+bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts, size_t batch,
+                                  int k);
 size_t moe_units_grouped_workspace_bytes(int gate_kind, int down_kind, size_t batch, int k, int n_experts, int hidden, int ffn);
 int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts,
                                  const float *x, size_t batch, const int32_t *ids, const float *weights, int k, float *out,

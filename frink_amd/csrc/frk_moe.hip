@@ -691,8 +691,8 @@ int launch_gemm_grouped(const frk_weights *w, size_t n_groups, const int32_t *gr
 // keeps its experts in MXFP4): every (token, slot) pair is a job of the integer decode kernel -- gate and up over the
 // token's quantized activation, silu(g) * u, that row quantized, down -- and the weighted sum in the reference's order
 // for the batch size.  Q8_0 activation blocks for Q5_0 and MXFP4 projections, Q8_K for IQ4_XS ones.  (A batch of
-// hundreds of tokens would read an expert's matrices once per pair here: from 32 tokens on the layer takes the
-// bucketed path below instead, where the kinds have a decoded form.)
+// hundreds of tokens would read an expert's matrices once per pair here: from 32 tokens on, and MXFP4 experts from two
+// pairs an expert on, the layer takes the bucketed path below instead, where the kinds have a decoded form.)
 struct UnitsActs {
     int8_t *q;
     float *d;
@@ -746,15 +746,33 @@ int launch_moe_ffn_units(const frk_weights *gate, const frk_weights *up, const f
     return FRK_OK;
 }
 
-// The same layer from 32 tokens on, when every projection's kind has a decoded form the matrix cores read (Q5_0;
+// The same layer from 32 tokens on (MXFP4: moe_units_takes_grouped_path), when every projection's kind has a decoded form the matrix cores read (Q5_0;
 // MXFP4 with scales that are f16 values; IQ4_XS): the reference's bucket path (crates/frink-models/src/decoder/
 // ffn_batch.rs:343-434) -- the pairs bucketed by expert, every expert's rows read once.  MXFP4 experts go to the
 // block-scaled matrix cores as they are (frk_gemm_mx.hip); the others are decoded into signed bytes in the call's scratch
 // memory for the grouped form of the Q8_0 matrix-core kernel.  The
 // activations are quantized per token (gate and up) and per grouped row (down) exactly as the per-pair jobs
 // quantize them, and the integers are the same: the two paths differ in the order of the float additions only.
-bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, size_t batch) {
-    return batch >= MOE_BUCKET_ORDER_FROM && units_have_planar_form(gate) && units_have_planar_form(up) && units_have_planar_form(down);
+// which projections multiply MXFP4 experts as they are (frk_gemm_mx.hip): no decoded copy, gate and up in one launch
+struct UnitsNative {
+    bool gate_up, down;
+};
+static UnitsNative units_native(int gate_kind, int down_kind, size_t batch, size_t rows, size_t hidden, size_t ffn) {
+    UnitsNative n;
+    n.gate_up = gate_kind == FRK_KIND_MXFP4 && mx_gemm_fits(std::max(batch, rows), ffn, hidden);
+    n.down = n.gate_up && down_kind == FRK_KIND_MXFP4 && mx_gemm_fits(rows, hidden, ffn);
+    return n;
+}
+bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts, size_t batch,
+                                  int k) {
+    if (!units_have_planar_form(gate) || !units_have_planar_form(up) || !units_have_planar_form(down)) return false;
+    if (batch >= MOE_BUCKET_ORDER_FROM) return true;
+    // Below 32 tokens a job per pair reads an expert once for every pair, the grouped kernel once.  It pays from about two
+    // pairs an expert on, and from 32 pairs (per pair / grouped, us): 32 experts top-4 of 2880 / 2880 at 8, 12, 16 tokens
+    // 143 / 187, 207 / 196, 263 / 197; 16 top-4 of 1440 / 2880 at 6, 8 77 / 82, 97 / 83; 16 top-2 of 2048 / 1440 at 12, 16
+    // 56 / 58, 67 / 59; 8 top-2 of 1024 / 1024 at 12, 16, 24 39 / 42, 45 / 42, 59 / 43.
+    const size_t pairs = batch * (size_t)k, ffn = down->cols;
+    return pairs >= std::max<size_t>(2 * (size_t)n_experts, 32) && units_native(gate->kind, down->kind, batch, moe_max_rows(pairs, n_experts), gate->cols, ffn).down;
 }
 struct UnitsGroupedScratch {
     uint8_t *gate_w, *up_w, *down_w;  // decoded experts (not of projections in their own form)
@@ -767,16 +785,6 @@ struct UnitsGroupedScratch {
 static size_t units_grouped_acts_bytes(size_t rows, size_t cols) {
     const size_t q8k = round_up(rows * cols, 256) + round_up(rows * cols / QK_K * 4 + 4, 256) + round_up(rows * cols / 16 * 2 + 2, 256);
     return std::max(q8_0_gemm_acts_bytes(rows, cols), q8k);
-}
-// which projections multiply MXFP4 experts as they are (frk_gemm_mx.hip): no decoded copy, gate and up in one launch
-struct UnitsNative {
-    bool gate_up, down;
-};
-static UnitsNative units_native(int gate_kind, int down_kind, size_t batch, size_t rows, size_t hidden, size_t ffn) {
-    UnitsNative n;
-    n.gate_up = gate_kind == FRK_KIND_MXFP4 && mx_gemm_fits(std::max(batch, rows), ffn, hidden);
-    n.down = n.gate_up && down_kind == FRK_KIND_MXFP4 && mx_gemm_fits(rows, hidden, ffn);
-    return n;
 }
 static UnitsGroupedScratch units_grouped_carve(void *base, UnitsNative native, size_t batch, int k, int n_experts, int hidden, int ffn,
                                                size_t *end) {
@@ -952,7 +960,7 @@ int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up,
     }
     if (rc) return rc;
     hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)batch, (unsigned)((hidden + 1023) / 1024)), dim3(256), 0, s, m.down_out, ids,
-                       weights, m.pos_of, k, hidden, n_experts, 1, out);
+                       weights, m.pos_of, k, hidden, n_experts, (int)(batch >= MOE_BUCKET_ORDER_FROM), out);
     FRK_LAUNCH_CHECK("moe_combine");
     return FRK_OK;
 }

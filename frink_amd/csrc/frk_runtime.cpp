@@ -1117,7 +1117,7 @@ int frk_hip_moe_ffn_dev(const frk_weights *gate, const frk_weights *up, const fr
                          gate->rows, gate->cols, up->rows, up->cols, down->rows, down->cols, n_experts, hidden, ffn);
     if (batch * k > (size_t)1 << 30) return set_error(FRK_ERR_SHAPE, "batch*k = %zu pairs is too many", batch * k);
     WorkspaceLease lease;
-    if (unit_experts && moe_units_takes_grouped_path(gate, up, down, batch)) {
+    if (unit_experts && moe_units_takes_grouped_path(gate, up, down, (int)n_experts, batch, (int)k)) {
         int rc = workspace(moe_units_grouped_workspace_bytes(gate->kind, down->kind, batch, (int)k, (int)n_experts, (int)hidden, (int)ffn), (hipStream_t)stream, lease);
         if (rc) return rc;
         return launch_moe_ffn_units_grouped(gate, up, down, (int)n_experts, x, batch, ids, weights, (int)k, out, lease.ptr,

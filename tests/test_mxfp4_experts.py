@@ -70,7 +70,7 @@ def test_activations_whose_scale_leaves_f16(fa):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_experts,k,hidden,ffn,batch", [(64, 2, 160, 1056, 40), (3, 2, 544, 288, 33)])
+@pytest.mark.parametrize("n_experts,k,hidden,ffn,batch", [(64, 2, 160, 1056, 40), (3, 2, 544, 288, 33), (8, 2, 288, 544, 16), (16, 2, 96, 160, 15)])
 def test_moe_layer_at_the_edges_of_its_tiles(fa, n_experts, k, hidden, ffn, batch):
     _moe_case(fa, fo.MXFP4, fo.MXFP4, n_experts, k, hidden, ffn, batch)
 
