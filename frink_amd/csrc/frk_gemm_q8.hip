@@ -395,23 +395,31 @@ static int q8_0_split(size_t rows, size_t M, size_t nb32) {
     while (ks < Q8_MAX_SPLIT && wgs * ks * 2 <= fill && pairs / (size_t)(ks * 2) >= 2) ks *= 2;
     return ks;
 }
-// the quantized activations, their scales, and room for the parts' sums where the chunks are split
-size_t gemm_q8_0_workspace_bytes(size_t M, size_t cols, size_t rows) {
-    const int ks = q8_0_split(rows, M, cols / 32);
-    return round_up(M * cols, 256) + round_up(M * round_up(cols / 32, 8) * 2, 256) + (ks > 1 ? (size_t)ks * M * rows * sizeof(float) : 0);
+// Which kernel, and the scratch memory it takes: the quantized activations, their scales, and room for the parts' sums
+// where the columns are split -- in `limit` bytes where the larger tiles' own split is what would exceed them.
+Q8GemmPlan gemm_q8_0_plan(size_t M, size_t cols, size_t rows, bool q4, size_t limit) {
+    const size_t acts = round_up(M * cols, 256) + round_up(M * round_up(cols / 32, 8) * 2, 256), part = M * rows * sizeof(float);
+    const int split = q8_0_split(rows, M, cols / 32);
+    Q8GemmPlan p;
+    p.pipe = Q8PipePlan{0, 0, 0};
+    p.bytes = acts + (split > 1 ? (size_t)split * part : 0);
+    if (q4 || p.bytes > limit) return p;
+    p.pipe = q8_pipe_plan(rows, M, cols / 32, layout_for(FRK_KIND_Q8_0, cols).row_stride, split, (limit - acts) / part);
+    if (p.pipe.rows_wg) p.bytes = acts + (p.pipe.k_split > 1 ? (size_t)p.pipe.k_split * part : 0);
+    return p;
 }
 
 static int launch_q8_mfma(Q8GemmArgs g, bool q4, bool sub, hipStream_t s);
 
-int launch_gemm_q8_0(const frk_weights *w, const float *x, size_t M, float *y, void *ws, hipStream_t s) {
-    return launch_gemm_q8_0_planar(w->dev, w->layout.row_stride, w->layout.off_a, w->rows, w->cols, w->kind == FRK_KIND_Q4_0, x, M, y,
-                                   ws, s);
+int launch_gemm_q8_0(const frk_weights *w, const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s) {
+    return launch_gemm_q8_0_planar(w->dev, w->layout.row_stride, w->layout.off_a, w->rows, w->cols, w->kind == FRK_KIND_Q4_0, plan, x, M,
+                                   y, ws, s);
 }
 
 // The same over any rows in the planar form -- quants [nb][32] (q4: nibbles [nb][16]), then the f16 scales [nb] at
 // off_d of every row: the resident Q8_0 / Q4_0 matrices, and other 32-element kinds decoded into that form.
-int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t cols, bool q4, const float *x,
-                            size_t M, float *y, void *ws, hipStream_t s) {
+int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t cols, bool q4,
+                            const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s) {
     if (M > (size_t)1 << 30 || rows > (size_t)1 << 30)
         return set_error(FRK_ERR_SHAPE, "gemm_q8_0: %zu activation rows x %zu weight rows is too many", M, rows);
     struct {
@@ -438,6 +446,11 @@ int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, s
     g.tiles = nullptr;
     g.n_tiles = nullptr;
     g.src_rows = nullptr;
+    if (const Q8PipePlan &p = plan.pipe; p.rows_wg) {
+        const int rc = launch_gemm_q8_0_pipe(p, W, row_stride, off_d, rows, cols / 32, aq, ad, M, p.k_split > 1 ? g.partial : y, s);
+        if (rc || p.k_split == 1) return rc;
+        return launch_sum_parts(g.partial, p.k_split, M * rows, y, s);
+    }
     return launch_q8_mfma(g, q4, false, s);
 }
 

@@ -1,0 +1,261 @@
+// The batched Q8_0 GEMM from 65 rows on: the arithmetic of frk_gemm_q8.hip (an exact int8 MFMA per 32-wide block, the
+// block scales' outer product from the f16 matrix core, a conversion and a fused multiply-add per sum, blocks in order),
+// over larger tiles that come into LDS without passing through registers.
+//
+// What bounds it is the vector ALU: 32 instructions for a tile's two MFMAs.  A wavefront owns 32 weight rows and MT tiles
+// of 32 tokens, so a weight fragment is read once for MT products (the kernel it replaces read two fragments a product and
+// moved 816 bytes a product through registers into LDS; 256 x 128 tiles move 408, and no instruction touches them).
+// The columns go by in halves of a chunk (128 columns, four blocks), three stages in LDS, requested two ahead, the
+// requests spread over the arithmetic; block scales come a chunk (256 columns) at a time.  One barrier a half chunk.
+#include "frk_device.hpp"
+
+#include <type_traits>
+
+namespace frk {
+
+typedef int qp_v4i __attribute__((ext_vector_type(4)));
+typedef int qp_v16i __attribute__((ext_vector_type(16)));
+typedef float qp_v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 qp_v4h __attribute__((ext_vector_type(4)));
+
+struct Q8PipeArgs {
+    const uint8_t *W;  // rows: quants [nb][32], then the f16 scales [nb] at off_d
+    size_t row_stride, off_d;
+    const int8_t *aq;    // [M][nb * 32]
+    const uint16_t *ad;  // [M][nb rounded up to 8], zeros in the padding
+    float *y;            // [k_split][M][rows]
+    int rows, nb, M;
+    int row_tiles, tok_tiles, k_split;
+};
+
+// RG x TG wavefronts of 32 rows x MT tiles of tokens
+template <int RG, int TG, int MT>
+struct Q8PipeLds {
+    static_assert(RG * TG == 8, "eight wavefronts");
+    static constexpr int ROWS = 32 * RG, TOKS = 32 * TG * MT, LINES = ROWS + TOKS;
+    static constexpr int STAGE = LINES * 128, STAGES = 3;
+    static constexpr int OFF_SCALES = STAGES * STAGE, SCALES = LINES * 16;  // two slots of a chunk's scales
+    static constexpr int REQUESTS = LINES / 64;                            // of a wavefront and half chunk
+    static constexpr int SCALE_REQUESTS = LINES / 64;                      // of a chunk, one a wavefront
+    static constexpr size_t BYTES = OFF_SCALES + 2 * SCALES;
+    static_assert(LINES % 64 == 0 && SCALE_REQUESTS <= 8 && BYTES <= 160 * 1024, "whole requests, LDS of a CU");
+};
+
+template <int RG, int TG, int MT>
+__global__ __launch_bounds__(512, 2) void gemm_q8_0_pipe_kernel(Q8PipeArgs g) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using L = Q8PipeLds<RG, TG, MT>;
+    constexpr int R = L::REQUESTS;
+    extern __shared__ __align__(16) uint8_t qp_lds[];
+    const uint32_t lds0 = lds_address(qp_lds);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int li = lane & 31, lg = lane >> 5;
+    const int rg = wave % RG, tg = wave / RG;
+
+    // an XCD (block id mod 8) takes a run of the (row tile, token tile) list: its workgroups share weight rows
+    const int total = g.row_tiles * g.tok_tiles, per_xcd = (total + 7) / 8;
+    const int index = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+    if (((int)blockIdx.x >> 3) >= per_xcd || index >= total) return;  // (uniform)
+    const int row0 = index / g.tok_tiles * L::ROWS, tok0 = index % g.tok_tiles * L::TOKS;
+    const int n_chunks = (g.nb + 7) / 8;
+    const int chunk0 = n_chunks * (int)blockIdx.y / g.k_split, chunk1 = n_chunks * ((int)blockIdx.y + 1) / g.k_split;
+    // half chunks h0 .. h1 - 1 (the last chunk's second half may have no block)
+    const int h0 = 2 * chunk0, h1 = min(2 * chunk1, (g.nb + 3) / 4);
+    const size_t nbp = (size_t)n_chunks * 8;
+
+    // ---- the requests.  Lines 0 .. ROWS - 1 of a stage are weight rows, the others tokens, 128 bytes each; piece p of
+    // line r sits in place p ^ (r / 2) % 8, so that sixteen lines' reads of one piece fall in different banks.  Request n
+    // brings lines 8n .. 8n + 7.  (Lines past the operands repeat the last one: their results are not stored.  The last
+    // half chunk may reach past a row, into its scales or the next row: those products meet zero scales.  Past the last
+    // row there are the resident copy's 256 bytes of slack, and behind the quants of the last token the scales.)
+    auto line_offset = [&](int line) -> uint32_t {
+        return line < L::ROWS ? (uint32_t)min(row0 + line, g.rows - 1) * (uint32_t)g.row_stride
+                              : (uint32_t)min(tok0 + line - L::ROWS, g.M - 1) * (uint32_t)g.nb * 32u;
+    };
+    uint32_t off[R];
+#pragma unroll
+    for (int c = 0; c < R; c++) {
+        const int line = (wave * R + c) * 8 + (lane >> 3);
+        off[c] = line_offset(line) + (uint32_t)((lane & 7) ^ ((line >> 1) & 7)) * 16;
+    }
+    const bool fetches_scales = wave < L::SCALE_REQUESTS;
+    const int scale_line = wave * 64 + lane;  // (64 divides ROWS: a request is all rows or all tokens)
+    const uint32_t scale_off = scale_line < L::ROWS ? (uint32_t)min(row0 + scale_line, g.rows - 1) * (uint32_t)g.row_stride
+                                                    : (uint32_t)min(tok0 + scale_line - L::ROWS, g.M - 1) * (uint32_t)nbp * 2u;
+    const uint8_t *const scale_base = wave * 64 < L::ROWS ? g.W + g.off_d : reinterpret_cast<const uint8_t *>(g.ad);
+    int fill = 0;  // the stage the next half chunk goes into
+    auto fetch_quants = [&](int h, int c) {
+        const int n = wave * R + c;
+        const uint8_t *base = 8 * n < L::ROWS ? g.W : reinterpret_cast<const uint8_t *>(g.aq);
+        dma16(lds0 + (uint32_t)fill * L::STAGE + (uint32_t)n * 1024, base + (size_t)h * 128, off[c]);
+    };
+    auto fetch_scales = [&](int h) {  // in front of its chunk's first half
+        if (!(h & 1) && fetches_scales)
+            dma16(lds0 + L::OFF_SCALES + (uint32_t)((h >> 1) & 1) * L::SCALES + (uint32_t)wave * 1024, scale_base + (size_t)(h >> 1) * 16, scale_off);
+    };
+    auto filled = [&]() { fill = fill == L::STAGES - 1 ? 0 : fill + 1; };
+
+    qp_v16f acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++) acc[t] = qp_v16f{0.0f};
+    const qp_v16i zero_i = {0};
+    const qp_v16f zero_f = {0.0f};
+    // this lane's piece of block b in a line of its own row or token, less the line's tile
+    uint32_t piece[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++) piece[b] = (uint32_t)(li * 128 + ((2 * b + lg) ^ ((li >> 1) & 7)) * 16);
+
+#pragma unroll
+    for (int ahead = 0; ahead < 2; ahead++)
+        if (h0 + ahead < h1) {
+            fetch_scales(h0 + ahead);
+#pragma unroll
+            for (int c = 0; c < R; c++) fetch_quants(h0 + ahead, c);
+            filled();
+        }
+    int at = 0;
+    // MORE: half chunk h + 2 exists and is requested.  (Two copies of the body instead of branches in it: the compiler
+    // counts the wait states between an MFMA and a reader of its result within one basic block only.)
+    auto half_chunk = [&](auto more_c, int h) {
+        constexpr bool MORE = decltype(more_c)::value;
+        // half chunk h (and its chunk's scales) has landed; behind it only h + 1 was requested
+        if (h + 1 >= h1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if ((h & 1) && fetches_scales) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R + 1) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");
+        lds_barrier();
+        if (MORE) fetch_scales(h + 2);
+        const uint8_t *st = qp_lds + (size_t)at * L::STAGE, *sw_lines = st + rg * 32 * 128, *sa_lines = st + (L::ROWS + tg * MT * 32) * 128;
+        const uint8_t *sc = qp_lds + L::OFF_SCALES + ((h >> 1) & 1) * L::SCALES + (h & 1) * 8;
+        // the four blocks' scales, f16, two to a register; k = 0 of the outer product sits in lanes 0 .. 31
+        const int live = g.nb - 4 * h;  // blocks of the row from here on: a row's scales past its end are whatever lies there
+        uint2 sw = *reinterpret_cast<const uint2 *>(sc + (rg * 32 + li) * 16);
+        sw.x = lg ? 0u : sw.x & (live > 1 ? 0xffffffffu : 0xffffu);
+        sw.y = lg ? 0u : sw.y & (live > 3 ? 0xffffffffu : live > 2 ? 0xffffu : 0u);
+        uint2 sa[MT];
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+            sa[t] = *reinterpret_cast<const uint2 *>(sc + (L::ROWS + (tg * MT + t) * 32 + li) * 16);
+            sa[t].x = lg ? 0u : sa[t].x;
+            sa[t].y = lg ? 0u : sa[t].y;
+        }
+        auto k0 = [](uint2 s, int b) {  // {scale of block b, 0, 0, 0}
+            const uint32_t w = b < 2 ? s.x : s.y;
+            const uint2 u = make_uint2(b & 1 ? w >> 16 : w & 0xffffu, 0u);
+            qp_v4h v;
+            __builtin_memcpy(&v, &u, 8);
+            return v;
+        };
+        // A three-stage pipeline over the products (block by block, its MT tiles in turn): the reads of product n + 2, the
+        // matrix core's work for n + 1, the float step of n.
+        constexpr int N = 4 * MT;
+        auto read_w = [&](int b) { return *reinterpret_cast<const qp_v4i *>(sw_lines + piece[b]); };
+        auto read_a = [&](int n) { return *reinterpret_cast<const qp_v4i *>(sa_lines + (n % MT) * 4096 + piece[n / MT]); };
+        qp_v4i w1 = read_w(0), w2 = MT > 1 ? w1 : read_w(1), a1 = read_a(0), a2 = read_a(1);
+        qp_v16i isum_next = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, w1, zero_i, 0, 0, 0);
+        qp_v16f scale_next = __builtin_amdgcn_mfma_f32_32x32x8f16(k0(sa[0], 0), k0(sw, 0), zero_f, 0, 0, 0);
+        a1 = a2, w1 = w2;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < N; n++) {
+            const qp_v16i isum = isum_next;
+            const qp_v16f scale = scale_next;
+            if (n + 2 < N) {
+                a2 = read_a(n + 2);
+                w2 = (n + 2) % MT == 0 ? read_w((n + 2) / MT) : w1;
+            }
+            if (n + 1 < N) {
+                isum_next = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, w1, zero_i, 0, 0, 0);
+                scale_next = __builtin_amdgcn_mfma_f32_32x32x8f16(k0(sa[(n + 1) % MT], (n + 1) / MT), k0(sw, (n + 1) / MT), zero_f, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[n % MT][r] = __builtin_fmaf(scale[r], (float)isum[r], acc[n % MT][r]);
+            asm volatile("" : "+v"(acc[n % MT]));  // (the float step stays here: sunk to the end, every product's sums are alive at once)
+            if (n % (N / R) == 0 && n / (N / R) < R && MORE) fetch_quants(h + 2, n / (N / R));
+            __builtin_amdgcn_sched_barrier(0);
+            a1 = a2, w1 = w2;
+        }
+        static_assert(R <= N, "at most a request a product");
+        if (MORE) filled();
+        at = at == L::STAGES - 1 ? 0 : at + 1;
+    };
+    int h = h0;
+    for (; h + 2 < h1; h++) half_chunk(std::true_type(), h);
+    for (; h < h1; h++) half_chunk(std::false_type(), h);
+
+    // register r of a lane: token 8 * (r / 4) + 4 * (lane / 32) + r % 4 of the tile, weight row lane % 32
+    const int row = row0 + rg * 32 + li;
+    float *const dst = g.y + (size_t)blockIdx.y * g.M * g.rows;
+    if (row < g.rows) {
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int tok = tok0 + (tg * MT + t) * 32 + 8 * (r >> 2) + 4 * lg + (r & 3);
+                if (tok < g.M) dst[(size_t)tok * g.rows + row] = acc[t][r];
+            }
+    }
+#endif
+}
+
+template <int RG, int TG, int MT>
+static int launch_tile(const Q8PipeArgs &g, hipStream_t s) {
+    using L = Q8PipeLds<RG, TG, MT>;
+    static bool sized = false;  // a benign race: every thread sets the same attribute
+    if (!sized) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q8_0_pipe_kernel<RG, TG, MT>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::BYTES);
+        if (e != hipSuccess) return set_error(FRK_ERR_HIP, "hipFuncSetAttribute(LDS %zu): %s", L::BYTES, hipGetErrorString(e));
+        sized = true;
+    }
+    const unsigned grid = (unsigned)((g.row_tiles * g.tok_tiles + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_q8_0_pipe_kernel<RG, TG, MT>), dim3(grid, (unsigned)g.k_split), dim3(512), L::BYTES, s, g);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(FRK_ERR_HIP, "gemm_q8_0_pipe launch: %s", hipGetErrorString(e));
+    return FRK_OK;
+}
+
+// The tile and the split by estimated time, in us, `old_us` (without what all forms share) being the other kernel's.
+// Measured a half chunk (one workgroup a CU, one round of the chip): 256 x 128 tiles 2.64, 128 x 64 tiles 0.85 alone and
+// 1.47 in pairs (two fit a CU), the other kernel's 64 x 128 tiles 0.84 -- a 128 x 64 share of the work costs 0.66, 0.73 and
+// 0.84; a split's parts move at 6.2 TB/s.  With quantization, other kernel -> this one: 2048 x 4096 x 14336 388 -> 317 us,
+// 512 x 14336 x 4096 113 -> 91, 200 x 11008 x 4096 62 -> 49, 512 x 4096 x 14336 107 -> 98, 1000 x 4096 x 4096 64 -> 58;
+// grids of one round of the other kernel (2048 x 1024 x 4096: 40 against 42 us) stay there.
+Q8PipePlan q8_pipe_plan(size_t rows, size_t M, size_t nb, size_t row_stride, int old_split, size_t max_parts) {
+    Q8PipePlan best = {0, 0, 0};
+    if (M <= 64 || rows * row_stride > 0xffffffffu || M * nb * 32 > 0xffffffffu) return best;  // (32-bit lane offsets)
+    auto tiles = [](size_t n, size_t t) { return (n + t - 1) / t; };
+    auto parts = [&](size_t ks) { return ks > 1 ? 3.0 + (double)(2 * ks + 1) * (double)(M * rows) * 4.0 / 6.2e6 : 0.0; };
+    const size_t halves = (nb + 3) / 4, chunks = (nb + 7) / 8;
+    const double old_us = (double)tiles(tiles(rows, 64) * tiles(M, 128) * (size_t)old_split, 256) * 0.84 * (double)halves / old_split + parts(old_split);
+    double least = 0.97 * old_us - 2.0;  // (and two more to start)
+    for (size_t ks = 1; ks <= 4 && chunks / ks >= 2; ks *= 2) {
+        if (ks > 1 && ks > max_parts) break;
+        const double steps = (double)(2 * tiles(chunks, ks));
+        const size_t large = tiles(rows, 256) * tiles(M, 128) * ks, small = tiles(rows, 128) * tiles(M, 64) * ks, rest = small % 512;
+        const double large_us = (double)tiles(large, 256) * 2.64 * steps + parts(ks);
+        const double small_us = ((double)(small / 512) * 1.47 + (rest == 0 ? 0.0 : rest <= 256 ? 0.85 : 1.47)) * steps + parts(ks);
+        if (large_us < least) least = large_us, best = Q8PipePlan{256, 128, (int)ks};
+        if (small_us < least) least = small_us, best = Q8PipePlan{128, 64, (int)ks};
+    }
+    return best;
+}
+int launch_gemm_q8_0_pipe(const Q8PipePlan &p, const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t nb,
+                          const int8_t *aq, const uint16_t *ad, size_t M, float *y, hipStream_t s) {
+    Q8PipeArgs g;
+    g.W = W;
+    g.row_stride = row_stride;
+    g.off_d = off_d;
+    g.aq = aq;
+    g.ad = ad;
+    g.y = y;
+    g.rows = (int)rows;
+    g.nb = (int)nb;
+    g.M = (int)M;
+    g.row_tiles = (int)((rows + p.rows_wg - 1) / p.rows_wg);
+    g.tok_tiles = (int)((M + p.tok_wg - 1) / p.tok_wg);
+    g.k_split = p.k_split;
+    if (p.rows_wg == 256) return launch_tile<8, 1, 4>(g, s);
+    return launch_tile<4, 2, 1>(g, s);
+}
+
+}  // namespace frk

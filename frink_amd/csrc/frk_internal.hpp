@@ -230,12 +230,24 @@ int launch_pipe_gemm(const frk_weights *w, const float *x, size_t M, float *y, v
 // the same over activations already quantized into the tiled form; `parts` holds the parts' sums of a split
 int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, size_t parts_bytes, hipStream_t s);
 // the same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time
-size_t gemm_q8_0_workspace_bytes(size_t M, size_t cols, size_t rows);
 // y[n] = partial[0][n] + partial[1][n] + ... in that order (the split GEMMs' second step; frk_gemm_q6.hip)
 int launch_sum_parts(const float *partial, int parts, size_t n, float *y, hipStream_t s);
-int launch_gemm_q8_0(const frk_weights *w, const float *x, size_t M, float *y, void *ws, hipStream_t s);
-int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t cols, bool q4, const float *x,
-                            size_t M, float *y, void *ws, hipStream_t s);
+// its form over large tiles (frk_gemm_q8_pipe.hip): weight rows x tokens of a workgroup, and how many workgroups share a
+// row's columns; rows_wg = 0: the other kernel
+struct Q8PipePlan {
+    int rows_wg, tok_wg, k_split;
+};
+Q8PipePlan q8_pipe_plan(size_t rows, size_t M, size_t nb, size_t row_stride, int old_split, size_t max_parts);
+int launch_gemm_q8_0_pipe(const Q8PipePlan &p, const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t nb,
+                          const int8_t *aq, const uint16_t *ad, size_t M, float *y, hipStream_t s);
+struct Q8GemmPlan {
+    Q8PipePlan pipe;
+    size_t bytes;  // of scratch memory
+};
+Q8GemmPlan gemm_q8_0_plan(size_t M, size_t cols, size_t rows, bool q4, size_t limit);
+int launch_gemm_q8_0(const frk_weights *w, const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s);
+int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t cols, bool q4,
+                            const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s);
 // IQ4_XS on the matrix cores: the rows decoded to signed bytes with their block scales (launch_iq4_xs_to_sub_planar,
 // rows of layout_for(FRK_KIND_Q8_0, cols)'s stride) against Q8_K activations
 int launch_iq4_xs_to_sub_planar(const frk_weights *w, uint8_t *dst, size_t dst_stride, size_t off_d, hipStream_t s);

@@ -671,12 +671,14 @@ static int gemm_units_int(const frk_weights *w, const float *x, size_t batch, fl
         // (no room for the decoded rows where a copy of them is kept)
         const size_t planar_bytes = w->decoded.load(std::memory_order_acquire) ? 0 : round_up(planar.row_stride * w->rows + 256, 256);
         void *ws = nullptr;
-        int rc = scratch.get(planar_bytes + gemm_q8_0_workspace_bytes(batch, w->cols, w->rows), s, &ws);
+        const size_t limit = scratch.limit();
+        const Q8GemmPlan plan = gemm_q8_0_plan(batch, w->cols, w->rows, false, limit > planar_bytes ? limit - planar_bytes : 0);
+        int rc = scratch.get(planar_bytes + plan.bytes, s, &ws);
         if (rc) return rc;
         const uint8_t *decoded = nullptr;
         rc = units_decoded(w, (uint8_t *)ws, s, &decoded);
         if (rc) return rc;
-        return launch_gemm_q8_0_planar(decoded, planar.row_stride, planar.off_a, w->rows, w->cols, false, x, batch, y,
+        return launch_gemm_q8_0_planar(decoded, planar.row_stride, planar.off_a, w->rows, w->cols, false, plan, x, batch, y,
                                        (char *)ws + planar_bytes, s);
     }
     if (!gemv_units_int_fits(w))
@@ -742,9 +744,10 @@ static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *
     // crates/frink-core/src/weight_matrix.rs:2701-2829); a single row keeps the f32 dot of its decode path
     if ((w->kind == FRK_KIND_Q8_0 || w->kind == FRK_KIND_Q4_0) && batch >= 2) {  // (Q4_0: the same kernel, dot_q4_0_q8)
         void *ws = nullptr;
-        int rc = scratch.get(gemm_q8_0_workspace_bytes(batch, w->cols, w->rows), (hipStream_t)stream, &ws);
+        const Q8GemmPlan plan = gemm_q8_0_plan(batch, w->cols, w->rows, w->kind == FRK_KIND_Q4_0, scratch.limit());
+        int rc = scratch.get(plan.bytes, (hipStream_t)stream, &ws);
         if (rc) return rc;
-        return launch_gemm_q8_0(w, x, batch, y, ws, (hipStream_t)stream);
+        return launch_gemm_q8_0(w, plan, x, batch, y, ws, (hipStream_t)stream);
     }
     // Q5_0 / IQ4_XS / MXFP4: a batch is the integer tier too, as in the reference (q8_row_dot / q8k_row_dot per
     // (row, activation) over activations quantized once, crates/frink-core/src/weight_matrix.rs:392-420)
