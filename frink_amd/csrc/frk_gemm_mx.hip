@@ -15,7 +15,7 @@
 //
 // Before, the experts were decoded to signed bytes with f16 scales on every call (83 us a projection of 32 x 2880 x
 // 2880) and multiplied by the Q8_0 kernel, whose float step is 32 vector instructions per MFMA (156 us).
-#include "frk_device.hpp"
+#include "frk_mx_quant.hpp"
 
 #include <type_traits>
 
@@ -31,12 +31,6 @@ typedef float mx_v16f __attribute__((ext_vector_type(16)));
         if (e_ != hipSuccess) return set_error(FRK_ERR_HIP, what " launch: %s", hipGetErrorString(e_)); \
     } while (0)
 
-// ---- activations: rows of blocks, a row padded with zero blocks to a multiple of eight.  A block: six 16-byte pieces --
-// dwords 0..3 of the planes 0..3, dwords 4 and 5 of planes 0 and 1, of planes 2 and 3 -- and one dword of the four planes'
-// E8M0 scales.  Four blocks' pieces lie together: the four first ones, the four second ones, ... ----
-constexpr int MX_BLOCK_BYTES = 96;
-static __host__ __device__ inline size_t mx_padded_blocks(size_t cols) { return (cols / 32 + 7) / 8 * 8; }
-
 MxActs mx_acts_carve(void *base, size_t rows, size_t cols) {
     const size_t blocks = rows * mx_padded_blocks(cols);
     MxActs a;
@@ -50,78 +44,14 @@ size_t mx_acts_bytes(size_t rows, size_t cols) {
     return round_up(blocks * MX_BLOCK_BYTES, 256) + round_up(blocks * 4, 256) + round_up(rows * 4, 256);
 }
 
-// quantize_activations_q8, Avx form (crates/frink-quant/src/act_quant.rs:157-189), and the digits of quant * scale.
-// A workgroup per row, four lanes per block, a lane elements 4i .. 4i+3 and 16+4i .. 16+4i+3: eight neighbours in the
-// digits' order, 48 bits of a plane.  `used`: a row whose entry is negative is left as it is.
-// A block whose scale overflows f16 (a largest value above 8.3e6) makes the row's results infinite (NaN where its sum
-// is zero): its digits are kept with a scale of 65536, the row's other blocks are zeroed, and `factor` carries the
-// infinity to the end.
+// `used`: a row whose entry is negative is left as it is
 __global__ __launch_bounds__(128) void quantize_mx_kernel(const float *__restrict__ x, int nb, const int *__restrict__ used, MxActs out) {
+    __shared__ int infinite;
     const int row = blockIdx.x;
     if (used && used[row] < 0) return;
-    const int nbp = (nb + 7) & ~7, part = threadIdx.x & 3;
-    const float *xr = x + (size_t)row * nb * 32;
-    bool row_infinite = false;
-    for (int pass = 0; pass < 2; pass++) {
-        int infinite = 0;
-        for (int b = threadIdx.x >> 2; b < nbp; b += 32) {
-            float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
-            if (b < nb) {
-                lo = reinterpret_cast<const float4 *>(xr + b * 32)[part];
-                hi = reinterpret_cast<const float4 *>(xr + b * 32)[4 + part];
-            }
-            const float e[8] = {lo.x, hi.x, lo.y, hi.y, lo.z, hi.z, lo.w, hi.w};
-            float amax = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(e[i]));
-            amax = fmaxf(amax, __shfl_xor(amax, 1));
-            amax = fmaxf(amax, __shfl_xor(amax, 2));
-            const float inv = amax != 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
-            const uint32_t d = f2h_bits(__fdiv_rn(amax, 127.0f));
-            const int ex = (int)(d >> 10);
-            int mant = (int)(d & 1023u) | (ex ? 1024 : 0);
-            infinite |= ex == 31;
-            if (pass && ex != 31) mant = 0;
-            uint64_t planes[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const float r = rintf(e[i] * inv);
-                int v = ((r != r) ? 0 : (int)fminf(fmaxf(r, -127.0f), 127.0f)) * mant;
-#pragma unroll
-                for (int p = 0; p < 4; p++) {
-                    const int digit = ((v + 16) & 31) - 16;
-                    v = (v - digit) >> 5;
-                    const int a = abs(digit);
-                    // E2M3 in units of a quarter: 0 .. 7 are 2a, 8 .. 16 are a + 8
-                    const uint32_t code = (uint32_t)(a < 8 ? 2 * a : a + 8) | (digit < 0 ? 32u : 0u);
-                    planes[p] |= (uint64_t)code << (6 * i);
-                }
-            }
-            // lanes in pairs: the even one writes planes 0 and 1 of the pair's 96 bits, the odd one planes 2 and 3
-            const bool odd = part & 1;
-            const size_t at = (size_t)row * nbp + b;
-            uint32_t *dst = reinterpret_cast<uint32_t *>(out.digits + (at & ~(size_t)3) * MX_BLOCK_BYTES) + (b & 3) * 4;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const uint64_t own = odd ? planes[2 + h] : planes[h];
-                const uint64_t other = __shfl_xor((unsigned long long)(odd ? planes[h] : planes[2 + h]), 1);
-                const uint64_t first = odd ? other : own, second = odd ? own : other;
-                const uint32_t w[3] = {(uint32_t)first, (uint32_t)(first >> 32) | (uint32_t)(second << 16), (uint32_t)(second >> 16)};
-                const int p = (odd ? 2 : 0) + h;
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    const int j = 3 * (part >> 1) + k;
-                    dst[j < 4 ? 16 * p + j : 64 + 16 * (p >> 1) + 2 * (p & 1) + j - 4] = w[k];
-                }
-            }
-            // 2^(ex - 25) a unit, a digit's code is a quarter of its value, plane p times 32^p
-            if (part == 0) out.scales[at] = 0x0f0a0500u + 0x01010101u * (uint32_t)(max(ex, 1) + 104);
-        }
-        if (pass) break;
-        row_infinite = __syncthreads_or(infinite) != 0;
-        if (!row_infinite) break;
-    }
-    if (threadIdx.x == 0) out.factor[row] = row_infinite ? __builtin_inff() : 1.0f;
+    if (threadIdx.x == 0) infinite = 0;
+    __syncthreads();
+    quantize_mx_row(x, row, nb, threadIdx.x, &infinite, out);
 }
 int launch_quantize_mx(const float *x, size_t rows, size_t cols, const int *used, const MxActs &out, hipStream_t s) {
     if (rows == 0) return FRK_OK;
@@ -135,27 +65,18 @@ int launch_quantize_mx(const float *x, size_t rows, size_t cols, const int *used
 // whose results meet in the epilogue as silu(gate) * up.
 //
 // The columns go by four blocks at a time: step s (0, 1) multiplies blocks s and 2 + s, a lane block s or 2 + s of its
-// row by its half (k = 64).  Everything comes straight into LDS: the activations' digits (25 KB) two quads of blocks ahead
-// in a ring of three stages that the workgroup shares, with one barrier a quad; the weights one quad ahead into a
-// wavefront's own two slots, their scale bytes four quads at a time.
-// What bounds the kernel is the way of those bytes into LDS (60 KB a quad of 2048 clocks of matrix core): neighbouring
-// lanes of a request fetch neighbouring pieces of memory (384 bytes of digits, 64 of codes a row), the LDS images are
-// swizzled so that a fragment's reads -- one piece of sixteen rows each -- fall in different banks, and the requests are
-// spread over the quad's arithmetic.  Gate and up of 32 experts of 2880 x 2880 over 2048 pairs: weights loaded into
-// registers, a row a lane, 227 us; weights in LDS but a lane per activation row 208 us; as it is now 171 us (the bytes
-// from memory take 50, the matrix core 40).  Eight wavefronts a workgroup where that still fills the chip: a stage of
-// digits then serves twice the rows (the down projection 137 -> 96 us). ----
-struct MxGemmArgs {
-    const uint8_t *W, *W2;  // GLU: gate and up
-    size_t row_stride, group_stride;
-    int rows, nb;  // of one group
-    MxActs acts;
-    const int *src_rows;  // the activation row of a row of the grouped order (negative: none); null: the row itself
-    const int4 *tiles;    // {group, first row of the grouped order, rows in use, first row of y}
-    const int *n_tiles;
-    int row_groups;  // workgroups a tile
-    float *y;
-};
+// row by its half (k = 64).  Everything comes straight into LDS, two quads of blocks ahead: the activations' digits (25 KB)
+// into a ring of three stages that the workgroup shares, with one barrier a quad; the weights into a wavefront's own two
+// slots, their scale bytes four quads at a time.
+// A quad takes about 2.4 us: 64 products a SIMD at the 24 ns that a chain of E2M3 x E2M1 products alone was measured at
+// are 1.5, its 60 KB on their way into LDS most of the rest (1.9 us without them).  So neighbouring lanes of a request
+// fetch neighbouring pieces of memory (384 bytes of digits, 64 of codes a row), the LDS images are swizzled so that a
+// fragment's reads -- one piece of sixteen rows each -- fall in different banks, and the requests are spread over the
+// arithmetic.  Gate and up of 32 experts of 2880 x 2880 over 2048 pairs: weights loaded into registers, a row a lane, 227
+// us; weights in LDS but a lane per activation row 208; every request at the head of its quad 181; operands of the next
+// quad read behind the barrier instead of in front of the last step 171; as it is now 164 (the bytes from memory take 50).
+// Eight wavefronts a workgroup where that still fills the chip: a stage of digits then serves twice the rows (the down
+// projection 137 -> 97 us). ----
 constexpr int MX_ROW = 4 * MX_BLOCK_BYTES;             // an activation row's digits of one quad, 24 pieces
 constexpr int MX_STAGE_SCALES = 64 * MX_ROW;           // [64 rows][4 blocks] dwords
 constexpr int MX_STAGE = MX_STAGE_SCALES + 64 * 16;
@@ -227,21 +148,20 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
     auto fetch_act_scales = [&](int i) {
         if (wave == 0) dma16(lds0 + (uint32_t)(i % MX_STAGES) * MX_STAGE + MX_STAGE_SCALES, g.acts.scales + (size_t)i * 4, scales_off);
     };
-    // What a wavefront requests during quad i, in four portions (the address unit takes a clock per lane of a request:
-    // all at once, the requests of eight wavefronts hold each other up for longer than the quad's arithmetic takes):
-    // the weights of quad i + 1, then the digits of quad i + 2.
-    auto request = [&](auto portion_c, int i) {
-        constexpr int P = decltype(portion_c)::value;
-        if (P < 2 && i + 1 < quads) {
-            fetch_codes(i + 1, 2 * P);
-            fetch_codes(i + 1, 2 * P + 1);
-            if (P == 1 && ((i + 1) & 3) == 0) fetch_weight_scales(i + 1);
-        }
-        if (P >= 2 && i + 2 < quads) {
+    // What a wavefront requests during quad i, spread over its arithmetic (all at once, the requests of eight wavefronts
+    // hold each other up): the codes of quad i + 2, whose slot is that of quad i, in its registers by then, and the
+    // digits of quad i + 2, whose stage everybody left before quad i.
+    auto request_codes = [&](int i, int c) {
+        if (i + 2 >= quads) return;
+        fetch_codes(i + 2, c);
+        fetch_codes(i + 2, c + 1);
+        if (c == 0 && ((i + 2) & 3) == 0) fetch_weight_scales(i + 2);
+    };
+    auto request_digits = [&](int i) {
+        if (i + 2 >= quads) return;
 #pragma unroll
-            for (int c = (P - 2) * ((REQUESTS + 1) / 2); c < (P == 2 ? (REQUESTS + 1) / 2 : REQUESTS); c++) fetch_digits(i + 2, c);
-            if (P == 3) fetch_act_scales(i + 2);
-        }
+        for (int c = 0; c < REQUESTS; c++) fetch_digits(i + 2, c);
+        fetch_act_scales(i + 2);
     };
     // where this lane's pieces of step k sit in a half's 32 rows: piece 4n + block in place (4n + block) ^ x, so the even n
     // 128 bytes apart from here, the odd ones from there
@@ -257,87 +177,110 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
 #pragma unroll
         for (int r = 0; r < 2; r++) acc[h][r] = mx_v16f{0.0f};
 
-    // one quad: per half two steps of four planes of digits, smallest first, their sum added onto the running one; a
-    // step's operands are read while the one before is multiplied
-    auto multiply = [&](int i) {
-        constexpr int E2M3 = 2, E2M1 = 4;
-        const uint8_t *st = lds + (size_t)(i % MX_STAGES) * MX_STAGE;
-        const uint8_t *w_wave = lds + MX_STAGES * MX_STAGE + (size_t)wave * MX_W_WAVE, *ws = w_wave + (i & 1) * 4096;
-        const uint8_t *w_scales = w_wave + MX_W_SCALES + ((i >> 2) & 1) * 1024 + (i & 3) * 4;
-        // the codes of step k and row group r, and the scale bytes of the lane's two blocks (a block past the row's end: 2^-127)
-        auto codes = [&](int k, int r) {
-            const mx_v4i v = *reinterpret_cast<const mx_v4i *>(ws + (32 * r + li) * 64 + ((2 * lg + k) ^ ((li >> 2) & 3)) * 16);
-            return mx_v8i{v[0], v[1], v[2], v[3], 0, 0, 0, 0};
-        };
+    // One quad: per half (TWO: both, else the first) two steps of four planes of digits, smallest first, their sum added
+    // onto the running one.  A step's operands are read while the one before is multiplied -- across the quads too: before
+    // the last step the next quad is waited for (and everybody has read the present one), and its codes and first operands
+    // are read behind that step's products.
+    // (macros: as a struct handed between lambdas the operands end up in scratch memory)
+    constexpr int E2M3 = 2, E2M1 = 4;
+    const uint8_t *const w_wave = lds + MX_STAGES * MX_STAGE + (size_t)wave * MX_W_WAVE;
+    auto codes = [&](int i, int k, int r) {  // of step k and row group r
+        return *reinterpret_cast<const mx_v4i *>(w_wave + (i & 1) * 4096 + (32 * r + li) * 64 + ((2 * lg + k) ^ ((li >> 2) & 3)) * 16);
+    };
+    auto scales = [&](int i, int r) {  // the scale bytes of the lane's two blocks (a block past the row's end: 2^-127)
         const int left = nb - (4 * i + 2 * lg);
         const uint32_t live = left > 1 ? 0xffffu : left > 0 ? 0xffu : 0u;
-        auto scales = [&](int r) { return (int)((*reinterpret_cast<const uint32_t *>(w_scales + (32 * r + li) * 16) >> (16 * lg)) & live); };
-        const mx_v8i b00 = codes(0, 0), b01 = codes(0, 1), b10 = codes(1, 0), b11 = codes(1, 1);
-        const int scale0 = scales(0), scale1 = scales(1);
-        // (macros: as a struct handed between lambdas the operands end up in scratch memory)
-        auto piece = [&](int h, int k, int n) { return *reinterpret_cast<const mx_v4i *>(st + h * 32 * MX_ROW + (n >> 1) * 128 + piece_at[k][n & 1]); };
-        // step K's operands of half H, requested here, ahead of the products in front of theirs: the planes' dwords 0..3,
-        // dwords 4 and 5 of planes 0 and 1, of planes 2 and 3, and the planes' scales
+        const uint32_t four = *reinterpret_cast<const uint32_t *>(w_wave + MX_W_SCALES + ((i >> 2) & 1) * 1024 + (i & 3) * 4 + (32 * r + li) * 16);
+        return (int)((four >> (16 * lg)) & live);
+    };
+    auto piece = [&](const uint8_t *st, int h, int k, int n) {
+        return *reinterpret_cast<const mx_v4i *>(st + h * 32 * MX_ROW + (n >> 1) * 128 + piece_at[k][n & 1]);
+    };
+    auto act_scales = [&](const uint8_t *st, int h, int k) {
+        return *reinterpret_cast<const int *>(st + MX_STAGE_SCALES + (32 * h + li) * 16 + (2 * lg + k) * 4);
+    };
+    // step K's operands of half H, requested here, ahead of the products in front of theirs: the planes' dwords 0..3,
+    // dwords 4 and 5 of planes 0 and 1, of planes 2 and 3, and the planes' scales
 #define FRK_MX_READ(o, H, K)                                                                                           \
-    const mx_v4i o##0 = piece(H, K, 0), o##1 = piece(H, K, 1), o##2 = piece(H, K, 2), o##3 = piece(H, K, 3),           \
-                 o##01 = piece(H, K, 4), o##23 = piece(H, K, 5);                                                       \
-    const int o##_scales = *reinterpret_cast<const int *>(st + MX_STAGE_SCALES + (32 * H + li) * 16 + (2 * lg + K) * 4); \
+    o##0 = piece(st, H, K, 0), o##1 = piece(st, H, K, 1), o##2 = piece(st, H, K, 2), o##3 = piece(st, H, K, 3),        \
+    o##01 = piece(st, H, K, 4), o##23 = piece(st, H, K, 5), o##_scales = act_scales(st, H, K);                         \
     __builtin_amdgcn_sched_barrier(0)
 #define FRK_MX_PLANE(o, K, P, head, tail, T)                                                                           \
     {                                                                                                                  \
         const mx_v8i x = {head[0], head[1], head[2], head[3], tail[T], tail[T + 1], 0, 0};                             \
-        part0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, b##K##0, part0, E2M3, E2M1, P, o##_scales, K, scale0); \
-        part1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, b##K##1, part1, E2M3, E2M1, P, o##_scales, K, scale1); \
+        const mx_v8i y0 = {b##K##0[0], b##K##0[1], b##K##0[2], b##K##0[3], 0, 0, 0, 0};                                \
+        const mx_v8i y1 = {b##K##1[0], b##K##1[1], b##K##1[2], b##K##1[3], 0, 0, 0, 0};                                \
+        part0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y0, part0, E2M3, E2M1, P, o##_scales, K, scale0);   \
+        part1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y1, part1, E2M3, E2M1, P, o##_scales, K, scale1);   \
     }
-#define FRK_MX_STEP(o, K)                   \
-    FRK_MX_PLANE(o, K, 0, o##0, o##01, 0) \
+#define FRK_MX_FIRST(o, K) FRK_MX_PLANE(o, K, 0, o##0, o##01, 0)
+#define FRK_MX_REST(o, K)                   \
     FRK_MX_PLANE(o, K, 1, o##1, o##01, 2) \
     FRK_MX_PLANE(o, K, 2, o##2, o##23, 0) \
     FRK_MX_PLANE(o, K, 3, o##3, o##23, 2) \
     asm volatile("" : "+v"(part0), "+v"(part1));  // (stays in front of the requests behind it)
-        const std::integral_constant<int, 0> c0;
-        const std::integral_constant<int, 1> c1;
-        const std::integral_constant<int, 2> c2;
-        const std::integral_constant<int, 3> c3;
-        FRK_MX_READ(p, 0, 0);
-        FRK_MX_READ(q, 0, 1);
-        request(c0, i);
-        mx_v16f part0 = mx_v16f{0.0f}, part1 = part0;
-        FRK_MX_STEP(p, 0)
-        request(c1, i);
-        FRK_MX_READ(u, 1, 0);  // (the stage has the second half's place in any case)
-        FRK_MX_STEP(q, 1)
-        acc[0][0] += part0;
-        acc[0][1] += part1;
-        request(c2, i);
-        if (two) {
-            FRK_MX_READ(v, 1, 1);
-            part0 = part1 = mx_v16f{0.0f};
-            FRK_MX_STEP(u, 0)
-            FRK_MX_STEP(v, 1)
-            acc[1][0] += part0;
-            acc[1][1] += part1;
+    // quad I has landed: behind its digits the wavefront requested four times codes and its share of digits, of quad I + 1
+    // (and now and then scales: then a little more is waited for); afterwards its codes (step 0's in place, step 1's
+    // beside the present ones) and first operands
+#define FRK_MX_ARRIVE(I)                                                                                               \
+    if ((I) + 1 < quads && wave == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(REQUESTS + 5) : "memory");              \
+    else if ((I) + 1 < quads) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(REQUESTS + 4) : "memory");                      \
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                                              \
+    lds_barrier();                                                                                                     \
+    st = lds + (size_t)((I) % MX_STAGES) * MX_STAGE;                                                                   \
+    b00 = codes(I, 0, 0), b01 = codes(I, 0, 1), next10 = codes(I, 1, 0), next11 = codes(I, 1, 1);                      \
+    next_scale0 = scales(I, 0), next_scale1 = scales(I, 1);                                                            \
+    __builtin_amdgcn_sched_barrier(0);                                                                                 \
+    FRK_MX_READ(p, 0, 0)
+    auto all_quads = [&](auto two_c) {
+        constexpr bool TWO = decltype(two_c)::value;
+        const uint8_t *st;
+        mx_v4i b00, b01, b10, b11, next10, next11, p0, p1, p2, p3, p01, p23, q0, q1, q2, q3, q01, q23;
+        int scale0, scale1, next_scale0, next_scale1, p_scales, q_scales;
+        FRK_MX_ARRIVE(0);
+        b10 = next10, b11 = next11, scale0 = next_scale0, scale1 = next_scale1;
+        for (int i = 0; i < quads; i++) {
+            mx_v16f part0 = mx_v16f{0.0f}, part1 = part0;
+            FRK_MX_FIRST(p, 0)
+            FRK_MX_READ(q, 0, 1);
+            request_codes(i, 0);
+            FRK_MX_REST(p, 0)
+            request_codes(i, 2);
+            if (TWO) {
+                FRK_MX_FIRST(q, 1)
+                FRK_MX_READ(p, 1, 0);
+                FRK_MX_REST(q, 1)
+                acc[0][0] += part0;
+                acc[0][1] += part1;
+                request_digits(i);
+                part0 = part1 = mx_v16f{0.0f};
+                FRK_MX_FIRST(p, 0)
+                FRK_MX_READ(q, 1, 1);
+                FRK_MX_REST(p, 0)
+            } else {
+                request_digits(i);
+            }
+            FRK_MX_ARRIVE(i + 1);  // (behind the last quad: whatever lies there, unused)
+            FRK_MX_FIRST(q, 1)
+            FRK_MX_REST(q, 1)
+            acc[TWO][0] += part0;
+            acc[TWO][1] += part1;
+            b10 = next10, b11 = next11, scale0 = next_scale0, scale1 = next_scale1;
         }
-        request(c3, i);
-#undef FRK_MX_READ
-#undef FRK_MX_PLANE
-#undef FRK_MX_STEP
     };
-    // A quad: its digits and weights have landed (behind them only the digits of quad i + 1 were requested), everybody
-    // has left the stage that the next request overwrites.
     for (int c = 0; c < 4; c++) fetch_codes(0, c);
     fetch_weight_scales(0);
-    request(std::integral_constant<int, 2>(), -2);
-    request(std::integral_constant<int, 3>(), -2);
-    request(std::integral_constant<int, 2>(), -1);
-    request(std::integral_constant<int, 3>(), -1);
-    for (int i = 0; i < quads; i++) {
-        if (i + 1 < quads && wave == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(REQUESTS + 1) : "memory");
-        else if (i + 1 < quads) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(REQUESTS) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        lds_barrier();
-        multiply(i);
-    }
+    request_digits(-2);
+    request_codes(-1, 0);
+    request_codes(-1, 2);
+    request_digits(-1);
+    if (two) all_quads(std::true_type());
+    else all_quads(std::false_type());
+#undef FRK_MX_READ
+#undef FRK_MX_PLANE
+#undef FRK_MX_FIRST
+#undef FRK_MX_REST
+#undef FRK_MX_ARRIVE
 
     // the factor of row `lane` of the tile
     float factor = 1.0f;

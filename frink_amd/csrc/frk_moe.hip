@@ -3,7 +3,7 @@
 //   bucket (token, slot) pairs by expert  ->  gate/up grouped GEMM over gathered token rows
 //   ->  silu(gate)*up, quantized to Q8_K  ->  down grouped GEMM  ->  out[tok] = sum_e w * down
 // with each token's experts added in the order the reference adds them (moe_combine_kernel).
-#include "frk_device.hpp"
+#include "frk_mx_quant.hpp"
 
 namespace frk {
 
@@ -250,6 +250,21 @@ __global__ __launch_bounds__(1024) void moe_group_quantize_kernel(GroupArgs a, c
         if ((lane & 3) == 0) out.bs[(size_t)b * 16 + (lane >> 2)] = (_Float16)bs;
         if (lane == 0) out.d[b] = dd;
     }
+}
+
+// The same beside the digits of MXFP4 expert layers: eight token rows a workgroup (one after the other, the bucketing
+// 9 us and the digits 8 stood in front of every such layer).
+__global__ __launch_bounds__(1024) void moe_group_quantize_mx_kernel(GroupArgs a, const float *__restrict__ x, int rows, int nb, MxActs out) {
+    __shared__ int infinite[8];
+    if (blockIdx.x == 0) {
+        moe_group(a);
+        return;
+    }
+    const int sub = threadIdx.x >> 7;
+    if (threadIdx.x < 8) infinite[threadIdx.x] = 0;
+    __syncthreads();
+    // (past the end the last row again: the same bytes)
+    quantize_mx_row(x, min(((int)blockIdx.x - 1) * 8 + sub, rows - 1), nb, threadIdx.x & 127, &infinite[sub], out);
 }
 
 // The grouped GEMM with the groups given (enqueue_mul_mm_grouped_dev, crates/frink-cuda/src/mul_mm_launch.rs:391-470):
@@ -910,20 +925,24 @@ int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up,
     if (!sized) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_kernel),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GroupLds));
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_quantize_mx_kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GroupLds));
         if (e != hipSuccess) return set_error(FRK_ERR_HIP, "hipFuncSetAttribute(moe_group): %s", hipGetErrorString(e));
         sized = true;
     }
     const GroupArgs ga{ids, (int)pairs, k, n_experts, m.group_off, m.gather, m.pos_of, m.cpos_of, m.tiles, m.n_tiles, (int)rows};
-    hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), sizeof(GroupLds), s, ga);
-    FRK_LAUNCH_CHECK("moe_group");
     int rc;
     if (native.gate_up) {
         const MxActs xa = mx_acts_carve(m.x_acts, batch, hidden);
-        rc = launch_quantize_mx(x, batch, (size_t)hidden, nullptr, xa, s);
-        if (rc) return rc;
+        hipLaunchKernelGGL(moe_group_quantize_mx_kernel, dim3(1 + (unsigned)((batch + 7) / 8)), dim3(1024), sizeof(GroupLds), s, ga, x,
+                           (int)batch, hidden / 32, xa);
+        FRK_LAUNCH_CHECK("moe_group_quantize_mx");
         rc = launch_gemm_mx_grouped(gate, up, (size_t)ffn, xa, m.gather, m.tiles, m.n_tiles, max_tiles, m.gate_out, s);
         if (rc) return rc;
     } else {
+        hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), sizeof(GroupLds), s, ga);
+        FRK_LAUNCH_CHECK("moe_group");
         const uint8_t *gate_w = nullptr, *up_w = nullptr;
         rc = units_decoded(gate, m.gate_w, s, &gate_w);
         if (rc) return rc;
