@@ -77,6 +77,17 @@ int launch_quantize_mx(const float *x, size_t rows, size_t cols, const int *used
 // quad read behind the barrier instead of in front of the last step 171; as it is now 164 (the bytes from memory take 50).
 // Eight wavefronts a workgroup where that still fills the chip: a stage of digits then serves twice the rows (the down
 // projection 137 -> 97 us). ----
+struct MxGemmArgs {
+    const uint8_t *W, *W2;  // GLU: gate and up
+    size_t row_stride, group_stride;
+    int rows, nb;  // of one group
+    MxActs acts;
+    const int *src_rows;  // the activation row of a row of the grouped order (negative: none); null: the row itself
+    const int4 *tiles;    // {group, first row of the grouped order, rows in use, first row of y}
+    const int *n_tiles;
+    int row_groups;  // workgroups a tile
+    float *y;
+};
 constexpr int MX_ROW = 4 * MX_BLOCK_BYTES;             // an activation row's digits of one quad, 24 pieces
 constexpr int MX_STAGE_SCALES = 64 * MX_ROW;           // [64 rows][4 blocks] dwords
 constexpr int MX_STAGE = MX_STAGE_SCALES + 64 * 16;
