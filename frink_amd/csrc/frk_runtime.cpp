@@ -618,7 +618,7 @@ static bool q4_k_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     const size_t q4k_thin_rows = w->rows * w->cols > (size_t)20 << 20 ? 16 : 32;
     return w->kind == FRK_KIND_Q4_K && batch > 16 && (batch > q4k_thin_rows || thin_gemm_max_batch(w) < 16);
 }
-// Q5_K: the same kernel with a third plane for the fifth bits, from the batch on where it is ahead of the
+// Q5_K: the same kernel, from the batch on where it is ahead of the
 // thin kernel's 16-row groups
 static bool q5_k_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     const size_t q5k_thin_rows = 32;
