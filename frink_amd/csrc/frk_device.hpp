@@ -254,8 +254,12 @@ struct Q8KRecordLds {
     _Float16 bs[512];
     float d[32];
 };
-template <int WAVES, class Load>
-__device__ __forceinline__ void quantize_q8k_record(const Q8KTiled &a, size_t rec, Q8KRecordLds &L, Load load) {
+// (`keep(r, quants, d, sum)` sees a lane's four values of row r as well, `sum` in every fourth lane)
+struct KeepNothing {
+    __device__ void operator()(int, uint32_t, float, int) const {}
+};
+template <int WAVES, class Load, class Keep = KeepNothing>
+__device__ __forceinline__ void quantize_q8k_record(const Q8KTiled &a, size_t rec, Q8KRecordLds &L, Load load, Keep keep = Keep()) {
     constexpr int RPW = 32 / WAVES;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float4 v[RPW];
@@ -272,6 +276,7 @@ __device__ __forceinline__ void quantize_q8k_record(const Q8KTiled &a, size_t re
         L.q[ks * 256 + (half * 32 + r) * 4 + (lane & 3)] = packed;
         if ((lane & 3) == 0) L.bs[((g >> 3) * 32 + r) * 8 + (g & 7)] = (_Float16)bs;
         if (lane == 0) L.d[r] = dd;
+        keep(r, packed, dd, bs);
     }
     __syncthreads();
     uint4 *dq = reinterpret_cast<uint4 *>(a.q + rec * 8192);

@@ -217,7 +217,14 @@ struct Q8KRows {
 size_t q8k_tiled_bytes(size_t rows, size_t cols);
 Q8KTiled q8k_tiled_carve(void *base, size_t rows, size_t cols);
 // out row r = x[r] quantized, r < rows; the rest of the last tile becomes zeros
-int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTiled out, hipStream_t s);
+// Q8KActs to be written; null pointers: none wanted
+struct Q8KActsOut {
+    int8_t *q = nullptr;
+    float *d = nullptr;
+    int16_t *bsums = nullptr;
+};
+// (`plain`: the same quants as plain rows too)
+int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTiled out, hipStream_t s, Q8KActsOut plain = Q8KActsOut());
 // out row r = x[gather[r]] quantized (zeros where gather[r] < 0), for the 32-row records of the first
 // max_rows rows whose first entry is not negative
 int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, size_t max_rows, Q8KTiled out,

@@ -610,30 +610,37 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
     return set_error(FRK_ERR_UNSUPPORTED, "Q8_K activations feed Q4_K, Q5_K and Q6_K weights only (kind %d)", w->kind);
 }
 
-// Q4_K: the thin kernel takes 16 rows a launch.  Measured (us; thin launches / the matrix-core GEMM, whose cost
-// is flat up to 64 rows): 4096x4096 8.8 at 16 rows, 14.5 at 32 / 17.6; 1024x4096 7.5, 12.9 / 15.0 -- two thin
-// launches are ahead for small matrices; 14336x4096 23.9, 44.9 / 24.9; 5120x5120 15.1, 26.8 / 20.4; 4096x11008
-// 25.3 at 16 rows / 23.7 -- from 20 M weights on a second thin launch is not.
-static bool q4_k_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
-    const size_t q4k_thin_rows = w->rows * w->cols > (size_t)20 << 20 ? 16 : 32;
-    return w->kind == FRK_KIND_Q4_K && batch > 16 && (batch > q4k_thin_rows || thin_gemm_max_batch(w) < 16);
-}
-// Q5_K: the same kernel, from the batch on where it is ahead of the
-// thin kernel's 16-row groups
-static bool q5_k_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
-    const size_t q5k_thin_rows = 32;
-    return w->kind == FRK_KIND_Q5_K && batch > q5k_thin_rows;
-}
-
-// Q6_K: the matrix-core GEMM (with its blocks split between workgroups for small batches: 53 us at
-// 4096x14336 and 31 us at 4096x4096 up to 64 rows) is ahead of the thin kernel's 8-row groups (15 us
-// and 6 us each) from four groups on for large matrices and from six on for small ones
-static bool q6_k_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
-    const size_t q6k_gemm_from = w->rows * w->cols > (size_t)2 * 4096 * 4096 ? 25 : 41;
-    return w->kind == FRK_KIND_Q6_K && batch >= q6k_gemm_from;
+// From how many rows on a batch takes the matrix-core GEMM, whose cost is flat up to 64 rows; below that the thin
+// kernels' groups of 16 (Q4_K, Q5_K) or 8 rows are ahead, by what a group costs at the matrix's shape.  Measured with
+// quantization (us; thin / GEMM), nb blocks a row, rules beyond 17 / 33 / 41 rows within 32768 columns:
+//   Q4_K  nb > 32, where a thin launch holds 8 rows: 4096x11008 at 8, 9, 16 rows 14.8 / 19.7, 21.9 / 19.4, 25.3 / 19.7;
+//         1024x14336 at 9, 16 23.5 / 18.8, 28.0 / 19.2.  nb 24 .. 32 past one workgroup a CU: 5120x6144 at 9, 16 19.3 /
+//         16.2, 20.7 / 16.8, 14336x8192 38.7 / 27.7, 44.8 / 27.2, but 2048x8192 14.1 / 15.6, 14336x6144
+//         18.8 / 24.2.  Then by size: 14336x4096 at 17 20.4 / 19.6; 4096x4096 at 17, 32 13.3 / 14.8, 13.3 / 16.1.
+//   Q5_K  nb >= 32: 4096x11008 at 8, 9, 32 rows 16.3 / 23.2, 25.3 / 23.0, 51.1 / 24.7; 2048x8192 at 9, 32 20.2 / 18.5,
+//         41.2 / 19.7.  nb 16 .. 31 of few rows: 4096x4096 at 16, 17, 32 11.0 / 16.3, 20.4 / 16.4, 20.7 / 17.7; 5120x6144 at
+//         17 27.5 / 19.6, but 14336x4096 at 17, 32 21.1 / 23.9, 21.2 / 25.6.
+//   Q6_K  odd nb (not the streamed thin kernel's): 4096x11008 at 8, 9, 24 rows 18.3 / 24.3, 28.9 / 24.2, 42.1 / 25.2;
+//         2048x11008 at 16, 17, 33 17.4 / 23.4, 27.3 / 23.1, 39.1 / 24.6.  Even: 4096x14336 at 16, 17 22.5 / 27.4, 28.9 / 27.6;
+//         5120x8192 at 17, 25 23.2 / 23.8, 35.0 / 25.1; 8192x4096 at 17, 25 20.4 / 21.2, 25.0 / 22.1; 4096x4096 at 40 15.3 / 19.6.
+// (No matrix starts below tiled_from(cols): a batch quantized without knowing its matrices has tiles from there on.)
+static size_t tiled_from(size_t cols) { return cols >= 24 * QK_K ? 9 : 17; }
+static size_t matrix_cores_from(const frk_weights *w) {
+    const size_t n = w->rows * w->cols, nb = w->cols / QK_K;
+    const bool measured = nb <= 128;
+    if (w->kind == FRK_KIND_Q4_K) {
+        if (measured && (nb > 32 || (nb >= 24 && w->rows > 4096 && (nb == 32 || w->rows <= 8192)))) return 9;
+        return n > (size_t)20 << 20 || thin_gemm_max_batch(w) < 16 ? 17 : 33;
+    }
+    if (w->kind == FRK_KIND_Q5_K) return measured && nb >= 32 ? 9 : measured && nb >= 16 && w->rows <= 6144 ? 17 : 33;
+    if (w->kind != FRK_KIND_Q6_K) return SIZE_MAX;
+    const bool large = n > (size_t)32 << 20;
+    if (measured && nb % 2) return large ? 9 : n > (size_t)20 << 20 ? 17 : 41;
+    if (measured && n > (size_t)48 << 20) return 17;
+    return large || (measured && n >= (size_t)30 << 20) ? 25 : 41;
 }
 static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
-    return q4_k_takes_the_matrix_cores(w, batch) || q5_k_takes_the_matrix_cores(w, batch) || q6_k_takes_the_matrix_cores(w, batch);
+    return batch >= std::max(matrix_cores_from(w), tiled_from(w->cols));
 }
 // whether a batch of this matrix multiplies on the thin kernels (over plain Q8_K rows)
 static bool batch_takes_the_thin_kernels(const frk_weights *w, size_t batch) {
@@ -841,8 +848,9 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
 // The object owns room for both forms the K-quant kernels read: plain Q8_K rows (the decode and thin kernels)
 // and the tiled form (the matrix-core GEMMs).  Which of them a batch gets depends on its size alone, so that
 // the quantization does not need to know the matrices: plain rows up to ACTS_PLAIN_MAX_BATCH rows (the thin
-// kernels take at most 40), tiles from ACTS_TILED_MIN_BATCH rows on (no matrix-core GEMM starts below 17).
-constexpr size_t ACTS_PLAIN_MAX_BATCH = 64, ACTS_TILED_MIN_BATCH = 17;
+// kernels take at most 40), tiles from tiled_from(cols) rows on, both out of one launch where a
+// batch has both.
+constexpr size_t ACTS_PLAIN_MAX_BATCH = 64;
 }  // extern "C"
 struct frk_batch_acts {
     size_t max_batch = 0, cols = 0;
@@ -874,7 +882,7 @@ int frk_hip_batch_acts_create(size_t max_batch, size_t cols, frk_batch_acts **ou
     a->max_batch = max_batch;
     a->cols = cols;
     a->tiled_off = round_up(acts_plain_bytes(std::min(max_batch, ACTS_PLAIN_MAX_BATCH), cols), 256);
-    const size_t bytes = a->tiled_off + (max_batch >= ACTS_TILED_MIN_BATCH ? round_up(q8k_tiled_bytes(max_batch, cols), 256) : 0);
+    const size_t bytes = a->tiled_off + (max_batch >= tiled_from(cols) ? round_up(q8k_tiled_bytes(max_batch, cols), 256) : 0);
     hipError_t e = hipMalloc(&a->base, bytes);
     if (e != hipSuccess) {
         delete a;
@@ -900,19 +908,18 @@ int frk_hip_quantize_batch_acts_dev(frk_batch_acts *a, const float *x, size_t ba
         return set_error(FRK_ERR_SHAPE, "a batch of %zu rows in an object made for at most %zu", batch, a->max_batch);
     hipStream_t s = (hipStream_t)stream;
     a->batch = 0;
+    const bool tiled = batch >= tiled_from(a->cols);
+    Q8KActsOut plain;
     if (batch <= ACTS_PLAIN_MAX_BATCH) {
         const size_t n = batch * a->cols;
-        int8_t *q = (int8_t *)a->base;
-        float *d = (float *)((char *)a->base + round_up(n, 256));
-        int16_t *b = (int16_t *)((char *)a->base + round_up(n, 256) + round_up(n / QK_K * 4, 256));
-        int rc = launch_quantize_q8_k(x, n, q, d, b, s);
-        if (rc) return rc;
-        a->plain = Q8KActs{q, d, b};
+        plain.q = (int8_t *)a->base;
+        plain.d = (float *)((char *)a->base + round_up(n, 256));
+        plain.bsums = (int16_t *)((char *)a->base + round_up(n, 256) + round_up(n / QK_K * 4, 256));
+        a->plain = Q8KActs{plain.q, plain.d, plain.bsums};
     }
-    if (batch >= ACTS_TILED_MIN_BATCH) {
-        int rc = launch_quantize_q8_k_tiled(x, batch, a->cols, q8k_tiled_carve((char *)a->base + a->tiled_off, batch, a->cols), s);
-        if (rc) return rc;
-    }
+    const int rc = tiled ? launch_quantize_q8_k_tiled(x, batch, a->cols, q8k_tiled_carve((char *)a->base + a->tiled_off, batch, a->cols), s, plain)
+                         : launch_quantize_q8_k(x, batch * a->cols, plain.q, plain.d, plain.bsums, s);
+    if (rc) return rc;
     a->batch = batch;
     return FRK_OK;
 }

@@ -33,3 +33,34 @@ def test_pipelined_gemm_at_the_edges_of_its_tiles(fa, kind, rows, cols, batch):
     room = np.abs(a).sum(axis=1)[:, None] * (3.0 * np.abs(wd).max(axis=1))[None, :]
     assert (np.abs(got - a @ wd.T) <= (cols // 256 + 9) * 2.0 ** -24 * room).all()
     w.release()
+
+
+@pytest.mark.parametrize("kind,rows,cols", [
+    (fo.Q4_K, 40, 8448),     # rows past 32 blocks: the matrix cores from 9 rows on
+    (fo.Q4_K, 4104, 6144),   # 24 blocks, past one workgroup a CU: from 9
+    (fo.Q5_K, 72, 8192),     # 32 blocks: from 9
+    (fo.Q5_K, 264, 4096),    # 16 blocks of few rows: from 17
+    (fo.Q6_K, 4104, 8448),   # large, an odd number of blocks: from 9
+    (fo.Q6_K, 8200, 4352),   # the same with 17 blocks, whose batches have no tiles below 17 rows: from 17
+])
+def test_batches_around_the_step_from_thin_to_tiled(fa, kind, rows, cols):
+    """Both sides of the batch size at which a matrix changes kernels, against 64-bit sums of the same quantized
+    operands; the activations' two forms come out of one launch, and a product over them is the plain call's bit for bit."""
+    from bench import random_blocks
+    from frink_amd import synth
+    data = random_blocks(kind, rows, cols, seed=rows + kind)
+    wd = fo.dequant(kind, data).reshape(rows, cols).astype(np.float64)
+    w = fa.Weights.from_host(kind, data, rows, cols)
+    acts = fa.BatchActs(33, cols)
+    for batch in (8, 9, 16, 17, 33):
+        x = synth.activations(7 + batch, batch, cols, outlier_frac=0.01)
+        xd = to_dev(x)
+        y = w.gemm(xd).cpu().numpy()
+        assert np.array_equal(w.gemm_acts(acts.quantize(xd)).cpu().numpy().view(np.uint32), y.view(np.uint32)), batch
+        q, d, _ = fo.quantize_q8_k(x.reshape(-1))
+        a = (q.reshape(-1, 256).astype(np.float64) * d.reshape(-1, 1).astype(np.float64)).reshape(batch, cols)
+        # (the bound of the test above, whose kernel adds a block at a time; the thin kernels' chains are no longer)
+        room = np.abs(a).sum(axis=1)[:, None] * (3.0 * np.abs(wd).max(axis=1))[None, :]
+        assert (np.abs(y.astype(np.float64) - a @ wd.T) <= (cols // 256 + 9) * 2.0 ** -24 * room).all(), batch
+    acts.release()
+    w.release()
