@@ -572,19 +572,18 @@ int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, 
 // Which tile and split a batch takes: the one that an estimate of the launch's time finds cheapest.  A workgroup of the
 // large tile (256 rows x 128 tokens) takes `step` microseconds per block of a row, one of the small tile (128 x 64) per two
 // blocks -- longer, by `load`, the more of the 256 CUs have a workgroup (L2 and the clock are shared) -- and `start` for its
-// first block and its stores; a launch is as many rounds of workgroups as the CUs take; splitting the blocks costs the
-// second launch and its bytes.  The constants are a fit to 870 launches (three kinds, six matrices of 1024 .. 14336 rows
-// and columns, 48 .. 1024 tokens, either tile, 1 .. 8 parts; 7 % rms): over those shapes the tile and split it picks are
-// 0.2 % behind the best one measured on average, 7 % at worst.  What it replaced (the large tile where it gave 200
-// workgroups, else the small one in 1, 2 or 4 parts up to 256 workgroups) was up to 1.5 times the best one's time: Q4_K
-// 4096x14336 at 512 tokens 83 us against 74 (large tile, four parts), 2048x8192 at 48 tokens 15.6 against 14.1.
+// first block and its stores; a launch is as many rounds of workgroups as the CUs take, which holds because every XCD has an
+// equal share of them (deal_entry); splitting the blocks costs the second launch and its bytes.  The constants are a fit
+// (4 % rms) to 6079 launches over 1200 drawn shapes: the three kinds, 1024 .. 14336 rows and columns, 8 .. 2048 tokens,
+// 1 .. 8 parts.  Over the 720 of them with 48 tokens and more the choice is 0.2 % behind the best one measured on average,
+// 8 % at worst; with the constants fitted to one half and tried on the other likewise.
 PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb, size_t parts_bytes) {
     struct Cost {
         float step, load, start;
     };
     // (a Q5_K or Q6_K block has three times Q4_K's vector instructions in its unpacking)
-    const Cost small = kind == FRK_KIND_Q4_K ? Cost{2.0f, 0.56f, 2.1f} : Cost{2.8f, 0.43f, 2.9f};
-    const Cost large = kind == FRK_KIND_Q4_K ? Cost{3.1f, 0.57f, 2.5f} : Cost{3.7f, 0.49f, 3.5f};
+    const Cost small = kind == FRK_KIND_Q4_K ? Cost{1.62f, 0.74f, 3.26f} : Cost{2.41f, 0.77f, 4.06f};
+    const Cost large = kind == FRK_KIND_Q4_K ? Cost{2.66f, 1.07f, 4.85f} : Cost{3.26f, 1.06f, 5.79f};
     PipePlan best = {128, 64, 1};
     float best_us = 0.0f;
     for (int big = 0; big < 2; big++)
@@ -592,10 +591,12 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb, size_t parts_byte
             const size_t bytes = (size_t)ks * M * rows * sizeof(float);
             if (ks > 1 && (nb / (size_t)ks < 2 || bytes > parts_bytes)) continue;
             const size_t wgs = (big ? ((rows + 255) / 256) * ((M + 127) / 128) : ((rows + 127) / 128) * ((M + 63) / 64)) * (size_t)ks;
-            const size_t blocks = (nb + (size_t)ks - 1) / (size_t)ks, steps = big ? blocks : (blocks + 1) / 2;
+            const size_t blocks = (nb + (size_t)ks - 1) / (size_t)ks;
+            const float steps = (float)(big ? blocks : (blocks + 1) / 2), last = (float)(wgs % 256) / 256.0f;
             const Cost c = big ? large : small;
-            float us = (float)((wgs + 255) / 256) * ((float)steps * (c.step + c.load * (wgs < 256 ? (float)wgs / 256.0f : 1.0f)) + c.start);
-            if (ks > 1) us += 4.9f + 3.6e-7f * (float)bytes;
+            float us = (float)(wgs / 256) * (steps * (c.step + c.load) + c.start);
+            if (wgs % 256) us += steps * (c.step + c.load * last) + c.start;
+            if (ks > 1) us += 1.3f + 2.6e-7f * (float)bytes;
             if (best_us == 0.0f || us < best_us) {
                 best_us = us;
                 best = big ? PipePlan{256, 128, ks} : PipePlan{128, 64, ks};

@@ -12,6 +12,7 @@
 // alone: 14336x4096 in Q5_K 131 -> 78 us, 4096x14336 in Q6_K 155 -> 83 us with the sum of its four parts.)
 #pragma once
 
+#include "frk_deal.hpp"
 #include "frk_device.hpp"
 
 #include <type_traits>
@@ -34,7 +35,7 @@ struct GemmArgs {
     Q8KTiled a;  // ceil(M / 32) tiles
     float *y;    // [M][rows]
     int row_tiles, tok_tiles;
-    int k_split;     // 1, or 2/4: blockIdx.y takes that share of a row's blocks and writes its sums to `partial`
+    int k_split;     // 1 .. 8 parts of a row's blocks; with more than one each writes its sums to `partial`
     float *partial;  // [k_split][M][rows], added up in order afterwards (launch_sum_parts)
 };
 
@@ -656,17 +657,19 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     const int li = lane & 31, lg = lane >> 5;
     const int rg = wave % RG, ks = wave / RG;
 
-    // workgroups that share weight rows (different token tiles) sit on one XCD (block id mod 8)
-    const int bid = blockIdx.x;
-    const int per_group = 8 * g.tok_tiles;
-    const int grp = bid / per_group, in_grp = bid % per_group;
-    const int row_tile = grp * 8 + (in_grp & 7);
-    if (row_tile >= g.row_tiles) return;  // uniform per workgroup
-    const int tok0 = (in_grp >> 3) * TM;
+    // An XCD takes an equal run of the list (part, row tile, token tile): its workgroups share weight rows and, where the
+    // blocks are split, the activations of a part or two.  (With XCD x given the row tiles congruent to x mod 8, the busiest
+    // one had a round more than the others wherever their number does not divide by eight: 2440 x 12032 in Q5_K at 146
+    // tokens, 20 row tiles, 53 -> 33 us; and with the parts in the middle of the list every XCD reads all activations: 1025
+    // x 13056 in Q4_K at 105 tokens in eight parts 23.4 -> 21.1.)
+    const int entry = deal_entry((int)blockIdx.x, g.row_tiles * g.tok_tiles * g.k_split);
+    if (entry < 0) return;  // uniform per workgroup
+    const int tile = entry / g.tok_tiles, part = tile / g.row_tiles;
+    const int row_tile = tile - part * g.row_tiles, tok0 = (entry - tile * g.tok_tiles) * TM;
     const int nb = g.nb;
     // this workgroup multiplies blocks kb0 .. kb1 - 1, its KS shares `steps` consecutive ones each (a
     // share that runs out of blocks idles through its last steps)
-    const int kb0 = nb * (int)blockIdx.y / g.k_split, kb1 = nb * ((int)blockIdx.y + 1) / g.k_split;
+    const int kb0 = nb * part / g.k_split, kb1 = nb * (part + 1) / g.k_split;
     const int steps = (kb1 - kb0 + KS - 1) / KS;
     const int tile0 = tok0 / 32, last_tile = (g.M - 1) / 32;
     auto tile_of = [&](int slot) { return min(tile0 + slot % MT, last_tile); };  // uniform
@@ -858,7 +861,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     }
     // store: a lane holds one weight row and 16 tokens per tile
     const int row = row_tile * ROWS + rg * 32 + li;
-    float *const dst = g.k_split > 1 ? g.partial + (size_t)blockIdx.y * g.M * g.rows : g.y;
+    float *const dst = g.k_split > 1 ? g.partial + (size_t)part * g.M * g.rows : g.y;
     const int rows_lim = g.rows;
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
@@ -887,8 +890,8 @@ int launch_pipe(void (*kernel)(GemmArgs), const GemmArgs &g, hipStream_t s) {
         if (e != hipSuccess) return set_error(FRK_ERR_HIP, "hipFuncSetAttribute(LDS %zu): %s", shmem, hipGetErrorString(e));
         sized = true;
     }
-    const unsigned grid = (unsigned)((g.row_tiles + 7) / 8 * 8 * g.tok_tiles);
-    hipLaunchKernelGGL(kernel, dim3(grid, (unsigned)g.k_split), dim3(512), shmem, s, g);
+    const unsigned grid = (unsigned)deal_grid(g.row_tiles * g.tok_tiles * g.k_split);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), shmem, s, g);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(FRK_ERR_HIP, "pipelined GEMM launch: %s", hipGetErrorString(e));
     if (g.k_split > 1) return launch_sum_parts(g.partial, g.k_split, (size_t)g.M * g.rows, g.y, s);
