@@ -577,7 +577,7 @@ int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, 
 // (4 % rms) to 6079 launches over 1200 drawn shapes: the three kinds, 1024 .. 14336 rows and columns, 8 .. 2048 tokens,
 // 1 .. 8 parts.  Over the 720 of them with 48 tokens and more the choice is 0.2 % behind the best one measured on average,
 // 8 % at worst; with the constants fitted to one half and tried on the other likewise.
-PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb, size_t parts_bytes) {
+PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     struct Cost {
         float step, load, start;
     };
@@ -589,7 +589,7 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb, size_t parts_byte
     for (int big = 0; big < 2; big++)
         for (int ks : {1, 2, 3, 4, 6, 8}) {
             const size_t bytes = (size_t)ks * M * rows * sizeof(float);
-            if (ks > 1 && (nb / (size_t)ks < 2 || bytes > parts_bytes)) continue;
+            if (ks > 1 && (nb / (size_t)ks < 2 || bytes > SPLIT_PARTS_BYTES)) continue;
             const size_t wgs = (big ? ((rows + 255) / 256) * ((M + 127) / 128) : ((rows + 127) / 128) * ((M + 63) / 64)) * (size_t)ks;
             const size_t blocks = (nb + (size_t)ks - 1) / (size_t)ks;
             const float steps = (float)(big ? blocks : (blocks + 1) / 2), last = (float)(wgs % 256) / 256.0f;
@@ -604,19 +604,16 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb, size_t parts_byte
         }
     return best;
 }
-static size_t pipe_parts_bytes(const PipePlan &p, size_t M, size_t rows) {
+size_t pipe_gemm_parts_bytes(int kind, size_t M, size_t cols, size_t rows) {
+    const PipePlan p = pipe_plan(kind, rows, M, cols / QK_K);
     return p.k_split > 1 ? (size_t)p.k_split * M * rows * sizeof(float) : 0;
 }
-size_t pipe_gemm_workspace_bytes(int kind, size_t M, size_t cols, size_t rows, size_t limit) {
-    const size_t acts = round_up(q8k_tiled_bytes(M, cols), 256);
-    return acts + pipe_parts_bytes(pipe_plan(kind, rows, M, cols / QK_K, limit > acts ? limit - acts : 0), M, rows);
-}
 
-int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, size_t parts_bytes, hipStream_t s) {
+int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, hipStream_t s) {
     // the kernel addresses a row group's weights with 32-bit lane offsets
     if ((uint64_t)w->layout.row_stride * 64 >= (1ull << 32))
         return set_error(FRK_ERR_SHAPE, "matrix-core GEMM: rows of %zu bytes are beyond the kernel's offsets", w->layout.row_stride);
-    const PipePlan p = pipe_plan(w->kind, w->rows, M, w->cols / QK_K, parts_bytes);
+    const PipePlan p = pipe_plan(w->kind, w->rows, M, w->cols / QK_K);
     const GemmArgs g = pipe_args(w, acts, M, y, (float *)parts, p);
     const bool big = p.rows_wg == 256;
     if (w->kind == FRK_KIND_Q6_K) return launch_pipe_q6_k(g, big, s);
@@ -625,14 +622,6 @@ int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *
                    : launch_pipe<FRK_KIND_Q5_K, 4, 2, 2>(gemm_q5_k_pipe_kernel<4, 2, 2>, g, s);
     return big ? launch_pipe<FRK_KIND_Q4_K, 8, 1, 4>(gemm_q4_k_pipe_kernel<8, 1, 4>, g, s)
                : launch_pipe<FRK_KIND_Q4_K, 4, 2, 2>(gemm_q4_k_pipe_kernel<4, 2, 2>, g, s);
-}
-
-int launch_pipe_gemm(const frk_weights *w, const float *x, size_t M, float *y, void *ws, size_t ws_bytes, hipStream_t s) {
-    const Q8KTiled acts = q8k_tiled_carve(ws, M, w->cols);
-    int rc = launch_quantize_q8_k_tiled(x, M, w->cols, acts, s);
-    if (rc) return rc;
-    const size_t acts_bytes = round_up(q8k_tiled_bytes(M, w->cols), 256);
-    return launch_pipe_gemm_acts(w, acts, M, y, (char *)ws + acts_bytes, ws_bytes - acts_bytes, s);
 }
 
 template <int KIND, bool GATHER>

@@ -875,11 +875,11 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
 // ------------------------------------------------------------------ host side
 
 // The workgroup tile of a batch: 256 rows x 128 tokens or 128 rows x 64 tokens, and how many workgroups share a row's
-// blocks (their sums, in `parts_bytes` of memory at most, are added in order afterwards).
+// blocks (their sums, in SPLIT_PARTS_BYTES of memory at most, are added in order afterwards).
 struct PipePlan {
     int rows_wg, tok_wg, k_split;
 };
-PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb, size_t parts_bytes);  // frk_gemm.hip
+PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb);  // frk_gemm.hip
 
 template <int KIND, int RG, int KS, int MT>
 int launch_pipe(void (*kernel)(GemmArgs), const GemmArgs &g, hipStream_t s) {

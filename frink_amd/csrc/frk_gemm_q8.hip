@@ -396,30 +396,30 @@ static int q8_0_split(size_t rows, size_t M, size_t nb32) {
     return ks;
 }
 // Which kernel, and the scratch memory it takes: the quantized activations, their scales, and room for the parts' sums
-// where the columns are split -- in `limit` bytes where the larger tiles' own split is what would exceed them.
-Q8GemmPlan gemm_q8_0_plan(size_t M, size_t cols, size_t rows, bool q4, size_t limit) {
-    const size_t acts = round_up(M * cols, 256) + round_up(M * round_up(cols / 32, 8) * 2, 256), part = M * rows * sizeof(float);
+// where the columns are split.
+Q8GemmPlan gemm_q8_0_plan(size_t M, size_t cols, size_t rows, bool q4) {
+    const size_t part = M * rows * sizeof(float);
     const int split = q8_0_split(rows, M, cols / 32);
     Q8GemmPlan p;
     p.pipe = Q8PipePlan{0, 0, 0};
-    p.bytes = acts + (split > 1 ? (size_t)split * part : 0);
-    if (q4 || p.bytes > limit) return p;
-    p.pipe = q8_pipe_plan(rows, M, cols / 32, layout_for(FRK_KIND_Q8_0, cols).row_stride, split, (limit - acts) / part);
-    if (p.pipe.rows_wg) p.bytes = acts + (p.pipe.k_split > 1 ? (size_t)p.pipe.k_split * part : 0);
+    p.acts_bytes = round_up(M * cols, 256) + round_up(M * round_up(cols / 32, 8) * 2, 256);
+    if (!q4) p.pipe = q8_pipe_plan(rows, M, cols / 32, layout_for(FRK_KIND_Q8_0, cols).row_stride, split, SPLIT_PARTS_BYTES / part);
+    const int parts = p.pipe.rows_wg ? p.pipe.k_split : split;
+    p.parts_bytes = parts > 1 ? (size_t)parts * part : 0;
     return p;
 }
 
 static int launch_q8_mfma(Q8GemmArgs g, bool q4, bool sub, hipStream_t s);
 
-int launch_gemm_q8_0(const frk_weights *w, const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s) {
+int launch_gemm_q8_0(const frk_weights *w, const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, void *parts, hipStream_t s) {
     return launch_gemm_q8_0_planar(w->dev, w->layout.row_stride, w->layout.off_a, w->rows, w->cols, w->kind == FRK_KIND_Q4_0, plan, x, M,
-                                   y, ws, s);
+                                   y, ws, parts, s);
 }
 
 // The same over any rows in the planar form -- quants [nb][32] (q4: nibbles [nb][16]), then the f16 scales [nb] at
 // off_d of every row: the resident Q8_0 / Q4_0 matrices, and other 32-element kinds decoded into that form.
 int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t cols, bool q4,
-                            const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s) {
+                            const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, void *parts, hipStream_t s) {
     if (M > (size_t)1 << 30 || rows > (size_t)1 << 30)
         return set_error(FRK_ERR_SHAPE, "gemm_q8_0: %zu activation rows x %zu weight rows is too many", M, rows);
     struct {
@@ -442,7 +442,7 @@ int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, s
     g.rows = (int)w->rows;
     g.nb = (int)(w->cols / 32);
     g.M = (int)M;
-    g.partial = reinterpret_cast<float *>((char *)ws + round_up(M * w->cols, 256) + round_up(M * round_up(w->cols / 32, 8) * 2, 256));
+    g.partial = (float *)parts;
     g.tiles = nullptr;
     g.n_tiles = nullptr;
     g.src_rows = nullptr;

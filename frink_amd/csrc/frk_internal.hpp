@@ -229,16 +229,17 @@ int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTile
 // max_rows rows whose first entry is not negative
 int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, size_t max_rows, Q8KTiled out,
                                 hipStream_t s);
-// batched GEMM of the K-quants on the int8 matrix cores; ws must hold pipe_gemm_workspace_bytes(...): the tiled
-// activations, then room for the parts' sums where the blocks are split between workgroups.  With a limit on the memory
-// the blocks are split no further than it allows.
-size_t pipe_gemm_workspace_bytes(int kind, size_t M, size_t cols, size_t rows, size_t limit = SIZE_MAX);
-int launch_pipe_gemm(const frk_weights *w, const float *x, size_t M, float *y, void *ws, size_t ws_bytes, hipStream_t s);
-// the same over activations already quantized into the tiled form; `parts` holds the parts' sums of a split
-int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, size_t parts_bytes, hipStream_t s);
-// the same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time
+// A GEMM that splits a row's columns between workgroups keeps the parts' sums in at most this much memory, whichever entry
+// point it runs for: how a shape is split does not depend on the memory a caller brings, so neither do the result's bits.
+// (Of 6000 drawn shapes up to 14336 x 14336 x 2048, 18 would split further with more: by estimate 8 % faster at most.)
+constexpr size_t SPLIT_PARTS_BYTES = (size_t)FRK_NOALLOC_PARTS_MIB << 20;
+// batched GEMM of the K-quants on the int8 matrix cores, over activations quantized into the tiled form; `parts` holds
+// pipe_gemm_parts_bytes(...) of the parts' sums where the blocks are split between workgroups (0: they are not)
+size_t pipe_gemm_parts_bytes(int kind, size_t M, size_t cols, size_t rows);
+int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, hipStream_t s);
 // y[n] = partial[0][n] + partial[1][n] + ... in that order (the split GEMMs' second step; frk_gemm_q6.hip)
 int launch_sum_parts(const float *partial, int parts, size_t n, float *y, hipStream_t s);
+// the same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time
 // its form over large tiles (frk_gemm_q8_pipe.hip): weight rows x tokens of a workgroup, and how many workgroups share a
 // row's columns; rows_wg = 0: the other kernel
 struct Q8PipePlan {
@@ -249,12 +250,12 @@ int launch_gemm_q8_0_pipe(const Q8PipePlan &p, const uint8_t *W, size_t row_stri
                           const int8_t *aq, const uint16_t *ad, size_t M, float *y, hipStream_t s);
 struct Q8GemmPlan {
     Q8PipePlan pipe;
-    size_t bytes;  // of scratch memory
+    size_t acts_bytes, parts_bytes;  // of scratch memory: the quantized activations, the parts' sums
 };
-Q8GemmPlan gemm_q8_0_plan(size_t M, size_t cols, size_t rows, bool q4, size_t limit);
-int launch_gemm_q8_0(const frk_weights *w, const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s);
+Q8GemmPlan gemm_q8_0_plan(size_t M, size_t cols, size_t rows, bool q4);
+int launch_gemm_q8_0(const frk_weights *w, const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, void *parts, hipStream_t s);
 int launch_gemm_q8_0_planar(const uint8_t *W, size_t row_stride, size_t off_d, size_t rows, size_t cols, bool q4,
-                            const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, hipStream_t s);
+                            const Q8GemmPlan &plan, const float *x, size_t M, float *y, void *ws, void *parts, hipStream_t s);
 // IQ4_XS on the matrix cores: the rows decoded to signed bytes with their block scales (launch_iq4_xs_to_sub_planar,
 // rows of layout_for(FRK_KIND_Q8_0, cols)'s stride) against Q8_K activations
 int launch_iq4_xs_to_sub_planar(const frk_weights *w, uint8_t *dst, size_t dst_stride, size_t off_d, hipStream_t s);

@@ -462,28 +462,35 @@ int frk_hip_read_shape_dev(const void *src, size_t bytes, void *sink, int span_k
     return launch_read_shape(src, bytes, sink, span_kb, waves, to_lds, policy, (hipStream_t)stream);
 }
 
-// Where one call's scratch memory comes from: the stream's leased buffer (grown on demand), or a fixed
-// region that has to suffice (the entry point that allocates nothing).  It must outlive the launches that
+// Where one call's scratch memory comes from: the stream's leased buffer (grown on demand), or fixed
+// regions that have to suffice (the entry point that allocates nothing).  It must outlive the launches that
 // use the memory; nested requests of one call get the same start address, as with the lease.
 struct Scratch {
     WorkspaceLease lease;
-    void *fixed = nullptr;
+    void *fixed = nullptr, *fixed_parts = nullptr;  // of fixed_bytes, of SPLIT_PARTS_BYTES
     size_t fixed_bytes = 0;
     Scratch() = default;
-    Scratch(void *region, size_t bytes) : fixed(region), fixed_bytes(bytes) {}
+    Scratch(void *region, size_t bytes, void *parts) : fixed(region), fixed_parts(parts), fixed_bytes(bytes) {}
     int get(size_t bytes, hipStream_t s, void **out) {
+        void *none = nullptr;
+        return get(bytes, 0, s, out, &none);
+    }
+    // `parts`: room for the parts' sums of a split GEMM besides
+    int get(size_t bytes, size_t parts_bytes, hipStream_t s, void **out, void **parts) {
         if (fixed) {
-            if (bytes > fixed_bytes)
-                return set_error(FRK_ERR_SHAPE, "this shape needs %zu bytes of scratch memory, the entry point that allocates nothing has %zu",
-                                 bytes, fixed_bytes);
+            if (bytes > fixed_bytes || parts_bytes > SPLIT_PARTS_BYTES)
+                return set_error(FRK_ERR_SHAPE, "this shape needs %zu + %zu bytes of scratch memory, the entry point that allocates nothing has %zu + %zu",
+                                 bytes, parts_bytes, fixed_bytes, SPLIT_PARTS_BYTES);
             *out = fixed;
+            *parts = fixed_parts;
             return FRK_OK;
         }
-        int rc = workspace(bytes, s, lease);
+        const size_t at = parts_bytes ? round_up(bytes, 256) : bytes;
+        int rc = workspace(at + parts_bytes, s, lease);
         *out = lease.ptr;
+        *parts = (char *)lease.ptr + at;
         return rc;
     }
-    size_t limit() const { return fixed ? fixed_bytes : SIZE_MAX; }
 };
 
 // Quantizes `batch` activation rows of w->cols values to Q8_K in the call's scratch memory.
@@ -677,16 +684,15 @@ static int gemm_units_int(const frk_weights *w, const float *x, size_t batch, fl
         const Layout planar = layout_for(FRK_KIND_Q8_0, w->cols);
         // (no room for the decoded rows where a copy of them is kept)
         const size_t planar_bytes = w->decoded.load(std::memory_order_acquire) ? 0 : round_up(planar.row_stride * w->rows + 256, 256);
-        void *ws = nullptr;
-        const size_t limit = scratch.limit();
-        const Q8GemmPlan plan = gemm_q8_0_plan(batch, w->cols, w->rows, false, limit > planar_bytes ? limit - planar_bytes : 0);
-        int rc = scratch.get(planar_bytes + plan.bytes, s, &ws);
+        void *ws = nullptr, *parts = nullptr;
+        const Q8GemmPlan plan = gemm_q8_0_plan(batch, w->cols, w->rows, false);
+        int rc = scratch.get(planar_bytes + plan.acts_bytes, plan.parts_bytes, s, &ws, &parts);
         if (rc) return rc;
         const uint8_t *decoded = nullptr;
         rc = units_decoded(w, (uint8_t *)ws, s, &decoded);
         if (rc) return rc;
         return launch_gemm_q8_0_planar(decoded, planar.row_stride, planar.off_a, w->rows, w->cols, false, plan, x, batch, y,
-                                       (char *)ws + planar_bytes, s);
+                                       (char *)ws + planar_bytes, parts, s);
     }
     if (!gemv_units_int_fits(w))
         return set_error(FRK_ERR_UNSUPPORTED, "the integer tier of quant kind %d does not take rows of %zu columns", w->kind, w->cols);
@@ -697,8 +703,8 @@ static int gemm_units_int(const frk_weights *w, const float *x, size_t batch, fl
         const size_t planar_bytes = w->decoded.load(std::memory_order_acquire) ? 0 : round_up(planar.row_stride * w->rows + 256, 256);
         const size_t n = batch * w->cols;
         const size_t q_bytes = round_up(n, 256), d_bytes = round_up(n / QK_K * 4, 256), b_bytes = round_up(n / 16 * 2, 256);
-        void *ws = nullptr;
-        int rc = scratch.get(planar_bytes + q_bytes + d_bytes + b_bytes + gemm_sub_partial_bytes(batch, w->cols, w->rows), s, &ws);
+        void *ws = nullptr, *parts = nullptr;
+        int rc = scratch.get(planar_bytes + q_bytes + d_bytes + b_bytes, gemm_sub_partial_bytes(batch, w->cols, w->rows), s, &ws, &parts);
         if (rc) return rc;
         const uint8_t *decoded = nullptr;
         int8_t *q = (int8_t *)((char *)ws + planar_bytes);
@@ -708,7 +714,7 @@ static int gemm_units_int(const frk_weights *w, const float *x, size_t batch, fl
         if (rc) return rc;
         rc = launch_quantize_q8_k(x, n, q, d, bs, s);
         if (rc) return rc;
-        return launch_gemm_sub_planar(decoded, planar.row_stride, planar.off_a, w->rows, w->cols, q, d, batch, y, (char *)bs + b_bytes, s);
+        return launch_gemm_sub_planar(decoded, planar.row_stride, planar.off_a, w->rows, w->cols, q, d, batch, y, parts, s);
     }
     if (w->kind == FRK_KIND_IQ4_XS) {  // one Q8_K quantization of the batch, the decode kernel per row
         Q8KActs a;
@@ -741,20 +747,23 @@ static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *
     // one row is the decode path, whatever the kind
     if (batch == 1) return gemv_impl(w, x, y, FRK_ACT_F32, (hipStream_t)stream, scratch);
     if (k_quant_takes_the_matrix_cores(w, batch)) {  // (frk_hip_gemm_pair_dev: the same test)
-        void *ws = nullptr;
-        const size_t bytes = pipe_gemm_workspace_bytes(w->kind, batch, w->cols, w->rows, scratch.limit());
-        int rc = scratch.get(bytes, (hipStream_t)stream, &ws);
+        hipStream_t s = (hipStream_t)stream;
+        void *ws = nullptr, *parts = nullptr;
+        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts);
         if (rc) return rc;
-        return launch_pipe_gemm(w, x, batch, y, ws, bytes, (hipStream_t)stream);
+        const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
+        rc = launch_quantize_q8_k_tiled(x, batch, w->cols, acts, s);
+        if (rc) return rc;
+        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
     }
     // Q8_0: a batch is the integer path, as in the reference (Q8_0 activation blocks and dot_q8_0_q8,
     // crates/frink-core/src/weight_matrix.rs:2701-2829); a single row keeps the f32 dot of its decode path
     if ((w->kind == FRK_KIND_Q8_0 || w->kind == FRK_KIND_Q4_0) && batch >= 2) {  // (Q4_0: the same kernel, dot_q4_0_q8)
-        void *ws = nullptr;
-        const Q8GemmPlan plan = gemm_q8_0_plan(batch, w->cols, w->rows, w->kind == FRK_KIND_Q4_0, scratch.limit());
-        int rc = scratch.get(plan.bytes, (hipStream_t)stream, &ws);
+        void *ws = nullptr, *parts = nullptr;
+        const Q8GemmPlan plan = gemm_q8_0_plan(batch, w->cols, w->rows, w->kind == FRK_KIND_Q4_0);
+        int rc = scratch.get(plan.acts_bytes, plan.parts_bytes, (hipStream_t)stream, &ws, &parts);
         if (rc) return rc;
-        return launch_gemm_q8_0(w, plan, x, batch, y, ws, (hipStream_t)stream);
+        return launch_gemm_q8_0(w, plan, x, batch, y, ws, parts, (hipStream_t)stream);
     }
     // Q5_0 / IQ4_XS / MXFP4: a batch is the integer tier too, as in the reference (q8_row_dot / q8k_row_dot per
     // (row, activation) over activations quantized once, crates/frink-core/src/weight_matrix.rs:392-420)
@@ -826,17 +835,17 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
     if (k_quant_takes_the_matrix_cores(w0, batch) && k_quant_takes_the_matrix_cores(w1, batch)) {
         // one quantization into the tiled form, then the two GEMMs (each with its own room for a split's parts)
         const size_t acts_bytes = round_up(q8k_tiled_bytes(batch, w0->cols), 256);
-        const size_t part0 = pipe_gemm_workspace_bytes(w0->kind, batch, w0->cols, w0->rows) - acts_bytes;
-        const size_t part1 = pipe_gemm_workspace_bytes(w1->kind, batch, w1->cols, w1->rows) - acts_bytes;
-        void *ws = nullptr;
-        int rc = scratch.get(acts_bytes + round_up(part0, 256) + part1, s, &ws);
+        const size_t part0 = round_up(pipe_gemm_parts_bytes(w0->kind, batch, w0->cols, w0->rows), 256);
+        const size_t part1 = pipe_gemm_parts_bytes(w1->kind, batch, w1->cols, w1->rows);
+        void *ws = nullptr, *parts = nullptr;
+        int rc = scratch.get(acts_bytes, part0 + part1, s, &ws, &parts);
         if (rc) return rc;
         const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
         rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
         if (rc) return rc;
-        rc = launch_pipe_gemm_acts(w0, acts, batch, y0, (char *)ws + acts_bytes, part0, s);
+        rc = launch_pipe_gemm_acts(w0, acts, batch, y0, parts, s);
         if (rc) return rc;
-        return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)ws + acts_bytes + round_up(part0, 256), part1, s);
+        return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)parts + part0, s);
     }
     // otherwise each matrix takes the path frk_hip_gemm_dev gives it (the same results, two quantizations)
     int rc = gemm_impl(w0, x, batch, y0, stream, scratch);
@@ -937,15 +946,14 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *a, float *
     hipStream_t s = (hipStream_t)stream;
     if (k_quant_takes_the_matrix_cores(w, batch)) {
         const Q8KTiled acts = q8k_tiled_carve((char *)a->base + a->tiled_off, batch, a->cols);
-        const size_t acts_bytes = round_up(q8k_tiled_bytes(batch, w->cols), 256);
-        const size_t need = pipe_gemm_workspace_bytes(w->kind, batch, w->cols, w->rows);
+        const size_t parts_bytes = pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows);
         void *parts = nullptr;
         Scratch scratch;
-        if (need > acts_bytes) {  // a split of the blocks between workgroups: room for the parts' sums
-            int rc = scratch.get(need - acts_bytes, s, &parts);
+        if (parts_bytes) {  // a split of the blocks between workgroups: room for the parts' sums
+            int rc = scratch.get(parts_bytes, s, &parts);
             if (rc) return rc;
         }
-        return launch_pipe_gemm_acts(w, acts, batch, y, parts, need - acts_bytes, s);
+        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
     }
     // (below the matrix-core GEMMs' batches the plain rows are there: ACTS_PLAIN_MAX_BATCH covers every such batch)
     if (batch > ACTS_PLAIN_MAX_BATCH)
@@ -961,11 +969,12 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *a, float *
 }
 
 // ---- the entry point that allocates nothing ----
-// Its scratch memory is this array in the library's device image: every GPU the library runs on holds
-// its own copy, at its own address, until the process ends.  In host code the array's name is only a
-// handle for hipGetSymbolAddress; what the kernels get is the address looked up once per device.
+// Its scratch memory is this array in the library's device image (the quantized activations and decoded rows, then the
+// parts' sums of a split GEMM): every GPU the library runs on holds its own copy, at its own address, until the process
+// ends.  In host code the array's name is only a handle for hipGetSymbolAddress; what the kernels get is the address
+// looked up once per device.
 constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)FRK_NOALLOC_SCRATCH_MIB << 20;
-static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES + SPLIT_PARTS_BYTES];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static void *g_scratch_addr[NOALLOC_MAX_DEVICES] = {nullptr};  // under g_dev.mu
 
@@ -991,7 +1000,7 @@ int frk_hip_gemm_noalloc_dev(const frk_weights *w, const float *x, size_t batch,
     void *region = nullptr;
     int rc = noalloc_scratch(&region);
     if (rc) return rc;
-    Scratch fixed(region, NOALLOC_SCRATCH_BYTES);
+    Scratch fixed(region, NOALLOC_SCRATCH_BYTES, (char *)region + NOALLOC_SCRATCH_BYTES);
     return gemm_impl(w, x, batch, y, stream, fixed);
 }
 

@@ -250,15 +250,16 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *acts, floa
 
 /* frk_hip_gemm_dev for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same arguments, same
- * kernels and bit for bit the same y (where the parts of a split GEMM fit; where they do not the blocks of a
- * row are split less and add up in another order), but the scratch memory (quantized activations, the parts of a
- * split GEMM) is a fixed array of FRK_NOALLOC_SCRATCH_MIB MiB inside the library's device image, looked
- * up on the first call on a device; the call never allocates or frees.  A shape whose scratch does not
- * fit returns FRK_ERR_SHAPE and launches nothing (it fits every batch of up to 64 rows of matrices up to
- * 16384 columns, and prefill batches of 512 rows of 4096 columns that need no split).  Every call on a
- * GPU shares that GPU's array: calls that overlap on one GPU (two streams, two threads) race -- enqueue
- * them on one stream. */
+ * kernels and bit for bit the same y, but the scratch memory is a fixed array inside the library's device
+ * image, looked up on the first call on a device: FRK_NOALLOC_SCRATCH_MIB MiB for quantized activations
+ * (and, for the kinds that are decoded on each call, the decoded rows), and FRK_NOALLOC_PARTS_MIB MiB for
+ * the parts of a split GEMM, which is as much as any call splits into.  The call never allocates or frees.
+ * A shape whose scratch does not fit returns FRK_ERR_SHAPE and launches nothing (K-quants and Q8_0: it fits
+ * every batch of up to 64 rows of matrices up to 16384 columns, and prefill batches of up to 1024 rows of
+ * 14336 columns).  Every call on a GPU shares that GPU's array: calls that overlap on one GPU (two streams,
+ * two threads) race -- enqueue them on one stream. */
 #define FRK_NOALLOC_SCRATCH_MIB 16
+#define FRK_NOALLOC_PARTS_MIB 64
 int frk_hip_gemm_noalloc_dev(const frk_weights *w, const float *x_dev, size_t batch, float *y_dev,
                              void *stream);
 

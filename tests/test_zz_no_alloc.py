@@ -54,6 +54,42 @@ def test_gemm_noalloc_gives_the_bits_of_gemm(fa, kind, rows, cols, batches):
     w.release()
 
 
+@pytest.mark.parametrize("kind,rows,cols,batch", [
+    (fo.Q4_K, 4096, 14336, 256),
+    (fo.Q4_K, 1536, 8192, 700),    # (this and the next two: the parts' sums alone take more than the activations' 16 MiB)
+    (fo.Q5_K, 2560, 12288, 300),
+    (fo.Q6_K, 4096, 14336, 512),
+    (fo.Q8_0, 1024, 16384, 512),
+    (fo.Q8_0, 3000, 14336, 400),
+    (fo.MXFP4, 700, 14336, 200),
+])
+def test_gemm_noalloc_splits_as_gemm_does(fa, kind, rows, cols, batch):
+    """A prefill batch whose rows are split between many workgroups: the same split and so the same bits, and those of
+    the exactly quantized operands' product."""
+    import torch
+    from bench import random_blocks
+    from frink_amd import synth
+    from test_gpu_parity import _other_kind_blocks
+    print("no-alloc split", kind, rows, cols, batch, flush=True)
+    if kind == fo.MXFP4:
+        data = _other_kind_blocks(kind, rows, cols, seed=3)
+        blocks = data.reshape(-1, 17)
+        blocks[:, 0] = 112 + blocks[:, 0] % 8
+    else:
+        data = random_blocks(kind, rows, cols, seed=rows)
+    w = fa.Weights.from_host(kind, data, rows, cols)
+    x = synth.activations(4200 + batch, batch, cols)
+    xd = torch.from_numpy(x).cuda()
+    want = w.gemm(xd)
+    got = torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda")
+    w.gemm_noalloc(xd, got)
+    assert np.array_equal(_bits(got), _bits(want))
+    ref = fo.gemm(kind, data[:data.size // rows * 24], 24, cols, x, fo.INT_DOT)
+    err = np.abs(got[:, :24].cpu().numpy() - ref).max(axis=1) / np.abs(ref).max(axis=1)
+    assert err.max() <= 1e-5, err.max()  # (the order of at most 448 f32 additions)
+    w.release()
+
+
 def test_gemm_noalloc_refuses_a_shape_beyond_its_scratch(fa):
     import torch
     from frink_amd import synth
