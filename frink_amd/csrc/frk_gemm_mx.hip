@@ -36,7 +36,7 @@ MxActs mx_acts_carve(void *base, size_t rows, size_t cols) {
     MxActs a;
     a.digits = (uint8_t *)base;
     a.scales = (uint32_t *)((char *)base + round_up(blocks * MX_BLOCK_BYTES, 256));
-    a.factor = (float *)((char *)a.scales + round_up(blocks * 4, 256));
+    a.infinite = (int *)((char *)a.scales + round_up(blocks * 4, 256));
     return a;
 }
 size_t mx_acts_bytes(size_t rows, size_t cols) {
@@ -293,15 +293,6 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
 #undef FRK_MX_REST
 #undef FRK_MX_ARRIVE
 
-    // the factor of row `lane` of the tile
-    float factor = 1.0f;
-    {
-        const int r = tile.y + lane, src = g.src_rows ? g.src_rows[r] : r;
-        if (lane < tile.z && src >= 0) factor = g.acts.factor[src];
-    }
-    const bool scaled_rows = __any(factor != 1.0f);
-
-
     // ---- register r of a lane: activation row 8 * (r / 4) + 4 * (lane / 32) + r % 4 of the half, weight row lane % 32
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -309,11 +300,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int tok = 32 * h + 8 * (r >> 2) + 4 * lg + (r & 3);
-            float v0 = acc[h][0][r], v1 = acc[h][1][r];
-            if (scaled_rows) {
-                const float f = __shfl(factor, tok);
-                v0 = f == 1.0f ? v0 : v0 * f, v1 = f == 1.0f ? v1 : v1 * f;
-            }
+            const float v0 = acc[h][0][r], v1 = acc[h][1][r];
             if (tok >= tile.z) continue;
             float *dst = g.y + (size_t)(tile.w + tok) * g.rows;
             if (GLU) {
@@ -322,6 +309,43 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
                 if (row0 < g.rows) dst[row0] = v0;
                 if (row0 + 32 < g.rows) dst[row0 + 32] = v1;
             }
+        }
+    }
+
+    // ---- the rows with infinite blocks again (hardly ever any): what decides is the sign of each such block's integer
+    // sum, an infinity each, NaN where the sum is zero or two differ.  Lanes 0 .. 31 take the first row group, the others
+    // the second.
+    bool again = false;
+    if (lane < tile.z) {
+        const int src = g.src_rows ? g.src_rows[tile.y + lane] : tile.y + lane;
+        again = src >= 0 && g.acts.infinite[src] != 0;
+    }
+    uint64_t left = __ballot(again);
+    if (left) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (their first results are out)
+    for (; left; left &= left - 1) {
+        const int tok = __builtin_ctzll(left);
+        const size_t first = (size_t)act_row(tok) * nbp;
+        const uint8_t *codes_row = (lg ? w_base[1] : w_base[0]) + weight_row(lane);
+        float sum = 0.0f;
+        for (int b = 0; b < nb; b++) {
+            if ((g.acts.scales[first + b] & 0xffu) != MX_INFINITE) continue;
+            const int8_t *q = reinterpret_cast<const int8_t *>(g.acts.digits + (first + b) * MX_BLOCK_BYTES);
+            int isum = 0;
+            for (int i = 0; i < 16; i++) {
+                auto times = [&](int code, int quant) {  // 0, 1, 2, 3, 4, 6, 8, 12 halves
+                    const int m = (int)(0xc8643210u >> (4 * (code & 7)) & 15u);
+                    return (code & 8 ? -m : m) * quant;
+                };
+                isum += times(codes_row[b * 16 + i] & 15, q[i]) + times(codes_row[b * 16 + i] >> 4, q[16 + i]);
+            }
+            sum += (float)isum * __builtin_inff();
+        }
+        float *dst = g.y + (size_t)(tile.w + tok) * g.rows;
+        if (GLU) {
+            const float up = __shfl_xor(sum, 32);
+            if (lg == 0 && row0 < g.rows) dst[row0] = silu_as_host(sum) * up;
+        } else if (row0 + 32 * lg < g.rows) {
+            dst[row0 + 32 * lg] = sum;
         }
     }
 #endif

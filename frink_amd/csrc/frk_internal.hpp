@@ -271,7 +271,7 @@ int launch_quantize_q8_0_gemm(const float *x, const float *up, size_t rows, size
 struct MxActs {
     uint8_t *digits;   // [rows][blocks of 32, padded to a multiple of 8][96]
     uint32_t *scales;  // [rows][blocks]: a byte per plane
-    float *factor;     // [rows]: 1, or infinity where a block's scale is
+    int *infinite;     // [rows]: 1 where a block's scale is infinite
 };
 MxActs mx_acts_carve(void *base, size_t rows, size_t cols);
 size_t mx_acts_bytes(size_t rows, size_t cols);

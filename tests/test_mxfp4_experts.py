@@ -70,6 +70,65 @@ def test_activations_whose_scale_leaves_f16(fa):
 
 
 @pytest.mark.gpu
+def test_rows_with_several_blocks_whose_scale_leaves_f16(fa):
+    """Every such block adds an infinity of its own: two that agree stay infinite, two that differ give NaN, as does one
+    whose integer sum is zero beside one whose sum is not."""
+    cols, rows_g = 416, 70
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((70, cols)).astype(np.float32)
+    x[3, [10, 200]] = 2.0e7
+    x[7, [10, 200, 415]] = 1.0e8, -3.0e7, 2.0e8
+    x[40, 64:96] = 9.0e6 * rng.standard_normal(32)
+    x[40, 96] = -1.0e9
+    x[66, [0, 33]] = np.inf, 2.0e7
+    off, per, got = _case(fa, [33, 37], rows_g, cols, x, seed=21)
+    large = [3, 7, 40, 66]
+    for g in range(2):
+        s = slice(int(off[g]), int(off[g + 1]))
+        want = fo.gemm(fo.MXFP4, per[g], rows_g, cols, x[s], fo.INT_DOT)
+        assert np.array_equal(np.isnan(got[s]), np.isnan(want)) and np.array_equal(np.isinf(got[s]), np.isinf(want))
+        inf = np.isinf(want)
+        assert np.array_equal(np.sign(got[s][inf]), np.sign(want[inf]))
+        fine = [r for r in range(want.shape[0]) if r + s.start not in large]
+        assert (np.abs(got[s][fine] - want[fine]).max(axis=1) <= 1e-5 * np.abs(want[fine]).max(axis=1)).all()
+    for r in (3, 7, 40):  # (rows with both outcomes)
+        assert np.isnan(got[r]).any() and np.isinf(got[r]).any()
+    assert np.isnan(got[66]).all()
+
+
+@pytest.mark.gpu
+def test_moe_layer_whose_intermediates_leave_f16(fa):
+    """The same between gate/up and the down projection: a layer of a few tokens runs a job per pair, a batch the grouped
+    kernels, and a token's results are of the same kind in both."""
+    import torch
+    n_experts, hidden, ffn, batch = 4, 416, 448, 40
+    rng = np.random.default_rng(12)
+    ws = []
+    for i, (rows, cols) in enumerate(((ffn, hidden), (ffn, hidden), (hidden, ffn))):
+        data = _other_kind_blocks(fo.MXFP4, n_experts * rows, cols, seed=30 + i)
+        data.reshape(-1, 17)[:, 0] = 118 + data.reshape(-1, 17)[:, 0] % 4
+        ws.append(fa.Weights.from_host(fo.MXFP4, data, n_experts * rows, cols))
+    x = rng.standard_normal((batch, hidden)).astype(np.float32)
+    x[5] *= 2.0e4       # finite gate and up, products past 8.3e6 in many blocks
+    x[9, [3, 300]] = 2.0e7   # infinite gate and up
+    ids = to_dev(rng.integers(0, n_experts, (batch, 1)).astype(np.int32))
+    weights = torch.ones((batch, 1), dtype=torch.float32, device="cuda")
+    xd = to_dev(x)
+    got = fa.moe_ffn(*ws, n_experts, xd, ids, weights).cpu().numpy()
+    want = np.concatenate([fa.moe_ffn(*ws, n_experts, xd[i:i + 8].contiguous(), ids[i:i + 8].contiguous(), weights[i:i + 8].contiguous()).cpu().numpy()
+                           for i in range(0, batch, 8)])
+    assert not np.isfinite(want[5]).all() and not np.isfinite(want[9]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    inf = np.isinf(want)
+    assert np.array_equal(np.sign(got[inf]), np.sign(want[inf]))
+    fine = [r for r in range(batch) if r not in (5, 9)]
+    # (an intermediate's last bit now and then moves a quant of the down projection's input to the next level)
+    assert (np.abs(got[fine] - want[fine]).max(axis=1) <= 2e-3 * np.abs(want[fine]).max(axis=1)).all()
+    for w in ws:
+        w.release()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n_experts,k,hidden,ffn,batch", [(64, 2, 160, 1056, 40), (3, 2, 544, 288, 33), (8, 2, 288, 544, 16), (16, 2, 96, 160, 15)])
 def test_moe_layer_at_the_edges_of_its_tiles(fa, n_experts, k, hidden, ffn, batch):
     _moe_case(fa, fo.MXFP4, fo.MXFP4, n_experts, k, hidden, ffn, batch)
