@@ -7,9 +7,9 @@
 // E8M0 byte its scale.  The activation block's  da * qa  is a 19-bit number (f16 scale: 11 bits of mantissa, 8-bit quant)
 // times a power of two, and goes through as four planes of signed base-32 digits, -16 .. 16: exact in E2M3 (six bits),
 // the power of two and the plane's 32^p in its E8M0 scale.  So every product is exact, sums are f32 inside the matrix
-// core, and the vector ALU has no float step at all -- it adds the sums of 128 columns onto the running ones, which keeps
-// the error against 64 bits below that of one addition a block (2-norm over 2-norm at 1024 / 1184 / 2048 columns: 5.8e-8,
-// 6.2e-8 and 7.9e-8, with an addition a block 7.6e-8, 8.2e-8 and 1.1e-7).
+// core, and the vector ALU has no float step at all -- it adds the sums of 128 columns onto the running ones.  From 384
+// columns on that keeps the error against 64 bits below that of one rounding a block, which shorter rows keep
+// (mx_gemm_takes).
 // (Byte i of a GGUF block holds elements i and i + 16; a lane's operand takes byte i as k = 2i and 2i + 1.  The order of
 // k within a block is free as long as both operands have it: the digits are stored in the weights' order.)
 //
@@ -351,7 +351,15 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
 #endif
 }
 
-bool mx_gemm_fits(size_t act_rows, size_t rows_g, size_t cols) {
+// Rows of 384 columns and more.  A matrix-core step rounds its 64 products several times within the last places of the
+// largest, and the vector ALU adds once a quad of blocks; the decoded form's kernel rounds once a block.  Errors against
+// 64-bit sums of the same quantized operands, this kernel's over the other one's (2-norm / largest; activations N(0, 1) with
+// scales of 4 powers of two, and the worst of that, of scales of 40 powers and of a 64th of the channels fifty times as
+// large): 64 columns 1.02 / 1.00 and 1.30 / 1.54, 128 1.01 / 0.94 and 1.25 / 1.52, 256 0.90 / 0.73 and 1.08 / 0.93, 320 0.91 /
+// 0.83 and 1.03 / 0.86, 384 0.85 / 0.71 and 0.99 / 0.84, 512 0.83 / 0.68 and 0.94 / 0.85, 1024 0.76 / 0.67 and 0.83 / 0.81, 2880
+// 0.68 / 0.51 and 0.76 / 0.56 (there 9.3e-8 against 1.4e-7 in the 2-norm).
+bool mx_gemm_takes(size_t act_rows, size_t rows_g, size_t cols) {
+    if (cols < 384) return false;
     // lane offsets are 32 bits wide
     return act_rows * mx_padded_blocks(cols) * MX_BLOCK_BYTES <= 0xffffffffu &&
            rows_g * layout_for(FRK_KIND_MXFP4, cols).row_stride <= 0xffffffffu;

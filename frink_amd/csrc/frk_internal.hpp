@@ -276,7 +276,7 @@ struct MxActs {
 MxActs mx_acts_carve(void *base, size_t rows, size_t cols);
 size_t mx_acts_bytes(size_t rows, size_t cols);
 int launch_quantize_mx(const float *x, size_t rows, size_t cols, const int *used, const MxActs &out, hipStream_t s);
-bool mx_gemm_fits(size_t act_rows, size_t rows_g, size_t cols);
+bool mx_gemm_takes(size_t act_rows, size_t rows_g, size_t cols);
 int launch_gemm_mx_grouped(const frk_weights *w, const frk_weights *up, size_t rows_g, const MxActs &acts, const int *src_rows,
                            const int4 *tiles, const int *n_tiles, size_t max_tiles, float *y, hipStream_t s);
 // the grouped GEMM over groups of Q5_0 / IQ4_XS / MXFP4 matrices that have a decoded form for the matrix cores

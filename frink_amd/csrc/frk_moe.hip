@@ -774,8 +774,8 @@ struct UnitsNative {
 };
 static UnitsNative units_native(int gate_kind, int down_kind, size_t batch, size_t rows, size_t hidden, size_t ffn) {
     UnitsNative n;
-    n.gate_up = gate_kind == FRK_KIND_MXFP4 && mx_gemm_fits(std::max(batch, rows), ffn, hidden);
-    n.down = n.gate_up && down_kind == FRK_KIND_MXFP4 && mx_gemm_fits(rows, hidden, ffn);
+    n.gate_up = gate_kind == FRK_KIND_MXFP4 && mx_gemm_takes(std::max(batch, rows), ffn, hidden);
+    n.down = n.gate_up && down_kind == FRK_KIND_MXFP4 && mx_gemm_takes(rows, hidden, ffn);
     return n;
 }
 bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts, size_t batch,
@@ -863,7 +863,7 @@ struct GroupedUnitsScratch {
     int4 *tiles;
 };
 static bool grouped_units_native(int kind, size_t rows_g, size_t x_rows, size_t cols) {
-    return kind == FRK_KIND_MXFP4 && mx_gemm_fits(x_rows, rows_g, cols);
+    return kind == FRK_KIND_MXFP4 && mx_gemm_takes(x_rows, rows_g, cols);
 }
 static GroupedUnitsScratch grouped_units_carve(void *base, bool native, size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs,
                                                size_t cols, size_t *end) {

@@ -26,7 +26,11 @@ def _case(fa, counts, rows_g, cols, x, seed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows_g,cols,counts", [
     (1, 32, [1, 64]), (63, 96, [0, 33, 2]), (65, 128, [32, 31, 65]), (257, 160, [64, 5]), (72, 544, [97, 1]),
-    (512, 1056, [40]), (1100, 160, [3, 0, 34] * 30),  # (the last: eight wavefronts a workgroup, three workgroups a tile)
+    (512, 1056, [40]), (1100, 160, [3, 0, 34] * 30),
+    # (rows from 384 columns on are frk_gemm_mx.hip's: three quads of blocks, and one to four blocks of a last one; the last:
+    # eight wavefronts a workgroup, three workgroups a tile)
+    (1, 384, [1, 64]), (63, 416, [0, 33, 2]), (65, 448, [32, 31, 65]), (257, 480, [64, 5]), (72, 512, [97, 1]),
+    (1100, 416, [3, 0, 34] * 30),
 ])
 def test_grouped_gemm_at_the_edges_of_its_tiles(fa, rows_g, cols, counts):
     from frink_amd import synth
@@ -46,6 +50,28 @@ def test_grouped_gemm_at_the_edges_of_its_tiles(fa, rows_g, cols, counts):
         wd = fo.dequant(fo.MXFP4, per[g]).reshape(rows_g, cols).astype(np.float64)
         room = (64 + cols // 128 + 1) * 2.0 ** -24 * (np.abs(a[s]) @ np.abs(wd).T)
         assert (np.abs(got[s] - a[s] @ wd.T) <= room).all(), g
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [64, 96, 352])
+def test_short_rows_round_once_a_block(fa, cols):
+    """Below 384 columns a block's sum is an exact integer with one rounding behind it, added in the blocks' order."""
+    from frink_amd import synth
+    rows_g, counts = 80, [70, 50]
+    x = synth.activations(77, sum(counts), cols, outlier_frac=0.02)
+    off, per, got = _case(fa, counts, rows_g, cols, x, seed=cols)
+    xb = x.reshape(-1, cols // 32, 32)
+    amax = np.abs(xb).max(axis=2)
+    inv = np.where(amax != 0, np.float32(127) / np.where(amax != 0, amax, 1), 0).astype(np.float32)
+    q = np.clip(np.rint(xb * inv[:, :, None]), -127, 127).astype(np.float64)
+    a = q * (amax / np.float32(127)).astype(np.float16).astype(np.float64)[:, :, None]
+    for g in range(len(counts)):
+        s = slice(int(off[g]), int(off[g + 1]))
+        wd = fo.dequant(fo.MXFP4, per[g]).reshape(rows_g, cols // 32, 32).astype(np.float64)
+        running = np.cumsum(np.einsum("tbi,rbi->trb", a[s], wd), axis=2)
+        # half a unit in the last place of every running sum, and of what the roundings before have made of it
+        room = 2.0 ** -24 * (np.abs(running).sum(axis=2) * (1 + 2.0 ** -20) + cols // 32 * 2.0 ** -24 * np.abs(running).max(axis=2))
+        assert (np.abs(got[s] - running[:, :, -1]) <= room).all(), g
 
 
 @pytest.mark.gpu
@@ -81,6 +107,9 @@ def test_rows_with_several_blocks_whose_scale_leaves_f16(fa):
     x[40, 64:96] = 9.0e6 * rng.standard_normal(32)
     x[40, 96] = -1.0e9
     x[66, [0, 33]] = np.inf, 2.0e7
+    x[9, 50] = np.nan       # (counts as zero)
+    x[11, :32] *= 1e-5      # (an f16 subnormal scale)
+    x[12] = 0.0
     off, per, got = _case(fa, [33, 37], rows_g, cols, x, seed=21)
     large = [3, 7, 40, 66]
     for g in range(2):
@@ -129,7 +158,8 @@ def test_moe_layer_whose_intermediates_leave_f16(fa):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_experts,k,hidden,ffn,batch", [(64, 2, 160, 1056, 40), (3, 2, 544, 288, 33), (8, 2, 288, 544, 16), (16, 2, 96, 160, 15)])
+@pytest.mark.parametrize("n_experts,k,hidden,ffn,batch", [(64, 2, 160, 1056, 40), (3, 2, 544, 288, 33), (8, 2, 288, 544, 16), (16, 2, 96, 160, 15),
+                                                            (64, 2, 416, 1056, 40), (3, 2, 544, 416, 33), (8, 2, 480, 544, 16)])
 def test_moe_layer_at_the_edges_of_its_tiles(fa, n_experts, k, hidden, ffn, batch):
     _moe_case(fa, fo.MXFP4, fo.MXFP4, n_experts, k, hidden, ffn, batch)
 
