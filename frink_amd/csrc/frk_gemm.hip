@@ -576,7 +576,8 @@ int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, 
 // equal share of them (deal_entry); splitting the blocks costs the second launch and its bytes.  The constants are a fit
 // (4 % rms) to 6079 launches over 1200 drawn shapes: the three kinds, 1024 .. 14336 rows and columns, 8 .. 2048 tokens,
 // 1 .. 8 parts.  Over the 720 of them with 48 tokens and more the choice is 0.2 % behind the best one measured on average,
-// 8 % at worst; with the constants fitted to one half and tried on the other likewise.
+// 8 % at worst; with the constants fitted to one half and tried on the other likewise.  (Up to 64 tokens the small tile, the
+// cheaper one there in every launch measured: its float step is the thin kernels', see fold_mins.)
 PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     struct Cost {
         float step, load, start;
@@ -586,7 +587,7 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     const Cost large = kind == FRK_KIND_Q4_K ? Cost{2.66f, 1.07f, 4.85f} : Cost{3.26f, 1.06f, 5.79f};
     PipePlan best = {128, 64, 1};
     float best_us = 0.0f;
-    for (int big = 0; big < 2; big++)
+    for (int big = 0; big < (M > 64 ? 2 : 1); big++)
         for (int ks : {1, 2, 3, 4, 6, 8}) {
             const size_t bytes = (size_t)ks * M * rows * sizeof(float);
             if (ks > 1 && (nb / (size_t)ks < 2 || bytes > SPLIT_PARTS_BYTES)) continue;

@@ -142,12 +142,14 @@ __device__ __forceinline__ void unpack_rest(const v4i &wh, const BlockScales &s,
     B.ndmin = -h2f(hx >> 16);
 }
 
-// The dense kernel's form of a tile's float step, one accumulator less: the mins' MFMA adds onto the
-// converted integer sums instead of into registers of its own.  With d' = d / (-dmin):
+// The large tile's form of the float step, one accumulator less (there are no registers for it): the mins' MFMA
+// adds onto the converted integer sums instead of into registers of its own.  With d' = d / (-dmin):
 //     d * S1 - dmin * S2 = (-dmin) * (d' * S1 + S2),
 // so the f16 MFMA takes d' * S1 as its C operand and the epilogue multiplies by -dmin (and the token's
-// scale).  A row whose dmin is zero keeps d and a factor of one, and zero mins.  (Not the same
-// rounding as the two-term form: both are within a few ulp of the exact sum.)
+// scale).  A row whose dmin is zero keeps d and a factor of one, and zero mins.  (Two roundings a block more than the
+// two-term form of the small tile, which every batch of up to 64 rows takes, and of the thin kernels: 2-norm against
+// 64-bit sums at 15 rows of Q4_K 2009x12032 1.3e-7 folded, 9.0e-8 apart, 9.2e-8 on the thin kernels; Q5_K 3594x8192 at 25
+// 1.3e-7, 9.2e-8 and 9.0e-8.  In time the small tile's two forms are within 1 % of each other.)
 __device__ __forceinline__ void fold_mins(BPlanes &B) {
     const bool z = B.ndmin == 0.0f;
     B.d = z ? B.d : B.d * __builtin_amdgcn_rcpf(B.ndmin);
@@ -336,28 +338,36 @@ __device__ __forceinline__ void read_tile_scales(TileScales &S, uint32_t sa) {
     ds_read16<SLOT * 128 + 96>(S.da3, sa);
 }
 
-// A finished tile's way into the float sums, in sixteen pieces.  With mins (the arithmetic fold_mins prepares):
+// A finished tile's way into the float sums, in sixteen pieces.  MINS_FOLDED (the arithmetic fold_mins prepares):
 //   pieces 0..7   c[r] = d' * float(S1[r]) for two results each,
 //   piece  7      then the mins' MFMA adds S2 onto c,
 //   pieces 8..15  sum[r] += (da[r] * -dmin) * c[r] for two results each.
-// Without: c[r] = float(S1[r]), then sum[r] += (da[r] * d) * c[r].
+// MINS_APART: piece 0 S2 into registers of its own, pieces 0..7 c[r] = d * float(S1[r]), pieces 8..15
+// sum[r] += da[r] * (c[r] - dmin * S2[r]).
+// NO_MINS: c[r] = float(S1[r]), then sum[r] += (da[r] * d) * c[r].
+enum { NO_MINS, MINS_FOLDED, MINS_APART };
 struct TileTail {
     v16i s1;      // the integer sums
-    v16f c;       // d' * S1, then + S2
+    v16f c;       // see above
+    v16f s2;      // MINS_APART
     v8h bs;       // the tile's 16-wide activation sums
     TileScales S; // the tile's activation scales
 };
-template <bool MINS>
+template <int FORM>
 __device__ __forceinline__ void tail_piece(int i, TileTail &E, const BPlanes &B, v16f &sum) {
     if (i < 8) {
-        E.c[2 * i] = MINS ? B.d * (float)E.s1[2 * i] : (float)E.s1[2 * i];
-        E.c[2 * i + 1] = MINS ? B.d * (float)E.s1[2 * i + 1] : (float)E.s1[2 * i + 1];
-        if (MINS && i == 7) E.c = __builtin_amdgcn_mfma_f32_32x32x16_f16(E.bs, B.m, E.c, 0, 0, 0);
+        if (FORM == MINS_APART && i == 0) E.s2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(E.bs, B.m, v16f{0.0f}, 0, 0, 0);
+        E.c[2 * i] = FORM != NO_MINS ? B.d * (float)E.s1[2 * i] : (float)E.s1[2 * i];
+        E.c[2 * i + 1] = FORM != NO_MINS ? B.d * (float)E.s1[2 * i + 1] : (float)E.s1[2 * i + 1];
+        if (FORM == MINS_FOLDED && i == 7) E.c = __builtin_amdgcn_mfma_f32_32x32x16_f16(E.bs, B.m, E.c, 0, 0, 0);
     } else {
         const v4f dav[4] = {E.S.da0, E.S.da1, E.S.da2, E.S.da3};
-        const float d = MINS ? B.ndmin : B.d;
+        const float d = FORM == MINS_FOLDED ? B.ndmin : B.d;
 #pragma unroll
-        for (int r = 2 * (i - 8); r < 2 * (i - 8) + 2; r++) sum[r] = fmaf(dav[r >> 2][r & 3] * d, E.c[r], sum[r]);
+        for (int r = 2 * (i - 8); r < 2 * (i - 8) + 2; r++) {
+            if (FORM == MINS_APART) sum[r] = fmaf(dav[r >> 2][r & 3], fmaf(B.ndmin, E.s2[r], E.c[r]), sum[r]);
+            else sum[r] = fmaf(dav[r >> 2][r & 3] * d, E.c[r], sum[r]);
+        }
     }
 }
 
@@ -514,10 +524,7 @@ struct WeightSide {  // Q4_K, Q5_K: the rows' 9 or 11 sixteen-byte pieces back t
         }
         wait_raw<0>(R);
     }
-    static __device__ __forceinline__ void unpack(const Raw &R, int lg, int, BPlanes &B) {
-        unpack_block(R, lg, B);
-        fold_mins(B);
-    }
+    static __device__ __forceinline__ void unpack(const Raw &R, int lg, int, BPlanes &B) { unpack_block(R, lg, B); }
     __device__ __forceinline__ void pin() {  // the lane offsets stay in registers as they are
 #pragma unroll
         for (int c = 0; c < NC; c++) asm volatile("" : "+v"(off[c]));
@@ -647,6 +654,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     using L = PipeLds<KIND, RG, KS, MT>;
     using Side = typename L::Side;
     constexpr bool MINS = Side::MINS;
+    constexpr int FORM = !MINS ? NO_MINS : MT == 4 ? MINS_FOLDED : MINS_APART;
     constexpr int NW = L::NW, NT = L::NT, ROWS = 32 * RG, TM = 32 * MT;
     static_assert(NW == 8 && NT == 4 && (MT == 2 || MT == 4), "eight wavefronts share the four tile slots of a stage");
     extern __shared__ uint4 smem_gemm[];
@@ -734,7 +742,10 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     int kb_raw = kb0 + ks * steps;  // the block that leaves the slot next
     // a raw block leaves this wavefront's slot for registers
     auto read_block = [&]() { Side::read(R, lds_w, li, lg); };
-    auto unpack = [&]() { Side::unpack(R, lg, kb_raw++, B); };
+    auto unpack = [&]() {
+        Side::unpack(R, lg, kb_raw++, B);
+        if (FORM == MINS_FOLDED) fold_mins(B);
+    };
 
     // prologue: activations of steps 0 and 1, weights of step 0; then the weights of step 1
     if (fetches_acts) {
@@ -786,7 +797,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
                         // they have landed once the chain has waited for everything, in front of MFMA 8, and
                         // only from here on may the compiler touch them
                         if (j == 8) wait_scales<0>(E.S);
-                        tail_piece<MINS>(j, E, B, sum[mt > 0 ? mt - 1 : 0]);
+                        tail_piece<FORM>(j, E, B, sum[mt > 0 ? mt - 1 : 0]);
                     }
                 };
                 auto next = [&](int j) {
@@ -820,7 +831,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
             // the last tile's tail is exposed
             wait_scales<0>(E.S);
 #pragma unroll
-            for (int j = 0; j < 16; j++) tail_piece<MINS>(j, E, B, sum[MT - 1]);
+            for (int j = 0; j < 16; j++) tail_piece<FORM>(j, E, B, sum[MT - 1]);
         } else if (fetch_now) {
             fetch_quants(0), fetch_quants(1), fetch_sums_scales(), acts_fetched();
         }

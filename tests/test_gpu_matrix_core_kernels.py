@@ -64,3 +64,22 @@ def test_batches_around_the_step_from_thin_to_tiled(fa, kind, rows, cols):
         assert (np.abs(y.astype(np.float64) - a @ wd.T) <= (cols // 256 + 9) * 2.0 ** -24 * room).all(), batch
     acts.release()
     w.release()
+
+
+@pytest.mark.parametrize("kind,rows,cols", [(fo.Q4_K, 640, 9728), (fo.Q5_K, 640, 8192), (fo.Q6_K, 4104, 8448)])
+def test_a_batch_past_the_thin_kernels_is_no_further_from_64_bit_sums(fa, kind, rows, cols):
+    """Eight rows run on the thin kernels and nine on the matrix cores: the larger batch must not be less precise.  The
+    2-norms of thousands of independent errors are within a few percent of their expectation, hence the tenth."""
+    from frink_amd import synth
+    # (encoded rows, whose offsets and scaled codes nearly cancel as a checkpoint's do)
+    distinct = fo.encode_matrix(kind, synth.weights(5 + kind, 160, cols))
+    data = np.resize(distinct.reshape(160, -1), (rows, distinct.size // 160)).reshape(-1)
+    x = synth.activations(9, 9, cols, outlier_frac=0.002)
+    q, d, _ = fo.quantize_q8_k(x.reshape(-1))
+    a = (q.reshape(-1, 256).astype(np.float64) * d.reshape(-1, 1).astype(np.float64)).reshape(9, cols)
+    exact = a @ fo.dequant(kind, distinct).reshape(160, cols).astype(np.float64).T
+    w = fa.Weights.from_host(kind, data, rows, cols)
+    nine = np.linalg.norm(w.gemm(to_dev(x)).cpu().numpy()[:8, :160] - exact[:8])
+    eight = np.linalg.norm(w.gemm(to_dev(x[:8])).cpu().numpy()[:, :160] - exact[:8])
+    w.release()
+    assert nine <= 1.1 * eight, (nine, eight)
