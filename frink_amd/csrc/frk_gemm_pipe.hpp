@@ -37,6 +37,7 @@ struct GemmArgs {
     int row_tiles, tok_tiles;
     int k_split;     // 1 .. 8 parts of a row's blocks; with more than one each writes its sums to `partial`
     float *partial;  // [k_split][M][rows], added up in order afterwards (launch_sum_parts)
+    int parts_inner; // a row tile's parts next to each other in the work list
 };
 
 // One block of a lane's weight row as MFMA B operands: the two pre-scaled planes of the 8 sub-blocks,
@@ -665,15 +666,17 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     const int li = lane & 31, lg = lane >> 5;
     const int rg = wave % RG, ks = wave / RG;
 
-    // An XCD takes an equal run of the list (part, row tile, token tile): its workgroups share weight rows and, where the
+    // An XCD takes an equal run of the list (part, row tile, token tile), or (row tile, part, token tile): its workgroups share weight rows and, where the
     // blocks are split, the activations of a part or two.  (With XCD x given the row tiles congruent to x mod 8, the busiest
     // one had a round more than the others wherever their number does not divide by eight: 2440 x 12032 in Q5_K at 146
     // tokens, 20 row tiles, 53 -> 33 us; and with the parts in the middle of the list every XCD reads all activations: 1025
-    // x 13056 in Q4_K at 105 tokens in eight parts 23.4 -> 21.1.)
+    // x 13056 in Q4_K at 105 tokens in eight parts 23.4 -> 21.1.  parts_inner: see pipe_args.)
     const int entry = deal_entry((int)blockIdx.x, g.row_tiles * g.tok_tiles * g.k_split);
     if (entry < 0) return;  // uniform per workgroup
-    const int tile = entry / g.tok_tiles, part = tile / g.row_tiles;
-    const int row_tile = tile - part * g.row_tiles, tok0 = (entry - tile * g.tok_tiles) * TM;
+    const int tile = entry / g.tok_tiles, inner = g.parts_inner ? g.k_split : g.row_tiles;
+    const int high = tile / inner, low = tile - high * inner;
+    const int part = g.parts_inner ? low : high, row_tile = g.parts_inner ? high : low;
+    const int tok0 = (entry - tile * g.tok_tiles) * TM;
     const int nb = g.nb;
     // this workgroup multiplies blocks kb0 .. kb1 - 1, its KS shares `steps` consecutive ones each (a
     // share that runs out of blocks idles through its last steps)
@@ -928,6 +931,10 @@ inline GemmArgs pipe_args(const frk_weights *w, Q8KTiled acts, size_t M, float *
     g.tok_tiles = (int)((M + p.tok_wg - 1) / p.tok_wg);
     g.k_split = p.k_split;
     g.partial = partial;
+    // A part of a Q6_K row is four runs that end inside cache lines (scales and d a few bytes each: 13 lines for 9 lines'
+    // worth of an eighth of 43 blocks): with few activations its row's parts share an L2 instead (4096x11008 at 13 rows 23.7
+    // -> 22.7 us; 9 .. 32 rows of 79 drawn matrices 0.2 % in the mean, 33 .. 128 rows would lose 0.8).
+    g.parts_inner = w->kind == FRK_KIND_Q6_K && M <= 32;
     return g;
 }
 
