@@ -655,6 +655,8 @@ bool gemm_q4_k_stream_gathers(size_t src_rows, size_t cols) {
 int launch_gemm_k_stream(const frk_weights *w0, const frk_weights *w1, size_t rows_e, Q8KTiled a,
                             const Q8KRows *src, const int *gather, const int4 *tiles, const int *n_tiles,
                             int max_tiles, float *y0, float *y1, hipStream_t s) {
+    if ((w0->kind != FRK_KIND_Q4_K && w0->kind != FRK_KIND_Q6_K) || (w1 && w1->kind != w0->kind))
+        return set_error(FRK_ERR_UNSUPPORTED, "the grouped K-quant GEMM takes Q4_K or Q6_K stacks (kinds %d and %d)", w0->kind, w1 ? w1->kind : w0->kind);
     StreamArgs g;
     g.W[0] = w0->dev;
     g.W[1] = w1 ? w1->dev : w0->dev;

@@ -537,10 +537,12 @@ struct WeightSide {  // Q4_K, Q5_K: the rows' 9 or 11 sixteen-byte pieces back t
         ScalePairs p;
     };
     static __device__ __forceinline__ Scales scales(const Raw &R, int) {
+        static_assert(!Q5, "in pieces: Q4_K's planes only");
         const BlockScales s = block_scales(R.wh);
         return {s, scale_pairs(s)};
     }
     static __device__ __forceinline__ void unpack_piece(int i, const Raw &R, const Scales &c, int lg, int, BPlanes &B) {
+        static_assert(!Q5, "in pieces: Q4_K's planes only");
         if (i == 0) unpack_pair_free(R.q0, c.p.p0, c.p.p1, B.H0, B.L0, B.H1, B.L1);
         if (i == 2) unpack_pair_free(R.q1, c.p.p2, c.p.p3, B.H2, B.L2, B.H3, B.L3);
         if (i == 4) unpack_pair_free(R.q2, c.p.p4, c.p.p5, B.H4, B.L4, B.H5, B.L5);
