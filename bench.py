@@ -613,7 +613,7 @@ def main():
             for w in experts:
                 w.release()
             # a layer of MXFP4 experts in gpt-oss-20b's shape (32 experts, top-4, 2880/2880), 512 tokens: the experts
-            # decoded to signed bytes per call, the grouped form of the Q8_0 matrix-core kernel
+            # as they are stored on the block-scaled matrix cores
             E4, K4, H4, F4 = 32, 4, 2880, 2880
             ex4 = [fa.Weights.from_device(fa.MXFP4, torch.from_numpy(random_blocks(fa.MXFP4, r, c, seed=90 + j)).to(dev), r, c)
                    for j, (r, c) in enumerate(((E4 * F4, H4), (E4 * F4, H4), (E4 * H4, F4)))]

@@ -19,8 +19,8 @@
 // l % 32, the 16 k-values 16*(l/32) .. +15 (8*(l/32) .. +7 for the K=16 f16 form); result register
 // r of lane l is D[8*(r/4) + 4*(l/32) + r%4][l % 32].
 //
-// Data movement: everything a block needs -- the workgroup's 128 weight rows (raw 144-byte blocks)
-// and its activation tile -- goes from global memory straight into LDS with global_load_lds_dwordx4
+// Data movement: everything a block needs -- the workgroup's weight rows (raw blocks) and its
+// activation tile -- goes from global memory straight into LDS with global_load_lds_dwordx4
 // (the 64 lanes' 16-byte pieces land in 1 KB of consecutive LDS; each lane chooses which piece it
 // fetches, so the LDS image is whatever order the consumer wants), several blocks ahead, in rings of
 // stages.  No prefetch lives in registers, and the only waits on memory are "the stage issued P

@@ -196,8 +196,6 @@ __device__ __forceinline__ void unpack_pair_sel(const v4i q, uint32_t pair0, uin
 }
 // The same in plain vector arithmetic (the compiler finds the op_sel forms itself), for a kernel that leaves
 // the place of the unpacking to the compiler: statements of inline assembly stay where they are written.
-// The same in plain vector arithmetic (the compiler finds the op_sel forms itself), for a kernel that leaves
-// the place of the unpacking to the compiler: statements of inline assembly stay where they are written.
 __device__ __forceinline__ void unpack_pair_free(const v4i q, uint32_t pair0, uint32_t pair1, v4i &H0, v4i &L0, v4i &H1, v4i &L1) {
     us2 p0, p1;
     __builtin_memcpy(&p0, &pair0, 4);

@@ -216,14 +216,14 @@ struct Q8KRows {
 };
 size_t q8k_tiled_bytes(size_t rows, size_t cols);
 Q8KTiled q8k_tiled_carve(void *base, size_t rows, size_t cols);
-// out row r = x[r] quantized, r < rows; the rest of the last tile becomes zeros
 // Q8KActs to be written; null pointers: none wanted
 struct Q8KActsOut {
     int8_t *q = nullptr;
     float *d = nullptr;
     int16_t *bsums = nullptr;
 };
-// (`plain`: the same quants as plain rows too)
+// out row r = x[r] quantized, r < rows; the rest of the last tile becomes zeros (`plain`: the same quants as plain rows
+// too)
 int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTiled out, hipStream_t s, Q8KActsOut plain = Q8KActsOut());
 // out row r = x[gather[r]] quantized (zeros where gather[r] < 0), for the 32-row records of the first
 // max_rows rows whose first entry is not negative
@@ -239,8 +239,8 @@ size_t pipe_gemm_parts_bytes(int kind, size_t M, size_t cols, size_t rows);
 int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, hipStream_t s);
 // y[n] = partial[0][n] + partial[1][n] + ... in that order (the split GEMMs' second step; frk_gemm_q6.hip)
 int launch_sum_parts(const float *partial, int parts, size_t n, float *y, hipStream_t s);
-// the same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time
-// its form over large tiles (frk_gemm_q8_pipe.hip): weight rows x tokens of a workgroup, and how many workgroups share a
+// The same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time.
+// Its form over large tiles (frk_gemm_q8_pipe.hip): weight rows x tokens of a workgroup, and how many workgroups share a
 // row's columns; rows_wg = 0: the other kernel
 struct Q8PipePlan {
     int rows_wg, tok_wg, k_split;
@@ -289,7 +289,7 @@ int units_decoded(const frk_weights *w, uint8_t *room, hipStream_t s, const uint
 size_t grouped_units_workspace_bytes(int kind, size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs, size_t cols);
 int launch_gemm_grouped_units(const frk_weights *w, size_t n_groups, const int32_t *group_off, const int32_t *gather, const float *x,
                               size_t x_rows, size_t pairs, float *y, void *ws, hipStream_t s);
-// MoE layer over Q5_0 / IQ4_XS / MXFP4 experts by bucket, on the matrix cores (32 tokens and more)
+// MoE layer over Q5_0 / IQ4_XS / MXFP4 experts by bucket, on the matrix cores (32 tokens and more; MXFP4 earlier)
 bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts, size_t batch,
                                   int k);
 size_t moe_units_grouped_workspace_bytes(int gate_kind, int down_kind, size_t batch, int k, int n_experts, int hidden, int ffn);

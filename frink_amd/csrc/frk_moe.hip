@@ -761,14 +761,15 @@ int launch_moe_ffn_units(const frk_weights *gate, const frk_weights *up, const f
     return FRK_OK;
 }
 
-// The same layer from 32 tokens on (MXFP4: moe_units_takes_grouped_path), when every projection's kind has a decoded form the matrix cores read (Q5_0;
-// MXFP4 with scales that are f16 values; IQ4_XS): the reference's bucket path (crates/frink-models/src/decoder/
-// ffn_batch.rs:343-434) -- the pairs bucketed by expert, every expert's rows read once.  MXFP4 experts go to the
-// block-scaled matrix cores as they are (frk_gemm_mx.hip); the others are decoded into signed bytes in the call's scratch
-// memory for the grouped form of the Q8_0 matrix-core kernel.  The
+// The same layer from 32 tokens on (MXFP4: moe_units_takes_grouped_path), when every projection's kind has a decoded form
+// the matrix cores read (Q5_0; MXFP4 with scales that are f16 values; IQ4_XS): the reference's bucket path
+// (crates/frink-models/src/decoder/ffn_batch.rs:343-434) -- the pairs bucketed by expert, every expert's rows read once.
+// MXFP4 experts go to the block-scaled matrix cores as they are (frk_gemm_mx.hip: rows of 384 columns and more); the others
+// are decoded into signed bytes in the call's scratch memory for the grouped form of the Q8_0 matrix-core kernel.  The
 // activations are quantized per token (gate and up) and per grouped row (down) exactly as the per-pair jobs
-// quantize them, and the integers are the same: the two paths differ in the order of the float additions only.
-// which projections multiply MXFP4 experts as they are (frk_gemm_mx.hip): no decoded copy, gate and up in one launch
+// quantize them, and the products are the same: the two paths differ in the float additions only.
+
+// Which projections multiply MXFP4 experts as they are (frk_gemm_mx.hip): no decoded copy, gate and up in one launch
 struct UnitsNative {
     bool gate_up, down;
 };

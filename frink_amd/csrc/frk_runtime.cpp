@@ -620,7 +620,7 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
 // From how many rows on a batch takes the matrix-core GEMM, whose cost is flat up to 64 rows; below that the thin
 // kernels' groups of 16 (Q4_K, Q5_K) or 8 rows are ahead, by what a group costs at the matrix's shape.  Measured with
 // quantization (us; thin / GEMM), nb blocks a row, rules beyond 17 / 33 / 41 rows within 32768 columns:
-//   Q4_K  nb > 32, where a thin launch holds 8 rows: 4096x11008 at 8, 9, 16 rows 14.8 / 19.7, 21.9 / 19.4, 25.3 / 19.7;
+//   Q4_K  a thin launch holds 8 rows from 32 blocks on.  nb > 32: 4096x11008 at 8, 9, 16 rows 14.8 / 19.7, 21.9 / 19.4, 25.3 / 19.7;
 //         1024x14336 at 9, 16 23.5 / 18.8, 28.0 / 19.2.  nb 24 .. 32 past one workgroup a CU: 5120x6144 at 9, 16 19.3 /
 //         16.2, 20.7 / 16.8, 14336x8192 38.7 / 27.7, 44.8 / 27.2, but 2048x8192 14.1 / 15.6, 14336x6144
 //         18.8 / 24.2.  Then by size: 14336x4096 at 17 20.4 / 19.6; 4096x4096 at 17, 32 13.3 / 14.8, 13.3 / 16.1.
@@ -630,14 +630,18 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
 //   Q6_K  odd nb (not the streamed thin kernel's): 4096x11008 at 8, 9, 24 rows 18.3 / 24.3, 28.9 / 24.2, 42.1 / 25.2;
 //         2048x11008 at 16, 17, 33 17.4 / 23.4, 27.3 / 23.1, 39.1 / 24.6.  Even: 4096x14336 at 16, 17 22.5 / 27.4, 28.9 / 27.6;
 //         5120x8192 at 17, 25 23.2 / 23.8, 35.0 / 25.1; 8192x4096 at 17, 25 20.4 / 21.2, 25.0 / 22.1; 4096x4096 at 40 15.3 / 19.6.
+// Of 480 drawn matrices of 1024 .. 14336 rows and 2048 .. 14336 columns at 8 .. 40 rows, 273 take the GEMM here: the thin
+// kernels are ahead by more than 2 % for four of them, Q5_K of 8 .. 12 blocks past 33 rows (12 % at most).  Of the 207 that
+// stay, the GEMM would be ahead by more than 5 % for 52, most of them Q6_K of few rows and odd nb (1.8 times at most).
 // (No matrix starts below tiled_from(cols): a batch quantized without knowing its matrices has tiles from there on.)
 static size_t tiled_from(size_t cols) { return cols >= 24 * QK_K ? 9 : 17; }
 static size_t matrix_cores_from(const frk_weights *w) {
     const size_t n = w->rows * w->cols, nb = w->cols / QK_K;
     const bool measured = nb <= 128;
     if (w->kind == FRK_KIND_Q4_K) {
-        if (measured && (nb > 32 || (nb >= 24 && w->rows > 4096 && (nb == 32 || w->rows <= 8192)))) return 9;
-        return n > (size_t)20 << 20 || thin_gemm_max_batch(w) < 16 ? 17 : 33;
+        const bool eights = thin_gemm_max_batch(w) < 16;
+        if (measured && (nb > 32 || (nb >= 24 && w->rows > 4096 && (eights || w->rows <= 8192)))) return 9;
+        return n > (size_t)20 << 20 || eights ? 17 : 33;
     }
     if (w->kind == FRK_KIND_Q5_K) return measured && nb >= 32 ? 9 : measured && nb >= 16 && w->rows <= 6144 ? 17 : 33;
     if (w->kind != FRK_KIND_Q6_K) return SIZE_MAX;

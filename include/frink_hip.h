@@ -118,7 +118,8 @@ int frk_hip_weights_from_device(int kind, const void *dev_bytes, size_t len, siz
 int frk_hip_weights_release(frk_weights *w);
 /* Q5_0 / IQ4_XS / MXFP4 (scale bytes within 104..143) reach the matrix cores decoded to signed bytes; a batched call
  * (frk_hip_gemm_dev from four rows on, frk_hip_gemm_grouped_dev, frk_hip_moe_ffn_dev from 32 tokens on) decodes
- * into its scratch memory each time.  This keeps the decoded rows beside the resident ones until the handle is
+ * into its scratch memory each time -- but for MXFP4 groups and experts with rows of 384 columns and more, which
+ * are multiplied as they are stored.  This keeps the decoded rows beside the resident ones until the handle is
  * released -- twice the bytes of a Q8_0 matrix of that shape, for a part with HBM to spare -- and those calls skip
  * the decoding (same results, bit for bit).  Decodes on `stream` and synchronizes it.  The reference has no
  * counterpart: its GPU GEMM dequantizes inside the kernel (crates/frink-cuda/src/mul_mm.rs:146-205).  Other kinds:
@@ -278,9 +279,10 @@ int frk_hip_route_top_k_softmax_dev(const float *logits_dev, size_t batch, size_
  * crates/frink-moe/src/lib.rs:1246-1263).  gate/up/down hold the experts stacked row-wise
  * (expert e = rows [e*ffn, (e+1)*ffn) of gate and up, [e*hidden, (e+1)*hidden) of down); gate and up
  * are Q4_K, down is Q4_K or Q6_K; or all three of Q5_0 / IQ4_XS / MXFP4 (gate and up of one kind): below 32 tokens
- * every (token, slot) pair runs on the integer decode kernel of its kind, from 32 on the pairs are bucketed by
- * expert and the experts, decoded to signed bytes in scratch memory, run on the grouped matrix-core kernel (an MXFP4
- * stack with scale bytes outside 104..143 keeps the per-pair jobs).  Other combinations: FRK_ERR_UNSUPPORTED.
+ * every (token, slot) pair runs on the integer decode kernel of its kind (MXFP4: until there are two pairs an expert
+ * and 32 pairs), from there on the pairs are bucketed by expert and the experts run on a grouped matrix-core kernel,
+ * decoded to signed bytes in scratch memory or (MXFP4 rows of 384 columns and more) as they are stored; an MXFP4
+ * stack with scale bytes outside 104..143 keeps the per-pair jobs.  Other combinations: FRK_ERR_UNSUPPORTED.
  * ids[batch][k] / weights[batch][k] are a RoutingDecision per token (lib.rs:112-115); an id outside
  * [0, n_experts) contributes nothing. */
 int frk_hip_moe_ffn_dev(const frk_weights *gate, const frk_weights *up, const frk_weights *down,
@@ -291,7 +293,7 @@ int frk_hip_moe_ffn_dev(const frk_weights *gate, const frk_weights *up, const fr
  * enqueue_mul_mm_grouped_dev (crates/frink-cuda/src/mul_mm_launch.rs:391-470) and enqueue_mmq_grouped
  * (crates/frink-cuda/src/mmq/mod.rs:144-217).  Group g's matrix is rows [g*R, (g+1)*R) of `stacked` (R = rows /
  * n_groups; the reference's table[g], here one resident stack), Q4_K or Q6_K, or Q5_0 / IQ4_XS / MXFP4 with scale
- * bytes within 104..143 (decoded to signed bytes per call); others: FRK_ERR_UNSUPPORTED;
+ * bytes within 104..143 (decoded to signed bytes per call; MXFP4 rows of 384 columns and more as they are stored); others: FRK_ERR_UNSUPPORTED;
  * group_off_dev[n_groups + 1] are non-decreasing pair indices from 0 to pairs; pair p of group g reads activation
  * row gather_dev[p] of x_dev[x_rows][cols] (row p when gather_dev is null) and writes y_dev[p][R] -- every pair of
  * every group, no gaps.  Everything is read on the device, so the call can follow the kernel that built the

@@ -425,7 +425,7 @@ def test_q5_k_decode_and_batches_at_full_size(fa):
     arbitrary block bytes (every bit pattern of the fifth-bit plane) against the oracle on slices of
     rows, for one row (the decode kernel), 3, 16, 17 and 32 rows (the thin matrix-core kernel: 16 rows
     a workgroup, wider batches as a grid of 16-row groups in one launch), 33, 70 and 512 rows (the tiled
-    matrix-core kernel with the fifth bits as a third int8 plane, its blocks split between workgroups for
+    matrix-core kernel, a scaled code's two bytes as its int8 planes, its blocks split between workgroups for
     the small batches), and the whole output of a row against dequantized weights in float64."""
     from frink_amd import synth
     rows, cols = 14336, 4096
@@ -802,8 +802,8 @@ def test_grouped_gemm_over_more_rows_than_the_gathering_kernel_addresses(fa):
 @pytest.mark.parametrize("kind,cols", [(fo.Q5_0, 96), (fo.MXFP4, 2880), (fo.IQ4_XS, 768), (fo.MXFP4, 256)])
 @pytest.mark.parametrize("with_gather", [True, False])
 def test_grouped_gemm_over_the_other_kinds(fa, kind, cols, with_gather):
-    """The grouped entry over stacks of Q5_0 / MXFP4 / IQ4_XS matrices: the stack decoded to signed bytes per call, the
-    activation rows quantized once (Q8_0 blocks; Q8_K for IQ4_XS), the grouped matrix-core kernel gathering through the
+    """The grouped entry over stacks of Q5_0 / MXFP4 / IQ4_XS matrices: the stack decoded to signed bytes per call (MXFP4
+    rows of 384 columns and more: as they are), the activation rows quantized once (Q8_0 blocks; Q8_K for IQ4_XS), the grouped matrix-core kernel gathering through the
     list -- every pair against the integer tier of its kind (q8_row_dot / q8k_row_dot,
     crates/frink-core/src/weight_matrix.rs:392-420)."""
     from frink_amd import synth
@@ -839,8 +839,8 @@ def test_grouped_gemm_over_the_other_kinds(fa, kind, cols, with_gather):
 @pytest.mark.parametrize("kind", [fo.Q5_0, fo.IQ4_XS, fo.MXFP4])
 def test_a_kept_decoded_copy_changes_no_bit(fa, kind):
     """frk_hip_weights_keep_decoded: the batched GEMM, the grouped GEMM and the MoE layer read the kept rows instead of
-    decoding per call -- the same kernels over the same bytes, so every output bit is the same; kinds without a decoded
-    form are refused."""
+    decoding per call (MXFP4 groups of 384 columns and more read the codes either way) -- the same kernels over the same
+    bytes, so every output bit is the same; kinds without a decoded form are refused."""
     from frink_amd import synth
     import torch
     E, k, hidden, ffn, batch = 4, 2, 512, 256, 70
@@ -1122,9 +1122,10 @@ def test_moe_ffn_with_experts_of_the_other_kinds(fa, gate_kind, down_kind, n_exp
     """Experts in MXFP4 / Q5_0 / IQ4_XS (run_expert takes any WeightMatrix, crates/frink-moe/src/lib.rs:1068-1165):
     every (token, slot) pair on the integer tier of its kind, the slots added in the reference's order for the batch
     size (routing order below 32 tokens, ascending expert id from 32 on), an id outside the experts left out.  Below 32
-    tokens a decode job per pair; from 32 on the pairs bucketed by expert and the experts, decoded to signed bytes, on
-    the grouped matrix-core kernel (tiles of every fill, several tiles an expert, experts nobody chose, rows that are
-    not a multiple of the kernel's 256-column step)."""
+    tokens a decode job per pair (MXFP4: until two pairs an expert and 32 pairs); from there on the pairs bucketed by
+    expert and the experts on a grouped matrix-core kernel, decoded to signed bytes or (MXFP4 rows of 384 columns and
+    more) as they are (tiles of every fill, several tiles an expert, experts nobody chose, rows that are not a multiple
+    of the kernel's 256-column step)."""
     from frink_amd import synth
     print("moe, other kinds", gate_kind, down_kind, n_experts, k, hidden, ffn, batch, flush=True)
     gate = _other_kind_blocks(gate_kind, n_experts * ffn, hidden, seed=41)
@@ -1781,7 +1782,7 @@ def test_dev_calls_on_two_streams_from_two_threads(fa):
     ((fo.Q4_K, fo.Q4_K), (96, 256), 2048, 40),     # the blocks split between workgroups: each GEMM its own parts
     ((fo.Q4_K, fo.Q4_K), (64, 64), 512, 8),        # thin kernel
     ((fo.Q4_K, fo.Q6_K), (128, 96), 1024, 64),     # kinds that do not share a quantized form
-    ((fo.Q5_K, fo.Q4_K), (200, 136), 1024, 70),    # Q5_K's three planes beside Q4_K's two, one quantization
+    ((fo.Q5_K, fo.Q4_K), (200, 136), 1024, 70),    # Q5_K's planes beside Q4_K's, one quantization
     ((fo.Q5_K, fo.Q5_K), (96, 160), 2048, 40),     # both with their blocks split
 ])
 def test_gemm_pair_is_two_gemms_over_one_quantization(fa, kinds, rows, cols, batch):
