@@ -2,11 +2,18 @@
 // block scales' outer product from the f16 matrix core, a conversion and a fused multiply-add per sum, blocks in order),
 // over larger tiles that come into LDS without passing through registers.
 //
-// What bounds it is the vector ALU: 32 instructions for a tile's two MFMAs.  A wavefront owns 32 weight rows and MT tiles
+// What bounds it is the issue of the vector ALU beside the matrix core: 32 instructions for a tile's two MFMAs, 64 ns a product
+// and SIMD alone (76 in this kernel; the chip holds about 2 GHz under it).  A wavefront owns 32 weight rows and MT tiles
 // of 32 tokens, so a weight fragment is read once for MT products (the kernel it replaces read two fragments a product and
 // moved 816 bytes a product through registers into LDS; 256 x 128 tiles move 408, and no instruction touches them).
 // The columns go by in halves of a chunk (128 columns, four blocks), three stages in LDS, requested two ahead, the
-// requests spread over the arithmetic; block scales come a chunk (256 columns) at a time.  One barrier a half chunk.
+// requests spread over the arithmetic; block scales come a chunk (256 columns) at a time.  One barrier a half chunk, and
+// the pipeline of reads, matrix instructions and float steps runs across it: started anew behind every barrier, the wait
+// for the first operands and products stood open on both wavefronts of a SIMD (2048 x 4096 x 14336 in tokens x rows x
+// columns, with quantization, 310 us; across 301; 512 x 14336 x 4096 87.7 -> 82.7, 200 x 11008 x 4096 46.3 -> 45.5, 512 x
+// 4096 x 14336 93.4 -> 90.9).  Tried beside it without gain: the conversion as a subtraction from a sum that starts at 1.5 *
+// 2^23 (302), the scales' MFMA in the middle of the float step (303), quants as f16 planes whose sums need no conversion
+// (the products alone 60 against 64 ns, for twice the LDS traffic).
 #include "frk_device.hpp"
 
 #include <type_traits>
@@ -113,74 +120,99 @@ __global__ __launch_bounds__(512, 2) void gemm_q8_0_pipe_kernel(Q8PipeArgs g) {
             for (int c = 0; c < R; c++) fetch_quants(h0 + ahead, c);
             filled();
         }
+    // ---- A three-stage pipeline over the products (block by block, its MT tiles in turn): the reads of product n + 2, the
+    // matrix core's work for n + 1, the float step of n.  It runs across the half chunks: the next one is waited for behind
+    // the last product's matrix instructions, its scales and first operands are read in front of the float step before.
+    constexpr int N = 4 * MT;
     int at = 0;
-    // MORE: half chunk h + 2 exists and is requested.  (Two copies of the body instead of branches in it: the compiler
-    // counts the wait states between an MFMA and a reader of its result within one basic block only.)
-    auto half_chunk = [&](auto more_c, int h) {
-        constexpr bool MORE = decltype(more_c)::value;
-        // half chunk h (and its chunk's scales) has landed; behind it only h + 1 was requested
+    const uint8_t *sw_lines, *sa_lines;
+    uint2 sw, sa[MT];  // the four blocks' scales, f16, two to a register; k = 0 of the outer product sits in lanes 0 .. 31
+    uint2 sw_next, sa_next[MT];
+    auto arrive = [&](int h) {
+        // half chunk h (and its chunk's scales) has landed, and everybody has read the one before; behind it only h + 1
+        // was requested
         if (h + 1 >= h1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         else if ((h & 1) && fetches_scales) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R + 1) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R) : "memory");
         lds_barrier();
-        if (MORE) fetch_scales(h + 2);
-        const uint8_t *st = qp_lds + (size_t)at * L::STAGE, *sw_lines = st + rg * 32 * 128, *sa_lines = st + (L::ROWS + tg * MT * 32) * 128;
+        const uint8_t *st = qp_lds + (size_t)at * L::STAGE;
+        at = at == L::STAGES - 1 ? 0 : at + 1;
+        sw_lines = st + rg * 32 * 128;
+        sa_lines = st + (L::ROWS + tg * MT * 32) * 128;
         const uint8_t *sc = qp_lds + L::OFF_SCALES + ((h >> 1) & 1) * L::SCALES + (h & 1) * 8;
-        // the four blocks' scales, f16, two to a register; k = 0 of the outer product sits in lanes 0 .. 31
-        const int live = g.nb - 4 * h;  // blocks of the row from here on: a row's scales past its end are whatever lies there
-        uint2 sw = *reinterpret_cast<const uint2 *>(sc + (rg * 32 + li) * 16);
-        sw.x = lg ? 0u : sw.x & (live > 1 ? 0xffffffffu : 0xffffu);
-        sw.y = lg ? 0u : sw.y & (live > 3 ? 0xffffffffu : live > 2 ? 0xffffu : 0u);
-        uint2 sa[MT];
+        sw_next = *reinterpret_cast<const uint2 *>(sc + (rg * 32 + li) * 16);
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
-            sa[t] = *reinterpret_cast<const uint2 *>(sc + (L::ROWS + (tg * MT + t) * 32 + li) * 16);
-            sa[t].x = lg ? 0u : sa[t].x;
-            sa[t].y = lg ? 0u : sa[t].y;
-        }
-        auto k0 = [](uint2 s, int b) {  // {scale of block b, 0, 0, 0}
-            const uint32_t w = b < 2 ? s.x : s.y;
-            const uint2 u = make_uint2(b & 1 ? w >> 16 : w & 0xffffu, 0u);
-            qp_v4h v;
-            __builtin_memcpy(&v, &u, 8);
-            return v;
-        };
-        // A three-stage pipeline over the products (block by block, its MT tiles in turn): the reads of product n + 2, the
-        // matrix core's work for n + 1, the float step of n.
-        constexpr int N = 4 * MT;
-        auto read_w = [&](int b) { return *reinterpret_cast<const qp_v4i *>(sw_lines + piece[b]); };
-        auto read_a = [&](int n) { return *reinterpret_cast<const qp_v4i *>(sa_lines + (n % MT) * 4096 + piece[n / MT]); };
-        qp_v4i w1 = read_w(0), w2 = MT > 1 ? w1 : read_w(1), a1 = read_a(0), a2 = read_a(1);
-        qp_v16i isum_next = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, w1, zero_i, 0, 0, 0);
-        qp_v16f scale_next = __builtin_amdgcn_mfma_f32_32x32x8f16(k0(sa[0], 0), k0(sw, 0), zero_f, 0, 0, 0);
-        a1 = a2, w1 = w2;
-        __builtin_amdgcn_sched_barrier(0);
+        for (int t = 0; t < MT; t++) sa_next[t] = *reinterpret_cast<const uint2 *>(sc + (L::ROWS + (tg * MT + t) * 32 + li) * 16);
+    };
+    auto use_scales = [&](int h) {
+        const int live = g.nb - 4 * h;  // blocks of the row from here on: a row's scales past its end are whatever lies there
+        const uint32_t both = lg ? 0u : 0xffffffffu;
+        sw.x = sw_next.x & (live > 1 ? both : both & 0xffffu);
+        sw.y = sw_next.y & (live > 3 ? both : live > 2 ? both & 0xffffu : 0u);
+#pragma unroll
+        for (int t = 0; t < MT; t++) sa[t] = make_uint2(sa_next[t].x & both, sa_next[t].y & both);
+    };
+    auto k0 = [](uint2 s, int b) {  // {scale of block b, 0, 0, 0}
+        const uint32_t w = b < 2 ? s.x : s.y;
+        const uint2 u = make_uint2(b & 1 ? w >> 16 : w & 0xffffu, 0u);
+        qp_v4h v;
+        __builtin_memcpy(&v, &u, 8);
+        return v;
+    };
+    auto read_w = [&](int b) { return *reinterpret_cast<const qp_v4i *>(sw_lines + piece[b]); };
+    auto read_a = [&](int n) { return *reinterpret_cast<const qp_v4i *>(sa_lines + (n % MT) * 4096 + piece[n / MT]); };
+    qp_v4i w1, w2, a1, a2;
+    qp_v16i isum_next;
+    qp_v16f scale_next;
+    auto multiply = [&](int n) {
+        isum_next = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, w1, zero_i, 0, 0, 0);
+        scale_next = __builtin_amdgcn_mfma_f32_32x32x8f16(k0(sa[n % MT], n / MT), k0(sw, n / MT), zero_f, 0, 0, 0);
+    };
+    // MORE: half chunk h + 2 exists and is requested, NEXT: h + 1 exists.  (Copies of the body instead of branches in it:
+    // the compiler counts the wait states between an MFMA and a reader of its result within one basic block only; over the
+    // loop's edge 32 vector instructions lie between the two.)
+    auto half_chunk = [&](auto more_c, auto next_c, int h) {
+        constexpr bool MORE = decltype(more_c)::value, NEXT = decltype(next_c)::value;
+        if (MORE) fetch_scales(h + 2);
 #pragma unroll
         for (int n = 0; n < N; n++) {
             const qp_v16i isum = isum_next;
             const qp_v16f scale = scale_next;
+            if (n == N - 1 && NEXT) use_scales(h + 1);
             if (n + 2 < N) {
                 a2 = read_a(n + 2);
                 w2 = (n + 2) % MT == 0 ? read_w((n + 2) / MT) : w1;
             }
-            if (n + 1 < N) {
-                isum_next = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, w1, zero_i, 0, 0, 0);
-                scale_next = __builtin_amdgcn_mfma_f32_32x32x8f16(k0(sa[(n + 1) % MT], (n + 1) / MT), k0(sw, (n + 1) / MT), zero_f, 0, 0, 0);
+            if (n + 1 < N || NEXT) multiply((n + 1) % N);
+            if (n % (N / R) == 0 && n / (N / R) < R && MORE) fetch_quants(h + 2, n / (N / R));
+            if (n == N - 2 && MORE) filled();
+            if (n + 2 >= N && NEXT) {
+                if (n == N - 2) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    arrive(h + 1);
+                }
+                a2 = read_a(n + 2 - N);
+                w2 = (n + 2 - N) % MT == 0 ? read_w((n + 2 - N) / MT) : w1;
             }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[n % MT][r] = __builtin_fmaf(scale[r], (float)isum[r], acc[n % MT][r]);
             asm volatile("" : "+v"(acc[n % MT]));  // (the float step stays here: sunk to the end, every product's sums are alive at once)
-            if (n % (N / R) == 0 && n / (N / R) < R && MORE) fetch_quants(h + 2, n / (N / R));
             __builtin_amdgcn_sched_barrier(0);
             a1 = a2, w1 = w2;
         }
-        static_assert(R <= N, "at most a request a product");
-        if (MORE) filled();
-        at = at == L::STAGES - 1 ? 0 : at + 1;
+        static_assert((R - 1) * (N / R) <= N - 2, "a half chunk's requests in front of the next one's wait");
     };
     int h = h0;
-    for (; h + 2 < h1; h++) half_chunk(std::true_type(), h);
-    for (; h < h1; h++) half_chunk(std::false_type(), h);
+    arrive(h0);
+    use_scales(h0);
+    a1 = read_a(0), w1 = read_w(0);
+    a2 = read_a(1), w2 = MT > 1 ? w1 : read_w(1);
+    multiply(0);
+    a1 = a2, w1 = w2;
+    for (; h + 2 < h1; h++) half_chunk(std::true_type(), std::true_type(), h);
+    if (h + 1 < h1) half_chunk(std::false_type(), std::true_type(), h++);
+    half_chunk(std::false_type(), std::false_type(), h);
 
     // register r of a lane: token 8 * (r / 4) + 4 * (lane / 32) + r % 4 of the tile, weight row lane % 32
     const int row = row0 + rg * 32 + li;
