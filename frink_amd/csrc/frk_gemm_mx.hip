@@ -60,21 +60,24 @@ int launch_quantize_mx(const float *x, size_t rows, size_t cols, const int *used
     return FRK_OK;
 }
 
-// ---- the GEMM.  A workgroup of NW wavefronts multiplies one tile (at most 64 activation rows of one group, two halves
+// ---- the GEMM.  A workgroup of NW wavefronts multiplies one tile (at most 96 activation rows of one group, halves
 // of 32) with 64 weight rows a wavefront, as two groups of 32: of one matrix, or (GLU) the same rows of gate and up,
 // whose results meet in the epilogue as silu(gate) * up.
 //
 // The columns go by four blocks at a time: step s (0, 1) multiplies blocks s and 2 + s, a lane block s or 2 + s of its
-// row by its half (k = 64).  Everything comes straight into LDS, two quads of blocks ahead: the activations' digits (25 KB)
-// into a ring of three stages that the workgroup shares, with one barrier a quad; the weights into a wavefront's own two
-// slots, their scale bytes four quads at a time.
-// A quad takes about 2.4 us: 64 products a SIMD at the 24 ns that a chain of E2M3 x E2M1 products alone was measured at
-// are 1.5, its 60 KB on their way into LDS most of the rest (1.9 us without them).  So neighbouring lanes of a request
+// row by its half (k = 64).  Everything comes straight into LDS: the activations' digits (37 KB) into two stages that the
+// workgroup shares, a quad refilled as soon as everybody has read it, with one barrier a quad; the weights two quads of
+// blocks ahead into a wavefront's own two slots, their scale bytes four quads at a time.
+// A quad of a full tile takes about 2.9 us: 96 products a SIMD at the 22 ns that a chain of E2M3 x E2M1 products alone was
+// measured at (the chip holds 1.6 GHz under it) are 2.1; without its requests 2.5.  So neighbouring lanes of a request
 // fetch neighbouring pieces of memory (384 bytes of digits, 64 of codes a row), the LDS images are swizzled so that a
 // fragment's reads -- one piece of sixteen rows each -- fall in different banks, and the requests are spread over the
 // arithmetic.  Gate and up of 32 experts of 2880 x 2880 over 2048 pairs: weights loaded into registers, a row a lane, 227
 // us; weights in LDS but a lane per activation row 208; every request at the head of its quad 181; operands of the next
-// quad read behind the barrier instead of in front of the last step 171; as it is now 164 (the bytes from memory take 50).
+// quad read behind the barrier instead of in front of the last step 171; tiles of 64 rows 152-159; tiles of 96 rows (half of
+// the experts have more than 64 pairs and read their weights a second time for a few rows otherwise) 145, with silu ahead of
+// the stores 142, an XCD's last jobs cut in two 132; the down projection 90 -> 72 (the bytes from memory take 50 and 27).
+// A step's operands are read in two parts of twelve registers, as three halves' sums leave no room for a second step's.
 // Eight wavefronts a workgroup where that still fills the chip: a stage of digits then serves twice the rows (the down
 // projection 137 -> 97 us). ----
 struct MxGemmArgs {
@@ -89,13 +92,15 @@ struct MxGemmArgs {
     float *y;
 };
 constexpr int MX_ROW = 4 * MX_BLOCK_BYTES;             // an activation row's digits of one quad, 24 pieces
-constexpr int MX_STAGE_SCALES = 64 * MX_ROW;           // [64 rows][4 blocks] dwords
-constexpr int MX_STAGE = MX_STAGE_SCALES + 64 * 16;
-constexpr int MX_STAGES = 3;
+constexpr int MX_STAGE_SCALES = MX_TILE * MX_ROW;      // [MX_TILE rows][4 blocks] dwords
+constexpr int MX_STAGE = MX_STAGE_SCALES + MX_TILE * 16;
+constexpr int MX_STAGES = 2;
+constexpr int XCD_CUS = 32;
+static_assert(MX_TILE == 96, "three halves");
 constexpr int MX_W_SCALES = 2 * 4096;                  // two slots of codes [64 rows][4 blocks], two of scales [64 rows][16]
 constexpr int MX_W_WAVE = MX_W_SCALES + 2 * 1024;
 template <int NW>
-constexpr size_t mx_lds_bytes() { return (size_t)MX_STAGES * MX_STAGE + (size_t)NW * MX_W_WAVE; }
+constexpr size_t mx_lds_bytes() { return (size_t)MX_STAGES * MX_STAGE + (size_t)NW * MX_W_WAVE + sizeof(EXPF_TABLE); }
 static_assert(mx_lds_bytes<8>() <= 160 * 1024, "LDS of a CU");
 
 template <int NW, bool GLU>
@@ -103,20 +108,39 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
 #if defined(__HIP_DEVICE_COMPILE__)
     extern __shared__ __align__(16) uint8_t mx_lds[];
     uint8_t *const lds = mx_lds;
-    // the workgroups of a tile sit on one XCD (block id mod 8), whose L2 then serves the tile's digits
-    const int j = (int)blockIdx.x >> 3, t = ((int)blockIdx.x & 7) + 8 * (j / g.row_groups);
-    if (t >= *g.n_tiles) return;
+    // The workgroups of a tile sit on one XCD (block id mod 8), whose L2 then serves the tile's digits.  One workgroup fits a
+    // CU, so an XCD's jobs go in rounds of 32; where the last round is half empty, its jobs are cut in two: half the
+    // rows each, four wavefronts to the first tokens and four to the others of the same rows.
+    const int xcd = (int)blockIdx.x & 7, jobs = max(*g.n_tiles - xcd + 7, 0) / 8 * g.row_groups;
+    int j = (int)blockIdx.x >> 3, part = -1;
+    if (NW == 8) {
+        const int last = jobs % XCD_CUS;
+        if (last <= XCD_CUS / 2 && j >= jobs - last) {
+            part = (j - (jobs - last)) & 1;
+            j = jobs - last + ((j - (jobs - last)) >> 1);
+        }
+    }
+    if (j >= jobs) return;
+    const int t = xcd + 8 * (j / g.row_groups);
     const int4 tile = g.tiles[t];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int li = lane & 31, lg = lane >> 5;
     const int nb = g.nb, nbp = (nb + 7) & ~7;
     const int quads = (nb + 3) >> 2;
-    const bool two = tile.z > 32;
+    uint64_t *const expf_table = reinterpret_cast<uint64_t *>(lds + MX_STAGES * MX_STAGE + NW * MX_W_WAVE);
+    if (GLU && threadIdx.x < 32) expf_table[threadIdx.x] = EXPF_TABLE[threadIdx.x];  // (read behind the first barrier)
+    const int halves = (tile.z + 31) >> 5;  // of 32 rows, three at most
+    // this wavefront's: all of them; where a job's rows are cut in two, the first two (of two: one) or what is left
+    // (nothing left: the first again, not stored)
+    const int lower = halves > 2 ? 2 : 1;
+    const bool upper = part >= 0 && wave >= 4;
+    const int h_first = upper && halves > 1 ? lower : 0, h_count = part < 0 ? halves : upper ? max(halves - lower, 1) : lower;
+    const bool stores = !(upper && halves == 1);
 
     const uint32_t lds0 = lds_address(lds);
     // ---- weights: rows row0 + lane % 32 of the two groups.  Request c of a quad brings rows 16c .. 16c + 15 of the 64:
     // slot p of row r holds block p ^ (r / 4) % 4, so that the reads of one block of 32 rows fall in different banks.
-    const int row_wave = ((j % g.row_groups) * NW + wave) * (GLU ? 32 : 64), row0 = row_wave + li;
+    const int row_wave = ((j % g.row_groups) * NW + (part < 0 ? wave : part * 4 + (wave & 3))) * (GLU ? 32 : 64), row0 = row_wave + li;
     const uint8_t *const w_base[2] = {g.W + (size_t)tile.x * g.group_stride, (GLU ? g.W2 : g.W) + (size_t)tile.x * g.group_stride};
     auto weight_row = [&](int r) {  // row r of the wavefront's 64 as a row of its matrix
         return (uint32_t)min(GLU ? row_wave + (r & 31) : row_wave + r, g.rows - 1) * (uint32_t)g.row_stride;
@@ -139,40 +163,36 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
         else dma16(to, w_base[1] + at, w_scales_off);
     };
 
-    // ---- activations: a stage's digits are 64 rows of 24 pieces, piece s of row r in place s ^ (r / 2) % 8 (sixteen rows reading one
-    // piece each then touch sixteen different pieces of the 64 banks); each wavefront
-    // fetches its share of the 24 requests, the first one the scales too
-    constexpr int REQUESTS = 24 / NW;
-    static_assert(24 % NW == 0, "whole requests");
+    // ---- activations: a stage's digits are rows of 24 pieces, piece s of row r in place s ^ (r / 2) % 8 (sixteen rows reading one
+    // piece each then touch sixteen different pieces of the 64 banks).  A half is twelve requests, dealt out to the wavefronts;
+    // the first two fetch the scales.
+    constexpr int REQUESTS = 36 / NW + (36 % NW != 0);
     auto act_row = [&](int r) { return (uint32_t)(g.src_rows ? max(g.src_rows[tile.y + r], 0) : tile.y + r); };
     uint32_t digits_off[REQUESTS];
 #pragma unroll
     for (int c = 0; c < REQUESTS; c++) {
-        const int at = (wave * REQUESTS + c) * 64 + lane, r = at / 24;
+        const int at = min(wave + c * NW, 12 * halves - 1) * 64 + lane, r = at / 24;
         digits_off[c] = act_row(r) * (uint32_t)nbp * MX_BLOCK_BYTES + (uint32_t)((at % 24) ^ ((r >> 1) & 7)) * 16;
     }
-    const uint32_t scales_off = act_row(lane) * (uint32_t)nbp * 4;
-    auto fetch_digits = [&](int i, int c) {
-        dma16(lds0 + (uint32_t)(i % MX_STAGES) * MX_STAGE + (uint32_t)(wave * REQUESTS + c) * 1024, g.acts.digits + (size_t)i * MX_ROW,
-              digits_off[c]);
+    const int scales_row = (wave & 1) * 64 + lane;
+    const bool fetches_scales = wave < 2 && scales_row < 32 * halves;
+    const uint32_t scales_off = fetches_scales ? act_row(scales_row) * (uint32_t)nbp * 4 : 0u;
+    auto request_digits = [&](int i) {  // of quad i + 2, when everybody has read quad i's
+        if (i + 2 >= quads) return;
+        const uint32_t to = lds0 + (uint32_t)(i & 1) * MX_STAGE;
+#pragma unroll
+        for (int c = 0; c < REQUESTS; c++)
+            if (wave + c * NW < 12 * halves)
+                dma16(to + (uint32_t)(wave + c * NW) * 1024, g.acts.digits + (size_t)(i + 2) * MX_ROW, digits_off[c]);
+        if (fetches_scales) dma16(to + MX_STAGE_SCALES + (uint32_t)(wave & 1) * 1024, g.acts.scales + (size_t)(i + 2) * 4, scales_off);
     };
-    auto fetch_act_scales = [&](int i) {
-        if (wave == 0) dma16(lds0 + (uint32_t)(i % MX_STAGES) * MX_STAGE + MX_STAGE_SCALES, g.acts.scales + (size_t)i * 4, scales_off);
-    };
-    // What a wavefront requests during quad i, spread over its arithmetic (all at once, the requests of eight wavefronts
-    // hold each other up): the codes of quad i + 2, whose slot is that of quad i, in its registers by then, and the
-    // digits of quad i + 2, whose stage everybody left before quad i.
+    // the codes of quad i + 2, whose slot is that of quad i, in the wavefront's registers by then; spread over the arithmetic (all at once, the
+    // requests of eight wavefronts hold each other up)
     auto request_codes = [&](int i, int c) {
         if (i + 2 >= quads) return;
         fetch_codes(i + 2, c);
         fetch_codes(i + 2, c + 1);
         if (c == 0 && ((i + 2) & 3) == 0) fetch_weight_scales(i + 2);
-    };
-    auto request_digits = [&](int i) {
-        if (i + 2 >= quads) return;
-#pragma unroll
-        for (int c = 0; c < REQUESTS; c++) fetch_digits(i + 2, c);
-        fetch_act_scales(i + 2);
     };
     // where this lane's pieces of step k sit in a half's 32 rows: piece 4n + block in place (4n + block) ^ x, so the even n
     // 128 bytes apart from here, the odd ones from there
@@ -180,18 +200,18 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
 #pragma unroll
     for (int k = 0; k < 2; k++)
 #pragma unroll
-        for (int n = 0; n < 2; n++) piece_at[k][n] = (uint32_t)(li * MX_ROW + ((4 * n + 2 * lg + k) ^ ((li >> 1) & 7)) * 16);
+        for (int n = 0; n < 2; n++) piece_at[k][n] = (uint32_t)((32 * h_first + li) * MX_ROW + ((4 * n + 2 * lg + k) ^ ((li >> 1) & 7)) * 16);
 
-    mx_v16f acc[2][2];  // [half][row group]
+    mx_v16f acc[3][2];  // [half][row group]
 #pragma unroll
-    for (int h = 0; h < 2; h++)
+    for (int h = 0; h < 3; h++)
 #pragma unroll
         for (int r = 0; r < 2; r++) acc[h][r] = mx_v16f{0.0f};
 
-    // One quad: per half (TWO: both, else the first) two steps of four planes of digits, smallest first, their sum added
-    // onto the running one.  A step's operands are read while the one before is multiplied -- across the quads too: before
-    // the last step the next quad is waited for (and everybody has read the present one), and its codes and first operands
-    // are read behind that step's products.
+    // One quad: per half two steps of four planes of digits, smallest first, their sum added onto the running one.  Operands
+    // are read while others are multiplied -- across the quads too: before the last step's second part the next quad is
+    // waited for (and everybody has read the present one), and its codes and first operands are read behind that part's
+    // products.
     // (macros: as a struct handed between lambdas the operands end up in scratch memory)
     constexpr int E2M3 = 2, E2M1 = 4;
     const uint8_t *const w_wave = lds + MX_STAGES * MX_STAGE + (size_t)wave * MX_W_WAVE;
@@ -208,122 +228,133 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
         return *reinterpret_cast<const mx_v4i *>(st + h * 32 * MX_ROW + (n >> 1) * 128 + piece_at[k][n & 1]);
     };
     auto act_scales = [&](const uint8_t *st, int h, int k) {
-        return *reinterpret_cast<const int *>(st + MX_STAGE_SCALES + (32 * h + li) * 16 + (2 * lg + k) * 4);
+        return *reinterpret_cast<const int *>(st + MX_STAGE_SCALES + (32 * (h_first + h) + li) * 16 + (2 * lg + k) * 4);
     };
-    // step K's operands of half H, requested here, ahead of the products in front of theirs: the planes' dwords 0..3,
-    // dwords 4 and 5 of planes 0 and 1, of planes 2 and 3, and the planes' scales
-#define FRK_MX_READ(o, H, K)                                                                                           \
-    o##0 = piece(st, H, K, 0), o##1 = piece(st, H, K, 1), o##2 = piece(st, H, K, 2), o##3 = piece(st, H, K, 3),        \
-    o##01 = piece(st, H, K, 4), o##23 = piece(st, H, K, 5), o##_scales = act_scales(st, H, K);                         \
+    // A step's operands come in two parts, planes 0 and 1 (A: dwords 0..3 of each, then dwords 4 and 5 of both; with the
+    // planes' scales) and planes 2 and 3 (B): one is read while the other is multiplied.
+#define FRK_MX_READ_A(H, K)                                                                                            \
+    a0 = piece(st, H, K, 0), a1 = piece(st, H, K, 1), a01 = piece(st, H, K, 4), next_scales = act_scales(st, H, K);    \
     __builtin_amdgcn_sched_barrier(0)
-#define FRK_MX_PLANE(o, K, P, head, tail, T)                                                                           \
+#define FRK_MX_READ_B(H, K)                                                                                            \
+    b2 = piece(st, H, K, 2), b3 = piece(st, H, K, 3), b23 = piece(st, H, K, 5);                                        \
+    __builtin_amdgcn_sched_barrier(0)
+#define FRK_MX_PLANE(K, P, head, tail, T)                                                                              \
     {                                                                                                                  \
         const mx_v8i x = {head[0], head[1], head[2], head[3], tail[T], tail[T + 1], 0, 0};                             \
-        const mx_v8i y0 = {b##K##0[0], b##K##0[1], b##K##0[2], b##K##0[3], 0, 0, 0, 0};                                \
-        const mx_v8i y1 = {b##K##1[0], b##K##1[1], b##K##1[2], b##K##1[3], 0, 0, 0, 0};                                \
-        part0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y0, part0, E2M3, E2M1, P, o##_scales, K, scale0);   \
-        part1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y1, part1, E2M3, E2M1, P, o##_scales, K, scale1);   \
+        const mx_v8i y0 = {w##K##0[0], w##K##0[1], w##K##0[2], w##K##0[3], 0, 0, 0, 0};                                \
+        const mx_v8i y1 = {w##K##1[0], w##K##1[1], w##K##1[2], w##K##1[3], 0, 0, 0, 0};                                \
+        part0 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y0, part0, E2M3, E2M1, P, act_scale, K, scale0);    \
+        part1 = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, y1, part1, E2M3, E2M1, P, act_scale, K, scale1);    \
     }
-#define FRK_MX_FIRST(o, K) FRK_MX_PLANE(o, K, 0, o##0, o##01, 0)
-#define FRK_MX_REST(o, K)                   \
-    FRK_MX_PLANE(o, K, 1, o##1, o##01, 2) \
-    FRK_MX_PLANE(o, K, 2, o##2, o##23, 0) \
-    FRK_MX_PLANE(o, K, 3, o##3, o##23, 2) \
+#define FRK_MX_MULTIPLY_A(K)                          \
+    act_scale = next_scales;                          \
+    FRK_MX_PLANE(K, 0, a0, a01, 0)                    \
+    FRK_MX_PLANE(K, 1, a1, a01, 2)                    \
+    asm volatile("" : "+v"(part0), "+v"(part1));
+#define FRK_MX_MULTIPLY_B(K)                          \
+    FRK_MX_PLANE(K, 2, b2, b23, 0)                    \
+    FRK_MX_PLANE(K, 3, b3, b23, 2)                    \
     asm volatile("" : "+v"(part0), "+v"(part1));  // (stays in front of the requests behind it)
-    // quad I has landed: behind its digits the wavefront requested four times codes and its share of digits, of quad I + 1
-    // (and now and then scales: then a little more is waited for); afterwards its codes (step 0's in place, step 1's
-    // beside the present ones) and first operands
+    // quad I has landed: behind its digits the wavefront requested the codes of quad I + 1 (four times, and now and then
+    // scales: then a little more is waited for); afterwards its codes (step 0's in place, step 1's beside the present ones)
+    // and first operands
 #define FRK_MX_ARRIVE(I)                                                                                               \
-    if ((I) + 1 < quads && wave == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(REQUESTS + 5) : "memory");              \
-    else if ((I) + 1 < quads) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(REQUESTS + 4) : "memory");                      \
+    if ((I) + 1 < quads) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");                                              \
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                                              \
     lds_barrier();                                                                                                     \
-    st = lds + (size_t)((I) % MX_STAGES) * MX_STAGE;                                                                   \
-    b00 = codes(I, 0, 0), b01 = codes(I, 0, 1), next10 = codes(I, 1, 0), next11 = codes(I, 1, 1);                      \
+    st = lds + (size_t)((I) & 1) * MX_STAGE;                                                                           \
+    w00 = codes(I, 0, 0), w01 = codes(I, 0, 1);                                                                    \
     next_scale0 = scales(I, 0), next_scale1 = scales(I, 1);                                                            \
     __builtin_amdgcn_sched_barrier(0);                                                                                 \
-    FRK_MX_READ(p, 0, 0)
-    auto all_quads = [&](auto two_c) {
-        constexpr bool TWO = decltype(two_c)::value;
+    FRK_MX_READ_A(0, 0)
+    auto all_quads = [&](auto halves_c) {
+        constexpr int H = decltype(halves_c)::value;
         const uint8_t *st;
-        mx_v4i b00, b01, b10, b11, next10, next11, p0, p1, p2, p3, p01, p23, q0, q1, q2, q3, q01, q23;
-        int scale0, scale1, next_scale0, next_scale1, p_scales, q_scales;
+        mx_v4i w00, w01, w10, w11, a0, a1, a01, b2, b3, b23;
+        int scale0, scale1, next_scale0, next_scale1, act_scale, next_scales;
         FRK_MX_ARRIVE(0);
-        b10 = next10, b11 = next11, scale0 = next_scale0, scale1 = next_scale1;
+        request_digits(-1);
+        scale0 = next_scale0, scale1 = next_scale1;
         for (int i = 0; i < quads; i++) {
-            mx_v16f part0 = mx_v16f{0.0f}, part1 = part0;
-            FRK_MX_FIRST(p, 0)
-            FRK_MX_READ(q, 0, 1);
-            request_codes(i, 0);
-            FRK_MX_REST(p, 0)
-            request_codes(i, 2);
-            if (TWO) {
-                FRK_MX_FIRST(q, 1)
-                FRK_MX_READ(p, 1, 0);
-                FRK_MX_REST(q, 1)
-                acc[0][0] += part0;
-                acc[0][1] += part1;
-                request_digits(i);
-                part0 = part1 = mx_v16f{0.0f};
-                FRK_MX_FIRST(p, 0)
-                FRK_MX_READ(q, 1, 1);
-                FRK_MX_REST(p, 0)
-            } else {
-                request_digits(i);
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                mx_v16f part0 = mx_v16f{0.0f}, part1 = part0;
+                FRK_MX_READ_B(h, 0);
+                FRK_MX_MULTIPLY_A(0)
+                if (h == 0) w10 = codes(i, 1, 0), w11 = codes(i, 1, 1);
+                FRK_MX_READ_A(h, 1);
+                FRK_MX_MULTIPLY_B(0)
+                FRK_MX_READ_B(h, 1);
+                FRK_MX_MULTIPLY_A(1)
+                if (h == 0) request_codes(i, 0);
+                if (H == 1) request_codes(i, 2);
+                if (h < H - 1) {
+                    FRK_MX_READ_A(h + 1, 0);
+                } else {
+                    FRK_MX_ARRIVE(i + 1);  // (behind the last quad: whatever lies there, unused)
+                    request_digits(i);
+                }
+                FRK_MX_MULTIPLY_B(1)
+                acc[h][0] += part0;
+                acc[h][1] += part1;
+                if (H == 3) asm volatile("" : "+v"(acc[h][0]), "+v"(acc[h][1]));  // (sunk further down, two halves' sums are alive at once)
+                if (h == 0 && H > 1) request_codes(i, 2);
             }
-            FRK_MX_ARRIVE(i + 1);  // (behind the last quad: whatever lies there, unused)
-            FRK_MX_FIRST(q, 1)
-            FRK_MX_REST(q, 1)
-            acc[TWO][0] += part0;
-            acc[TWO][1] += part1;
-            b10 = next10, b11 = next11, scale0 = next_scale0, scale1 = next_scale1;
+            scale0 = next_scale0, scale1 = next_scale1;
         }
     };
+    request_digits(-2);
     for (int c = 0; c < 4; c++) fetch_codes(0, c);
     fetch_weight_scales(0);
-    request_digits(-2);
     request_codes(-1, 0);
     request_codes(-1, 2);
-    request_digits(-1);
-    if (two) all_quads(std::true_type());
-    else all_quads(std::false_type());
-#undef FRK_MX_READ
+    if (h_count > 2) all_quads(std::integral_constant<int, 3>());
+    else if (h_count > 1) all_quads(std::integral_constant<int, 2>());
+    else all_quads(std::integral_constant<int, 1>());
+#undef FRK_MX_READ_A
+#undef FRK_MX_READ_B
 #undef FRK_MX_PLANE
-#undef FRK_MX_FIRST
-#undef FRK_MX_REST
+#undef FRK_MX_MULTIPLY_A
+#undef FRK_MX_MULTIPLY_B
 #undef FRK_MX_ARRIVE
 
     // ---- register r of a lane: activation row 8 * (r / 4) + 4 * (lane / 32) + r % 4 of the half, weight row lane % 32
+    // (silu ahead of the stores and their conditions, so that several values' chains of operations run beside each other)
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        if (h == 1 && !two) break;
+    for (int h = 0; h < 3; h++) {
+        if (h >= h_count || !stores) break;
+        if (GLU) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[h][0][r] = silu_as_host(acc[h][0][r], expf_table) * acc[h][1][r];
+        }
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const int tok = 32 * h + 8 * (r >> 2) + 4 * lg + (r & 3);
-            const float v0 = acc[h][0][r], v1 = acc[h][1][r];
+            const int tok = 32 * (h_first + h) + 8 * (r >> 2) + 4 * lg + (r & 3);
             if (tok >= tile.z) continue;
             float *dst = g.y + (size_t)(tile.w + tok) * g.rows;
-            if (GLU) {
-                if (row0 < g.rows) dst[row0] = silu_as_host(v0) * v1;
-            } else {
-                if (row0 < g.rows) dst[row0] = v0;
-                if (row0 + 32 < g.rows) dst[row0 + 32] = v1;
-            }
+            if (row0 < g.rows) dst[row0] = acc[h][0][r];
+            if (!GLU && row0 + 32 < g.rows) dst[row0 + 32] = acc[h][1][r];
         }
     }
 
     // ---- the rows with infinite blocks again (hardly ever any): what decides is the sign of each such block's integer
     // sum, an infinity each, NaN where the sum is zero or two differ.  Lanes 0 .. 31 take the first row group, the others
     // the second.
-    bool again = false;
-    if (lane < tile.z) {
-        const int src = g.src_rows ? g.src_rows[tile.y + lane] : tile.y + lane;
-        again = src >= 0 && g.acts.infinite[src] != 0;
-    }
-    uint64_t left = __ballot(again);
-    if (left) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (their first results are out)
-    for (; left; left &= left - 1) {
-        const int tok = __builtin_ctzll(left);
+    auto infinite_rows = [&](int first) {  // of 64 rows
+        bool again = false;
+        const int half = (first + lane) >> 5;
+        if (stores && first + lane < tile.z && half >= h_first && half < h_first + h_count) {
+            const int src = g.src_rows ? g.src_rows[tile.y + first + lane] : tile.y + first + lane;
+            again = src >= 0 && g.acts.infinite[src] != 0;
+        }
+        return __ballot(again);
+    };
+    uint64_t left = infinite_rows(0), left_high = tile.z > 64 ? infinite_rows(64) : 0;
+    if (left | left_high) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (their first results are out)
+    while (left | left_high) {
+        const int tok = left ? __builtin_ctzll(left) : 64 + __builtin_ctzll(left_high);
+        if (left) left &= left - 1;
+        else left_high &= left_high - 1;
         const size_t first = (size_t)act_row(tok) * nbp;
         const uint8_t *codes_row = (lg ? w_base[1] : w_base[0]) + weight_row(lane);
         float sum = 0.0f;
@@ -343,7 +374,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
         float *dst = g.y + (size_t)(tile.w + tok) * g.rows;
         if (GLU) {
             const float up = __shfl_xor(sum, 32);
-            if (lg == 0 && row0 < g.rows) dst[row0] = silu_as_host(sum) * up;
+            if (lg == 0 && row0 < g.rows) dst[row0] = silu_as_host(sum, expf_table) * up;
         } else if (row0 + 32 * lg < g.rows) {
             dst[row0 + 32 * lg] = sum;
         }
@@ -364,9 +395,22 @@ bool mx_gemm_takes(size_t act_rows, size_t rows_g, size_t cols) {
     return act_rows * mx_padded_blocks(cols) * MX_BLOCK_BYTES <= 0xffffffffu &&
            rows_g * layout_for(FRK_KIND_MXFP4, cols).row_stride <= 0xffffffffu;
 }
+// Wavefronts of a workgroup: eight where 64-row tiles of as many groups as may be partly used fill the chip.
+static int mx_waves(size_t pairs, size_t groups, size_t rows_g, bool glu) {
+    const size_t rows = 8 * (glu ? 32 : 64);
+    return (pairs / 64 + groups) * ((rows_g + rows - 1) / rows) >= 256 ? 8 : 4;
+}
+// Tiles of 96 rows where the workgroups of 64-row tiles would not fit the chip at once: an expert of 65 to 96 pairs then reads
+// its weights once, not a second time for a few rows.  Tiles of 64 rows where they do: there a job's length is the launch's.
+// (64-row tiles / 96, us a layer: 32 experts top-4 of 2880 / 2880 at 512 and 768 tokens 286 / 244 and 352 / 304, 16 top-2 of
+// 2880 / 1536 at 700 152 / 118, 8 top-4 of 2048 / 1440 at 300 98 / 87, 8 top-2 of 1024 / 1024 at 512 57.5 / 65.9.)
+int mx_tile(size_t pairs, size_t groups, size_t rows_g, bool glu) {
+    const size_t rows = (size_t)mx_waves(pairs, groups, rows_g, glu) * (glu ? 32 : 64);
+    return (pairs / 64 + groups / 2) * ((rows_g + rows - 1) / rows) > 256 ? MX_TILE : MOE_TILE;
+}
 // up: the second matrix (y = silu(gate) * up), or null
 int launch_gemm_mx_grouped(const frk_weights *w, const frk_weights *up, size_t rows_g, const MxActs &acts, const int *src_rows,
-                           const int4 *tiles, const int *n_tiles, size_t max_tiles, float *y, hipStream_t s) {
+                           const int4 *tiles, const int *n_tiles, size_t max_tiles, size_t pairs, size_t groups, float *y, hipStream_t s) {
     if (max_tiles == 0) return FRK_OK;
     MxGemmArgs g;
     g.W = w->dev;
@@ -381,9 +425,9 @@ int launch_gemm_mx_grouped(const frk_weights *w, const frk_weights *up, size_t r
     g.n_tiles = n_tiles;
     g.y = y;
     const size_t rows_wave = up ? 32 : 64, tiles8 = (max_tiles + 7) / 8 * 8;
-    const bool wide = max_tiles * ((rows_g + 8 * rows_wave - 1) / (8 * rows_wave)) >= 256;
+    const bool wide = mx_waves(pairs, groups, rows_g, up != nullptr) == 8;
     g.row_groups = (int)((rows_g + (wide ? 8 : 4) * rows_wave - 1) / ((wide ? 8 : 4) * rows_wave));
-    const size_t grid = tiles8 * (size_t)g.row_groups;
+    const size_t grid = tiles8 * (size_t)g.row_groups + (wide ? 8 * XCD_CUS / 2 : 0);
     if (grid > 0x7fffffffu) return set_error(FRK_ERR_SHAPE, "grouped gemm: %zu rows a group, %zu tiles", rows_g, max_tiles);
     static bool sized = false;  // a benign race: every thread sets the same attribute
     if (!sized) {

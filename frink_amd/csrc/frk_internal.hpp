@@ -277,8 +277,9 @@ MxActs mx_acts_carve(void *base, size_t rows, size_t cols);
 size_t mx_acts_bytes(size_t rows, size_t cols);
 int launch_quantize_mx(const float *x, size_t rows, size_t cols, const int *used, const MxActs &out, hipStream_t s);
 bool mx_gemm_takes(size_t act_rows, size_t rows_g, size_t cols);
+int mx_tile(size_t pairs, size_t groups, size_t rows_g, bool glu);  // rows of a tile: MX_TILE or MOE_TILE
 int launch_gemm_mx_grouped(const frk_weights *w, const frk_weights *up, size_t rows_g, const MxActs &acts, const int *src_rows,
-                           const int4 *tiles, const int *n_tiles, size_t max_tiles, float *y, hipStream_t s);
+                           const int4 *tiles, const int *n_tiles, size_t max_tiles, size_t pairs, size_t groups, float *y, hipStream_t s);
 // the grouped GEMM over groups of Q5_0 / IQ4_XS / MXFP4 matrices that have a decoded form for the matrix cores
 bool units_have_planar_form(const frk_weights *w);
 // that form: rows of layout_for(FRK_KIND_Q8_0, cols) -- signed bytes, then f16 scales per 32 (IQ4_XS: per block of
@@ -304,6 +305,7 @@ int launch_gemm_sub_planar(const uint8_t *W, size_t row_stride, size_t off_d, si
 // same activations.  (64 rows: an expert's weights are then fetched and unpacked once for up to 64
 // of its rows; the second half of a tile costs nothing when it is not in use.)
 constexpr int MOE_TILE = 64;
+constexpr int MX_TILE = 96;  // the MXFP4 kernel's larger tile (mx_tile)
 // Up to this many tokens the MoE layer runs per (token, slot) pair on the decode kernels.  Measured
 // on the 128-expert, top-8, 2048/768 layer: 8 tokens 47 us against 94 us on the grouped path, 16
 // tokens 79 against 123, 32 tokens 146 against 140.

@@ -122,6 +122,7 @@ struct GroupArgs {
     int *n_tiles;
     int max_rows;
 };
+template <int TILE>
 __device__ __forceinline__ void moe_group(const GroupArgs &a) {
     const int32_t *__restrict__ ids = a.ids;
     const int pairs = a.pairs, k = a.k, n_experts = a.n_experts, max_rows = a.max_rows;
@@ -152,9 +153,9 @@ __device__ __forceinline__ void moe_group(const GroupArgs &a) {
     __syncthreads();
     {
         const int c = tid < n_experts ? L.cnt[tid] : 0;
-        const int nt = (c + MOE_TILE - 1) / MOE_TILE;
-        const int last = c - MOE_TILE * (nt - 1);  // rows in use of the last tile (nt > 0)
-        const int big = nt == 0 ? 0 : nt - 1 + (last > 32);
+        const int nt = (c + TILE - 1) / TILE;
+        const int last = c - TILE * (nt - 1);  // rows in use of the last tile (nt > 0)
+        const int big = nt == 0 ? 0 : nt - 1 + (last > TILE - 32);
         const int small = nt - big;  // 0 or 1
         int total, total_big, total_small;
         const int o = block_exclusive_scan(c, L.wave_tot, total);
@@ -168,8 +169,8 @@ __device__ __forceinline__ void moe_group(const GroupArgs &a) {
             group_off[tid] = o;
             for (int i = 0; i < nt; i++) {
                 const int t = i < big ? tb + i : ts;
-                const int used = min(MOE_TILE, c - MOE_TILE * i);
-                tiles[t] = make_int4(tid, MOE_TILE * t, used, MOE_TILE * t);
+                const int used = min(TILE, c - TILE * i);
+                tiles[t] = make_int4(tid, TILE * t, used, TILE * t);
             }
         }
         if (tid == 0) {
@@ -216,8 +217,8 @@ __device__ __forceinline__ void moe_group(const GroupArgs &a) {
             if (e >= 0 && e < n_experts) {
                 const int w = (j >> 5) * n_experts + e;
                 const int rank = L.run[e] + L.before[w] + __popc(L.bits[w] & ((1u << (j & 31)) - 1u));
-                const int j = rank / MOE_TILE;
-                const int pos = MOE_TILE * (j < L.n_big[e] ? L.tile_big[e] + j : L.tile_small[e]) + rank % MOE_TILE;
+                const int j = rank / TILE;
+                const int pos = TILE * (j < L.n_big[e] ? L.tile_big[e] + j : L.tile_small[e]) + rank % TILE;
                 gather[pos] = p / k;
                 pos_of[p] = pos;
                 cpos_of[p] = L.off_cmp[e] + rank;
@@ -228,7 +229,7 @@ __device__ __forceinline__ void moe_group(const GroupArgs &a) {
         __syncthreads();
     }
 }
-__global__ __launch_bounds__(1024) void moe_group_kernel(GroupArgs a) { moe_group(a); }
+__global__ __launch_bounds__(1024) void moe_group_kernel(GroupArgs a) { moe_group<MOE_TILE>(a); }
 
 // The bucketing and the quantization of the token rows do not depend on each other: in one launch, workgroup
 // 0 buckets while the others quantize (quantize_activations_q8_k, crates/frink-quant/src/act_quant.rs:69-104;
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(GroupArgs a) { moe_grou
 __global__ __launch_bounds__(1024) void moe_group_quantize_kernel(GroupArgs a, const float *__restrict__ x, int n_blocks,
                                                                   Q8KRows out) {
     if (blockIdx.x == 0) {
-        moe_group(a);
+        moe_group<MOE_TILE>(a);
         return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -254,10 +255,11 @@ __global__ __launch_bounds__(1024) void moe_group_quantize_kernel(GroupArgs a, c
 
 // The same beside the digits of MXFP4 expert layers: eight token rows a workgroup (one after the other, the bucketing
 // 9 us and the digits 8 stood in front of every such layer).
+template <int TILE>
 __global__ __launch_bounds__(1024) void moe_group_quantize_mx_kernel(GroupArgs a, const float *__restrict__ x, int rows, int nb, MxActs out) {
     __shared__ int infinite[8];
     if (blockIdx.x == 0) {
-        moe_group(a);
+        moe_group<TILE>(a);
         return;
     }
     const int sub = threadIdx.x >> 7;
@@ -284,6 +286,7 @@ struct GroupedTilesLds {
     int off[1025], tile_big[1024], n_big[1024], tile_small[1024];
     int wave_tot[16];
 };
+template <int TILE>
 __device__ __forceinline__ void grouped_tiles(const GroupedTilesArgs &a) {
     __shared__ GroupedTilesLds L;
     const int tid = threadIdx.x;
@@ -293,9 +296,9 @@ __device__ __forceinline__ void grouped_tiles(const GroupedTilesArgs &a) {
     __syncthreads();
     {
         const int c = tid < a.n_groups ? max(L.off[tid + 1] - L.off[tid], 0) : 0;
-        const int nt = (c + MOE_TILE - 1) / MOE_TILE;
-        const int last = c - MOE_TILE * (nt - 1);
-        const int big = nt == 0 ? 0 : nt - 1 + (last > 32);
+        const int nt = (c + TILE - 1) / TILE;
+        const int last = c - TILE * (nt - 1);
+        const int big = nt == 0 ? 0 : nt - 1 + (last > TILE - 32);
         const int small = nt - big;  // 0 or 1
         int total_big, total_small;
         const int tb = block_exclusive_scan(big, L.wave_tot, total_big);
@@ -305,7 +308,7 @@ __device__ __forceinline__ void grouped_tiles(const GroupedTilesArgs &a) {
         L.tile_small[tid] = ts;
         for (int i = 0; i < nt; i++) {
             const int t = i < big ? tb + i : ts;
-            a.tiles[t] = make_int4(tid, MOE_TILE * t, min(MOE_TILE, c - MOE_TILE * i), L.off[tid] + MOE_TILE * i);
+            a.tiles[t] = make_int4(tid, TILE * t, min(TILE, c - TILE * i), L.off[tid] + TILE * i);
         }
         if (tid == 0) *a.n_tiles = total_big + total_small;
     }
@@ -319,18 +322,19 @@ __device__ __forceinline__ void grouped_tiles(const GroupedTilesArgs &a) {
         }
         const int rank = p - L.off[lo];
         if (rank < 0 || p >= L.off[lo + 1]) continue;  // (a pair before the first group or in a clamped hole)
-        const int i = rank / MOE_TILE;
+        const int i = rank / TILE;
         const int t = i < L.n_big[lo] ? L.tile_big[lo] + i : L.tile_small[lo];
         const int src = a.gather ? a.gather[p] : p;
-        a.src_rows[MOE_TILE * t + rank % MOE_TILE] = min(max(src, 0), a.x_rows - 1);
+        a.src_rows[TILE * t + rank % TILE] = min(max(src, 0), a.x_rows - 1);
     }
 }
-__global__ __launch_bounds__(1024) void grouped_tiles_kernel(GroupedTilesArgs a) { grouped_tiles(a); }
+template <int TILE>
+__global__ __launch_bounds__(1024) void grouped_tiles_kernel(GroupedTilesArgs a) { grouped_tiles<TILE>(a); }
 // the same beside the quantization of the activation rows, as in moe_group_quantize_kernel
 __global__ __launch_bounds__(1024) void grouped_tiles_quantize_kernel(GroupedTilesArgs a, const float *__restrict__ x, int n_blocks,
                                                                       Q8KRows out) {
     if (blockIdx.x == 0) {
-        grouped_tiles(a);
+        grouped_tiles<MOE_TILE>(a);
         return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -490,8 +494,8 @@ struct MoeScratch {
 };
 
 // rows of the grouped order at most: every bucket may end in a partly used tile
-static size_t moe_max_rows(size_t pairs, int n_experts) {
-    return (pairs / MOE_TILE + (size_t)n_experts) * MOE_TILE;
+static size_t moe_max_rows(size_t pairs, int n_experts, int tile = MOE_TILE) {
+    return (pairs / (size_t)tile + (size_t)n_experts) * (size_t)tile;
 }
 
 // Carves the workspace; with base == nullptr the returned pointers are offsets and `end` the size.
@@ -695,7 +699,7 @@ int launch_gemm_grouped(const frk_weights *w, size_t n_groups, const int32_t *gr
         FRK_LAUNCH_CHECK("grouped_tiles_quantize");
         return launch_gemm_k_stream(w, nullptr, rows_g, m.xa, &m.xr, m.src_rows, m.tiles, m.n_tiles, max_tiles, y, nullptr, s);
     }
-    hipLaunchKernelGGL(grouped_tiles_kernel, dim3(1), dim3(1024), 0, s, ta);
+    hipLaunchKernelGGL(grouped_tiles_kernel<MOE_TILE>, dim3(1), dim3(1024), 0, s, ta);
     FRK_LAUNCH_CHECK("grouped_tiles");
     int rc = launch_quantize_q8_k_gather(x, cols, m.src_rows, rows, m.xa, s);
     if (rc) return rc;
@@ -770,13 +774,23 @@ int launch_moe_ffn_units(const frk_weights *gate, const frk_weights *up, const f
 // quantize them, and the products are the same: the two paths differ in the float additions only.
 
 // Which projections multiply MXFP4 experts as they are (frk_gemm_mx.hip): no decoded copy, gate and up in one launch
+// (tiles of MX_TILE rows only where every projection does: the decoded form's kernel walks tiles of MOE_TILE)
 struct UnitsNative {
     bool gate_up, down;
+    int tile;
+    size_t rows;  // of the grouped order
 };
-static UnitsNative units_native(int gate_kind, int down_kind, size_t batch, size_t rows, size_t hidden, size_t ffn) {
+static UnitsNative units_native(int gate_kind, int down_kind, size_t batch, size_t pairs, int n_experts, size_t hidden, size_t ffn) {
     UnitsNative n;
-    n.gate_up = gate_kind == FRK_KIND_MXFP4 && mx_gemm_takes(std::max(batch, rows), ffn, hidden);
-    n.down = n.gate_up && down_kind == FRK_KIND_MXFP4 && mx_gemm_takes(rows, hidden, ffn);
+    n.tile = MOE_TILE;
+    n.rows = moe_max_rows(pairs, n_experts);
+    n.gate_up = gate_kind == FRK_KIND_MXFP4 && mx_gemm_takes(std::max(batch, n.rows), ffn, hidden);
+    n.down = n.gate_up && down_kind == FRK_KIND_MXFP4 && mx_gemm_takes(n.rows, hidden, ffn);
+    const int tile = mx_tile(pairs, (size_t)n_experts, ffn, true);
+    if (n.down && mx_gemm_takes(moe_max_rows(pairs, n_experts, tile), hidden, ffn)) {
+        n.tile = tile;
+        n.rows = moe_max_rows(pairs, n_experts, tile);
+    }
     return n;
 }
 bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts, size_t batch,
@@ -788,7 +802,7 @@ bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up
     // 143 / 187, 207 / 196, 263 / 197; 16 top-4 of 1440 / 2880 at 6, 8 77 / 82, 97 / 83; 16 top-2 of 2048 / 1440 at 12, 16
     // 56 / 58, 67 / 59; 8 top-2 of 1024 / 1024 at 12, 16, 24 39 / 42, 45 / 42, 59 / 43.
     const size_t pairs = batch * (size_t)k, ffn = down->cols;
-    return pairs >= std::max<size_t>(2 * (size_t)n_experts, 32) && units_native(gate->kind, down->kind, batch, moe_max_rows(pairs, n_experts), gate->cols, ffn).down;
+    return pairs >= std::max<size_t>(2 * (size_t)n_experts, 32) && units_native(gate->kind, down->kind, batch, pairs, n_experts, gate->cols, ffn).down;
 }
 struct UnitsGroupedScratch {
     uint8_t *gate_w, *up_w, *down_w;  // decoded experts (not of projections in their own form)
@@ -804,7 +818,7 @@ static size_t units_grouped_acts_bytes(size_t rows, size_t cols) {
 }
 static UnitsGroupedScratch units_grouped_carve(void *base, UnitsNative native, size_t batch, int k, int n_experts, int hidden, int ffn,
                                                size_t *end) {
-    const size_t pairs = batch * (size_t)k, rows = moe_max_rows(pairs, n_experts);
+    const size_t pairs = batch * (size_t)k, rows = native.rows;
     char *p = (char *)base;
     auto take = [&](size_t bytes) {
         char *r = p;
@@ -825,13 +839,13 @@ static UnitsGroupedScratch units_grouped_carve(void *base, UnitsNative native, s
     m.pos_of = (int *)take(pairs * 4);
     m.cpos_of = (int *)take(pairs * 4);
     m.n_tiles = (int *)take(256);
-    m.tiles = (int4 *)take((rows / MOE_TILE + 1) * 16);
+    m.tiles = (int4 *)take((rows / (size_t)native.tile + 1) * 16);
     if (end) *end = (size_t)(p - (char *)base);
     return m;
 }
 size_t moe_units_grouped_workspace_bytes(int gate_kind, int down_kind, size_t batch, int k, int n_experts, int hidden, int ffn) {
     size_t end = 0;
-    const UnitsNative native = units_native(gate_kind, down_kind, batch, moe_max_rows(batch * (size_t)k, n_experts), hidden, ffn);
+    const UnitsNative native = units_native(gate_kind, down_kind, batch, batch * (size_t)k, n_experts, hidden, ffn);
     (void)units_grouped_carve(nullptr, native, batch, k, n_experts, hidden, ffn, &end);
     return end;
 }
@@ -868,7 +882,8 @@ static bool grouped_units_native(int kind, size_t rows_g, size_t x_rows, size_t 
 }
 static GroupedUnitsScratch grouped_units_carve(void *base, bool native, size_t n_groups, size_t w_rows, size_t x_rows, size_t pairs,
                                                size_t cols, size_t *end) {
-    const size_t rows = moe_max_rows(pairs, (int)n_groups);
+    const int tile = native ? mx_tile(pairs, n_groups, w_rows / n_groups, false) : MOE_TILE;
+    const size_t rows = moe_max_rows(pairs, (int)n_groups, tile);
     char *p = (char *)base;
     auto take = [&](size_t bytes) {
         char *r = p;
@@ -880,7 +895,7 @@ static GroupedUnitsScratch grouped_units_carve(void *base, bool native, size_t n
     m.acts = take(native ? mx_acts_bytes(x_rows, cols) : units_grouped_acts_bytes(x_rows, cols));
     m.src_rows = (int *)take(rows * 4);
     m.n_tiles = (int *)take(256);
-    m.tiles = (int4 *)take((rows / MOE_TILE + 1) * 16);
+    m.tiles = (int4 *)take((rows / (size_t)tile + 1) * 16);
     if (end) *end = (size_t)(p - (char *)base);
     return m;
 }
@@ -891,18 +906,20 @@ size_t grouped_units_workspace_bytes(int kind, size_t n_groups, size_t w_rows, s
 }
 int launch_gemm_grouped_units(const frk_weights *w, size_t n_groups, const int32_t *group_off, const int32_t *gather, const float *x,
                               size_t x_rows, size_t pairs, float *y, void *ws, hipStream_t s) {
-    const size_t rows_g = w->rows / n_groups, cols = w->cols, rows = moe_max_rows(pairs, (int)n_groups);
+    const size_t rows_g = w->rows / n_groups, cols = w->cols;
     const bool native = grouped_units_native(w->kind, rows_g, x_rows, cols);
+    const size_t tile = native ? (size_t)mx_tile(pairs, n_groups, rows_g, false) : MOE_TILE, rows = moe_max_rows(pairs, (int)n_groups, (int)tile);
     const GroupedUnitsScratch m = grouped_units_carve(ws, native, n_groups, w->rows, x_rows, pairs, cols, nullptr);
     const GroupedTilesArgs ta{group_off, gather, (int)n_groups, (int)pairs, (int)x_rows, (int)rows, m.src_rows, m.tiles, m.n_tiles};
-    hipLaunchKernelGGL(grouped_tiles_kernel, dim3(1), dim3(1024), 0, s, ta);
+    if (tile == MX_TILE) hipLaunchKernelGGL(grouped_tiles_kernel<MX_TILE>, dim3(1), dim3(1024), 0, s, ta);
+    else hipLaunchKernelGGL(grouped_tiles_kernel<MOE_TILE>, dim3(1), dim3(1024), 0, s, ta);
     FRK_LAUNCH_CHECK("grouped_tiles");
     int rc;
     if (native) {
         const MxActs xa = mx_acts_carve(m.acts, x_rows, cols);
         rc = launch_quantize_mx(x, x_rows, cols, nullptr, xa, s);
         if (rc) return rc;
-        return launch_gemm_mx_grouped(w, nullptr, rows_g, xa, m.src_rows, m.tiles, m.n_tiles, rows / MOE_TILE, y, s);
+        return launch_gemm_mx_grouped(w, nullptr, rows_g, xa, m.src_rows, m.tiles, m.n_tiles, rows / tile, pairs, n_groups, y, s);
     }
     const uint8_t *decoded = nullptr;
     rc = units_decoded(w, m.decoded, s, &decoded);
@@ -912,22 +929,26 @@ int launch_gemm_grouped_units(const frk_weights *w, size_t n_groups, const int32
     if (rc) return rc;
     const Layout l = layout_for(FRK_KIND_Q8_0, cols);
     return launch_gemm_planar_grouped(decoded, l.row_stride, l.off_a, rows_g, cols, w->kind == FRK_KIND_IQ4_XS, xa.q, xa.d, m.src_rows,
-                                      m.tiles, m.n_tiles, rows / MOE_TILE, y, s);
+                                      m.tiles, m.n_tiles, rows / tile, y, s);
 }
 
 int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts,
                                  const float *x, size_t batch, const int32_t *ids, const float *weights, int k, float *out,
                                  void *ws, hipStream_t s) {
     const int hidden = (int)gate->cols, ffn = (int)down->cols;
-    const size_t pairs = batch * (size_t)k, rows = moe_max_rows(pairs, n_experts), max_tiles = rows / MOE_TILE;
-    const UnitsNative native = units_native(gate->kind, down->kind, batch, rows, hidden, ffn);
+    const size_t pairs = batch * (size_t)k;
+    const UnitsNative native = units_native(gate->kind, down->kind, batch, pairs, n_experts, hidden, ffn);
+    const size_t rows = native.rows, max_tiles = rows / (size_t)native.tile;
     const UnitsGroupedScratch m = units_grouped_carve(ws, native, batch, k, n_experts, hidden, ffn, nullptr);
     static bool sized = false;  // a benign race: every thread sets the same attribute
     if (!sized) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_kernel),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GroupLds));
         if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_quantize_mx_kernel),
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_quantize_mx_kernel<MOE_TILE>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GroupLds));
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(&moe_group_quantize_mx_kernel<MX_TILE>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GroupLds));
         if (e != hipSuccess) return set_error(FRK_ERR_HIP, "hipFuncSetAttribute(moe_group): %s", hipGetErrorString(e));
         sized = true;
@@ -936,10 +957,13 @@ int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up,
     int rc;
     if (native.gate_up) {
         const MxActs xa = mx_acts_carve(m.x_acts, batch, hidden);
-        hipLaunchKernelGGL(moe_group_quantize_mx_kernel, dim3(1 + (unsigned)((batch + 7) / 8)), dim3(1024), sizeof(GroupLds), s, ga, x,
-                           (int)batch, hidden / 32, xa);
+        const dim3 grid(1 + (unsigned)((batch + 7) / 8));
+        if (native.tile == MX_TILE)
+            hipLaunchKernelGGL(moe_group_quantize_mx_kernel<MX_TILE>, grid, dim3(1024), sizeof(GroupLds), s, ga, x, (int)batch, hidden / 32, xa);
+        else
+            hipLaunchKernelGGL(moe_group_quantize_mx_kernel<MOE_TILE>, grid, dim3(1024), sizeof(GroupLds), s, ga, x, (int)batch, hidden / 32, xa);
         FRK_LAUNCH_CHECK("moe_group_quantize_mx");
-        rc = launch_gemm_mx_grouped(gate, up, (size_t)ffn, xa, m.gather, m.tiles, m.n_tiles, max_tiles, m.gate_out, s);
+        rc = launch_gemm_mx_grouped(gate, up, (size_t)ffn, xa, m.gather, m.tiles, m.n_tiles, max_tiles, pairs, (size_t)n_experts, m.gate_out, s);
         if (rc) return rc;
     } else {
         hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), sizeof(GroupLds), s, ga);
@@ -966,7 +990,7 @@ int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up,
         const MxActs aa = mx_acts_carve(m.a_acts, rows, ffn);
         rc = launch_quantize_mx(m.gate_out, rows, (size_t)ffn, m.gather, aa, s);
         if (rc) return rc;
-        rc = launch_gemm_mx_grouped(down, nullptr, (size_t)hidden, aa, nullptr, m.tiles, m.n_tiles, max_tiles, m.down_out, s);
+        rc = launch_gemm_mx_grouped(down, nullptr, (size_t)hidden, aa, nullptr, m.tiles, m.n_tiles, max_tiles, pairs, (size_t)n_experts, m.down_out, s);
     } else {
         const uint8_t *down_w = nullptr;
         rc = units_decoded(down, m.down_w, s, &down_w);

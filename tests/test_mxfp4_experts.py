@@ -164,6 +164,22 @@ def test_moe_layer_at_the_edges_of_its_tiles(fa, n_experts, k, hidden, ffn, batc
     _moe_case(fa, fo.MXFP4, fo.MXFP4, n_experts, k, hidden, ffn, batch)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows_g,cols,counts", [
+    (1500, 416, [96, 97, 65, 64, 128, 192, 193, 0, 1] * 3),  # four wavefronts a workgroup, one to three halves, last tiles of a row
+    (4097, 416, [96, 65, 33, 1, 97, 32, 64, 200] * 4),  # nine workgroups a tile, an XCD's last round of jobs cut in two
+])
+def test_tiles_of_96_rows(fa, rows_g, cols, counts):
+    test_grouped_gemm_at_the_edges_of_its_tiles(fa, rows_g, cols, counts)
+
+
+@pytest.mark.gpu
+def test_layer_whose_last_round_of_jobs_is_cut_in_two(fa):
+    """Sixteen workgroups a tile: the XCDs with one tile (or three) cut a round of sixteen jobs in two, tiles of one to
+    three halves among them, the last 32 rows missing."""
+    _moe_case(fa, fo.MXFP4, fo.MXFP4, 9, 2, 416, 4064, 420)
+
+
 def test_no_result_of_the_matrix_core_is_read_too_soon(tmp_path):
     import isa_mfma_lint
     from test_isa_waits import _assembly
