@@ -9,7 +9,7 @@
 // the activation first, because a wavefront's loads return in issue order and the activation comes from L2,
 // then its weights from HBM -- are issued before any arithmetic, so a CU holds tens of kilobytes in flight
 // instead of one loop iteration's worth.  Rows too long for either fall back to the looping kernels.
-#include "frk_device.hpp"
+#include "frk_experts_down.hpp"
 
 namespace frk {
 
@@ -365,6 +365,57 @@ __global__ __launch_bounds__(256) void gemv_q6_k_experts_kernel(const uint8_t *_
     }
 }
 
+// The same with the weighted sum of a token's experts (frk_experts_down.hpp): a lane's 64 weights of a row.
+struct Q6Unit {
+    static constexpr int PER_BLOCK = 4;
+    uint4 qla, qlb, qh;
+    uint2 sc;
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t *W, uint32_t row, const Layout &lay, int u) {
+        const uint32_t b = u >> 2, h = (u >> 1) & 1, t = u & 1;
+        qla = *reinterpret_cast<const uint4 *>(W + (row + b * 128 + h * 64 + t * 16));
+        qlb = *reinterpret_cast<const uint4 *>(W + (row + b * 128 + h * 64 + t * 16 + 32));
+        qh = *reinterpret_cast<const uint4 *>(W + (row + (uint32_t)lay.off_a + b * 64 + h * 32 + t * 16));
+        sc = *reinterpret_cast<const uint2 *>(W + (row + (uint32_t)lay.off_b + b * 16 + h * 8));
+        d = *reinterpret_cast<const uint16_t *>(W + (row + (uint32_t)lay.off_c + b * 2));
+    }
+    struct Act {
+        uint4 a0, a1, a2, a3;
+        int b1, b2, b3, b4, t;
+        float da;
+        __device__ __forceinline__ void load(const int8_t *q, const int16_t *sums, const float *scales, int u) {
+            const int b = u >> 2, h = (u >> 1) & 1;
+            t = u & 1;
+            const int8_t *at = q + b * QK_K + h * 128 + t * 16;
+            a0 = *reinterpret_cast<const uint4 *>(at), a1 = *reinterpret_cast<const uint4 *>(at + 32);
+            a2 = *reinterpret_cast<const uint4 *>(at + 64), a3 = *reinterpret_cast<const uint4 *>(at + 96);
+            const uint4 bs = *reinterpret_cast<const uint4 *>(sums + b * 16 + h * 8);
+            const int sh = 16 * t;
+            b1 = (int)(int16_t)(bs.x >> sh), b2 = (int)(int16_t)(bs.y >> sh);
+            b3 = (int)(int16_t)(bs.z >> sh), b4 = (int)(int16_t)(bs.w >> sh);
+            da = scales[b];
+        }
+    };
+    __device__ __forceinline__ float dot(const Act &a) const {
+        int d1 = 0, d2 = 0, d3 = 0, d4 = 0;
+#define FRK_Q6_STEP(c)                                                                      \
+    d1 = dot4((qla.c & 0x0f0f0f0fu) | ((qh.c << 4) & 0x30303030u), a.a0.c, d1);        \
+    d2 = dot4((qlb.c & 0x0f0f0f0fu) | ((qh.c << 2) & 0x30303030u), a.a1.c, d2);        \
+    d3 = dot4(((qla.c >> 4) & 0x0f0f0f0fu) | (qh.c & 0x30303030u), a.a2.c, d3);        \
+    d4 = dot4(((qlb.c >> 4) & 0x0f0f0f0fu) | ((qh.c >> 2) & 0x30303030u), a.a3.c, d4);
+        FRK_Q6_STEP(x)
+        FRK_Q6_STEP(y)
+        FRK_Q6_STEP(z)
+        FRK_Q6_STEP(w)
+#undef FRK_Q6_STEP
+        const uint32_t slo = a.t ? (sc.x >> 8) : sc.x, shi = a.t ? (sc.y >> 8) : sc.y;
+        const int s1 = (int)(int8_t)(slo & 0xff), s2 = (int)(int8_t)((slo >> 16) & 0xff);
+        const int s3 = (int)(int8_t)(shi & 0xff), s4 = (int)(int8_t)((shi >> 16) & 0xff);
+        const int isum = s1 * (d1 - 32 * a.b1) + s2 * (d2 - 32 * a.b2) + s3 * (d3 - 32 * a.b3) + s4 * (d4 - 32 * a.b4);
+        return (h2f(d) * a.da) * (float)isum;
+    }
+};
+
 // ------------------------------------------------------------------ Q8_0 x f32
 // dot_q8_0_f32 (crates/frink-quant/src/lib.rs:663-686) over the planar resident layout.
 // Unit = 16 quants (half a block).
@@ -665,6 +716,14 @@ int launch_gemv_q6_k_experts(const frk_weights *w, int n_experts, size_t rows_e,
 #undef FRK_GO
     FRK_LAUNCH_CHECK("gemv_q6_k_experts");
     return FRK_OK;
+}
+
+// out[token][rows_e] = sum over the slots of weights * (rows of expert ids) . act[token][slot]; rows of at most 8 blocks
+int launch_q6_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids, const float *weights,
+                             size_t batch, int k, float *out, hipStream_t s) {
+    if (w->cols <= 4 * QK_K) return launch_experts_down_as<Q6Unit, 16, 2, 4>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
+    if (w->cols <= 6 * QK_K) return launch_experts_down_as<Q6Unit, 32, 4, 6>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
+    return launch_experts_down_as<Q6Unit, 32, 4, 8>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
 }
 
 int launch_gemv_q8_0_f32_direct(const frk_weights *w, const float *x, float *y, hipStream_t s) {

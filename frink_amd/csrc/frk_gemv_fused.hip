@@ -9,7 +9,7 @@
 // return in order); the workgroup barrier in front of the arithmetic waits for LDS only, never
 // for the weight loads.  A lane multiplies the same columns in every row, so its slice of the
 // quantized activation is read once into registers.
-#include "frk_device.hpp"
+#include "frk_experts_down.hpp"
 
 namespace frk {
 
@@ -128,6 +128,32 @@ __device__ __forceinline__ float q4_k_unit_dot(const uint4 h, const uint4 w0, co
     const float d = h2f(h.x & 0xffffu), dmin = h2f(h.x >> 16);
     return (d * U.da) * (float)s1 - (dmin * U.da) * (float)s2;
 }
+
+// The unit for frk_experts_down.hpp.
+struct Q4ExpertsUnit {
+    static constexpr int PER_BLOCK = 2;
+    uint4 h, w0, w1, w2, w3;
+    __device__ __forceinline__ void load(const uint8_t *W, uint32_t row, const Layout &, int u) {
+        const uint4 *blk = reinterpret_cast<const uint4 *>(W + (row + (uint32_t)(u >> 1) * (uint32_t)Q4_K_BYTES));
+        const int q2 = 2 * (u & 1);
+        h = blk[0], w0 = blk[1 + q2], w1 = blk[2 + q2], w2 = blk[5 + q2], w3 = blk[6 + q2];
+    }
+    struct Act {
+        Q4Unit U;
+        __device__ __forceinline__ void load(const int8_t *q, const int16_t *sums, const float *scales, int u) {
+            const int b = u >> 1, half = u & 1;
+            const uint4 *ap = reinterpret_cast<const uint4 *>(q + b * QK_K + half * 64);
+#pragma unroll
+            for (int i = 0; i < 4; i++) U.a[i] = ap[i], U.a[4 + i] = ap[8 + i];
+            const int16_t *bp = sums + b * 16 + half * 4;
+            U.bs[0] = (int)bp[0] + (int)bp[1], U.bs[1] = (int)bp[2] + (int)bp[3];
+            U.bs[2] = (int)bp[8] + (int)bp[9], U.bs[3] = (int)bp[10] + (int)bp[11];
+            U.da = scales[b];
+            U.sh = half * 16;
+        }
+    };
+    __device__ __forceinline__ float dot(const Act &a) const { return q4_k_unit_dot(h, w0, w1, w2, w3, a.U); }
+};
 
 // dot_q5_k_q8 (crates/frink-quant/src/lib.rs:886-938) for one unit of one row: the same with every weight's fifth
 // bit put over its nibble (fa, fb: the block's 32 bytes of fifth bits, byte l holding weight l of every sub-block,
@@ -1146,6 +1172,13 @@ int launch_gemv_q4_k_experts(const frk_weights *w, const frk_weights *w2, int n_
     const Q8KActs none = {nullptr, nullptr, nullptr};
     if (w2) return launch_q4_k_fused<MODE_FUSED, true, false, true>(w, w2, x, none, y, s, rows_e, &ma, (unsigned)jobs, (unsigned)per_job);
     return launch_q4_k_fused<MODE_FUSED, false, false, true>(w, nullptr, x, none, y, s, rows_e, &ma, (unsigned)jobs, (unsigned)per_job);
+}
+// out[token][rows_e] = sum over the slots of weights * (rows of expert ids) . act[token][slot]; rows of at most 8 blocks
+int launch_q4_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids, const float *weights,
+                             size_t batch, int k, float *out, hipStream_t s) {
+    if (w->cols <= 4 * QK_K) return launch_experts_down_as<Q4ExpertsUnit, 8, 1, 4>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
+    if (w->cols <= 6 * QK_K) return launch_experts_down_as<Q4ExpertsUnit, 16, 2, 6>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
+    return launch_experts_down_as<Q4ExpertsUnit, 16, 2, 8>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
 }
 // act[r] = silu(gate[r] . x) * (up[r] . x): both matrices Q4_K of one shape, fused_gemv_fits
 int launch_gemv_q4_k_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s) {

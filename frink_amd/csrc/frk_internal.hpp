@@ -368,6 +368,12 @@ int launch_gemv_kquant_f32(const frk_weights *w, const float *x, float *y, hipSt
 bool q6_k_experts_gemv_fits(const frk_weights *w);
 int launch_gemv_q6_k_experts(const frk_weights *w, int n_experts, size_t rows_e, const float *x, size_t x_stride,
                              const int32_t *ids, size_t jobs, float *y, hipStream_t s);
+// a token's (or a few tokens') down projection with the weighted sum of its experts; down rows of at most 8 blocks
+constexpr size_t EXPERTS_DOWN_MAX_COLS = 8 * QK_K;
+int launch_q6_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids, const float *weights,
+                             size_t batch, int k, float *out, hipStream_t s);
+int launch_q4_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids, const float *weights,
+                             size_t batch, int k, float *out, hipStream_t s);
 int launch_gemv_q8_0_f32_direct(const frk_weights *w, const float *x, float *y, hipStream_t s);
 // thin batched GEMM of the K-quants: 1 <= batch <= thin_gemm_max_batch(w) rows per launch (0: does not fit)
 int thin_gemm_max_batch(const frk_weights *w);

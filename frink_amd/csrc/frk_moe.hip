@@ -602,6 +602,16 @@ static int launch_moe_ffn_per_token(const frk_weights *gate, const frk_weights *
     float *act = m.gate_out;  // [batch*k][ffn]
     int rc = launch_gemv_q4_k_experts(gate, up, n_experts, (size_t)ffn, x, (size_t)hidden, ids, batch, (size_t)k, act, s);
     if (rc) return rc;
+    // The weighted sum in the down projection's launch (frk_experts_down.hpp; offsets within an expert are 32 bits wide).
+    // Layer before / with it, us: one token of 128 experts top-8 of 2048 / 768 23.5 / 20.6 (bound by the host's calls), 16
+    // tokens 75 / 64 (Q6_K) and 77 / 61 (Q4_K), 8 tokens of 60 top-4 of 2048 / 1280 42 / 36.  Not for longer Q6_K rows of
+    // five to seven slots, whose wavefronts share a CU's SIMDs unevenly (top-6 of 2048 / 1536 at 3 tokens 34.0 / 34.4, of
+    // 2048 / 1280 at 6 46.4 / 48.2, at 12 78.3 / 79.3; top-8 at 3 tokens 40.8 / 39.6).
+    const bool uneven = down->kind == FRK_KIND_Q6_K && ffn > 4 * QK_K && k > 4 && k < 8 && batch > 2;
+    if (down->cols <= EXPERTS_DOWN_MAX_COLS && (size_t)hidden * down->layout.row_stride <= 0xffffffffu && !uneven)
+        return down->kind == FRK_KIND_Q6_K
+                   ? launch_q6_k_experts_down(down, n_experts, (size_t)hidden, act, ids, weights, batch, k, out, s)
+                   : launch_q4_k_experts_down(down, n_experts, (size_t)hidden, act, ids, weights, batch, k, out, s);
     rc = down->kind == FRK_KIND_Q6_K
              ? launch_gemv_q6_k_experts(down, n_experts, (size_t)hidden, act, (size_t)ffn, ids, batch * (size_t)k, m.down_out, s)
              : launch_gemv_q4_k_experts(down, nullptr, n_experts, (size_t)hidden, act, (size_t)ffn, ids, batch * (size_t)k, 1,
