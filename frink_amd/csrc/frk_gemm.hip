@@ -561,6 +561,28 @@ int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTile
     return n_rec <= 1024 ? launch_quantize_records<16>(x, rows, nb, nullptr, n_rec, out, s, plain)
                          : launch_quantize_records<4>(x, rows, nb, nullptr, n_rec, out, s, plain);
 }
+// Q8_K rows as the quantizer of a thin batch leaves them, in the tiled form: a record a workgroup
+__global__ __launch_bounds__(256) void tile_q8_k_kernel(Q8KActs a, int rows, int nb, Q8KTiled out) {
+    const int t32 = blockIdx.x / nb, kb = blockIdx.x % nb;
+    const size_t rec = (size_t)t32 * nb + kb;
+    for (int i = threadIdx.x; i < 512; i += 256) {  // 16-byte piece: slice i / 64, half i / 32 % 2, row i % 32
+        const int row = t32 * 32 + (i & 31);
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (row < rows) v = *reinterpret_cast<const uint4 *>(a.q + ((size_t)row * nb + kb) * QK_K + (i >> 6) * 32 + ((i >> 5) & 1) * 16);
+        reinterpret_cast<uint4 *>(out.q + rec * 8192)[i] = v;
+        const int sum_row = t32 * 32 + ((i >> 3) & 31), g = (i >> 8) * 8 + (i & 7);
+        out.bs[rec * 512 + i] = sum_row < rows ? (_Float16)a.bsums[((size_t)sum_row * nb + kb) * 16 + g] : (_Float16)0.0f;
+    }
+    const int row = t32 * 32 + (int)threadIdx.x;
+    if (threadIdx.x < 32) out.d[rec * 32 + threadIdx.x] = row < rows ? a.d[(size_t)row * nb + kb] : 0.0f;
+}
+int launch_tile_q8_k(const Q8KActs &a, size_t rows, size_t cols, Q8KTiled out, hipStream_t s) {
+    const size_t nb = cols / QK_K, n_rec = (rows + 31) / 32 * nb;
+    if (n_rec == 0) return FRK_OK;
+    hipLaunchKernelGGL(tile_q8_k_kernel, dim3((unsigned)n_rec), dim3(256), 0, s, a, (int)rows, (int)nb, out);
+    FRK_LAUNCH_CHECK("tile_q8_k");
+    return FRK_OK;
+}
 int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, size_t max_rows, Q8KTiled out,
                                 hipStream_t s) {
     const size_t nb = cols / QK_K, n_rec = max_rows / 32 * nb;
@@ -576,7 +598,7 @@ int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, 
 // equal share of them (deal_entry); splitting the blocks costs the second launch and its bytes.  The constants are a fit
 // (4 % rms) to 6079 launches over 1200 drawn shapes: the three kinds, 1024 .. 14336 rows and columns, 8 .. 2048 tokens,
 // 1 .. 8 parts.  Over the 720 of them with 48 tokens and more the choice is 0.2 % behind the best one measured on average,
-// 8 % at worst; with the constants fitted to one half and tried on the other likewise.  (Up to 64 tokens the small tile, the
+// 8 % at worst; with the constants fitted to one half and tried on the other likewise.  (33 .. 64 tokens the small tile, the
 // cheaper one there in every launch measured: its float step is the thin kernels', see fold_mins.)
 PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     struct Cost {
@@ -585,18 +607,36 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     // (a Q5_K or Q6_K block has three times Q4_K's vector instructions in its unpacking)
     const Cost small = kind == FRK_KIND_Q4_K ? Cost{1.62f, 0.74f, 3.26f} : Cost{2.41f, 0.77f, 4.06f};
     const Cost large = kind == FRK_KIND_Q4_K ? Cost{2.66f, 1.07f, 4.85f} : Cost{3.26f, 1.06f, 5.79f};
+    auto rounds_us = [](size_t wgs, float steps, Cost c) {
+        const float last = (float)(wgs % 256) / 256.0f;
+        return (float)(wgs / 256) * (steps * (c.step + c.load) + c.start) + (wgs % 256 ? steps * (c.step + c.load * last) + c.start : 0.0f);
+    };
     PipePlan best = {128, 64, 1};
     float best_us = 0.0f;
+    // Up to 32 tokens a tile of 64 rows x 32 tokens, four blocks a step: half the small tile's matrix instructions for the same
+    // weights.  The same estimate, fitted (3.6 % rms) to 1700 launches over 130 shapes: its choice is 0.1 % behind the
+    // best measured split on average and 3 % at worst.  With quantization, the small tile -> this one, us: Q4_K 14336x4096
+    // at 9 and 32 rows 20.0 -> 14.9 and 21.6 -> 15.9, 4096x11008 at 16 20.0 -> 16.9, Q5_K 4096x4096 at 32 17.7 -> 14.4, Q6_K
+    // 4096x11008 at 32 24.3 -> 21.3.
+    if (M <= 32) {
+        const Cost c = kind == FRK_KIND_Q4_K ? Cost{1.06f, 0.65f, 2.47f} : Cost{1.91f, 0.68f, 2.95f};
+        best = {64, 32, 1};
+        for (int ks : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
+            const size_t bytes = (size_t)ks * M * rows * sizeof(float);
+            if (ks > 1 && (nb / (size_t)ks < 2 || bytes > SPLIT_PARTS_BYTES)) continue;
+            const size_t wgs = (rows + 63) / 64 * (size_t)ks, blocks = (nb + (size_t)ks - 1) / (size_t)ks;
+            const float us = rounds_us(wgs, (float)((blocks + 3) / 4), c) + (ks > 1 ? 1.6f + 2.6e-7f * (float)bytes : 0.0f);
+            if (best_us == 0.0f || us < best_us) best_us = us, best.k_split = ks;
+        }
+        return best;
+    }
     for (int big = 0; big < (M > 64 ? 2 : 1); big++)
         for (int ks : {1, 2, 3, 4, 6, 8}) {
             const size_t bytes = (size_t)ks * M * rows * sizeof(float);
             if (ks > 1 && (nb / (size_t)ks < 2 || bytes > SPLIT_PARTS_BYTES)) continue;
             const size_t wgs = (big ? ((rows + 255) / 256) * ((M + 127) / 128) : ((rows + 127) / 128) * ((M + 63) / 64)) * (size_t)ks;
             const size_t blocks = (nb + (size_t)ks - 1) / (size_t)ks;
-            const float steps = (float)(big ? blocks : (blocks + 1) / 2), last = (float)(wgs % 256) / 256.0f;
-            const Cost c = big ? large : small;
-            float us = (float)(wgs / 256) * (steps * (c.step + c.load) + c.start);
-            if (wgs % 256) us += steps * (c.step + c.load * last) + c.start;
+            float us = rounds_us(wgs, (float)(big ? blocks : (blocks + 1) / 2), big ? large : small);
             if (ks > 1) us += 1.3f + 2.6e-7f * (float)bytes;
             if (best_us == 0.0f || us < best_us) {
                 best_us = us;
@@ -616,13 +656,13 @@ int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *
         return set_error(FRK_ERR_SHAPE, "matrix-core GEMM: rows of %zu bytes are beyond the kernel's offsets", w->layout.row_stride);
     const PipePlan p = pipe_plan(w->kind, w->rows, M, w->cols / QK_K);
     const GemmArgs g = pipe_args(w, acts, M, y, (float *)parts, p);
-    const bool big = p.rows_wg == 256;
-    if (w->kind == FRK_KIND_Q6_K) return launch_pipe_q6_k(g, big, s);
-    if (w->kind == FRK_KIND_Q5_K)
-        return big ? launch_pipe<FRK_KIND_Q5_K, 8, 1, 4>(gemm_q5_k_pipe_kernel<8, 1, 4>, g, s)
-                   : launch_pipe<FRK_KIND_Q5_K, 4, 2, 2>(gemm_q5_k_pipe_kernel<4, 2, 2>, g, s);
-    return big ? launch_pipe<FRK_KIND_Q4_K, 8, 1, 4>(gemm_q4_k_pipe_kernel<8, 1, 4>, g, s)
-               : launch_pipe<FRK_KIND_Q4_K, 4, 2, 2>(gemm_q4_k_pipe_kernel<4, 2, 2>, g, s);
+    if (w->kind == FRK_KIND_Q6_K) return launch_pipe_q6_k(g, p.rows_wg, s);
+#define FRK_GO(KIND, KERNEL)                                                                                       \
+    return p.rows_wg == 256   ? launch_pipe<KIND, 8, 1, 4>(KERNEL<8, 1, 4>, g, s)                                  \
+           : p.rows_wg == 128 ? launch_pipe<KIND, 4, 2, 2>(KERNEL<4, 2, 2>, g, s) : launch_pipe<KIND, 2, 4, 1>(KERNEL<2, 4, 1>, g, s)
+    if (w->kind == FRK_KIND_Q5_K) FRK_GO(FRK_KIND_Q5_K, gemm_q5_k_pipe_kernel);
+    FRK_GO(FRK_KIND_Q4_K, gemm_q4_k_pipe_kernel);
+#undef FRK_GO
 }
 
 template <int KIND, bool GATHER>

@@ -467,8 +467,8 @@ __device__ __forceinline__ v16i tile_chain(TileOperands &T, const BPlanes &B, Be
 //
 // A workgroup = 8 wavefronts = RG row groups of 32 weight rows x KS shares of the blocks; a wavefront
 // runs MT 32-token tiles against its rows' current block.  KS = 2 (small matrices: 128 rows x 64 tokens
-// per workgroup fill the chip where 256 x 128 would not) halves the blocks between two wavefronts whose
-// sums are added through LDS at the end, always the first half's plus the second half's.
+// per workgroup fill the chip where 256 x 128 would not) and KS = 4 (64 rows x 32 tokens) share the blocks
+// between wavefronts whose sums are added through LDS at the end, in the order of the shares.
 //
 // LDS: activations in a ring of 3 stages (requested two steps ahead), their scales in a ring of 4
 // (they are read by an epilogue that may run a step later), the raw weights in ONE slot per
@@ -657,7 +657,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     constexpr bool MINS = Side::MINS;
     constexpr int FORM = !MINS ? NO_MINS : MT == 4 ? MINS_FOLDED : MINS_APART;
     constexpr int NW = L::NW, NT = L::NT, ROWS = 32 * RG, TM = 32 * MT;
-    static_assert(NW == 8 && NT == 4 && (MT == 2 || MT == 4), "eight wavefronts share the four tile slots of a stage");
+    static_assert(NW == 8 && NT == 4 && (MT == 1 || MT == 2 || MT == 4), "eight wavefronts share the four tile slots of a stage");
     extern __shared__ uint4 smem_gemm[];
     uint8_t *lds = reinterpret_cast<uint8_t *>(smem_gemm);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
@@ -692,9 +692,9 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     // other four -- fetch the activations: wavefront f the record of tile slot f (8 KB of quants, 1 KB of
     // sums), wavefronts 0 and 1 the scales of two slots each.  Every wavefront fetches its own weight rows.
     const bool fetches_acts = wave < NT;
-    const bool fetches_scales = wave < 2;
+    const bool fetches_scales = wave < (MT == 1 ? 4 : 2);  // (MT 1: two slots are two shares' blocks, not two tiles of one)
     const uint32_t lane16 = (uint32_t)lane * 16;
-    const int slot_f = wave & 3, slot_d = (wave & 1) * 2;
+    const int slot_f = wave & 3, slot_d = MT == 1 ? wave & 3 : (wave & 1) * 2;
     // (a share past its last block keeps requesting that block: nobody multiplies it)
     int next_kb_a = kb0 + (slot_f / MT) * steps;  // the block of this wavefront's activation slot at the next request
     int next_kb_d = kb0 + (slot_d / MT) * steps;
@@ -706,7 +706,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     const uint8_t *src_d = (const uint8_t *)scalar_pointer(reinterpret_cast<const uint8_t *>(g.a.d) +
                                                            ((size_t)tile_of(slot_d) * nb + min(next_kb_d, kb1 - 1)) * 128);
     const uint32_t lane_d = (uint32_t)(lane & 31) * 4 +
-                            (lane >= 32 ? (uint32_t)(tile_of(slot_d + 1) - tile_of(slot_d)) * (uint32_t)nb * 128u : 0u);
+                            (MT > 1 && lane >= 32 ? (uint32_t)(tile_of(slot_d + 1) - tile_of(slot_d)) * (uint32_t)nb * 128u : 0u);
     Side wside;
     const int row_base = min(row_tile * ROWS + rg * 32, g.rows - 1);
     wside.offsets((uint32_t)g.row_stride, g.rows - 1 - row_base, lane);
@@ -720,7 +720,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     };
     auto fetch_sums_scales = [&]() {
         if (MINS) dma16_run<1>(st_fill + L::OFF_BS + slot_f * 1024, src_s, lane16, 0, 0, 0);
-        if (fetches_scales) dma4(da_fill + slot_d * 128, src_d, lane_d);
+        if (fetches_scales && (MT > 1 || lane < 32)) dma4(da_fill + slot_d * 128, src_d, lane_d);
     };
     auto acts_fetched = [&]() {  // the request for a step is out: everything moves on to the step after
         const bool adv_a = next_kb_a + 1 < kb1, adv_d = next_kb_d + 1 < kb1;
@@ -857,21 +857,23 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
         }
     }
 
-    // two shares of the blocks: the second half's sums go through LDS and are added onto the first's
-    if (KS == 2) {
-        float *xch = reinterpret_cast<float *>(lds) + (size_t)rg * MT * 16 * 64;
-        if (ks == 1) {
+    // several shares of the blocks: the later ones' sums go through LDS and are added onto the first's, in order
+    if (KS > 1) {
+        float *xch = reinterpret_cast<float *>(lds) + (size_t)rg * (KS - 1) * MT * 16 * 64;
+        if (ks > 0) {
 #pragma unroll
             for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) xch[(mt * 16 + r) * 64 + lane] = sum[mt][r];
+                for (int r = 0; r < 16; r++) xch[(((ks - 1) * MT + mt) * 16 + r) * 64 + lane] = sum[mt][r];
         }
         __syncthreads();
-        if (ks == 1) return;
+        if (ks > 0) return;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
+        for (int k = 0; k < KS - 1; k++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) sum[mt][r] += xch[(mt * 16 + r) * 64 + lane];
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) sum[mt][r] += xch[((k * MT + mt) * 16 + r) * 64 + lane];
     }
     // store: a lane holds one weight row and 16 tokens per tile
     const int row = row_tile * ROWS + rg * 32 + li;
@@ -888,7 +890,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
 
 // ------------------------------------------------------------------ host side
 
-// The workgroup tile of a batch: 256 rows x 128 tokens or 128 rows x 64 tokens, and how many workgroups share a row's
+// The workgroup tile of a batch: 256 rows x 128 tokens, 128 x 64 or 64 x 32, and how many workgroups share a row's
 // blocks (their sums, in SPLIT_PARTS_BYTES of memory at most, are added in order afterwards).
 struct PipePlan {
     int rows_wg, tok_wg, k_split;
@@ -912,7 +914,7 @@ int launch_pipe(void (*kernel)(GemmArgs), const GemmArgs &g, hipStream_t s) {
     return FRK_OK;
 }
 
-int launch_pipe_q6_k(const GemmArgs &g, bool big, hipStream_t s);  // frk_gemm_q6.hip
+int launch_pipe_q6_k(const GemmArgs &g, int rows_wg, hipStream_t s);  // frk_gemm_q6.hip
 
 // what a launch of one matrix over tiled activations needs, by its plan
 inline GemmArgs pipe_args(const frk_weights *w, Q8KTiled acts, size_t M, float *y, float *partial, const PipePlan &p) {

@@ -13,6 +13,9 @@ __global__ __launch_bounds__(512) void gemm_q6_k_pipe_kernel(GemmArgs g) {
     pipe_gemm<FRK_KIND_Q6_K, RG, KS, MT>(g);
 }
 
+// 64 rows x 32 tokens, for batches of up to 32 rows
+__global__ __launch_bounds__(512) void batch_q6_k_pipe_kernel(GemmArgs g) { pipe_gemm<FRK_KIND_Q6_K, 2, 4, 1>(g); }
+
 // y = the parts' sums added in the order of the parts: the same bits on every run
 __global__ __launch_bounds__(256) void sum_parts_kernel(const float *__restrict__ partial, int parts, size_t n,
                                                         float *__restrict__ y) {
@@ -30,9 +33,10 @@ int launch_sum_parts(const float *partial, int parts, size_t n, float *y, hipStr
     return FRK_OK;
 }
 
-int launch_pipe_q6_k(const GemmArgs &g, bool big, hipStream_t s) {
-    return big ? launch_pipe<FRK_KIND_Q6_K, 8, 1, 4>(gemm_q6_k_pipe_kernel<8, 1, 4>, g, s)
-               : launch_pipe<FRK_KIND_Q6_K, 4, 2, 2>(gemm_q6_k_pipe_kernel<4, 2, 2>, g, s);
+int launch_pipe_q6_k(const GemmArgs &g, int rows_wg, hipStream_t s) {
+    return rows_wg == 256   ? launch_pipe<FRK_KIND_Q6_K, 8, 1, 4>(gemm_q6_k_pipe_kernel<8, 1, 4>, g, s)
+           : rows_wg == 128 ? launch_pipe<FRK_KIND_Q6_K, 4, 2, 2>(gemm_q6_k_pipe_kernel<4, 2, 2>, g, s)
+                            : launch_pipe<FRK_KIND_Q6_K, 2, 4, 1>(batch_q6_k_pipe_kernel, g, s);
 }
 
 }  // namespace frk

@@ -227,6 +227,7 @@ struct Q8KActsOut {
 int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTiled out, hipStream_t s, Q8KActsOut plain = Q8KActsOut());
 // out row r = x[gather[r]] quantized (zeros where gather[r] < 0), for the 32-row records of the first
 // max_rows rows whose first entry is not negative
+int launch_tile_q8_k(const Q8KActs &a, size_t rows, size_t cols, Q8KTiled out, hipStream_t s);  // plain rows, tiled
 int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, size_t max_rows, Q8KTiled out,
                                 hipStream_t s);
 // A GEMM that splits a row's columns between workgroups keeps the parts' sums in at most this much memory, whichever entry

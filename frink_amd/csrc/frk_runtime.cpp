@@ -617,48 +617,66 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
     return set_error(FRK_ERR_UNSUPPORTED, "Q8_K activations feed Q4_K, Q5_K and Q6_K weights only (kind %d)", w->kind);
 }
 
-// From how many rows on a batch takes the matrix-core GEMM, whose cost is flat up to 64 rows; below that the thin
-// kernels' groups of 16 (Q4_K, Q5_K) or 8 rows are ahead, by what a group costs at the matrix's shape.  Measured with
-// quantization (us; thin / GEMM), nb blocks a row, rules beyond 17 / 33 / 41 rows within 32768 columns:
-//   Q4_K  a thin launch holds 8 rows from 32 blocks on.  nb > 32: 4096x11008 at 8, 9, 16 rows 14.8 / 19.7, 21.9 / 19.4, 25.3 / 19.7;
-//         1024x14336 at 9, 16 23.5 / 18.8, 28.0 / 19.2.  nb 24 .. 32 past one workgroup a CU: 5120x6144 at 9, 16 19.3 /
-//         16.2, 20.7 / 16.8, 14336x8192 38.7 / 27.7, 44.8 / 27.2, but 2048x8192 14.1 / 15.6, 14336x6144
-//         18.8 / 24.2.  Then by size: 14336x4096 at 17 20.4 / 19.6; 4096x4096 at 17, 32 13.3 / 14.8, 13.3 / 16.1.
-//   Q5_K  nb >= 32: 4096x11008 at 8, 9, 32 rows 16.3 / 23.2, 25.3 / 23.0, 51.1 / 24.7; 2048x8192 at 9, 32 20.2 / 18.5,
-//         41.2 / 19.7.  nb 16 .. 31 of few rows: 4096x4096 at 16, 17, 32 11.0 / 16.3, 20.4 / 16.4, 20.7 / 17.7; 5120x6144 at
-//         17 27.5 / 19.6, but 14336x4096 at 17, 32 21.1 / 23.9, 21.2 / 25.6.
-//   Q6_K  odd nb (not the streamed thin kernel's): 4096x11008 at 8, 9, 24 rows 18.3 / 24.3, 28.9 / 24.2, 42.1 / 25.2;
-//         2048x11008 at 16, 17, 33 17.4 / 23.4, 27.3 / 23.1, 39.1 / 24.6.  Even: 4096x14336 at 16, 17 22.5 / 27.4, 28.9 / 27.6;
-//         5120x8192 at 17, 25 23.2 / 23.8, 35.0 / 25.1; 8192x4096 at 17, 25 20.4 / 21.2, 25.0 / 22.1; 4096x4096 at 40 15.3 / 19.6.
-// Of 480 drawn matrices of 1024 .. 14336 rows and 2048 .. 14336 columns at 8 .. 40 rows, 273 take the GEMM here: the thin
-// kernels are ahead by more than 2 % for four of them, Q5_K of 8 .. 12 blocks past 33 rows (12 % at most).  Of the 207 that
-// stay, the GEMM would be ahead by more than 5 % for 52, most of them Q6_K of few rows and odd nb (1.8 times at most).
-// (No matrix starts below tiled_from(cols): a batch quantized without knowing its matrices has tiles from there on.)
+// Whether a batch takes the matrix-core GEMM.  Its cost is flat up to 32 rows (64 x 32 tiles) and up to 64; below, the thin
+// kernels' groups of 16 (Q4_K, Q5_K) or 8 rows are ahead by what a group costs at the matrix's shape.  nb blocks a row, with
+// quantization (us; thin / GEMM), within 32768 columns:
+//   Q4_K  from 17 rows on always (of 71 drawn matrices the GEMM is ahead for all: 14336x4096 at 17 19.6 / 14.9; 3335x5120, the
+//         closest, 0.92 of the time).  From 9 on rows of 30 blocks and more (1861x7680 at 9 0.98, 4096x11008 19.9 / 16.6) and,
+//         past one workgroup a CU, of 24: 4771x7168 0.72, but 1798x6144 1.07, 7986x5120 1.15.
+//   Q5_K  from 17 rows on (62 of 65 drawn ahead; 14257x2304 1.09, 4096x4096 at 17 20.4 / 13.4), and from 9 on rows of 32 blocks
+//         and more (4096x11008 25.3 / 19.3) and, past 4608 rows, of 24: 5230x6144 0.78, but 2491x6912 1.20.
+//   Q6_K  odd nb (not the streamed thin kernel's): from 9 on matrices of 18 M weights (4096x11008 at 13 28.9 / 19.7, 2631x7936
+//         0.67, but 1914x8960 at 16 1.08), at 17 of 8 M and more than 1280 rows (1822x5376 0.68, but 1144x8448 1.07), at 33 of 5 M.
+//         Even: from 9 on past 48 M and 4096 rows (4207x12288 0.81, but 4096x14336 20.1 / 22.2), at 17 past 23 M (6574x6144
+//         0.79, 2015x12800 0.92, but 4788x4096 1.11), at 25 past 17 M (4788x4096 0.98, but 1897x6656 1.05).
+// (Below tiled_from(cols) none: a batch quantized without knowing its matrices has tiles from there on.)
 static size_t tiled_from(size_t cols) { return cols >= 24 * QK_K ? 9 : 17; }
-static size_t matrix_cores_from(const frk_weights *w) {
-    const size_t n = w->rows * w->cols, nb = w->cols / QK_K;
+static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
+    if (batch < tiled_from(w->cols)) return false;
+    const size_t n = w->rows * w->cols, nb = w->cols / QK_K, M = (size_t)1 << 20;
     const bool measured = nb <= 128;
     if (w->kind == FRK_KIND_Q4_K) {
-        const bool eights = thin_gemm_max_batch(w) < 16;
-        if (measured && (nb > 32 || (nb >= 24 && w->rows > 4096 && (eights || w->rows <= 8192)))) return 9;
-        return n > (size_t)20 << 20 || eights ? 17 : 33;
+        const bool eights = thin_gemm_max_batch(w) < 16;  // rows of a thin launch
+        if (batch >= 17) return measured || batch >= 33 || n > 20 * M || eights;
+        return measured && (nb >= 30 || (nb >= 24 && w->rows > 4096 && (eights || w->rows <= 8192)));
     }
-    if (w->kind == FRK_KIND_Q5_K) return measured && nb >= 32 ? 9 : measured && nb >= 16 && w->rows <= 6144 ? 17 : 33;
-    if (w->kind != FRK_KIND_Q6_K) return SIZE_MAX;
-    const bool large = n > (size_t)32 << 20;
-    if (measured && nb % 2) return large ? 9 : n > (size_t)20 << 20 ? 17 : 41;
-    if (measured && n > (size_t)48 << 20) return 17;
-    return large || (measured && n >= (size_t)30 << 20) ? 25 : 41;
+    if (w->kind == FRK_KIND_Q5_K) {
+        if (batch >= 17) return batch >= 33 || (measured && (nb >= 10 || w->rows <= 8192));
+        return measured && (nb >= 32 || (nb >= 24 && w->rows > 4608));
+    }
+    if (w->kind != FRK_KIND_Q6_K) return false;
+    if (batch >= 41) return true;
+    if (measured && nb % 2) {
+        if (batch >= 33) return n > 5 * M;
+        return n > 18 * M || (batch >= 17 && n > 8 * M && w->rows > 1280);
+    }
+    if (batch >= 25) return n > 32 * M || (measured && n > (batch >= 33 ? 23 : 17) * M);
+    if (batch >= 17) return measured && n > 23 * M;
+    return measured && n > 48 * M && w->rows > 4096;
 }
-static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
-    return batch >= std::max(matrix_cores_from(w), tiled_from(w->cols));
+// The crossings against the 128 x 64 tiles, higher than those above.  frk_hip_gemm_q8k_dev takes the batches below them (a
+// batch between the two is put into the tiled form first, so that it has frk_hip_gemm_dev's bits), and a batch between
+// the two whose scratch memory cannot be had -- a stream under capture -- goes where it went before.
+static bool matrix_cores_only(const frk_weights *w, size_t batch) {
+    const size_t n = w->rows * w->cols, nb = w->cols / QK_K, M = (size_t)1 << 20;
+    const bool measured = nb <= 128;
+    size_t from;
+    if (w->kind == FRK_KIND_Q4_K) {
+        const bool eights = thin_gemm_max_batch(w) < 16;
+        from = measured && (nb > 32 || (nb >= 24 && w->rows > 4096 && (eights || w->rows <= 8192))) ? 9 : n > 20 * M || eights ? 17 : 33;
+    } else if (w->kind == FRK_KIND_Q5_K) {
+        from = measured && nb >= 32 ? 9 : measured && nb >= 16 && w->rows <= 6144 ? 17 : 33;
+    } else if (measured && nb % 2) {
+        from = n > 32 * M ? 9 : n > 20 * M ? 17 : 41;
+    } else {
+        from = measured && n > 48 * M ? 17 : n > 32 * M || (measured && n >= 30 * M) ? 25 : 41;
+    }
+    return batch >= std::max(from, tiled_from(w->cols));
 }
-// whether a batch of this matrix multiplies on the thin kernels (over plain Q8_K rows)
-static bool batch_takes_the_thin_kernels(const frk_weights *w, size_t batch) {
+// whether the thin kernels hold a batch of this matrix (over plain Q8_K rows)
+static bool thin_kernels_hold(const frk_weights *w, size_t batch) {
     const bool k_quant = w->kind == FRK_KIND_Q4_K || w->kind == FRK_KIND_Q5_K || w->kind == FRK_KIND_Q6_K;
-    if (!k_quant || batch < 2) return false;
-    if (k_quant_takes_the_matrix_cores(w, batch)) return false;
-    return thin_gemm_max_batch(w) >= 2;
+    return k_quant && batch >= 2 && !matrix_cores_only(w, batch) && thin_gemm_max_batch(w) >= 2;
 }
 
 // a thin batch over activations already in Q8_K: `thin` rows a launch (thin_gemm_max_batch), or one launch over a
@@ -754,11 +772,14 @@ static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *
         hipStream_t s = (hipStream_t)stream;
         void *ws = nullptr, *parts = nullptr;
         int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts);
-        if (rc) return rc;
-        const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
-        rc = launch_quantize_q8_k_tiled(x, batch, w->cols, acts, s);
-        if (rc) return rc;
-        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        if (rc == FRK_OK) {
+            const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
+            rc = launch_quantize_q8_k_tiled(x, batch, w->cols, acts, s);
+            if (rc) return rc;
+            return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        }
+        if (matrix_cores_only(w, batch)) return rc;
+        clear_error();
     }
     // Q8_0: a batch is the integer path, as in the reference (Q8_0 activation blocks and dot_q8_0_q8,
     // crates/frink-core/src/weight_matrix.rs:2701-2829); a single row keeps the f32 dot of its decode path
@@ -773,7 +794,7 @@ static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *
     // (row, activation) over activations quantized once, crates/frink-core/src/weight_matrix.rs:392-420)
     if (is_unit_kind(w->kind) && batch >= 2) return gemm_units_int(w, x, batch, y, (hipStream_t)stream, scratch);
     // thin batches of the K-quants: the weights are read once per 8 (Q6_K) or 16 (Q4_K) activation rows
-    if (batch_takes_the_thin_kernels(w, batch)) {
+    if (thin_kernels_hold(w, batch)) {
         const int thin = thin_gemm_max_batch(w);
         Q8KActs a;
         int rc = quantize_acts_q8_k(w, x, batch, (hipStream_t)stream, scratch, &a);
@@ -819,12 +840,25 @@ int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
     if (batch == 1) return frk_hip_gemv_q8k_dev(w, q, d, bsums, y, stream);
     const bool k_quant = w->kind == FRK_KIND_Q4_K || w->kind == FRK_KIND_Q5_K || w->kind == FRK_KIND_Q6_K;
     if (!k_quant) return set_error(FRK_ERR_UNSUPPORTED, "Q8_K activations feed Q4_K, Q5_K and Q6_K weights only (kind %d)", w->kind);
-    if (!batch_takes_the_thin_kernels(w, batch))
+    if (!thin_kernels_hold(w, batch))
         return set_error(FRK_ERR_UNSUPPORTED,
                          "a batch of %zu rows of this matrix does not multiply on the thin kernels (the matrix-core GEMM "
                          "quantizes into a tiled form of its own): frk_hip_gemm_dev / frk_hip_gemm_pair_dev", batch);
     Q8KActs a{q, d, bsums};
-    return thin_gemm_acts(w, a, batch, thin_gemm_max_batch(w), y, (hipStream_t)stream);
+    hipStream_t s = (hipStream_t)stream;
+    if (k_quant_takes_the_matrix_cores(w, batch)) {
+        void *ws = nullptr, *parts = nullptr;
+        Scratch scratch;
+        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts);
+        if (rc == FRK_OK) {
+            const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
+            rc = launch_tile_q8_k(a, batch, w->cols, acts, s);
+            if (rc) return rc;
+            return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        }
+        clear_error();
+    }
+    return thin_gemm_acts(w, a, batch, thin_gemm_max_batch(w), y, s);
 }
 
 int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const float *x, size_t batch, float *y0, float *y1,
@@ -843,13 +877,16 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
         const size_t part1 = pipe_gemm_parts_bytes(w1->kind, batch, w1->cols, w1->rows);
         void *ws = nullptr, *parts = nullptr;
         int rc = scratch.get(acts_bytes, part0 + part1, s, &ws, &parts);
-        if (rc) return rc;
-        const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
-        rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
-        if (rc) return rc;
-        rc = launch_pipe_gemm_acts(w0, acts, batch, y0, parts, s);
-        if (rc) return rc;
-        return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)parts + part0, s);
+        if (rc == FRK_OK) {
+            const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
+            rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
+            if (rc) return rc;
+            rc = launch_pipe_gemm_acts(w0, acts, batch, y0, parts, s);
+            if (rc) return rc;
+            return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)parts + part0, s);
+        }
+        if (matrix_cores_only(w0, batch) && matrix_cores_only(w1, batch)) return rc;
+        clear_error();
     }
     // otherwise each matrix takes the path frk_hip_gemm_dev gives it (the same results, two quantizations)
     int rc = gemm_impl(w0, x, batch, y0, stream, scratch);
@@ -953,17 +990,17 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *a, float *
         const size_t parts_bytes = pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows);
         void *parts = nullptr;
         Scratch scratch;
-        if (parts_bytes) {  // a split of the blocks between workgroups: room for the parts' sums
-            int rc = scratch.get(parts_bytes, s, &parts);
-            if (rc) return rc;
-        }
-        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        int rc = FRK_OK;
+        if (parts_bytes) rc = scratch.get(parts_bytes, s, &parts);  // a split of the blocks between workgroups: room for the parts' sums
+        if (rc == FRK_OK) return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        if (matrix_cores_only(w, batch)) return rc;
+        clear_error();
     }
     // (below the matrix-core GEMMs' batches the plain rows are there: ACTS_PLAIN_MAX_BATCH covers every such batch)
     if (batch > ACTS_PLAIN_MAX_BATCH)
         return set_error(FRK_ERR_UNSUPPORTED, "a batch of %zu rows of this matrix has no kernel over quantized activations", batch);
     if (batch == 1) return frk_hip_gemv_q8k_dev(w, a->plain.q, a->plain.d, a->plain.bsums, y, stream);
-    if (batch_takes_the_thin_kernels(w, batch)) return thin_gemm_acts(w, a->plain, batch, thin_gemm_max_batch(w), y, s);
+    if (thin_kernels_hold(w, batch)) return thin_gemm_acts(w, a->plain, batch, thin_gemm_max_batch(w), y, s);
     const size_t nb = w->cols / QK_K;  // rows too long for the thin kernels: a decode launch per row
     for (size_t b = 0; b < batch; b++) {
         int rc = frk_hip_gemv_q8k_dev(w, a->plain.q + b * w->cols, a->plain.d + b * nb, a->plain.bsums + b * nb * 16, y + b * w->rows, stream);
