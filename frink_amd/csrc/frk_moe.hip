@@ -101,6 +101,28 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *wave_tot, int &t
     return base + inc - v;
 }
 
+// The same for three counts at once, packed: `count` below 2^24 in all, `big` and `small` below 2^20 each.
+__device__ __forceinline__ uint64_t block_exclusive_scan3(uint64_t v, uint64_t *wave_tot, uint64_t &total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint64_t inc = v;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        const uint64_t o = __shfl_up(inc, m);
+        if (lane >= m) inc += o;
+    }
+    if (lane == 63) wave_tot[wave] = inc;
+    lds_barrier();
+    uint64_t base = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < 16; w++) {
+        const uint64_t t = wave_tot[w];
+        if (w < wave) base += t;
+        tot += t;
+    }
+    total = tot;
+    return base + inc - v;
+}
+
 // Buckets the batch*k (token, slot) pairs by expert, pairs ascending inside a bucket (which is tokens
 // ascending: pairs are token-major).  A bucket is cut into tiles of MOE_TILE rows; tile t is rows
 // [MOE_TILE*t, MOE_TILE*(t+1)) of the grouped order and belongs to one expert, so the order has gaps.
@@ -124,6 +146,7 @@ struct GroupLds {
     int cnt[1024], off_cmp[1024], run[1024];
     int tile_big[1024], n_big[1024], tile_small[1024], seg_sum[1024];  // first heavy tile, their number, the light tile
     int wave_tot[16];
+    uint64_t wave_tot3[16];
 };
 struct GroupArgs {
     const int32_t *ids;
@@ -133,6 +156,98 @@ struct GroupArgs {
     int *n_tiles;
     int max_rows;
 };
+constexpr int HELD_IDS = 4;  // a thread's (eight, for 8192 pairs: 2 to 4 us slower at any size)
+// Up to 4096 pairs whose bits fit one round: the counts come out of the bit matrix itself, the three scans are one, a
+// row's words are read once and all of a thread's together, and the barriers wait for LDS only.  (512 tokens top-8 of 128 experts,
+// with the quantization beside it: 12.8 us under the profiler, now 9.9.)
+template <int TILE>
+__device__ __forceinline__ void moe_group_one_round(const GroupArgs &a, GroupLds &L, const int (&held)[HELD_IDS], int rw) {
+    const int pairs = a.pairs, n_experts = a.n_experts, tid = threadIdx.x;
+    for (int r = tid; r < a.max_rows; r += 1024) a.gather[r] = -1;
+    for (int i = tid; i < rw * n_experts; i += 1024) L.bits[i] = 0;
+    L.cnt[tid] = 0;
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < HELD_IDS; i++) {
+        const int p = tid + 1024 * i, e = held[i];
+        if (e >= 0 && e < n_experts) atomicOr(&L.bits[(p >> 5) * n_experts + e], 1u << (p & 31));
+    }
+    lds_barrier();
+    // the set bits of a run of every row's words, a thread a run
+    const int segs = max(1, 1024 / n_experts), ws = (rw + segs - 1) / segs;
+    const int e = tid % n_experts, seg = tid / n_experts;
+    const int w0 = min(rw, seg * ws), w1 = seg < segs ? min(rw, w0 + ws) : w0;
+    uint32_t words[16];  // (a second set where a run is longer: at most 32, n_experts > 512)
+    int sum = 0;
+    for (int half = 0; half < 2; half++) {
+        if (16 * half >= ws) break;  // uniform
+#pragma unroll
+        for (int i = 0; i < 16; i++) words[i] = L.bits[min(w0 + 16 * half + i, rw - 1) * n_experts + e];
+#pragma unroll
+        for (int i = 0; i < 16; i++) sum += w0 + 16 * half + i < w1 ? __popc(words[i]) : 0;
+    }
+    L.seg_sum[tid] = sum;
+    if (seg < segs) atomicAdd(&L.cnt[e], sum);
+    lds_barrier();
+    const int c = tid < n_experts ? L.cnt[tid] : 0;
+    const int nt = (c + TILE - 1) / TILE;
+    const int last = c - TILE * (nt - 1);  // rows in use of the last tile (nt > 0)
+    const int big = nt == 0 ? 0 : nt - 1 + (last > TILE - 32);
+    const int small = nt - big;  // 0 or 1
+    uint64_t total;
+    const uint64_t at = block_exclusive_scan3((uint64_t)c | (uint64_t)big << 24 | (uint64_t)small << 44, L.wave_tot3, total);
+    const int total_big = (int)(total >> 24) & 0xfffff, n_tiles = total_big + (int)(total >> 44);
+    const int o = (int)at & 0xffffff, tb = (int)(at >> 24) & 0xfffff, ts = total_big + (int)(at >> 44);
+    L.off_cmp[tid] = o;
+    L.tile_big[tid] = tb;
+    L.n_big[tid] = big;
+    L.tile_small[tid] = ts;
+    {
+        int run = 0;
+        for (int s2 = 0; s2 < seg && seg < segs; s2++) run += L.seg_sum[s2 * n_experts + e];
+        for (int half = 0; half < 2; half++) {
+            if (16 * half >= ws) break;  // uniform
+            if (ws > 16) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) words[i] = L.bits[min(w0 + 16 * half + i, rw - 1) * n_experts + e];
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int w = w0 + 16 * half + i;
+                if (w < w1) L.before[w * n_experts + e] = (unsigned short)run;
+                run += __popc(words[i]);
+            }
+        }
+    }
+    __syncthreads();  // (and the fill of the gather list is behind)
+    if (tid < n_experts) {
+        a.group_off[tid] = o;
+        for (int i = 0; i < nt; i++) {
+            const int t = i < big ? tb + i : ts;
+            a.tiles[t] = make_int4(tid, TILE * t, min(TILE, c - TILE * i), TILE * t);
+        }
+    }
+    if (tid == 0) {
+        a.group_off[n_experts] = (int)total & 0xffffff;
+        *a.n_tiles = n_tiles;
+    }
+#pragma unroll
+    for (int i = 0; i < HELD_IDS; i++) {
+        const int p = tid + 1024 * i, id = held[i];
+        if (p >= pairs) break;
+        if (id < 0 || id >= n_experts) {
+            a.pos_of[p] = a.cpos_of[p] = -1;
+            continue;
+        }
+        const int w = (p >> 5) * n_experts + id;
+        const int rank = L.before[w] + __popc(L.bits[w] & ((1u << (p & 31)) - 1u));
+        const int j = rank / TILE;
+        const int pos = TILE * (j < L.n_big[id] ? L.tile_big[id] + j : L.tile_small[id]) + rank % TILE;
+        a.gather[pos] = p / a.k;
+        a.pos_of[p] = pos;
+        a.cpos_of[p] = L.off_cmp[id] + rank;
+    }
+}
 template <int TILE>
 __device__ __forceinline__ void moe_group(const GroupArgs &a) {
     const int32_t *__restrict__ ids = a.ids;
@@ -143,15 +258,22 @@ __device__ __forceinline__ void moe_group(const GroupArgs &a) {
     extern __shared__ uint4 smem_group[];
     GroupLds &L = *reinterpret_cast<GroupLds *>(smem_group);
     const int tid = threadIdx.x;
+    // the first 4096 ids stay in registers for all passes (each pass from memory costs a
+    // round trip this one-workgroup kernel has nothing to hide behind)
+    int held[HELD_IDS];
+#pragma unroll
+    for (int i = 0; i < HELD_IDS; i++) held[i] = tid + 1024 * i < pairs ? ids[tid + 1024 * i] : -1;
+    // words per row; `before` is 16 bits wide, so a round stays below 65536 pairs
+    const int rw = max(1, min(min(GROUP_BIT_WORDS / n_experts, 2047), (pairs + 31) / 32));
+    const int round = rw * 32;
+    if (round >= pairs && pairs <= 1024 * HELD_IDS) {
+        moe_group_one_round<TILE>(a, L, held, rw);
+        return;
+    }
     L.cnt[tid] = 0;
     L.run[tid] = 0;
     for (int r = tid; r < max_rows; r += 1024) gather[r] = -1;
     __syncthreads();
-    // the first 4096 ids stay in registers for all three passes (each pass from memory costs a
-    // round trip this one-workgroup kernel has nothing to hide behind)
-    int held[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) held[i] = tid + 1024 * i < pairs ? ids[tid + 1024 * i] : -1;
     auto id_of = [&](int p) {  // p = tid (mod 1024)
         const int i = p >> 10;
         return i == 0 ? held[0] : i == 1 ? held[1] : i == 2 ? held[2] : i == 3 ? held[3] : ids[p];
@@ -189,9 +311,6 @@ __device__ __forceinline__ void moe_group(const GroupArgs &a) {
             *n_tiles = total_big + total_small;
         }
     }
-    // words per row; `before` is 16 bits wide, so a round stays below 65536 pairs
-    const int rw = max(1, min(min(GROUP_BIT_WORDS / n_experts, 2047), (pairs + 31) / 32));
-    const int round = rw * 32;
     for (int p0 = 0; p0 < pairs; p0 += round) {
         for (int i = tid; i < rw * n_experts; i += 1024) L.bits[i] = 0;
         __syncthreads();
