@@ -383,20 +383,23 @@ __global__ __launch_bounds__(1024) void moe_group_quantize_kernel(GroupArgs a, c
     }
 }
 
-// The same beside the digits of MXFP4 expert layers: eight token rows a workgroup (one after the other, the bucketing
-// 9 us and the digits 8 stood in front of every such layer).
+// The same beside the digits of MXFP4 expert layers: two token rows a workgroup (one after the other, the bucketing
+// 9 us and the digits 8 stood in front of every such layer; eight rows of 128 threads each, in three trips to memory on a
+// quarter of the CUs, 13.5 us for 512 rows of 2880 columns, now 11.4).
+constexpr int MX_TOKENS = 2;
 template <int TILE>
 __global__ __launch_bounds__(1024) void moe_group_quantize_mx_kernel(GroupArgs a, const float *__restrict__ x, int rows, int nb, MxActs out) {
-    __shared__ int infinite[8];
+    __shared__ int infinite[MX_TOKENS];
     if (blockIdx.x == 0) {
         moe_group<TILE>(a);
         return;
     }
-    const int sub = threadIdx.x >> 7;
-    if (threadIdx.x < 8) infinite[threadIdx.x] = 0;
+    constexpr int THREADS = 1024 / MX_TOKENS;
+    const int sub = threadIdx.x / THREADS;
+    if (threadIdx.x < MX_TOKENS) infinite[threadIdx.x] = 0;
     __syncthreads();
     // (past the end the last row again: the same bytes)
-    quantize_mx_row(x, min(((int)blockIdx.x - 1) * 8 + sub, rows - 1), nb, threadIdx.x & 127, &infinite[sub], out);
+    quantize_mx_row(x, min(((int)blockIdx.x - 1) * MX_TOKENS + sub, rows - 1), nb, threadIdx.x % THREADS, THREADS, &infinite[sub], out);
 }
 
 // The grouped GEMM with the groups given (enqueue_mul_mm_grouped_dev, crates/frink-cuda/src/mul_mm_launch.rs:391-470):
@@ -1101,7 +1104,7 @@ int launch_moe_ffn_units_grouped(const frk_weights *gate, const frk_weights *up,
     int rc;
     if (native.gate_up) {
         const MxActs xa = mx_acts_carve(m.x_acts, batch, hidden);
-        const dim3 grid(1 + (unsigned)((batch + 7) / 8));
+        const dim3 grid(1 + (unsigned)((batch + MX_TOKENS - 1) / MX_TOKENS));
         if (native.tile == MX_TILE)
             hipLaunchKernelGGL(moe_group_quantize_mx_kernel<MX_TILE>, grid, dim3(1024), sizeof(GroupLds), s, ga, x, (int)batch, hidden / 32, xa);
         else

@@ -25,14 +25,14 @@ __device__ __forceinline__ uint32_t mx_digit_codes(int v) {
 }
 
 // quantize_activations_q8, Avx form (crates/frink-quant/src/act_quant.rs:157-189), and the digits of quant * scale.
-// 128 threads (tid) of a workgroup per row, four lanes per block, a lane elements 4i .. 4i+3 and 16+4i .. 16+4i+3: eight
+// `threads` threads (tid; whole wavefronts) of a workgroup per row, four lanes per block, a lane elements 4i .. 4i+3 and 16+4i .. 16+4i+3: eight
 // neighbours in the digits' order, 48 bits of a plane.  `flag`: a word of LDS per row, zero before; a workgroup's rows meet
 // at one barrier.
 // A block whose scale overflows f16 (a largest value above 8.3e6; its E8M0 bytes start at MX_INFINITE) makes an infinity of
 // its integer sum, NaN where that is zero.  A row with such blocks is marked in `infinite`, and they keep their 32 quants as
 // bytes where the digits of a block would start: the GEMM ends with such rows on their own.
 constexpr uint32_t MX_INFINITE = 31 + 104;
-__device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int row, int nb, int tid, int *flag, const MxActs &out) {
+__device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int row, int nb, int tid, int threads, int *flag, const MxActs &out) {
     const int nbp = (nb + 7) & ~7, part = tid & 3;
     const float *xr = x + (size_t)row * nb * 32;
     float e[8];  // this lane's elements of a block
@@ -57,7 +57,7 @@ __device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int
         return (r != r) ? 0 : (int)fminf(fmaxf(r, -127.0f), 127.0f);
     };
     int infinite = 0;
-    for (int b = tid >> 2; b < nbp; b += 32) {
+    for (int b = tid >> 2; b < nbp; b += threads >> 2) {
         const uint32_t d = load(b);
         const int ex = (int)(d >> 10), mant = (int)(d & 1023u) | (ex ? 1024 : 0);
         infinite |= ex == 31;
@@ -106,7 +106,7 @@ __device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int
     __syncthreads();
     const bool row_infinite = *flag != 0;
     if (row_infinite)  // (over digits of the row that nobody will look at)
-        for (int b = tid >> 2; b < nb; b += 32) {
+        for (int b = tid >> 2; b < nb; b += threads >> 2) {
             if (load(b) >> 10 != 31) continue;
             auto bytes = [&](int i) {
                 return (uint32_t)(quant(i) & 0xff) | (uint32_t)(quant(i + 2) & 0xff) << 8 | (uint32_t)(quant(i + 4) & 0xff) << 16 | (uint32_t)(quant(i + 6) & 0xff) << 24;
