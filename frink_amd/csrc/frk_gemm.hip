@@ -558,8 +558,9 @@ static int launch_quantize_records(const float *x, size_t rows, size_t nb, const
 int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTiled out, hipStream_t s, Q8KActsOut plain) {
     const size_t nb = cols / QK_K, n_rec = (rows + 31) / 32 * nb;
     if (n_rec == 0) return FRK_OK;
-    return n_rec <= 1024 ? launch_quantize_records<16>(x, rows, nb, nullptr, n_rec, out, s, plain)
-                         : launch_quantize_records<4>(x, rows, nb, nullptr, n_rec, out, s, plain);
+    // (sixteen wavefronts a record, two rows each, at every size, us under the profiler, sixteen / eight / four: 512x4096 5.9 / 7.1 /
+    // 10.2, 512x14336 10.4 / 12.0 / 14.0, 700x12288 10.6 / 12.0 / 13.5, 2000x8192 16.8 / 18.6 / 22.0)
+    return launch_quantize_records<16>(x, rows, nb, nullptr, n_rec, out, s, plain);
 }
 // Q8_K rows as the quantizer of a thin batch leaves them, in the tiled form: a record a workgroup
 __global__ __launch_bounds__(256) void tile_q8_k_kernel(Q8KActs a, int rows, int nb, Q8KTiled out) {
