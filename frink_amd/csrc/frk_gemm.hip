@@ -601,6 +601,11 @@ int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, 
 // 1 .. 8 parts.  Over the 720 of them with 48 tokens and more the choice is 0.2 % behind the best one measured on average,
 // 8 % at worst; with the constants fitted to one half and tried on the other likewise.  (33 .. 64 tokens the small tile, the
 // cheaper one there in every launch measured: its float step is the thin kernels', see fold_mins.)
+// The last token tile of 128 multiplies only the 32-token tiles that have rows in use (three, two and one of four measured at 0.85, 0.7
+// and 0.55 of a full block's time) and may be split into parts of its own number, so that its workgroups take about as long as the
+// others: 197 tokens of 11008 x 4096 in Q5_K, three parts of the first tile and two of the second in one round of 215 workgroups,
+// 47.9 -> 44.7 us; 96 of 14336 x 8192 in Q4_K 50.3 -> 42.4.  Over 350 drawn shapes of 33 .. 2048 tokens 0.984 of the time, 0.79 at
+// best; none slower by more than two runs differ (4 %).
 PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     struct Cost {
         float step, load, start;
@@ -612,7 +617,7 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
         const float last = (float)(wgs % 256) / 256.0f;
         return (float)(wgs / 256) * (steps * (c.step + c.load) + c.start) + (wgs % 256 ? steps * (c.step + c.load * last) + c.start : 0.0f);
     };
-    PipePlan best = {128, 64, 1};
+    PipePlan best = {128, 64, 1, 1};
     float best_us = 0.0f;
     // Up to 32 tokens a tile of 64 rows x 32 tokens, four blocks a step: half the small tile's matrix instructions for the same
     // weights.  The same estimate, fitted (3.6 % rms) to 1700 launches over 130 shapes: its choice is 0.1 % behind the
@@ -621,34 +626,52 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     // 4096x11008 at 32 24.3 -> 21.3.
     if (M <= 32) {
         const Cost c = kind == FRK_KIND_Q4_K ? Cost{1.06f, 0.65f, 2.47f} : Cost{1.91f, 0.68f, 2.95f};
-        best = {64, 32, 1};
+        best = {64, 32, 1, 1};
         for (int ks : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
             const size_t bytes = (size_t)ks * M * rows * sizeof(float);
             if (ks > 1 && (nb / (size_t)ks < 2 || bytes > SPLIT_PARTS_BYTES)) continue;
             const size_t wgs = (rows + 63) / 64 * (size_t)ks, blocks = (nb + (size_t)ks - 1) / (size_t)ks;
             const float us = rounds_us(wgs, (float)((blocks + 3) / 4), c) + (ks > 1 ? 1.6f + 2.6e-7f * (float)bytes : 0.0f);
-            if (best_us == 0.0f || us < best_us) best_us = us, best.k_split = ks;
+            if (best_us == 0.0f || us < best_us) best_us = us, best.k_split = best.k_last = ks;
         }
         return best;
     }
-    for (int big = 0; big < (M > 64 ? 2 : 1); big++)
-        for (int ks : {1, 2, 3, 4, 6, 8}) {
-            const size_t bytes = (size_t)ks * M * rows * sizeof(float);
-            if (ks > 1 && (nb / (size_t)ks < 2 || bytes > SPLIT_PARTS_BYTES)) continue;
-            const size_t wgs = (big ? ((rows + 255) / 256) * ((M + 127) / 128) : ((rows + 127) / 128) * ((M + 63) / 64)) * (size_t)ks;
-            const size_t blocks = (nb + (size_t)ks - 1) / (size_t)ks;
-            float us = rounds_us(wgs, (float)(big ? blocks : (blocks + 1) / 2), big ? large : small);
-            if (ks > 1) us += 1.3f + 2.6e-7f * (float)bytes;
-            if (best_us == 0.0f || us < best_us) {
-                best_us = us;
-                best = big ? PipePlan{256, 128, ks} : PipePlan{128, 64, ks};
+    for (int big = 0; big < (M > 64 ? 2 : 1); big++) {
+        const Cost c = big ? large : small;
+        const size_t row_tiles = big ? (rows + 255) / 256 : (rows + 127) / 128, tok_tiles = big ? (M + 127) / 128 : (M + 63) / 64;
+        // the last token tile's 32-token tiles in use, and what a block of it costs of a full one's
+        const size_t before = (tok_tiles - 1) * (big ? 128 : 64), in_use = (M - before + 31) / 32;
+        const float share = !big || in_use == 4 ? 1.0f : in_use == 3 ? 0.85f : in_use == 2 ? 0.7f : 0.55f;
+        for (int ks : {1, 2, 3, 4, 5, 6, 8})
+            for (int last : {1, 2, 3, 4, 5, 6, 8}) {
+                const size_t wgs = row_tiles * ((tok_tiles - 1) * (size_t)ks + (size_t)last), most = (size_t)std::max(ks, last);
+                // (five parts, and other parts for the last token tile, where all workgroups are there at once)
+                if (last != ks && (!big || tok_tiles == 1 || in_use == 4)) continue;
+                if ((last != ks || ks == 5) && wgs > 256) continue;
+                if (most > 1 && (nb / most < 2 || most * M * rows * sizeof(float) > SPLIT_PARTS_BYTES)) continue;
+                auto steps = [&](int parts) {
+                    const size_t blocks = (nb + (size_t)parts - 1) / (size_t)parts;
+                    return (float)(big ? blocks : (blocks + 1) / 2);
+                };
+                float us = rounds_us(wgs, steps(ks) * (tok_tiles == 1 ? share : 1.0f), c);
+                if (last != ks) {
+                    const float step = c.step + c.load * (float)wgs / 256.0f;
+                    us = std::max(steps(ks), steps(last) * share) * step + c.start;
+                }
+                if (most > 1) us += 1.3f + 2.6e-7f * (float)(((size_t)ks * before + (size_t)last * (M - before)) * rows * sizeof(float));
+                if (last != ks) us *= 1.03f;  // (the full tiles and the last one share no weights in an XCD's L2)
+                if (best_us == 0.0f || us < best_us) {
+                    best_us = us;
+                    best = big ? PipePlan{256, 128, ks, last} : PipePlan{128, 64, ks, last};
+                }
             }
-        }
+    }
     return best;
 }
 size_t pipe_gemm_parts_bytes(int kind, size_t M, size_t cols, size_t rows) {
     const PipePlan p = pipe_plan(kind, rows, M, cols / QK_K);
-    return p.k_split > 1 ? (size_t)p.k_split * M * rows * sizeof(float) : 0;
+    const size_t parts = (size_t)std::max(p.k_split, p.k_last);
+    return parts > 1 ? parts * M * rows * sizeof(float) : 0;
 }
 
 int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, hipStream_t s) {

@@ -35,7 +35,8 @@ struct GemmArgs {
     Q8KTiled a;  // ceil(M / 32) tiles
     float *y;    // [M][rows]
     int row_tiles, tok_tiles;
-    int k_split;     // 1 .. 8 parts of a row's blocks; with more than one each writes its sums to `partial`
+    int k_split;     // parts of a row's blocks; with more than one each writes its sums to `partial`
+    int k_last;      // the parts of the last token tile
     float *partial;  // [k_split][M][rows], added up in order afterwards (launch_sum_parts)
     int parts_inner; // a row tile's parts next to each other in the work list
 };
@@ -650,8 +651,33 @@ struct PipeLds {
     static_assert(BYTES <= 160 * 1024, "LDS of a CU");
 };
 
-template <int KIND, int RG, int KS, int MT>
-__device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
+// A workgroup's entry of the work list.  The last token tile may be split into parts of its own number (k_last: it has fewer rows in
+// use, so a part of it may have more blocks): its entries then come behind all others.
+struct PipeEntry {
+    int part, parts, row_tile, tok_tile;  // part < 0: none
+};
+template <bool APART>  // whether that may be
+__device__ __forceinline__ PipeEntry pipe_entry(const GemmArgs &g) {
+    int tok_tiles = g.tok_tiles, i;
+    if (!APART || g.k_last == g.k_split) {
+        i = deal_entry((int)blockIdx.x, g.row_tiles * tok_tiles * g.k_split);
+    } else {
+        const int first = g.row_tiles * --tok_tiles * g.k_split;
+        i = deal_entry((int)blockIdx.x, first + g.row_tiles * g.k_last);
+        if (i >= first) {
+            i -= first;
+            return {i / g.row_tiles, g.k_last, i % g.row_tiles, tok_tiles};
+        }
+    }
+    if (i < 0) return {-1, 1, 0, 0};
+    const int tile = i / tok_tiles, inner = g.parts_inner ? g.k_split : g.row_tiles;
+    const int high = tile / inner, low = tile - high * inner;
+    return {g.parts_inner ? low : high, g.k_split, g.parts_inner ? high : low, i - tile * tok_tiles};
+}
+
+// ACT: the workgroup's token tiles with rows in use (the last one of a batch may have fewer than MT)
+template <int KIND, int RG, int KS, int MT, int ACT>
+__device__ __forceinline__ void pipe_gemm_tiles(const GemmArgs &g, const PipeEntry &entry) {
     using L = PipeLds<KIND, RG, KS, MT>;
     using Side = typename L::Side;
     constexpr bool MINS = Side::MINS;
@@ -671,16 +697,11 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
     // one had a round more than the others wherever their number does not divide by eight: 2440 x 12032 in Q5_K at 146
     // tokens, 20 row tiles, 53 -> 33 us; and with the parts in the middle of the list every XCD reads all activations: 1025
     // x 13056 in Q4_K at 105 tokens in eight parts 23.4 -> 21.1.  parts_inner: see pipe_args.)
-    const int entry = deal_entry((int)blockIdx.x, g.row_tiles * g.tok_tiles * g.k_split);
-    if (entry < 0) return;  // uniform per workgroup
-    const int tile = entry / g.tok_tiles, inner = g.parts_inner ? g.k_split : g.row_tiles;
-    const int high = tile / inner, low = tile - high * inner;
-    const int part = g.parts_inner ? low : high, row_tile = g.parts_inner ? high : low;
-    const int tok0 = (entry - tile * g.tok_tiles) * TM;
+    const int part = entry.part, row_tile = entry.row_tile, tok0 = entry.tok_tile * TM;
     const int nb = g.nb;
     // this workgroup multiplies blocks kb0 .. kb1 - 1, its KS shares `steps` consecutive ones each (a
     // share that runs out of blocks idles through its last steps)
-    const int kb0 = nb * part / g.k_split, kb1 = nb * (part + 1) / g.k_split;
+    const int kb0 = nb * part / entry.parts, kb1 = nb * (part + 1) / entry.parts;
     const int steps = (kb1 - kb0 + KS - 1) / KS;
     const int tile0 = tok0 / 32, last_tile = (g.M - 1) / 32;
     auto tile_of = [&](int slot) { return min(tile0 + slot % MT, last_tile); };  // uniform
@@ -737,9 +758,9 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
         next_kb_w++;
     };
 
-    v16f sum[MT];
+    v16f sum[ACT];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) sum[mt] = v16f{0.0f};
+    for (int mt = 0; mt < ACT; mt++) sum[mt] = v16f{0.0f};
     BPlanes B;
     typename Side::Raw R;
     int kb_raw = kb0 + ks * steps;  // the block that leaves the slot next
@@ -804,8 +825,8 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
                     }
                 };
                 auto next = [&](int j) {
-                    if (mt + 1 < MT) {
-                        constexpr int nx = mt + 1 < MT ? mt + 1 : mt;
+                    if (mt + 1 < ACT) {
+                        constexpr int nx = mt + 1 < ACT ? mt + 1 : mt;
                         if (j == 0) read_tile_operand<nx, 0>(Tn, qa);
                         if (j == 1) read_tile_operand<nx, 1>(Tn, qa);
                         if (j == 2) read_tile_operand<nx, 2>(Tn, qa);
@@ -820,21 +841,21 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
                 constexpr int LATER = (MINS ? 1 : 0) + (mt > 0 ? 4 : 0);
                 E.s1 = tile_chain<LATER, MINS, Side::SHIFT>(T, B, between, next);
                 if (MINS) E.bs = T.bs;
-                if (MINS && mt + 1 < MT) {
-                    constexpr int nx = mt + 1 < MT ? mt + 1 : mt;
+                if (MINS && mt + 1 < ACT) {
+                    constexpr int nx = mt + 1 < ACT ? mt + 1 : mt;
                     read_tile_sums<nx>(Tn, ba);
                 }
                 read_tile_scales<mt>(E.S, sa);
-                if (mt + 1 < MT) T = Tn;
+                if (mt + 1 < ACT) T = Tn;
             };
             run_tile(std::integral_constant<int, 0>());
-            if (MT > 1) run_tile(std::integral_constant<int, 1 < MT ? 1 : 0>());
-            if (MT > 2) run_tile(std::integral_constant<int, 2 < MT ? 2 : 0>());
-            if (MT > 3) run_tile(std::integral_constant<int, 3 < MT ? 3 : 0>());
+            if (ACT > 1) run_tile(std::integral_constant<int, 1 < ACT ? 1 : 0>());
+            if (ACT > 2) run_tile(std::integral_constant<int, 2 < ACT ? 2 : 0>());
+            if (ACT > 3) run_tile(std::integral_constant<int, 3 < ACT ? 3 : 0>());
             // the last tile's tail is exposed
             wait_scales<0>(E.S);
 #pragma unroll
-            for (int j = 0; j < 16; j++) tail_piece<FORM>(j, E, B, sum[MT - 1]);
+            for (int j = 0; j < 16; j++) tail_piece<FORM>(j, E, B, sum[ACT - 1]);
         } else if (fetch_now) {
             fetch_quants(0), fetch_quants(1), fetch_sums_scales(), acts_fetched();
         }
@@ -862,7 +883,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
         float *xch = reinterpret_cast<float *>(lds) + (size_t)rg * (KS - 1) * MT * 16 * 64;
         if (ks > 0) {
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++)
+            for (int mt = 0; mt < ACT; mt++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) xch[(((ks - 1) * MT + mt) * 16 + r) * 64 + lane] = sum[mt][r];
         }
@@ -871,16 +892,16 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
 #pragma unroll
         for (int k = 0; k < KS - 1; k++)
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++)
+            for (int mt = 0; mt < ACT; mt++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) sum[mt][r] += xch[((k * MT + mt) * 16 + r) * 64 + lane];
     }
     // store: a lane holds one weight row and 16 tokens per tile
     const int row = row_tile * ROWS + rg * 32 + li;
-    float *const dst = g.k_split > 1 ? g.partial + (size_t)part * g.M * g.rows : g.y;
+    float *const dst = entry.parts > 1 ? g.partial + (size_t)part * g.M * g.rows : g.y;
     const int rows_lim = g.rows;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
+    for (int mt = 0; mt < ACT; mt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int tok = tok0 + mt * 32 + (r >> 2) * 8 + lg * 4 + (r & 3);
@@ -888,12 +909,23 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
         }
 }
 
+template <int KIND, int RG, int KS, int MT>
+__device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
+    const PipeEntry entry = pipe_entry<MT == 4>(g);
+    if (entry.part < 0) return;  // uniform per workgroup
+    const int in_use = (g.M + 31) / 32 - entry.tok_tile * MT;
+    if (MT < 4 || in_use >= MT) pipe_gemm_tiles<KIND, RG, KS, MT, MT>(g, entry);
+    else if (in_use == 3) pipe_gemm_tiles<KIND, RG, KS, MT, MT == 4 ? 3 : MT>(g, entry);
+    else if (in_use == 2) pipe_gemm_tiles<KIND, RG, KS, MT, MT == 4 ? 2 : MT>(g, entry);
+    else pipe_gemm_tiles<KIND, RG, KS, MT, MT == 4 ? 1 : MT>(g, entry);
+}
+
 // ------------------------------------------------------------------ host side
 
 // The workgroup tile of a batch: 256 rows x 128 tokens, 128 x 64 or 64 x 32, and how many workgroups share a row's
 // blocks (their sums, in SPLIT_PARTS_BYTES of memory at most, are added in order afterwards).
 struct PipePlan {
-    int rows_wg, tok_wg, k_split;
+    int rows_wg, tok_wg, k_split, k_last;
 };
 PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb);  // frk_gemm.hip
 
@@ -906,12 +938,14 @@ int launch_pipe(void (*kernel)(GemmArgs), const GemmArgs &g, hipStream_t s) {
         if (e != hipSuccess) return set_error(FRK_ERR_HIP, "hipFuncSetAttribute(LDS %zu): %s", shmem, hipGetErrorString(e));
         sized = true;
     }
-    const unsigned grid = (unsigned)deal_grid(g.row_tiles * g.tok_tiles * g.k_split);
+    const unsigned grid = (unsigned)deal_grid(g.row_tiles * ((g.tok_tiles - 1) * g.k_split + g.k_last));
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), shmem, s, g);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(FRK_ERR_HIP, "pipelined GEMM launch: %s", hipGetErrorString(e));
-    if (g.k_split > 1) return launch_sum_parts(g.partial, g.k_split, (size_t)g.M * g.rows, g.y, s);
-    return FRK_OK;
+    const size_t n = (size_t)g.M * g.rows, last = (size_t)(g.tok_tiles - 1) * (32 * MT) * g.rows;  // where the last token tile begins
+    if (g.k_split == g.k_last) return g.k_split > 1 ? launch_sum_parts(g.partial, g.k_split, n, g.y, s) : FRK_OK;
+    if (g.k_split == 1) return launch_sum_parts_apart(g.partial, n, last, n, last, 1, g.k_last, g.y, s);
+    return launch_sum_parts_apart(g.partial, n, 0, g.k_last > 1 ? n : last, last, g.k_split, g.k_last, g.y, s);
 }
 
 int launch_pipe_q6_k(const GemmArgs &g, int rows_wg, hipStream_t s);  // frk_gemm_q6.hip
@@ -932,6 +966,7 @@ inline GemmArgs pipe_args(const frk_weights *w, Q8KTiled acts, size_t M, float *
     g.row_tiles = (int)((w->rows + p.rows_wg - 1) / p.rows_wg);
     g.tok_tiles = (int)((M + p.tok_wg - 1) / p.tok_wg);
     g.k_split = p.k_split;
+    g.k_last = p.k_last;
     g.partial = partial;
     // A part of a Q6_K row is four runs that end inside cache lines (scales and d a few bytes each: 13 lines for 9 lines'
     // worth of an eighth of 43 blocks): with few activations its row's parts share an L2 instead (4096x11008 at 13 rows 23.7

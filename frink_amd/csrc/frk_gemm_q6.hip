@@ -39,6 +39,36 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float *__restrict_
     *reinterpret_cast<vec *>(y + i) = acc;
 }
 
+// Sums begin .. end - 1 of n, parts0 parts of those in front of `split` and parts1 of the others
+template <int V>
+__global__ __launch_bounds__(256) void sum_parts_apart_kernel(const float *__restrict__ partial, size_t n, size_t begin, size_t end, size_t split,
+                                                              int parts0, int parts1, float *__restrict__ y) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const size_t i = begin + ((size_t)blockIdx.x * 256 + threadIdx.x) * V;
+    if (i >= end) return;
+    const int parts = i < split ? parts0 : parts1;
+    vec acc = *reinterpret_cast<const vec *>(partial + i);
+    for (int p0 = 1; p0 < parts; p0 += 4) {  // four asked for together
+        vec v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = *reinterpret_cast<const vec *>(partial + (size_t)min(p0 + k, parts - 1) * n + i);
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc = p0 + k < parts ? acc + v[k] : acc;
+    }
+    *reinterpret_cast<vec *>(y + i) = acc;
+}
+int launch_sum_parts_apart(const float *partial, size_t n, size_t begin, size_t end, size_t split, int parts0, int parts1, float *y, hipStream_t s) {
+    if (end <= begin) return FRK_OK;
+    const bool by_four = (n | begin | end | split) % 4 == 0 && ((reinterpret_cast<uintptr_t>(partial) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+    const size_t per_wg = by_four ? 1024 : 256;
+    const dim3 grid((unsigned)((end - begin + per_wg - 1) / per_wg));
+    if (by_four) hipLaunchKernelGGL(sum_parts_apart_kernel<4>, grid, dim3(256), 0, s, partial, n, begin, end, split, parts0, parts1, y);
+    else hipLaunchKernelGGL(sum_parts_apart_kernel<1>, grid, dim3(256), 0, s, partial, n, begin, end, split, parts0, parts1, y);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(FRK_ERR_HIP, "launch of the sum of a split GEMM's parts: %s", hipGetErrorString(e));
+    return FRK_OK;
+}
+
 template <int V>
 static void go_sum_parts(const float *partial, int parts, size_t n, float *y, hipStream_t s) {
     const dim3 grid((unsigned)((n / V + 255) / 256));
@@ -46,8 +76,11 @@ static void go_sum_parts(const float *partial, int parts, size_t n, float *y, hi
     if (parts == 2) FRK_GO(2);
     else if (parts == 3) FRK_GO(3);
     else if (parts == 4) FRK_GO(4);
+    else if (parts == 5) FRK_GO(5);
     else if (parts == 6) FRK_GO(6);
     else if (parts == 8) FRK_GO(8);
+    else if (parts == 12) FRK_GO(12);
+    else if (parts == 16) FRK_GO(16);
     else FRK_GO(0);
 #undef FRK_GO
 }

@@ -1,5 +1,6 @@
-"""Batches of 9 to 32 rows on the 64 x 32 tiles of the pipelined K-quant GEMM: rows past the last whole tile, blocks that do not
-divide by a step's four shares, parts of few blocks, and the sizes on both sides of the rule that sends a batch there."""
+"""The pipelined K-quant GEMM where its tiles are not filled.  Batches of 9 to 32 rows on the 64 x 32 tiles: rows past the last whole
+tile, blocks that do not divide by a step's four shares, parts of few blocks, and the sizes on both sides of the rule that
+sends a batch there.  Larger ones whose last token tile has few rows in use."""
 import numpy as np
 import pytest
 
@@ -15,6 +16,10 @@ from test_gpu_parity import fa, to_dev  # noqa: F401 (fa: the module's fixture)
     (fo.Q6_K, 4161, 12288, 9), (fo.Q6_K, 700, 7936, 33),
 ])
 def test_batches_match_exact_arithmetic(fa, kind, rows, cols, batch):
+    _check(fa, kind, rows, cols, batch)
+
+
+def _check(fa, kind, rows, cols, batch):
     from bench import random_blocks
     from frink_amd import synth
     print("batch tiles", kind, rows, cols, batch, flush=True)
@@ -36,3 +41,13 @@ def test_batches_match_exact_arithmetic(fa, kind, rows, cols, batch):
         mag = mag + np.abs(a).sum(1)[:, None] * np.abs(wd).max(1)[None, :]
     room = (cols // 256 + 24) * 2.0 ** -24 * mag
     assert (np.abs(got - a @ wd.T) <= room).all(), float((np.abs(got - a @ wd.T) / room).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,cols,batch", [
+    (fo.Q4_K, 3000, 8192, 65), (fo.Q5_K, 2000, 8192, 97), (fo.Q6_K, 1024, 11008, 96), (fo.Q4_K, 2600, 8192, 129), (fo.Q5_K, 11008, 4096, 197),
+    (fo.Q6_K, 11000, 4096, 170), (fo.Q4_K, 5000, 4352, 161), (fo.Q5_K, 8200, 2048, 225), (fo.Q6_K, 2900, 8192, 290), (fo.Q4_K, 3300, 6400, 321),
+])
+def test_last_token_tile_with_fewer_rows_in_use(fa, kind, rows, cols, batch):
+    """One to three 32-token tiles of the last 128 in use, with and without parts of its own number."""
+    _check(fa, kind, rows, cols, batch)
