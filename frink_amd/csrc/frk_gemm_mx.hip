@@ -46,7 +46,7 @@ size_t mx_acts_bytes(size_t rows, size_t cols) {
 
 // `used`: a row whose entry is negative is left as it is
 // A block of the row a quad of lanes, all of them at once: with 128 threads a row its blocks were three trips to memory one
-// after the other (2048 rows of 2880 columns are bound by the vector ALU either way, 19 us under the profiler; with the token rows'
+// after the other (2048 rows of 2880 columns are bound by the vector ALU either way; with the token rows'
 // digits likewise, 32 experts top-4 of 2880 / 2880 at 64 tokens, the layer, 184 -> 175 us, 16 experts at 24 117 -> 110.5).
 __global__ __launch_bounds__(512) void quantize_mx_kernel(const float *__restrict__ x, int nb, const int *__restrict__ used, MxActs out) {
     __shared__ int infinite;

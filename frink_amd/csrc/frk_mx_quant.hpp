@@ -11,17 +11,29 @@ namespace frk {
 constexpr int MX_BLOCK_BYTES = 96;
 static __host__ __device__ inline size_t mx_padded_blocks(size_t cols) { return (cols / 32 + 7) / 8 * 8; }
 
-// |v| <= 127 * 2047 as four signed base-32 digits, digit p's E2M3 code in byte p.  With 16 added at every place the digits
-// are the number's own bits; x = digit + 16 (0 .. 31) a byte each, then four codes at a time: the magnitude a = |x - 16| in
-// units of a quarter is 2a up to 7 and a + 8 from 8 on, under the sign.
-__device__ __forceinline__ uint32_t mx_digit_codes(int v) {
-    const uint32_t u = (uint32_t)(v + 16 * (1 + 32 + 32 * 32 + 32 * 32 * 32));
-    const uint32_t t = (u & 0x3ffu) | ((u << 6) & 0x03ff0000u);
-    const uint32_t x = (t & 0x001f001fu) | ((t << 3) & 0x1f001f00u);
-    const uint32_t n = (~x >> 4) & 0x01010101u;                                    // negative
-    const uint32_t a = ((x & 0x0f0f0f0fu) ^ ((n << 5) - n)) - ((n << 4) - n);      // n: (31 - low) - 15
-    const uint32_t g = ((a >> 3) | (a >> 4)) & 0x01010101u;                        // 8 or more
-    return (a + ((a & (0x07070707u ^ ((g << 3) - g))) | (g << 3))) | (n << 5);
+typedef _Float16 mx_v32h __attribute__((ext_vector_type(32)));
+typedef uint32_t mx_v6u __attribute__((ext_vector_type(6)));
+
+// Eight numbers, |v| <= 127 * 2047, as four signed base-32 digits each: 48 bits of E2M3 codes a plane, in units of a quarter.
+// (In units of an eighth the codes would be the digits' magnitudes, but the matrix core drops low places of such products
+// sooner: up to 1.12 times the error against 64 bits.)  With 16 added at every place the digits are the number's own bits, 0 ..
+// 31 each; as the bits of an f16 those are multiples of 2^-24, from which 16 are taken away again and 32 digits go through one
+// conversion, all exact.
+__device__ __forceinline__ mx_v6u mx_digit_codes(const int v[8]) {
+    uint32_t digits[4][4];  // [plane][two numbers]
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        constexpr int EACH = 16 * (1 + 32 + 32 * 32 + 32 * 32 * 32);
+        const uint32_t u0 = (uint32_t)(v[2 * j] + EACH), u1 = (uint32_t)(v[2 * j + 1] + EACH);
+        const uint32_t low = __builtin_amdgcn_perm(u1, u0, 0x05040100u), high = __builtin_amdgcn_perm(u1, u0, 0x06050201u);  // bits 0 .. 15, 8 .. 23
+        digits[0][j] = low & 0x001f001fu, digits[1][j] = (low >> 5) & 0x001f001fu;
+        digits[2][j] = (high >> 2) & 0x001f001fu, digits[3][j] = (high >> 7) & 0x001f001fu;
+    }
+    mx_v32h all;
+    __builtin_memcpy(&all, digits, sizeof all);
+    const _Float16 sixteen = (_Float16)(16.0f / 16777216.0f);
+    all -= sixteen;
+    return __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(all, 4.0f / 16777216.0f);
 }
 
 // quantize_activations_q8, Avx form (crates/frink-quant/src/act_quant.rs:157-189), and the digits of quant * scale.
@@ -31,6 +43,9 @@ __device__ __forceinline__ uint32_t mx_digit_codes(int v) {
 // A block whose scale overflows f16 (a largest value above 8.3e6; its E8M0 bytes start at MX_INFINITE) makes an infinity of
 // its integer sum, NaN where that is zero.  A row with such blocks is marked in `infinite`, and they keep their 32 quants as
 // bytes where the digits of a block would start: the GEMM ends with such rows on their own.
+// The vector ALU bounds it (41 MB for 2048 rows of 2880 columns, 8.7 us at a copy's rate): 18.9 us under the profiler with every
+// code made and packed by integer instructions, a float clamp and stores of single dwords, 11.6 so; 32 experts top-4 of 2880 / 2880 at
+// 512 tokens, the layer, 240 -> 230.  The same codes.
 constexpr uint32_t MX_INFINITE = 31 + 104;
 __device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int row, int nb, int tid, int threads, int *flag, const MxActs &out) {
     const int nbp = (nb + 7) & ~7, part = tid & 3;
@@ -54,51 +69,39 @@ __device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int
     };
     auto quant = [&](int i) {
         const float r = rintf(e[i] * inv);
-        return (r != r) ? 0 : (int)fminf(fmaxf(r, -127.0f), 127.0f);
+        int q;  // (the instruction's own ends: 0 for NaN, the largest integers for infinities)
+        asm("v_cvt_i32_f32 %0, %1" : "=v"(q) : "v"(r));
+        return min(max(q, -127), 127);
     };
     int infinite = 0;
     for (int b = tid >> 2; b < nbp; b += threads >> 2) {
         const uint32_t d = load(b);
         const int ex = (int)(d >> 10), mant = (int)(d & 1023u) | (ex ? 1024 : 0);
         infinite |= ex == 31;
-        uint32_t codes[8];  // an element's four digits' codes, plane p in byte p
+        int v[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) codes[i] = mx_digit_codes(quant(i) * mant);
-        uint32_t low[4], high[4];  // a plane's 48 bits
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t *c = codes + 4 * h;
-            const uint32_t a01 = __builtin_amdgcn_perm(c[1], c[0], 0x05010400u), b01 = __builtin_amdgcn_perm(c[1], c[0], 0x07030602u);
-            const uint32_t a23 = __builtin_amdgcn_perm(c[3], c[2], 0x05010400u), b23 = __builtin_amdgcn_perm(c[3], c[2], 0x07030602u);
-            const uint32_t by_plane[4] = {__builtin_amdgcn_perm(a23, a01, 0x05040100u), __builtin_amdgcn_perm(a23, a01, 0x07060302u),
-                                          __builtin_amdgcn_perm(b23, b01, 0x05040100u), __builtin_amdgcn_perm(b23, b01, 0x07060302u)};
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                const uint32_t w = by_plane[p];
-                const uint32_t bits24 = (w & 0x3fu) | ((w >> 2) & 0xfc0u) | ((w >> 4) & 0x3f000u) | ((w >> 6) & 0xfc0000u);
-                if (h == 0) low[p] = bits24;
-                else low[p] |= bits24 << 24, high[p] = bits24 >> 8;
-            }
-        }
-        // lanes in pairs: the even one writes planes 0 and 1 of the pair's 96 bits, the odd one planes 2 and 3
+        for (int i = 0; i < 8; i++) v[i] = quant(i) * mant;
+        const mx_v6u own = mx_digit_codes(v);  // a plane's 48 bits after the other's
+        // lanes in pairs: the even one has planes 0 and 1 of the pair's 96 bits, the odd one planes 2 and 3
         const bool odd = part & 1;
         const size_t at = (size_t)row * nbp + b;
-        uint32_t *dst = reinterpret_cast<uint32_t *>(out.digits + (at & ~(size_t)3) * MX_BLOCK_BYTES) + (b & 3) * 4;
+        uint32_t first[3], second[3];  // the even lane's share of the two planes, the odd lane's
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t own_low = odd ? low[2 + h] : low[h], own_high = odd ? high[2 + h] : high[h];
-            const uint32_t other_low = (uint32_t)dpp_i<DPP_QUAD_XOR1>((int)(odd ? low[h] : low[2 + h]));
-            const uint32_t other_high = (uint32_t)dpp_i<DPP_QUAD_XOR1>((int)(odd ? high[h] : high[2 + h]));
-            const uint32_t first_low = odd ? other_low : own_low, first_high = odd ? other_high : own_high;
-            const uint32_t second_low = odd ? own_low : other_low, second_high = odd ? own_high : other_high;
-            const uint32_t w[3] = {first_low, first_high | (second_low << 16), (second_low >> 16) | (second_high << 16)};
-            const int p = (odd ? 2 : 0) + h;
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const int j = 3 * (part >> 1) + k;
-                dst[j < 4 ? 16 * p + j : 64 + 16 * (p >> 1) + 2 * (p & 1) + j - 4] = w[k];
-            }
+        for (int k = 0; k < 3; k++) {
+            uint32_t low = own[k], high = own[3 + k];
+            asm("" : "+v"(low), "+v"(high));  // (else a choice of index, and a chain of compares)
+            const uint32_t from_even = (uint32_t)dpp_i<DPP_QUAD_XOR1>((int)high), from_odd = (uint32_t)dpp_i<DPP_QUAD_XOR1>((int)low);
+            first[k] = odd ? from_even : low, second[k] = odd ? high : from_odd;
         }
+        const uint32_t w[2][3] = {{first[0], (first[1] & 0xffffu) | (second[0] << 16), (second[0] >> 16) | (second[1] << 16)},
+                                  {(first[1] >> 16) | (first[2] << 16), (first[2] >> 16) | (second[1] & 0xffff0000u), second[2]}};
+        // (lanes 0 and 1 have dwords 0..2, 2 and 3 dwords 3..5: whole pieces from each)
+        const uint32_t third0 = (uint32_t)dpp_i<DPP_QUAD_XOR2>((int)w[0][0]), third1 = (uint32_t)dpp_i<DPP_QUAD_XOR2>((int)w[1][0]);
+        uint4 *dst = reinterpret_cast<uint4 *>(out.digits + (at & ~(size_t)3) * MX_BLOCK_BYTES) + (b & 3);
+        const bool tail = part & 2;
+        dst[4 * (tail ? 4 + (part & 1) : 2 * part)] =
+            tail ? make_uint4(w[0][1], w[0][2], w[1][1], w[1][2]) : make_uint4(w[0][0], w[0][1], w[0][2], third0);
+        if (!tail) dst[4 * (2 * part + 1)] = make_uint4(w[1][0], w[1][1], w[1][2], third1);
         // 2^(ex - 25) a unit, a digit's code is a quarter of its value, plane p times 32^p
         if (part == 0) out.scales[at] = 0x0f0a0500u + 0x01010101u * (uint32_t)(max(ex, 1) + 104);
     }

@@ -53,6 +53,30 @@ def test_grouped_gemm_at_the_edges_of_its_tiles(fa, rows_g, cols, counts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cols,scale", [(384, 1.0), (416, 2.0 ** -20), (1056, 6.0e4)])  # (the middle one: subnormal f16 scales)
+def test_digits_of_every_activation_are_exact(fa, cols, scale):
+    """A weight row that picks one column returns that activation's quant times scale: its digits' sum, no rounding."""
+    rng = np.random.default_rng(cols)
+    x = (rng.standard_normal((96, cols)) * scale * 2.0 ** rng.integers(-3, 4, (96, 1))).astype(np.float32)
+    x[0], x[1] = scale * 127, -scale * 127 * 2047 / 2048  # all ends, and all bits of a scale
+    x[2, ::3] = 0
+    x[3, 32:64] = 0
+    blk = np.zeros((cols, cols // 32, 17), np.uint8)
+    blk[:, :, 0] = 127
+    c = np.arange(cols)
+    blk[c, c // 32, 1 + c % 16] = np.where(c % 32 < 16, 0x02, 0x20)  # E2M1 one
+    w = fa.Weights.from_host(fo.MXFP4, blk.reshape(-1), cols, cols)
+    got = fa.gemm_grouped(w, 1, to_dev(np.array([0, 96], np.int32)), to_dev(x)).cpu().numpy()
+    w.release()
+    xb = x.reshape(96, cols // 32, 32)
+    amax = np.abs(xb).max(axis=2)
+    inv = np.where(amax != 0, np.float32(127) / np.where(amax != 0, amax, 1), 0).astype(np.float32)
+    q = np.clip(np.rint(xb * inv[:, :, None]), -127, 127)
+    a = q * (amax / np.float32(127)).astype(np.float16).astype(np.float32)[:, :, None]
+    assert np.array_equal(got, a.reshape(96, cols).astype(np.float32))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("cols", [64, 96, 352])
 def test_short_rows_round_once_a_block(fa, cols):
     """Below 384 columns a block's sum is an exact integer with one rounding behind it, added in the blocks' order."""
