@@ -209,13 +209,27 @@ __device__ __forceinline__ float silu_as_host(float x, const uint64_t *table = E
     return __fdiv_rn(x, 1.0f + expf_as_libm(-x, table));
 }
 
+// f32::clamp(-127, 127) of a value rounded half to even, `as i8`: a NaN, which the clamp keeps, becomes 0.  The conversion
+// instruction itself gives 0 for NaN and the ends of its range beyond it, so one integer median clamps.  (Three instructions in
+// place of seven; with the bytes by v_perm the batch quantization of 2048 x 14336 for Q8_0 30.3 -> 29.0 us under the profiler, SwiGLU
+// and Q8_K of 4096 rows of 768 12.8 -> 12.0, the token rows beside the bucketing 10.2 -> 9.5.)
+__device__ __forceinline__ int quant_of(float x) {
+    const float r = rintf(x);
+    int q;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(q) : "v"(r));
+    return min(max(q, -127), 127);
+}
+// four quants as bytes
+__device__ __forceinline__ uint32_t quants_of(int q0, int q1, int q2, int q3) {
+    return __builtin_amdgcn_perm((uint32_t)q1, (uint32_t)q0, 0x0c0c0400u) | __builtin_amdgcn_perm((uint32_t)q3, (uint32_t)q2, 0x04000c0cu);
+}
+
 // quantize_activations_q8_k (crates/frink-quant/src/act_quant.rs:69-104) for one 256-value block
 // held four consecutive values per lane by one wavefront.  Returns the lane's four quants packed
 // little-endian; d_out is the block scale (same in every lane); bsum16 is the sum of the 16-wide
 // group this lane belongs to (same in the four lanes of a quad).
-// BRANCHES false: an all-zero block is a select at the end instead of a branch around the arithmetic (the
-// same results: 127 / 0 is an infinity whose products are dropped by the select, and 1 / inf is the zero
-// scale), so that a wavefront quantizing several blocks can interleave their dependent chains.
+// BRANCHES false: no branch around the arithmetic for an all-zero block (the same results: 127 / 0 is an
+// infinity whose products with the zeros are NaN and so quants of 0, and 1 / inf is the zero scale), so that a wavefront quantizing several blocks can interleave their dependent chains.
 template <bool BRANCHES = true>
 __device__ __forceinline__ uint32_t quantize_q8_k_lane(float4 v, float &d_out, int &bsum16) {
     // f32::max ignores a NaN operand, as fmaxf does, and the fold starts from 0: a block of NaNs has the maximum 0
@@ -224,23 +238,17 @@ __device__ __forceinline__ uint32_t quantize_q8_k_lane(float4 v, float &d_out, i
     d_out = 0.0f;
     if (!BRANCHES || amax != 0.0f) {  // uniform across the wavefront
         const float iscale = __fdiv_rn(127.0f, amax);
-        auto quant = [&](float e) {
-            const float r = rintf(iscale * e);  // round half to even
-            // a NaN becomes 0: f32::clamp keeps it and `as i8` makes it 0 (fmaxf would turn it into -127)
-            return (r != r || (!BRANCHES && amax == 0.0f)) ? 0 : (int)fminf(fmaxf(r, -127.0f), 127.0f);
-        };
-        q0 = quant(v.x);
-        q1 = quant(v.y);
-        q2 = quant(v.z);
-        q3 = quant(v.w);
+        q0 = quant_of(iscale * v.x);
+        q1 = quant_of(iscale * v.y);
+        q2 = quant_of(iscale * v.z);
+        q3 = quant_of(iscale * v.w);
         d_out = __fdiv_rn(1.0f, iscale);
     }
     int s = q0 + q1 + q2 + q3;
     s += dpp_i<DPP_QUAD_XOR1>(s);
     s += dpp_i<DPP_QUAD_XOR2>(s);
     bsum16 = s;
-    return (uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8) | ((uint32_t)(q2 & 0xff) << 16) |
-           ((uint32_t)(q3 & 0xff) << 24);
+    return quants_of(q0, q1, q2, q3);
 }
 
 // One record of the tiled Q8_K form (32 rows x one 256-wide block) by a workgroup of WAVES wavefronts

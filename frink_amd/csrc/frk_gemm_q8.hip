@@ -77,7 +77,7 @@ __device__ __forceinline__ q8_v4h q8_as_k0(uint32_t h) {  // {h, 0, 0, 0}
 // Eight lanes per 32-value block.
 // GLU: what is quantized is silu(x) * up, element by element (the intermediate in front of a down projection).
 // Index: 32 bits wide where they hold the threads' numbers (a 64-bit division a thread and the block's maximum through LDS made
-// the vector ALU the bound: 512 rows of 14336 10.1 us under the profiler, now 9.2; 2048 rows 34.1, now 30.5).
+// the vector ALU the bound: 512 rows of 14336 10.1 us under the profiler without, 9.2 with them; 2048 rows 34.1, now 29.0).
 template <bool GLU, class Index>
 __global__ __launch_bounds__(256) void quantize_q8_0_gemm_kernel(const float *__restrict__ x, const float *__restrict__ up, Index n_blocks,
                                                                  int nb, int8_t *__restrict__ q, uint16_t *__restrict__ d) {
@@ -97,14 +97,7 @@ __global__ __launch_bounds__(256) void quantize_q8_0_gemm_kernel(const float *__
     if (!live) return;
     const float scale = __fdiv_rn(amax, 127.0f);
     const float inv = amax != 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
-    auto quant = [&](float e) {
-        const float r = rintf(e * inv);
-        // (f32::clamp keeps a NaN, which `as i8` turns into 0; fmaxf would turn it into -127)
-        return (r != r) ? 0 : (int)fminf(fmaxf(r, -127.0f), 127.0f);
-    };
-    const int q0 = quant(v.x), q1 = quant(v.y), q2 = quant(v.z), q3 = quant(v.w);
-    reinterpret_cast<uint32_t *>(q)[t] = (uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8) |
-                                         ((uint32_t)(q2 & 0xff) << 16) | ((uint32_t)(q3 & 0xff) << 24);
+    reinterpret_cast<uint32_t *>(q)[t] = quants_of(quant_of(v.x * inv), quant_of(v.y * inv), quant_of(v.z * inv), quant_of(v.w * inv));
     if ((t & 7) == 0) {
         const int stride = (nb + 7) & ~7;
         const Index tok = b / (Index)nb;

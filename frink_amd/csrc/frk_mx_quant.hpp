@@ -67,12 +67,7 @@ __device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int
         inv = amax != 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
         return f2h_bits(__fdiv_rn(amax, 127.0f));
     };
-    auto quant = [&](int i) {
-        const float r = rintf(e[i] * inv);
-        int q;  // (the instruction's own ends: 0 for NaN, the largest integers for infinities)
-        asm("v_cvt_i32_f32 %0, %1" : "=v"(q) : "v"(r));
-        return min(max(q, -127), 127);
-    };
+    auto quant = [&](int i) { return quant_of(e[i] * inv); };
     int infinite = 0;
     for (int b = tid >> 2; b < nbp; b += threads >> 2) {
         const uint32_t d = load(b);
@@ -112,7 +107,7 @@ __device__ __forceinline__ void quantize_mx_row(const float *__restrict__ x, int
         for (int b = tid >> 2; b < nb; b += threads >> 2) {
             if (load(b) >> 10 != 31) continue;
             auto bytes = [&](int i) {
-                return (uint32_t)(quant(i) & 0xff) | (uint32_t)(quant(i + 2) & 0xff) << 8 | (uint32_t)(quant(i + 4) & 0xff) << 16 | (uint32_t)(quant(i + 6) & 0xff) << 24;
+                return quants_of(quant(i), quant(i + 2), quant(i + 4), quant(i + 6));
             };
             uint32_t *dst = reinterpret_cast<uint32_t *>(out.digits + ((size_t)row * nbp + b) * MX_BLOCK_BYTES);
             dst[part] = bytes(0), dst[4 + part] = bytes(1);
