@@ -1,4 +1,4 @@
-// The batched Q8_0 GEMM (from 65 rows on; below, gemm_q8_0_rows_kernel for up to 32): the arithmetic of frk_gemm_q8.hip (an exact int8 MFMA per 32-wide block, the
+// The batched Q8_0 GEMM (from 65 rows on; below, gemm_q8_0_rows_kernel): the arithmetic of frk_gemm_q8.hip (an exact int8 MFMA per 32-wide block, the
 // block scales' outer product from the f16 matrix core, a conversion and a fused multiply-add per sum, blocks in order),
 // over larger tiles that come into LDS without passing through registers.
 //
@@ -229,27 +229,31 @@ __global__ __launch_bounds__(512, 2) void gemm_q8_0_pipe_kernel(Q8PipeArgs g) {
 #endif
 }
 
-// ---- Batches of up to 32 rows: a workgroup is 32 weight rows, its eight wavefronts shares of the columns in order (g.k_split
+// ---- Batches of up to 64 rows: a workgroup is 32 weight rows, its eight wavefronts shares of the columns in order (g.k_split
 // workgroups may share a row), whose sums meet in LDS.  The bytes of the weights bound it.  A wavefront brings its rows' and tokens' half
 // chunks, whole lines, into a slot of its own with global_load_lds and refills the slot as soon as it is in registers, so nothing
 // waits for another wavefront before the end, and rows are rarely split between workgroups, whose sums are a launch more.  TL lines
-// of tokens (8, 16, 32; products of lanes past them are not stored): six to nine KB a wavefront, two or three workgroups a CU.
+// of tokens (8, 16, 32, 64 as two tiles; products of lanes past them are not stored): 6 to 13 KB a wavefront, one to three workgroups a CU.
 // With quantization (us, tokens x rows x columns; one-wavefront workgroups over registers and LDS copies, in four or eight parts,
 // before): 8 x 4096 x 4096 14.2, now 8.0; 8 x 4096 x 14336 22.8, 15.5; 32 x 14336 x 4096 23.2, 15.9; 10 x 1100 x 14336 20.2, 10.5; over 45
-// shapes 0.66 of the time in the mean.  With weights past the 256 MB cache 4 x 4096 x 4096 14.7, 9.7, 16 x 14336 x 4096 24.6, 19.2.
-// Sixteen wavefronts a workgroup, four, two slots a wavefront, non-temporal weights and 64 rows a workgroup were slower or no faster over the range; a slot refilled behind the products instead of in
-// front of them 1.2 to 2.7 us slower.
+// shapes 0.66 of the time in the mean.  With weights past the 256 MB cache 4 x 4096 x 4096 14.7, 9.7, 16 x 14336 x 4096 24.6, 19.2.  33 .. 64
+// tokens (four wavefronts over 64 x 64 before): 48 x 14336 x 4096 30.3, 22.3; 30
+// shapes 0.73 of the time, 0.84 past the cache.
+// Sixteen wavefronts a workgroup, four, two slots a wavefront, non-temporal weights and 64 rows a workgroup were slower or no faster
+// over the range; a slot refilled behind the products instead of in front of them 1.2 to 2.7 us slower.
 constexpr int ROWS_WAVES = 8;
 template <int TL>
 struct Q8RowsLds {
-    static constexpr int TOKENS = 32 * 128, SCALES = TOKENS + TL * 128, SLOT = SCALES + 1024;
+    static constexpr int TT = TL > 32 ? 2 : 1;  // tiles of 32 tokens
+    static constexpr int TOKENS = 32 * 128, SCALES = TOKENS + TL * 128, TOKEN_SCALES = SCALES + 512, SLOT = TOKEN_SCALES + TT * 512;
     static constexpr size_t BYTES = (size_t)ROWS_WAVES * SLOT;
-    static_assert(SLOT >= 4096 && BYTES <= 160 * 1024, "a wavefront's sums in its slots, LDS of a CU");
+    static_assert(SLOT >= TT * 4096 && BYTES <= 160 * 1024, "a wavefront's sums in its slots, LDS of a CU");
 };
 template <int TL>
 __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_q8_0_rows_kernel(Q8PipeArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using L = Q8RowsLds<TL>;
+    constexpr int TT = L::TT;
     extern __shared__ __align__(16) uint8_t qp_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int li = lane & 31, lg = lane >> 5;
@@ -271,7 +275,8 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_q8_0_rows_kernel(Q8PipeA
         const int line = c * 8 + (lane >> 3);
         a_off[c] = (uint32_t)min(line, g.M - 1) * (uint32_t)g.nb * 32u + (uint32_t)((lane & 7) ^ ((line >> 1) & 7)) * 16;
     }
-    const uint32_t s_off = lg ? (uint32_t)min(li, g.M - 1) * nbp * 2u : (uint32_t)min(row0 + li, g.rows - 1) * (uint32_t)g.row_stride;
+    const uint32_t s_rows = (uint32_t)min(row0 + li, g.rows - 1) * (uint32_t)g.row_stride;
+    const uint32_t s_tokens = (uint32_t)min(TT == 2 ? lane : li, g.M - 1) * nbp * 2u;
     const uint8_t *const ad = reinterpret_cast<const uint8_t *>(g.ad);
     auto request = [&](int h) {
 #pragma unroll
@@ -279,31 +284,43 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_q8_0_rows_kernel(Q8PipeA
 #pragma unroll
         for (int c = 0; c < TL / 8; c++) dma16(slot_lds + L::TOKENS + c * 1024, reinterpret_cast<const uint8_t *>(g.aq) + (size_t)h * 128, a_off[c]);
         const size_t at = (size_t)(h >> 1) * 16;  // (a chunk's scales, with each of its halves)
-        if (lg) dma16(slot_lds + L::SCALES, ad + at, s_off);
-        else dma16(slot_lds + L::SCALES, g.W + g.off_d + at, s_off);
+        if (!lg) dma16(slot_lds + L::SCALES, g.W + g.off_d + at, s_rows);
+        if (TT == 2) dma16(slot_lds + L::TOKEN_SCALES, ad + at, s_tokens);
+        else if (lg) dma16(slot_lds + L::SCALES, ad + at, s_tokens);  // (lane 32 is 512 bytes further)
     };
-    qp_v16f acc = {0.0f};
+    qp_v16f acc[TT];
+#pragma unroll
+    for (int t = 0; t < TT; t++) acc[t] = qp_v16f{0.0f};
     const qp_v16i zero_i = {0};
     const qp_v16f zero_f = {0.0f};
     if (h0 < h1) request(h0);
     for (int h = h0; h < h1; h++) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         uint2 sw = *reinterpret_cast<const uint2 *>(slot + L::SCALES + li * 16 + (h & 1) * 8);
-        uint2 sa = *reinterpret_cast<const uint2 *>(slot + L::SCALES + (32 + li) * 16 + (h & 1) * 8);
-        qp_v4i w[4], a[4];
+        uint2 sa[TT];
+        qp_v4i w[4], a[TT][4];
+#pragma unroll
+        for (int t = 0; t < TT; t++) sa[t] = *reinterpret_cast<const uint2 *>(slot + L::TOKEN_SCALES + (32 * t + li) * 16 + (h & 1) * 8);
 #pragma unroll
         for (int b = 0; b < 4; b++) {
             w[b] = *reinterpret_cast<const qp_v4i *>(slot + li * 128 + ((2 * b + lg) ^ ((li >> 1) & 7)) * 16);
-            a[b] = *reinterpret_cast<const qp_v4i *>(slot + L::TOKENS + (li & (TL - 1)) * 128 + ((2 * b + lg) ^ (((li & (TL - 1)) >> 1) & 7)) * 16);
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                const int line = 32 * t + (li & (TL - 1));
+                a[t][b] = *reinterpret_cast<const qp_v4i *>(slot + L::TOKENS + line * 128 + ((2 * b + lg) ^ ((line >> 1) & 7)) * 16);
+            }
         }
         // the slot is in registers: the next half chunk travels beside the arithmetic
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sw), "+v"(sa), "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3])::"memory");
+#pragma unroll
+        for (int t = 0; t < TT; t++) asm volatile("" : "+v"(sa[t]), "+v"(a[t][0]), "+v"(a[t][1]), "+v"(a[t][2]), "+v"(a[t][3]));
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sw), "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3])::"memory");
         if (h + 1 < h1) request(h + 1);
         const int live = g.nb - 4 * h;  // blocks of the row from here on: behind its end lie other bytes
         const uint32_t both = lg ? 0u : 0xffffffffu;
         sw.x &= live > 1 ? both : both & 0xffffu;
         sw.y &= live > 3 ? both : live > 2 ? both & 0xffffu : 0u;
-        sa.x &= both, sa.y &= both;
+#pragma unroll
+        for (int t = 0; t < TT; t++) sa[t].x &= both, sa[t].y &= both;
         auto k0 = [](uint2 s, int b) {
             const uint32_t v = b < 2 ? s.x : s.y;
             const uint2 u = make_uint2(b & 1 ? v >> 16 : v & 0xffffu, 0u);
@@ -312,21 +329,25 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_q8_0_rows_kernel(Q8PipeA
             return o;
         };
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const qp_v16i isum = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[b], w[b], zero_i, 0, 0, 0);
-            const qp_v16f scale = __builtin_amdgcn_mfma_f32_32x32x8f16(k0(sa, b), k0(sw, b), zero_f, 0, 0, 0);
+        for (int b = 0; b < 4; b++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[r] = __builtin_fmaf(scale[r], (float)isum[r], acc[r]);
-        }
+            for (int t = 0; t < TT; t++) {
+                const qp_v16i isum = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[t][b], w[b], zero_i, 0, 0, 0);
+                const qp_v16f scale = __builtin_amdgcn_mfma_f32_32x32x8f16(k0(sa[t], b), k0(sw, b), zero_f, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[t][r] = __builtin_fmaf(scale[r], (float)isum[r], acc[t][r]);
+            }
     }
     // register r of a lane: token 8 * (r / 4) + 4 * (lane / 32) + r % 4, weight row lane % 32
 #pragma unroll
-    for (int r = 0; r < 16; r++) reinterpret_cast<float *>(slot)[r * 64 + lane] = acc[r];
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) reinterpret_cast<float *>(slot)[t * 1024 + r * 64 + lane] = acc[t][r];
     __syncthreads();
     float *const dst = g.y + (size_t)blockIdx.y * g.M * g.rows;
     for (int i = threadIdx.x; i < 32 * g.M; i += 64 * ROWS_WAVES) {
         const int tok = i >> 5, row = i & 31;
-        const int at = ((tok >> 3) * 4 + (tok & 3)) * 64 + ((tok >> 2) & 1) * 32 + row;
+        const int at = (tok >> 5) * 1024 + ((tok >> 3 & 3) * 4 + (tok & 3)) * 64 + ((tok >> 2) & 1) * 32 + row;
         float sum = 0.0f;
 #pragma unroll
         for (int v = 0; v < ROWS_WAVES; v++) {
@@ -371,13 +392,13 @@ static int launch_tile(const Q8PipeArgs &g, hipStream_t s) {
 }
 
 // The split of gemm_q8_0_rows_kernel: rounds of workgroups over 256 CUs times a wavefront's half chunks (0.9 us each with 8 lines of
-// tokens, 1.1 with 16, 1.35 with 32) against the second launch and the parts' bytes.  Measured (us; 1, 2, 4 workgroups a row, tokens x
+// tokens, 1.1 with 16, 1.35 with 32, 2.2 with 64) against the second launch and the parts' bytes.  Measured (us; 1, 2, 4 workgroups a row, tokens x
 // rows x columns): 8 x 4096 x 4096 8.0, 10.3, 10.6; 8 x 4096 x 14336 17.2, 15.5, 15.5; 16 x 1500 x 8192 12.6, 10.5, 10.3; 16 x 10240 x
 // 10240 41.2, 34.5, 34.3; 32 x 14336 x 4096 15.9, 18.5, 20.5.
 static Q8PipePlan q8_rows_plan(size_t rows, size_t M, size_t nb, size_t max_parts) {
     const size_t groups = (rows + 31) / 32, halves = (nb + 3) / 4;
-    const int lines = M <= 8 ? 8 : M <= 16 ? 16 : 32;
-    const double step = lines == 8 ? 0.9 : lines == 16 ? 1.1 : 1.35;
+    const int lines = M <= 8 ? 8 : M <= 16 ? 16 : M <= 32 ? 32 : 64;
+    const double step = lines == 8 ? 0.9 : lines == 16 ? 1.1 : lines == 32 ? 1.35 : 2.2;
     Q8PipePlan best = {32, lines, 1};
     double least = 0.0;
     for (size_t ks = 1; ks <= 8 && (ks == 1 || (ks <= max_parts && halves >= 8 * ks)); ks *= 2) {
@@ -396,10 +417,10 @@ static Q8PipePlan q8_rows_plan(size_t rows, size_t M, size_t nb, size_t max_part
 // grids of one round of the other kernel (2048 x 1024 x 4096: 40 against 42 us) stay there.
 Q8PipePlan q8_pipe_plan(size_t rows, size_t M, size_t nb, size_t row_stride, int old_split, size_t max_parts) {
     Q8PipePlan best = {0, 0, 0};
-    // (Past 80 M weights and 8 tokens the other kernel stays: there every workgroup's reads of all tokens cost what the sum's launch
+    // (Past 80 M weights the other kernel stays for 9 .. 32 and 45 .. 64 tokens, whose tiles it fills: there every workgroup's reads of all tokens cost what the sum's launch
     // did; 32 x 6000 x 13824 34.9 us, here 40.2, 16 x 14314 x 9984 47.9 and 50.2, but 4 x 6000 x 13824 32.8 and 30.4, 32 x 8000 x 8960
-    // 32.2 and 29.9, all from memory.)
-    if (M <= 32 && (M <= 8 || rows * nb * 32 <= (size_t)80 << 20) && rows * row_stride <= 0xffffffffu && M * nb * 32 <= 0xffffffffu)
+    // 32.2 and 29.9; 33, 48 and 64 x 14314 x 9984 66.5 and 61.7, 66.9 and 68.0, 67.3 and 73.7; all from memory.)
+    if (M <= 64 && (M <= 8 || (M > 32 && M <= 44) || rows * nb * 32 <= (size_t)80 << 20) && rows * row_stride <= 0xffffffffu && M * nb * 32 <= 0xffffffffu)
         return q8_rows_plan(rows, M, nb, max_parts);
     if (M <= 64 || rows * row_stride > 0xffffffffu || M * nb * 32 > 0xffffffffu) return best;  // (32-bit lane offsets)
     auto tiles = [](size_t n, size_t t) { return (n + t - 1) / t; };
@@ -433,7 +454,7 @@ int launch_gemm_q8_0_pipe(const Q8PipePlan &p, const uint8_t *W, size_t row_stri
     g.row_tiles = (int)((rows + p.rows_wg - 1) / p.rows_wg);
     g.tok_tiles = (int)((M + p.tok_wg - 1) / p.tok_wg);
     g.k_split = p.k_split;
-    if (p.rows_wg == 32) return p.tok_wg == 8 ? launch_rows<8>(g, s) : p.tok_wg == 16 ? launch_rows<16>(g, s) : launch_rows<32>(g, s);
+    if (p.rows_wg == 32) return p.tok_wg == 8 ? launch_rows<8>(g, s) : p.tok_wg == 16 ? launch_rows<16>(g, s) : p.tok_wg == 32 ? launch_rows<32>(g, s) : launch_rows<64>(g, s);
     if (p.rows_wg == 256) return launch_tile<8, 1, 4>(g, s);
     return launch_tile<4, 2, 1>(g, s);
 }

@@ -242,7 +242,7 @@ int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *
 int launch_sum_parts(const float *partial, int parts, size_t n, float *y, hipStream_t s);
 int launch_sum_parts_apart(const float *partial, size_t n, size_t begin, size_t end, size_t split, int parts0, int parts1, float *y, hipStream_t s);
 // The same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time.
-// Its forms over large tiles and, rows_wg = 32, for batches of up to 32 rows (frk_gemm_q8_pipe.hip): weight rows x tokens of a
+// Its forms over large tiles and, rows_wg = 32, for batches of up to 64 rows (frk_gemm_q8_pipe.hip): weight rows x tokens of a
 // workgroup, and how many workgroups share a row's columns; rows_wg = 0: the other kernel
 struct Q8PipePlan {
     int rows_wg, tok_wg, k_split;

@@ -1,4 +1,4 @@
-"""Q8_0 batches of up to 32 rows (gemm_q8_0_rows_kernel, frk_gemm_q8_pipe.hip) at the edges of its rows, lines of tokens, half
+"""Q8_0 batches of up to 64 rows (gemm_q8_0_rows_kernel, frk_gemm_q8_pipe.hip) at the edges of its rows, lines of tokens, half
 chunks of 128 columns and splits, against 64-bit sums of the same quants."""
 import numpy as np
 import pytest
@@ -10,7 +10,8 @@ from test_gpu_parity import fa, to_dev  # noqa: F401 (fa: a fixture)
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,rows,cols", [
     (2, 1, 32), (3, 31, 96), (8, 33, 128), (9, 32, 160), (16, 65, 1056), (17, 64, 992), (32, 97, 1024), (31, 1, 2144),
-    (5, 33, 14336), (12, 100, 8224), (32, 2048, 3104),  # rows split between workgroups; many of them
+    (33, 65, 1056), (40, 33, 2080), (64, 97, 992), (48, 32, 96),
+    (5, 33, 14336), (44, 100, 8224), (12, 100, 8224), (32, 2048, 3104),  # rows split between workgroups; many of them
 ])
 def test_small_batches(fa, batch, rows, cols):
     rng = np.random.default_rng(batch + rows + cols)
