@@ -604,8 +604,8 @@ int launch_quantize_q8_k_gather(const float *x, size_t cols, const int *gather, 
 // The last token tile of 128 multiplies only the 32-token tiles that have rows in use (three, two and one of four measured at 0.85, 0.7
 // and 0.55 of a full block's time) and may be split into parts of its own number, so that its workgroups take about as long as the
 // others: 197 tokens of 11008 x 4096 in Q5_K, three parts of the first tile and two of the second in one round of 215 workgroups,
-// 47.9 -> 44.7 us; 96 of 14336 x 8192 in Q4_K 50.3 -> 42.4.  Over 350 drawn shapes of 33 .. 2048 tokens 0.984 of the time, 0.79 at
-// best; none slower by more than two runs differ (4 %).
+// 47.9 -> 44.7 us.  Over 90 drawn shapes of 33 .. 2048 tokens whose plan these two change 0.92 of the time, 0.80 at best, 1.03 at
+// worst.
 PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
     struct Cost {
         float step, load, start;
@@ -636,35 +636,51 @@ PipePlan pipe_plan(int kind, size_t rows, size_t M, size_t nb) {
         }
         return best;
     }
-    for (int big = 0; big < (M > 64 ? 2 : 1); big++) {
-        const Cost c = big ? large : small;
-        const size_t row_tiles = big ? (rows + 255) / 256 : (rows + 127) / 128, tok_tiles = big ? (M + 127) / 128 : (M + 63) / 64;
-        // the last token tile's 32-token tiles in use, and what a block of it costs of a full one's
-        const size_t before = (tok_tiles - 1) * (big ? 128 : 64), in_use = (M - before + 31) / 32;
-        const float share = !big || in_use == 4 ? 1.0f : in_use == 3 ? 0.85f : in_use == 2 ? 0.7f : 0.55f;
-        for (int ks : {1, 2, 3, 4, 5, 6, 8})
-            for (int last : {1, 2, 3, 4, 5, 6, 8}) {
-                const size_t wgs = row_tiles * ((tok_tiles - 1) * (size_t)ks + (size_t)last), most = (size_t)std::max(ks, last);
-                // (five parts, and other parts for the last token tile, where all workgroups are there at once)
-                if (last != ks && (!big || tok_tiles == 1 || in_use == 4)) continue;
-                if ((last != ks || ks == 5) && wgs > 256) continue;
-                if (most > 1 && (nb / most < 2 || most * M * rows * sizeof(float) > SPLIT_PARTS_BYTES)) continue;
-                auto steps = [&](int parts) {
-                    const size_t blocks = (nb + (size_t)parts - 1) / (size_t)parts;
-                    return (float)(big ? blocks : (blocks + 1) / 2);
-                };
-                float us = rounds_us(wgs, steps(ks) * (tok_tiles == 1 ? share : 1.0f), c);
-                if (last != ks) {
-                    const float step = c.step + c.load * (float)wgs / 256.0f;
-                    us = std::max(steps(ks), steps(last) * share) * step + c.start;
+    // First at a full price for every token tile, then, within that plan's tile, with the last token tile at its own. Neither
+    // form of the choice is to cost precision.  2-norm against 64-bit sums, emulated with normal weights, rows of 32 blocks: the mins
+    // folded (the large tile, see fold_mins) 1.4e-7 as one sum, 1.2e-7 in four; apart (the small tile, two sums a part) 9.7e-8
+    // in two, 8.7e-8 in four; Q6_K 1.2e-7 as one sum, 1.0e-7 in two, 9.0e-8 in three, from five on 8.8e-8.  So the tile stays
+    // (96 x 14336 x 8192 in Q4_K, tokens first, 42.4 us in the large one and 50.3 in the small one; Q6_K, whose error is the same in both, was
+    // 0.95 to 1.04 of the time there), and no token tile's blocks are added up in fewer sums than before, or than five.
+    // (Another plan than the first where it is ahead by 2 %: 222 x 11624 x 3328 in Q6_K, 1 % ahead by the estimate, 46.3 -> 47.9 us.)
+    PipePlan full = best;
+    for (int pass = 0; pass < 2; pass++) {
+        best_us = 0.0f;
+        for (int big = 0; big < (M > 64 ? 2 : 1); big++) {
+            if (pass && (big ? 256 : 128) != full.rows_wg) continue;
+            const Cost c = big ? large : small;
+            const size_t row_tiles = big ? (rows + 255) / 256 : (rows + 127) / 128, tok_tiles = big ? (M + 127) / 128 : (M + 63) / 64;
+            // the last token tile's 32-token tiles in use, and what a block of it costs of a full one's
+            const size_t before = (tok_tiles - 1) * (big ? 128 : 64), in_use = (M - before + 31) / 32;
+            const float share = !pass || !big || in_use == 4 ? 1.0f : in_use == 3 ? 0.85f : in_use == 2 ? 0.7f : 0.55f;
+            for (int ks : {1, 2, 3, 4, 5, 6, 8})
+                for (int last : {1, 2, 3, 4, 5, 6, 8}) {
+                    const size_t wgs = row_tiles * ((tok_tiles - 1) * (size_t)ks + (size_t)last), most = (size_t)std::max(ks, last);
+                    // (five parts, and other parts for the last token tile, where all workgroups are there at once)
+                    if (last != ks && (!pass || !big || tok_tiles == 1 || in_use == 4)) continue;
+                    if ((last != ks || ks == 5) && (!pass || wgs > 256)) continue;
+                    if (most > 1 && (nb / most < 2 || most * M * rows * sizeof(float) > SPLIT_PARTS_BYTES)) continue;
+                    const int shares = big ? 1 : 2;  // (of a part, in a workgroup)
+                    if (pass && std::min(ks, last) * shares < std::min(full.k_split * shares, 5)) continue;
+                    auto steps = [&](int parts) {
+                        const size_t blocks = (nb + (size_t)parts - 1) / (size_t)parts;
+                        return (float)(big ? blocks : (blocks + 1) / 2);
+                    };
+                    float us = rounds_us(wgs, steps(ks) * (tok_tiles == 1 ? share : 1.0f), c);
+                    if (last != ks) {
+                        const float step = c.step + c.load * (float)wgs / 256.0f;
+                        us = std::max(steps(ks), steps(last) * share) * step + c.start;
+                    }
+                    if (most > 1) us += 1.3f + 2.6e-7f * (float)(((size_t)ks * before + (size_t)last * (M - before)) * rows * sizeof(float));
+                    if (last != ks) us *= 1.03f;  // (the full tiles and the last one share no weights in an XCD's L2)
+                    if (pass && (ks != full.k_split || last != ks)) us *= 1.02f;
+                    if (best_us == 0.0f || us < best_us) {
+                        best_us = us;
+                        best = big ? PipePlan{256, 128, ks, last} : PipePlan{128, 64, ks, last};
+                    }
                 }
-                if (most > 1) us += 1.3f + 2.6e-7f * (float)(((size_t)ks * before + (size_t)last * (M - before)) * rows * sizeof(float));
-                if (last != ks) us *= 1.03f;  // (the full tiles and the last one share no weights in an XCD's L2)
-                if (best_us == 0.0f || us < best_us) {
-                    best_us = us;
-                    best = big ? PipePlan{256, 128, ks, last} : PipePlan{128, 64, ks, last};
-                }
-            }
+        }
+        if (!pass) full = best;
     }
     return best;
 }

@@ -1,6 +1,8 @@
 """The pipelined K-quant GEMM where its tiles are not filled.  Batches of 9 to 32 rows on the 64 x 32 tiles: rows past the last whole
 tile, blocks that do not divide by a step's four shares, parts of few blocks, and the sizes on both sides of the rule that
 sends a batch there.  Larger ones whose last token tile has few rows in use."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -51,3 +53,86 @@ def _check(fa, kind, rows, cols, batch):
 def test_last_token_tile_with_fewer_rows_in_use(fa, kind, rows, cols, batch):
     """One to three 32-token tiles of the last 128 in use, with and without parts of its own number."""
     _check(fa, kind, rows, cols, batch)
+
+
+class _Plan(C.Structure):
+    _fields_ = [("rows_wg", C.c_int), ("tok_wg", C.c_int), ("k_split", C.c_int), ("k_last", C.c_int)]
+
+
+def _plan(kind, rows, batch, cols):
+    import frink_amd
+    f = frink_amd.lib()._ZN3frk9pipe_planEimmm  # frk::pipe_plan
+    f.restype, f.argtypes = _Plan, [C.c_int, C.c_size_t, C.c_size_t, C.c_size_t]
+    return f(kind, rows, batch, cols // 256)
+
+
+# shapes whose last token tile has one to three 32-token tiles in use; at a full price for it they take the small tile
+APART = [(fo.Q4_K, 5596, 68, 5632), (fo.Q4_K, 10897, 151, 2560), (fo.Q4_K, 14336, 96, 8192), (fo.Q5_K, 5816, 70, 4352), (fo.Q5_K, 5702, 144, 3840)]
+
+
+@pytest.mark.parametrize("kind,rows,batch,cols", APART)
+def test_a_partly_used_large_tile_takes_no_batch_from_the_small_one(kind, rows, batch, cols):
+    """The large tile folds the mins into the sums, with two roundings a block more than the small one's."""
+    assert _plan(kind, rows, batch, cols).rows_wg == 128
+
+
+@pytest.mark.parametrize("kind,rows,batch,cols,sums", [
+    (fo.Q6_K, 11516, 274, 12544, 3), (fo.Q6_K, 7777, 164, 8704, 4), (fo.Q5_K, 7196, 139, 5120, 4), (fo.Q5_K, 11008, 197, 4096, 2),
+])
+def test_no_token_tile_is_added_up_in_fewer_sums_than_at_a_full_price(kind, rows, batch, cols, sums):
+    p = _plan(kind, rows, batch, cols)
+    assert min(p.k_split, p.k_last) * (2 if p.rows_wg == 128 else 1) >= sums
+
+
+def _two_norm_errors(data, rows, cols, x, parts):
+    """The 2-norm errors against 64-bit sums of the float step with a block's mins apart and folded, a row's blocks in so
+    many sums added up in order: every operation of the kernel's float step in f32, in numpy."""
+    f = np.float32
+    nb = cols // 256
+    blk = data.reshape(rows, nb, 144)
+    d = blk[:, :, 0:2].copy().view(np.float16)[:, :, 0].astype(f)
+    dmin = blk[:, :, 2:4].copy().view(np.float16)[:, :, 0].astype(f)
+    s = blk[:, :, 4:16].astype(np.int64)
+    sc = np.concatenate((s[..., :4] & 63, (s[..., 8:] & 15) | (s[..., :4] >> 6 << 4)), -1)
+    m = np.concatenate((s[..., 4:8] & 63, (s[..., 8:] >> 4) | (s[..., 4:8] >> 6 << 4)), -1)
+    nib = blk[:, :, 16:].reshape(rows, nb, 4, 32)
+    q = np.stack((nib & 15, nib >> 4), 3).reshape(rows, nb, 8, 32)
+    aq, da = zip(*[fo.quantize_q8_k(r)[:2] for r in x])
+    aq = np.stack(aq).reshape(len(x), nb, 8, 32).astype(np.float64)
+    da = np.stack(da).reshape(len(x), nb).astype(f)
+
+    def fma(a, b, c):
+        return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(f)
+    exact, sums = 0.0, {"apart": [], "folded": []}
+    for p in range(parts):
+        acc = {k: np.zeros((len(x), rows), f) for k in sums}
+        for b in range(nb * p // parts, nb * (p + 1) // parts):
+            s1 = aq[:, b].reshape(len(x), 256) @ (q[:, b] * sc[:, b, :, None]).reshape(rows, 256).astype(np.float64).T
+            s2 = aq[:, b].sum(2) @ m[:, b].astype(np.float64).T
+            D, N, A = (np.broadcast_to(v, s1.shape) for v in (d[:, b], -dmin[:, b], da[:, b, None]))
+            exact = exact + A.astype(np.float64) * (D.astype(np.float64) * s1 + N.astype(np.float64) * s2)
+            acc["apart"] = fma(A, fma(N, s2.astype(f), D * s1.astype(f)), acc["apart"])
+            c = ((D * (f(1) / N)) * s1.astype(f) + s2).astype(f)
+            acc["folded"] = fma(A * N, c, acc["folded"])
+        for k in sums:
+            sums[k] = acc[k] if p == 0 else sums[k] + acc[k]
+    return exact, {k: np.linalg.norm(v - exact) / np.linalg.norm(exact) for k, v in sums.items()}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,batch,cols,parts", [APART[0][1:] + (4,), APART[1][1:] + (2,)])  # (two shares of two parts, of one)
+def test_batches_of_the_small_tile_are_as_exact_as_its_float_step(fa, rows, batch, cols, parts):
+    """The 2-norm error lies with the mins apart, not folded: below the middle of what the two float steps have."""
+    from bench import random_blocks
+    from frink_amd import synth
+    print("small tile's error", rows, cols, batch, flush=True)
+    data = random_blocks(fo.Q4_K, rows, cols, seed=rows)
+    x = synth.activations(batch, batch, cols)
+    w = fa.Weights.from_host(fo.Q4_K, data, rows, cols)
+    got = w.gemm(to_dev(x)).cpu().numpy()[:, :64].astype(np.float64)
+    w.release()
+    exact, want = _two_norm_errors(data.reshape(rows, -1)[:64], 64, cols, x, parts)
+    error = np.linalg.norm(got - exact) / np.linalg.norm(exact)
+    print(error, want, flush=True)
+    assert want["apart"] < 0.9 * want["folded"]
+    assert error < (want["apart"] * want["folded"]) ** 0.5
