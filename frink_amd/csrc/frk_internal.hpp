@@ -128,7 +128,7 @@ namespace frk {
 // apart; calls on different streams have different buffers.  A buffer that is too small is replaced, never
 // freed in place: the old one is kept until the outermost lease ends, then retired behind an event on the
 // stream and handed out again (to any stream) once that event has passed.  A stream that is being captured
-// cannot grow its buffer (the caller runs the shape once before capturing).
+// does not grow its buffer (the caller runs the shape once before capturing), but see workspace's `held`.
 struct StreamWorkspace;
 class WorkspaceLease {
   public:
@@ -139,12 +139,13 @@ class WorkspaceLease {
     void *ptr = nullptr;
 
   private:
-    friend int workspace(size_t, hipStream_t, WorkspaceLease &);
+    friend int workspace(size_t, hipStream_t, WorkspaceLease &, size_t);
     StreamWorkspace *held_ = nullptr;
     hipStream_t stream_ = nullptr;
 };
-// Leases at least `bytes` of the stream's buffer (the same start address for nested leases).
-int workspace(size_t bytes, hipStream_t stream, WorkspaceLease &lease);
+// Leases at least `bytes` of the stream's buffer (the same start address for nested leases).  A buffer of `held` bytes and more
+// grows during a capture too (0: and so does none at all).
+int workspace(size_t bytes, hipStream_t stream, WorkspaceLease &lease, size_t held = SIZE_MAX);
 hipStream_t own_stream();  // the stream host-buffer entry points run on
 
 // ---- launchers (each validates nothing: callers have checked shapes) ----

@@ -98,7 +98,7 @@ static int take_buffer_locked(size_t bytes, void **ptr, size_t *got) {
     return FRK_OK;
 }
 
-int workspace(size_t bytes, hipStream_t stream, WorkspaceLease &lease) {
+int workspace(size_t bytes, hipStream_t stream, WorkspaceLease &lease, size_t held) {
     StreamWorkspace *w = nullptr;
     {
         std::lock_guard<std::mutex> lk(g_dev.mu);
@@ -117,23 +117,28 @@ int workspace(size_t bytes, hipStream_t stream, WorkspaceLease &lease) {
     // nor reused after a growth -- it stays allocated, untouched by later calls, until the process ends.
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cs) != hipSuccess) (void)hipGetLastError();
-    if (cs != hipStreamCaptureStatusNone && bytes <= w->bytes) w->in_a_graph = true;
+    const bool capturing = cs != hipStreamCaptureStatusNone;
+    if (capturing && bytes <= w->bytes) w->in_a_graph = true;
     if (bytes > w->bytes) {
-        if (cs != hipStreamCaptureStatusNone)
+        if (capturing && w->bytes < held)
             return set_error(FRK_ERR_HIP,
                              "the stream's scratch buffer holds %zu bytes and this call needs %zu: it cannot grow while the "
                              "stream is being captured (run the shape once before capturing)", w->bytes, bytes);
         void *fresh = nullptr;
         size_t got = 0;
         {
+            // (during a capture only a thread in relaxed mode may allocate)
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            if (capturing) FRK_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
             std::lock_guard<std::mutex> lk(g_dev.mu);
             int rc = take_buffer_locked(bytes, &fresh, &got);
+            if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
             if (rc) return rc;
         }
         if (w->ptr && !w->in_a_graph) w->outgrown.emplace_back(w->ptr, w->bytes);  // (one a graph holds: kept, see above)
         w->ptr = fresh;
         w->bytes = got;
-        w->in_a_graph = false;
+        w->in_a_graph = capturing;
     }
     lease.ptr = w->ptr;
     return FRK_OK;
@@ -142,7 +147,10 @@ int workspace(size_t bytes, hipStream_t stream, WorkspaceLease &lease) {
 WorkspaceLease::~WorkspaceLease() {
     StreamWorkspace *w = held_;
     if (!w) return;
-    if (--w->depth == 0 && !w->outgrown.empty()) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (--w->depth == 0 && !w->outgrown.empty() && hipStreamIsCapturing(stream_, &cs) != hipSuccess) (void)hipGetLastError();
+    // (an event recorded during a capture would become a node of the graph: the next lease after it retires them)
+    if (w->depth == 0 && !w->outgrown.empty() && cs == hipStreamCaptureStatusNone) {
         // kernels enqueued under this lease may still read a replaced buffer: it is free once the
         // stream has passed this point
         std::lock_guard<std::mutex> lk(g_dev.mu);
@@ -475,8 +483,8 @@ struct Scratch {
         void *none = nullptr;
         return get(bytes, 0, s, out, &none);
     }
-    // `parts`: room for the parts' sums of a split GEMM besides
-    int get(size_t bytes, size_t parts_bytes, hipStream_t s, void **out, void **parts) {
+    // `parts`: room for the parts' sums of a split GEMM besides; `held`: see workspace
+    int get(size_t bytes, size_t parts_bytes, hipStream_t s, void **out, void **parts, size_t held = SIZE_MAX) {
         if (fixed) {
             if (bytes > fixed_bytes || parts_bytes > SPLIT_PARTS_BYTES)
                 return set_error(FRK_ERR_SHAPE, "this shape needs %zu + %zu bytes of scratch memory, the entry point that allocates nothing has %zu + %zu",
@@ -486,7 +494,7 @@ struct Scratch {
             return FRK_OK;
         }
         const size_t at = parts_bytes ? round_up(bytes, 256) : bytes;
-        int rc = workspace(at + parts_bytes, s, lease);
+        int rc = workspace(at + parts_bytes, s, lease, held);
         *out = lease.ptr;
         *parts = (char *)lease.ptr + at;
         return rc;
@@ -654,9 +662,8 @@ static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     if (batch >= 17) return measured && n > 23 * M;
     return measured && n > 48 * M && w->rows > 4096;
 }
-// The crossings against the 128 x 64 tiles, higher than those above.  frk_hip_gemm_q8k_dev takes the batches below them (a
-// batch between the two is put into the tiled form first, so that it has frk_hip_gemm_dev's bits), and a batch between
-// the two whose scratch memory cannot be had -- a stream under capture -- goes where it went before.
+// The crossings against the 128 x 64 tiles, higher than those above: below them the thin kernels hold a batch, and
+// frk_hip_gemm_q8k_dev takes it (one between the two is put into the tiled form first, so that it has frk_hip_gemm_dev's bits).
 static bool matrix_cores_only(const frk_weights *w, size_t batch) {
     const size_t n = w->rows * w->cols, nb = w->cols / QK_K, M = (size_t)1 << 20;
     const bool measured = nb <= 128;
@@ -672,6 +679,15 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
         from = measured && n > 48 * M ? 17 : n > 32 * M || (measured && n >= 30 * M) ? 25 : 41;
     }
     return batch >= std::max(from, tiled_from(w->cols));
+}
+static size_t acts_plain_bytes(size_t batch, size_t cols) {
+    const size_t n = batch * cols;
+    return round_up(n, 256) + round_up(n / QK_K * 4, 256) + round_up(n / 16 * 2, 256);
+}
+// A batch between the two crossings needs more scratch memory on the matrix cores than the thin kernels do (none of their own, or
+// plain rows): on a stream that is being captured its buffer grows where it would have done for those.
+static size_t held_for_capture(const frk_weights *w, size_t batch) {
+    return matrix_cores_only(w, batch) ? SIZE_MAX : acts_plain_bytes(batch, w->cols);
 }
 // whether the thin kernels hold a batch of this matrix (over plain Q8_K rows)
 static bool thin_kernels_hold(const frk_weights *w, size_t batch) {
@@ -771,15 +787,13 @@ static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *
     if (k_quant_takes_the_matrix_cores(w, batch)) {  // (frk_hip_gemm_pair_dev: the same test)
         hipStream_t s = (hipStream_t)stream;
         void *ws = nullptr, *parts = nullptr;
-        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts);
-        if (rc == FRK_OK) {
-            const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
-            rc = launch_quantize_q8_k_tiled(x, batch, w->cols, acts, s);
-            if (rc) return rc;
-            return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
-        }
-        if (matrix_cores_only(w, batch)) return rc;
-        clear_error();
+        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts,
+                             held_for_capture(w, batch));
+        if (rc) return rc;
+        const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
+        rc = launch_quantize_q8_k_tiled(x, batch, w->cols, acts, s);
+        if (rc) return rc;
+        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
     }
     // Q8_0: a batch is the integer path, as in the reference (Q8_0 activation blocks and dot_q8_0_q8,
     // crates/frink-core/src/weight_matrix.rs:2701-2829); a single row keeps the f32 dot of its decode path
@@ -849,14 +863,12 @@ int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
     if (k_quant_takes_the_matrix_cores(w, batch)) {
         void *ws = nullptr, *parts = nullptr;
         Scratch scratch;
-        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts);
-        if (rc == FRK_OK) {
-            const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
-            rc = launch_tile_q8_k(a, batch, w->cols, acts, s);
-            if (rc) return rc;
-            return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
-        }
-        clear_error();
+        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts, 0);
+        if (rc) return rc;
+        const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
+        rc = launch_tile_q8_k(a, batch, w->cols, acts, s);
+        if (rc) return rc;
+        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
     }
     return thin_gemm_acts(w, a, batch, thin_gemm_max_batch(w), y, s);
 }
@@ -875,18 +887,18 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
         const size_t acts_bytes = round_up(q8k_tiled_bytes(batch, w0->cols), 256);
         const size_t part0 = round_up(pipe_gemm_parts_bytes(w0->kind, batch, w0->cols, w0->rows), 256);
         const size_t part1 = pipe_gemm_parts_bytes(w1->kind, batch, w1->cols, w1->rows);
+        // (one matrix beyond the higher crossing: what it needs on its own)
+        auto alone = [&](const frk_weights *w, size_t parts) { return matrix_cores_only(w, batch) ? acts_bytes + parts : held_for_capture(w, batch); };
+        const bool only = matrix_cores_only(w0, batch) && matrix_cores_only(w1, batch);
         void *ws = nullptr, *parts = nullptr;
-        int rc = scratch.get(acts_bytes, part0 + part1, s, &ws, &parts);
-        if (rc == FRK_OK) {
-            const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
-            rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
-            if (rc) return rc;
-            rc = launch_pipe_gemm_acts(w0, acts, batch, y0, parts, s);
-            if (rc) return rc;
-            return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)parts + part0, s);
-        }
-        if (matrix_cores_only(w0, batch) && matrix_cores_only(w1, batch)) return rc;
-        clear_error();
+        int rc = scratch.get(acts_bytes, part0 + part1, s, &ws, &parts, only ? SIZE_MAX : std::max(alone(w0, part0), alone(w1, part1)));
+        if (rc) return rc;
+        const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
+        rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
+        if (rc) return rc;
+        rc = launch_pipe_gemm_acts(w0, acts, batch, y0, parts, s);
+        if (rc) return rc;
+        return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)parts + part0, s);
     }
     // otherwise each matrix takes the path frk_hip_gemm_dev gives it (the same results, two quantizations)
     int rc = gemm_impl(w0, x, batch, y0, stream, scratch);
@@ -909,12 +921,6 @@ struct frk_batch_acts {
     size_t batch = 0;           // rows of the last quantization (0: none yet)
     frk::Q8KActs plain{nullptr, nullptr, nullptr};
 };
-namespace {
-size_t acts_plain_bytes(size_t batch, size_t cols) {
-    const size_t n = batch * cols;
-    return frk::round_up(n, 256) + frk::round_up(n / frk::QK_K * 4, 256) + frk::round_up(n / 16 * 2, 256);
-}
-}  // namespace
 extern "C" {
 
 int frk_hip_batch_acts_create(size_t max_batch, size_t cols, frk_batch_acts **out) {
@@ -990,11 +996,12 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *a, float *
         const size_t parts_bytes = pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows);
         void *parts = nullptr;
         Scratch scratch;
-        int rc = FRK_OK;
-        if (parts_bytes) rc = scratch.get(parts_bytes, s, &parts);  // a split of the blocks between workgroups: room for the parts' sums
-        if (rc == FRK_OK) return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
-        if (matrix_cores_only(w, batch)) return rc;
-        clear_error();
+        if (parts_bytes) {  // a split of the blocks between workgroups: room for the parts' sums
+            void *none = nullptr;
+            int rc = scratch.get(parts_bytes, 0, s, &parts, &none, matrix_cores_only(w, batch) ? SIZE_MAX : 0);
+            if (rc) return rc;
+        }
+        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
     }
     // (below the matrix-core GEMMs' batches the plain rows are there: ACTS_PLAIN_MAX_BATCH covers every such batch)
     if (batch > ACTS_PLAIN_MAX_BATCH)

@@ -179,7 +179,11 @@ int frk_hip_launch_dense_ffn_swiglu(const frk_matvec_launch *gate, const frk_mat
  * capturing it (a call that would need to grow returns FRK_ERR_HIP and launches nothing) -- and a
  * buffer that was current during a capture belongs to that graph from then on: a later, larger call
  * on the stream gets a new buffer and the old one stays allocated and untouched until the process
- * ends, so replays of the graph stay valid (at the price of that memory).  Callers that capture
+ * ends, so replays of the graph stay valid (at the price of that memory).  One exception: a K-quant batch
+ * that frk_hip_gemm_q8k_dev takes and that runs on the matrix cores (see there) grows the buffer during a
+ * capture too -- in frk_hip_gemm_q8k_dev and frk_hip_gemm_acts_dev whatever it holds, in frk_hip_gemm_dev
+ * and frk_hip_gemm_pair_dev if it holds the batch's rows in Q8_K -- so that what a call returns
+ * does not depend on what ran on its stream before.  Callers that capture
  * without a warm call, or cannot have the library allocate at all, use frk_hip_gemm_noalloc_dev. */
 
 /* y[rows] = W x for one activation vector in HBM.  K-quants: x is quantized to Q8_K
@@ -218,7 +222,7 @@ int frk_hip_gemm_dev(const frk_weights *w, const float *x_dev, size_t batch, flo
  * crates/frink-core/src/weight_matrix.rs:757-768, handed to apply_batch_with_acts, :2481-2487).  Bit for bit
  * frk_hip_gemm_dev's result (one row: frk_hip_gemv_q8k_dev).  K-quants; the batches that the thin kernels hold (up to 16
  * or 32 rows for Q4_K and up to 24 or 40 for Q6_K by the matrix's size, 32 for Q5_K; those that frk_hip_gemm_dev multiplies on the
- * matrix cores are put into their tiled form first): FRK_ERR_UNSUPPORTED beyond, where the matrix-core GEMM quantizes for itself. */
+ * matrix cores are put into their tiled form in scratch memory first): FRK_ERR_UNSUPPORTED beyond, where the matrix-core GEMM quantizes for itself. */
 int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q_dev, const float *d_dev, const int16_t *bsums_dev,
                          size_t batch, float *y_dev, void *stream);
 
