@@ -20,6 +20,8 @@ int set_error(int code, const char *fmt, ...) {
     va_start(ap, fmt);
     vsnprintf(g_err, sizeof g_err, fmt, ap);
     va_end(ap);
+    // (what failed is reported here: left standing, the next call's launch check would find it and report it again)
+    if (code == FRK_ERR_HIP || code == FRK_ERR_OOM) (void)hipGetLastError();
     return code;
 }
 void clear_error() { g_err[0] = 0; }

@@ -1,5 +1,5 @@
 """K-quant batches under HIP graph capture that the matrix cores take and the thin kernels hold: their scratch buffer grows where
-it would have done for the thin kernels, with the bits of the same call outside of a capture; elsewhere it does not grow."""
+it would have done for the thin kernels, with the bits of the same call outside of a capture; elsewhere it does not grow.  And an allocation that fails."""
 import ctypes as C
 
 import numpy as np
@@ -97,4 +97,21 @@ def test_batches_on_a_stream_whose_scratch_buffer_is_too_small(fa):
     _captured(fa, lambda: w.gemm(x, out=y), [y], [eager], lambda: w.gemm(x[:2]))
     print("pair", flush=True)
     _captured(fa, lambda: fa.gemm_pair(w, w, x, outs=y2), y2, pair, lambda: w.gemm(x[:2]))
+    w.release()
+
+
+def test_a_failed_allocation_is_reported_once(fa):
+    """More memory than any device has: an error, and the next calls on the thread are not told of it again."""
+    import torch
+    from frink_amd import synth
+    w = fa.Weights.from_host(fo.Q4_K, make_weights(fo.Q4_K, 64, 512, seed=76), 64, 512)
+    x = to_dev(synth.activations(77, 3, 512))
+    want = w.gemm(x).clone()
+    torch.cuda.synchronize()
+    with pytest.raises(fa.BackendError) as e:
+        fa.BatchActs(10 ** 10, 32768)
+    assert e.value.code in (fa.ERR_HIP, fa.ERR_OOM)
+    got = w.gemm(x)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got.cpu().numpy()), bits(want.cpu().numpy()))
     w.release()
