@@ -17,6 +17,7 @@
 // 2880) and multiplied by the Q8_0 kernel, whose float step is 32 vector instructions per MFMA (156 us).
 #include "frk_mx_quant.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 namespace frk {
@@ -404,13 +405,24 @@ static int mx_waves(size_t pairs, size_t groups, size_t rows_g, bool glu) {
     const size_t rows = 8 * (glu ? 32 : 64);
     return (pairs / 64 + groups) * ((rows_g + rows - 1) / rows) >= 256 ? 8 : 4;
 }
-// Tiles of 96 rows where the workgroups of 64-row tiles would not fit the chip at once: an expert of 65 to 96 pairs then reads
-// its weights once, not a second time for a few rows.  Tiles of 64 rows where they do: there a job's length is the launch's.
-// (64-row tiles / 96, us a layer: 32 experts top-4 of 2880 / 2880 at 512 and 768 tokens 286 / 244 and 352 / 304, 16 top-2 of
-// 2880 / 1536 at 700 152 / 118, 8 top-4 of 2048 / 1440 at 300 98 / 87, 8 top-2 of 1024 / 1024 at 512 57.5 / 65.9.)
+// Tiles of so many rows that pairs dealt to the groups at random take: a group's number is about normal around the mean.
+static double expected_tiles(size_t pairs, size_t groups, double rows) {
+    const double mean = (double)pairs / (double)groups, spread = std::sqrt(2.0 * mean);
+    const double sure = std::max(0.0, std::floor((mean - 3.0 * spread) / rows));  // every group has these
+    double tiles = sure, p = 1.0;
+    for (double j = sure; p > 1e-3; j++) tiles += p = 0.5 * std::erfc((j * rows + 0.5 - mean) / spread);  // more than j * rows
+    return tiles * (double)groups;
+}
+// Tiles of 96 rows where the workgroups of 64-row tiles would not fit the chip's 256 CUs at once (with 1 % on top: the numbers
+// differ): an expert of 65 to 96 pairs then reads its weights once, not a second time for a few rows.  Tiles of 64 rows where they do:
+// there a job's length is the launch's.  As eight wavefronts a workgroup take over from four with more pairs (mx_waves), the
+// workgroups become half as many and fit again.  Measured in us a layer, 64-row tiles / 96: where they do not fit, 32 experts
+// top-4 of 2880 / 2880 at 517 tokens 242 / 212, 16 top-2 of 2240 / 1312 at 741 106 / 88, 8 top-2 of 2880 / 2880 at 768 182 / 152; where they just
+// fit, of four wavefronts, 8 top-2 of 2048 / 2048 at 416 72 / 87, of eight, 8 top-2 of 2880 / 2880 at 448 108 / 122, 16 top-2 of 1536 / 1536 at
+// 864 77 / 86.  Over 118 drawn layers the choice is 1.0 % behind the better one on average, 11 % at most.
 int mx_tile(size_t pairs, size_t groups, size_t rows_g, bool glu) {
     const size_t rows = (size_t)mx_waves(pairs, groups, rows_g, glu) * (glu ? 32 : 64);
-    return (pairs / 64 + groups / 2) * ((rows_g + rows - 1) / rows) > 256 ? MX_TILE : MOE_TILE;
+    return expected_tiles(pairs, groups, MOE_TILE) * (double)((rows_g + rows - 1) / rows) > 258.5 ? MX_TILE : MOE_TILE;
 }
 // up: the second matrix (y = silu(gate) * up), or null
 int launch_gemm_mx_grouped(const frk_weights *w, const frk_weights *up, size_t rows_g, const MxActs &acts, const int *src_rows,

@@ -197,6 +197,20 @@ def test_tiles_of_96_rows(fa, rows_g, cols, counts):
     test_grouped_gemm_at_the_edges_of_its_tiles(fa, rows_g, cols, counts)
 
 
+@pytest.mark.parametrize("pairs,groups,rows,glu,tile", [
+    (832, 8, 2048, True, 64), (896, 8, 2880, True, 64), (1728, 16, 1536, True, 64),  # two tiles an expert, one round of the chip
+    (1000, 16, 1536, True, 96), (2048, 32, 2880, True, 96), (2400, 8, 2880, True, 96),
+    (2508, 27, 1500, False, 96), (2352, 32, 4097, False, 96), (840, 9, 4064, True, 96),  # the tests of such tiles here
+])
+def test_tiles_of_96_rows_where_those_of_64_do_not_fit_the_chip_at_once(pairs, groups, rows, glu, tile):
+    import ctypes as C
+
+    import frink_amd
+    f = frink_amd.lib()._ZN3frk7mx_tileEmmmb  # frk::mx_tile
+    f.restype, f.argtypes = C.c_int, [C.c_size_t] * 3 + [C.c_bool]
+    assert f(pairs, groups, rows, glu) == tile
+
+
 @pytest.mark.gpu
 def test_layer_whose_last_round_of_jobs_is_cut_in_two(fa):
     """Sixteen workgroups a tile: the XCDs with one tile (or three) cut a round of sixteen jobs in two, tiles of one to
