@@ -197,10 +197,43 @@ def test_tiles_of_96_rows(fa, rows_g, cols, counts):
     test_grouped_gemm_at_the_edges_of_its_tiles(fa, rows_g, cols, counts)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows_g,cols,counts", [
+    (1500, 416, [96, 97, 65, 64, 128, 192, 193, 0, 1] * 3),
+    (4097, 416, [96, 65, 33, 1, 97, 32, 64, 200] * 4),  # among the jobs cut in two: tiles of one and two halves
+    (8190, 384, [96] * 9),                               # cut in two: all jobs of the XCDs with one tile, of three halves
+])
+def test_rows_whose_scale_leaves_f16_in_tiles_of_96(fa, rows_g, cols, counts):
+    """Infinite results where and with the signs the oracle has them, in every half of a tile; the other rows keep their bits."""
+    print("mxfp4 infinite rows", rows_g, cols, len(counts), flush=True)
+    rng = np.random.default_rng(rows_g)
+    x = rng.standard_normal((sum(counts), cols)).astype(np.float32)
+    large = x.copy()
+    off = np.concatenate(([0], np.cumsum(counts)))
+    rows = [sorted({r % n for r in (5, 31, 40, 63, 70, 95, n - 1)}) if n else [] for n in counts]
+    for g, picked in enumerate(rows):
+        for i, r in enumerate(picked):
+            large[off[g] + r, 7 * i + 1] = 2.0e7
+            large[off[g] + r, 370 - 9 * i] = (3.0e7, -3.0e7, 1.0, np.inf)[(g + i) % 4]
+    _, per, finite = _case(fa, counts, rows_g, cols, x, seed=41)
+    _, _, got = _case(fa, counts, rows_g, cols, large, seed=41)
+    untouched = np.ones(len(x), bool)
+    for g, picked in enumerate(rows):
+        if not picked:
+            continue
+        at = off[g] + np.array(picked)
+        untouched[at] = False
+        want = fo.gemm(fo.MXFP4, per[g], rows_g, cols, large[at], fo.INT_DOT)
+        assert not np.isfinite(want).any()
+        assert np.array_equal(np.isnan(got[at]), np.isnan(want)), g
+        assert np.array_equal(np.sign(got[at][np.isinf(want)]), np.sign(want[np.isinf(want)])), g
+    assert np.array_equal(got[untouched].view(np.uint32), finite[untouched].view(np.uint32))
+
+
 @pytest.mark.parametrize("pairs,groups,rows,glu,tile", [
     (832, 8, 2048, True, 64), (896, 8, 2880, True, 64), (1728, 16, 1536, True, 64),  # two tiles an expert, one round of the chip
     (1000, 16, 1536, True, 96), (2048, 32, 2880, True, 96), (2400, 8, 2880, True, 96),
-    (2508, 27, 1500, False, 96), (2352, 32, 4097, False, 96), (840, 9, 4064, True, 96),  # the tests of such tiles here
+    (2508, 27, 1500, False, 96), (2352, 32, 4097, False, 96), (840, 9, 4064, True, 96), (864, 9, 8190, False, 96),  # the tests of such tiles here
 ])
 def test_tiles_of_96_rows_where_those_of_64_do_not_fit_the_chip_at_once(pairs, groups, rows, glu, tile):
     import ctypes as C
