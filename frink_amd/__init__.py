@@ -149,9 +149,12 @@ def _stream():
     attention 7.5 -> 5.5 us a call, one token of a
     mixture-of-experts layer, its routing with it, 20.6 -> 16.2)."""
     import torch
-    if not torch.cuda.is_initialized():
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    if torch.cuda.is_initialized():
+        try:
+            return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+        except AttributeError:  # (private names: not every build of torch has them)
+            pass
+    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 def _np_ptr(a):

@@ -137,3 +137,16 @@ def test_cpp_host_mirror_without_a_device():
     r = subprocess.run([_host_check_binary()], env=env, text=True, capture_output=True, timeout=120)
     assert r.returncode == 0 and "FAIL" not in r.stdout, r.stdout + r.stderr
     assert "FRINK_HIP=off disables the backend" in r.stdout
+
+
+@pytest.mark.parametrize("missing", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_current_stream_without_torch_private_functions(monkeypatch, missing):
+    import types
+
+    import torch
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        monkeypatch.setattr(torch._C, name, lambda *_: 0, raising=False)
+    monkeypatch.delattr(torch._C, missing)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=1234))
+    assert fa._stream().value == 1234
