@@ -666,7 +666,9 @@ static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
 }
 // The crossings against the 128 x 64 tiles, higher than those above: below them the thin kernels hold a batch, and
 // frk_hip_gemm_q8k_dev takes it (one between the two is put into the tiled form first, so that it has frk_hip_gemm_dev's bits).
+// (The first test holds for every batch beyond them today; a batch that stays on the thin kernels is held by them in any case.)
 static bool matrix_cores_only(const frk_weights *w, size_t batch) {
+    if (!k_quant_takes_the_matrix_cores(w, batch)) return false;
     const size_t n = w->rows * w->cols, nb = w->cols / QK_K, M = (size_t)1 << 20;
     const bool measured = nb <= 128;
     size_t from;
