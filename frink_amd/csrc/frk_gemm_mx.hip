@@ -419,10 +419,17 @@ static double expected_tiles(size_t pairs, size_t groups, double rows) {
 // workgroups become half as many and fit again.  Measured in us a layer, 64-row tiles / 96: where they do not fit, 32 experts
 // top-4 of 2880 / 2880 at 517 tokens 242 / 212, 16 top-2 of 2240 / 1312 at 741 106 / 88, 8 top-2 of 2880 / 2880 at 768 182 / 152; where they just
 // fit, of four wavefronts, 8 top-2 of 2048 / 2048 at 416 72 / 87, of eight, 8 top-2 of 2880 / 2880 at 448 108 / 122, 16 top-2 of 1536 / 1536 at
-// 864 77 / 86.  Over 118 drawn layers the choice is 1.0 % behind the better one on average, 11 % at most.
+// 864 77 / 86.  Nor where four wavefronts' workgroups, whose jobs are not cut in two, need two rounds with either tile: 8
+// top-4 of 2304 / 1088 at 694 tokens 124 / 148.  Over 278 drawn layers the choice is 0.8 % behind the better one on average, 12 % at
+// most; none is slower than before there were tiles of 96 rows.
 int mx_tile(size_t pairs, size_t groups, size_t rows_g, bool glu) {
-    const size_t rows = (size_t)mx_waves(pairs, groups, rows_g, glu) * (glu ? 32 : 64);
-    return expected_tiles(pairs, groups, MOE_TILE) * (double)((rows_g + rows - 1) / rows) > 258.5 ? MX_TILE : MOE_TILE;
+    const int waves = mx_waves(pairs, groups, rows_g, glu);
+    const size_t rows = (size_t)waves * (glu ? 32 : 64);
+    const double row_groups = (double)((rows_g + rows - 1) / rows), round = 1.01 * 256.0;
+    const double of64 = expected_tiles(pairs, groups, MOE_TILE) * row_groups;
+    if (of64 <= round) return MOE_TILE;
+    if (waves == 4 && of64 <= 512.0 && expected_tiles(pairs, groups, MX_TILE) * row_groups > round) return MOE_TILE;
+    return MX_TILE;
 }
 // up: the second matrix (y = silu(gate) * up), or null
 int launch_gemm_mx_grouped(const frk_weights *w, const frk_weights *up, size_t rows_g, const MxActs &acts, const int *src_rows,

@@ -232,6 +232,7 @@ def test_rows_whose_scale_leaves_f16_in_tiles_of_96(fa, rows_g, cols, counts):
 
 @pytest.mark.parametrize("pairs,groups,rows,glu,tile", [
     (832, 8, 2048, True, 64), (896, 8, 2880, True, 64), (1728, 16, 1536, True, 64),  # two tiles an expert, one round of the chip
+    (2776, 8, 1088, True, 64),  # two rounds of four wavefronts' workgroups with either tile
     (1000, 16, 1536, True, 96), (2048, 32, 2880, True, 96), (2400, 8, 2880, True, 96),
     (2508, 27, 1500, False, 96), (2352, 32, 4097, False, 96), (840, 9, 4064, True, 96), (864, 9, 8190, False, 96),  # the tests of such tiles here
 ])
