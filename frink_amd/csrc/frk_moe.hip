@@ -12,8 +12,9 @@ namespace frk {
 // index order (the reference's sequential f32 sum); among equal probabilities the lowest index
 // wins (the reference's unstable sort leaves that case undefined).  n_experts <= 1024, k <= 64.
 // NR: registers a lane (expert i lives in lane i % 64, register i / 64), n_experts <= 64 * NR.  A launch is one wavefront's
-// chain of dependent steps: over 16 registers whatever the number of experts 6.4 us for one token of 128 experts top-8
-// (profiler; an empty launch takes 3), over two 4.3.
+// chain of dependent steps: over 16 registers whatever the number of experts (exponentials of those in use) one token of 128 /
+// 256 / 384 / 512 experts top-8 took 5.8 / 6.8 / 7.7 / 8.7 us, call after call under the profiler, over 2 / 4 / 8 / 8 it takes
+// 2.9 / 4.1 / 5.5 / 6.0; 576 experts over 16 8.4, before 9.3.
 template <int NR>
 __global__ __launch_bounds__(64) void route_top_k_softmax_kernel(const float *__restrict__ logits, int batch,
                                                                  int n_experts, int k, int norm,
@@ -615,6 +616,7 @@ int launch_route_top_k_softmax(const float *logits, int batch, int n_experts, in
     if (n_experts <= 64) FRK_GO(1);
     else if (n_experts <= 128) FRK_GO(2);
     else if (n_experts <= 256) FRK_GO(4);
+    else if (n_experts <= 512) FRK_GO(8);
     else FRK_GO(16);
 #undef FRK_GO
     FRK_LAUNCH_CHECK("route_top_k_softmax");

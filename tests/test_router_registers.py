@@ -7,7 +7,7 @@ from test_gpu_parity import fa, to_dev  # noqa: F401 (fa: the module's fixture)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_experts", [1, 2, 63, 64, 65, 128, 129, 256, 257, 1000, 1024])
+@pytest.mark.parametrize("n_experts", [1, 2, 63, 64, 65, 128, 129, 256, 257, 511, 512, 513, 1000, 1024])
 def test_router_at_the_edges_of_its_registers(fa, n_experts):
     """The oracle's weights bit for bit and its ids, ties to the lowest index, whatever the number of registers a lane."""
     rng = np.random.default_rng(n_experts)
