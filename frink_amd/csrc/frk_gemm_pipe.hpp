@@ -37,7 +37,7 @@ struct GemmArgs {
     int row_tiles, tok_tiles;
     int k_split;     // parts of a row's blocks; with more than one each writes its sums to `partial`
     int k_last;      // the parts of the last token tile
-    float *partial;  // [k_split][M][rows], added up in order afterwards (launch_sum_parts)
+    float *partial;  // [k_split][M][rows], added up afterwards (launch_sum_parts)
     int parts_inner; // a row tile's parts next to each other in the work list
 };
 
@@ -469,7 +469,7 @@ __device__ __forceinline__ v16i tile_chain(TileOperands &T, const BPlanes &B, Be
 // A workgroup = 8 wavefronts = RG row groups of 32 weight rows x KS shares of the blocks; a wavefront
 // runs MT 32-token tiles against its rows' current block.  KS = 2 (small matrices: 128 rows x 64 tokens
 // per workgroup fill the chip where 256 x 128 would not) and KS = 4 (64 rows x 32 tokens) share the blocks
-// between wavefronts whose sums are added through LDS at the end, in the order of the shares.
+// between wavefronts whose sums are added through LDS at the end, four of them as (0 + 1) + (2 + 3).
 //
 // LDS: activations in a ring of 3 stages (requested two steps ahead), their scales in a ring of 4
 // (they are read by an epilogue that may run a step later), the raw weights in ONE slot per
@@ -878,7 +878,7 @@ __device__ __forceinline__ void pipe_gemm_tiles(const GemmArgs &g, const PipeEnt
         }
     }
 
-    // several shares of the blocks: the later ones' sums go through LDS and are added onto the first's, in order
+    // several shares of the blocks: the later ones' sums go through LDS and are added onto the first's, two and two
     if (KS > 1) {
         float *xch = reinterpret_cast<float *>(lds) + (size_t)rg * (KS - 1) * MT * 16 * 64;
         if (ks > 0) {
@@ -889,12 +889,15 @@ __device__ __forceinline__ void pipe_gemm_tiles(const GemmArgs &g, const PipeEnt
         }
         __syncthreads();
         if (ks > 0) return;
+        static_assert(KS <= 2 || KS == 4, "shares");
 #pragma unroll
-        for (int k = 0; k < KS - 1; k++)
+        for (int mt = 0; mt < ACT; mt++)
 #pragma unroll
-            for (int mt = 0; mt < ACT; mt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) sum[mt][r] += xch[((k * MT + mt) * 16 + r) * 64 + lane];
+            for (int r = 0; r < 16; r++) {
+                auto share = [&](int k) { return xch[(((k - 1) * MT + mt) * 16 + r) * 64 + lane]; };
+                sum[mt][r] += share(1);
+                if (KS == 4) sum[mt][r] += share(2) + share(3);
+            }
     }
     // store: a lane holds one weight row and 16 tokens per tile
     const int row = row_tile * ROWS + rg * 32 + li;
@@ -923,7 +926,7 @@ __device__ __forceinline__ void pipe_gemm(const GemmArgs &g) {
 // ------------------------------------------------------------------ host side
 
 // The workgroup tile of a batch: 256 rows x 128 tokens, 128 x 64 or 64 x 32, and how many workgroups share a row's
-// blocks (their sums, in SPLIT_PARTS_BYTES of memory at most, are added in order afterwards).
+// blocks (their sums, in SPLIT_PARTS_BYTES of memory at most, are added afterwards).
 struct PipePlan {
     int rows_wg, tok_wg, k_split, k_last;
 };

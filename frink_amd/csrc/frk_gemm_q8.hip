@@ -44,7 +44,7 @@ struct Q8GemmArgs {
     float *y;           // [M][rows]
     int rows, nb, M;
     int k_split;     // 1, or 2/4/8: blockIdx.z takes that share of the 256-column chunks (whole pairs of them)
-    float *partial;  // [k_split][M][rows], added up in order afterwards
+    float *partial;  // [k_split][M][rows], added up afterwards
     // GROUPED: W stacks the groups' matrices of `rows` rows each; tile blockIdx.y = {group, first row of the grouped
     // order, rows in use, first row of y} multiplies the activation rows src_rows[first + r] (first + r without a list)
     const int4 *tiles;
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(64 * TT * RT) void gemm_q8_0_mfma_kernel(Q8GemmArgs
 
 constexpr int Q8_MAX_SPLIT = 8;
 // A small grid (few token tiles, a short matrix) splits the chunks of a row between 2, 4 or 8
-// workgroups, no finer than two pairs of chunks each; their sums are added in order afterwards.
+// workgroups, no finer than two pairs of chunks each; their sums are added afterwards.
 static int q8_0_split(size_t rows, size_t M, size_t nb32) {
     const size_t wgs = M > 32 ? ((rows + 63) / 64) * ((M + 127) / 128) : (rows + 31) / 32;
     const size_t pairs = ((nb32 + Q8_CHUNK_BLOCKS - 1) / Q8_CHUNK_BLOCKS + 1) / 2;

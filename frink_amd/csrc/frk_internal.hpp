@@ -239,7 +239,7 @@ constexpr size_t SPLIT_PARTS_BYTES = (size_t)FRK_NOALLOC_PARTS_MIB << 20;
 // pipe_gemm_parts_bytes(...) of the parts' sums where the blocks are split between workgroups (0: they are not)
 size_t pipe_gemm_parts_bytes(int kind, size_t M, size_t cols, size_t rows);
 int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, hipStream_t s);
-// y[n] = partial[0][n] + partial[1][n] + ... in that order (the split GEMMs' second step; frk_gemm_q6.hip)
+// y[n] = partial[0][n] + partial[1][n] + ..., always in the same pairs (the split GEMMs' second step; frk_gemm_q6.hip)
 int launch_sum_parts(const float *partial, int parts, size_t n, float *y, hipStream_t s);
 int launch_sum_parts_apart(const float *partial, size_t n, size_t begin, size_t end, size_t split, int parts0, int parts1, float *y, hipStream_t s);
 // The same for Q8_0 (frk_gemm_q8.hip), over activations quantized 32 at a time.

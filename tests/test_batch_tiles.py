@@ -84,9 +84,8 @@ def test_no_token_tile_is_added_up_in_fewer_sums_than_at_a_full_price(kind, rows
     assert min(p.k_split, p.k_last) * (2 if p.rows_wg == 128 else 1) >= sums
 
 
-def _two_norm_errors(data, rows, cols, x, parts):
-    """The 2-norm errors against 64-bit sums of the float step with a block's mins apart and folded, a row's blocks in so
-    many sums added up in order: every operation of the kernel's float step in f32, in numpy."""
+def _block_terms(data, rows, cols, x):
+    """(A, D, N, s1, s2) of every block: what the float step adds is A * (D * s1 + N * s2), s1 and s2 exact."""
     f = np.float32
     nb = cols // 256
     blk = data.reshape(rows, nb, 144)
@@ -100,16 +99,29 @@ def _two_norm_errors(data, rows, cols, x, parts):
     aq, da = zip(*[fo.quantize_q8_k(r)[:2] for r in x])
     aq = np.stack(aq).reshape(len(x), nb, 8, 32).astype(np.float64)
     da = np.stack(da).reshape(len(x), nb).astype(f)
+    terms = []
+    for b in range(nb):
+        s1 = aq[:, b].reshape(len(x), 256) @ (q[:, b] * sc[:, b, :, None]).reshape(rows, 256).astype(np.float64).T
+        s2 = aq[:, b].sum(2) @ m[:, b].astype(np.float64).T
+        terms.append(tuple(np.broadcast_to(v, s1.shape) for v in (da[:, b, None], d[:, b], -dmin[:, b])) + (s1, s2))
+    return terms
 
-    def fma(a, b, c):
-        return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(f)
+
+def _fma(a, b, c):
+    return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(np.float32)
+
+
+def _two_norm_errors(data, rows, cols, x, parts):
+    """The 2-norm errors against 64-bit sums of the float step with a block's mins apart and folded, a row's blocks in so
+    many sums added up in order: every operation of the kernel's float step in f32, in numpy."""
+    f, fma = np.float32, _fma
+    nb = cols // 256
+    terms = _block_terms(data, rows, cols, x)
     exact, sums = 0.0, {"apart": [], "folded": []}
     for p in range(parts):
         acc = {k: np.zeros((len(x), rows), f) for k in sums}
         for b in range(nb * p // parts, nb * (p + 1) // parts):
-            s1 = aq[:, b].reshape(len(x), 256) @ (q[:, b] * sc[:, b, :, None]).reshape(rows, 256).astype(np.float64).T
-            s2 = aq[:, b].sum(2) @ m[:, b].astype(np.float64).T
-            D, N, A = (np.broadcast_to(v, s1.shape) for v in (d[:, b], -dmin[:, b], da[:, b, None]))
+            A, D, N, s1, s2 = terms[b]
             exact = exact + A.astype(np.float64) * (D.astype(np.float64) * s1 + N.astype(np.float64) * s2)
             acc["apart"] = fma(A, fma(N, s2.astype(f), D * s1.astype(f)), acc["apart"])
             c = ((D * (f(1) / N)) * s1.astype(f) + s2).astype(f)
@@ -136,3 +148,48 @@ def test_batches_of_the_small_tile_are_as_exact_as_its_float_step(fa, rows, batc
     print(error, want, flush=True)
     assert want["apart"] < 0.9 * want["folded"]
     assert error < (want["apart"] * want["folded"]) ** 0.5
+
+
+def _in_pairs(v):
+    while len(v) > 1:
+        v = [v[i] + v[i + 1] if i + 1 < len(v) else v[i] for i in range(0, len(v), 2)]
+    return v[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,batch,cols", [(1304, 26, 11008), (1111, 28, 11520)])
+def test_twelve_parts_are_added_in_pairs(fa, rows, batch, cols):
+    """Twelve parts of a row, four shares each: below the middle of the 2-norm errors that adding them in order and in pairs have."""
+    from bench import random_blocks
+    from frink_amd import synth
+    print("twelve parts' error", rows, cols, batch, flush=True)
+    p = _plan(fo.Q4_K, rows, batch, cols)
+    assert (p.rows_wg, p.k_split) == (64, 12)
+    data = random_blocks(fo.Q4_K, rows, cols, seed=rows)
+    x = synth.activations(batch, batch, cols)
+    w = fa.Weights.from_host(fo.Q4_K, data, rows, cols)
+    got = w.gemm(to_dev(x)).cpu().numpy()[:, :256].astype(np.float64)
+    w.release()
+    nb = cols // 256
+    terms = _block_terms(data.reshape(rows, -1)[:256], 256, cols, x)
+    exact = sum(A.astype(np.float64) * (D.astype(np.float64) * s1 + N.astype(np.float64) * s2) for A, D, N, s1, s2 in terms)
+    parts = []
+    for i in range(12):
+        b0, b1 = nb * i // 12, nb * (i + 1) // 12
+        steps = -(-(b1 - b0) // 4)
+        shares = [np.zeros(exact.shape, np.float32) for _ in range(4)]
+        for b in range(b0, b1):
+            A, D, N, s1, s2 = terms[b]
+            k = (b - b0) // steps
+            shares[k] = _fma(A, _fma(N, s2.astype(np.float32), D * s1.astype(np.float32)), shares[k])
+        parts.append(shares)
+    order = sum(parts[0][1:], parts[0][0])
+    for s in parts[1:]:
+        order = order + sum(s[1:], s[0])
+    want = {"order": order, "pairs": _in_pairs([_in_pairs(s) for s in parts])}
+    assert all(v.dtype == np.float32 for v in want.values())
+    want = {k: np.linalg.norm(v - exact) / np.linalg.norm(exact) for k, v in want.items()}
+    error = np.linalg.norm(got - exact) / np.linalg.norm(exact)
+    print(error, want, flush=True)
+    assert want["pairs"] < 0.92 * want["order"]
+    assert error < (want["pairs"] * want["order"]) ** 0.5
