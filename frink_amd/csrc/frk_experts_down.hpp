@@ -19,8 +19,9 @@ namespace frk {
 constexpr int EXPERTS_DOWN_WAVES = 8, EXPERTS_DOWN_MAX_SLOTS = 64, EXPERTS_DOWN_ROWS = 8, EXPERTS_DOWN_MAX_ROWS = 64;
 static __host__ __device__ inline size_t experts_down_act_bytes(int nb) { return (size_t)nb * (256 + 32 + 16); }
 
-template <class Unit, int LPR, int STEPS, int XB>
-__global__ __launch_bounds__(64 * EXPERTS_DOWN_WAVES) void experts_down_kernel(const uint8_t *__restrict__ W, Layout lay, int rows_e,
+// SIMD_WAVES: wavefronts whose registers a SIMD holds.
+template <class Unit, int LPR, int STEPS, int XB, int SIMD_WAVES>
+__global__ __launch_bounds__(64 * EXPERTS_DOWN_WAVES, SIMD_WAVES) void experts_down_kernel(const uint8_t *__restrict__ W, Layout lay, int rows_e,
                                                                                int rows_wg, int nb, int n_experts, int k,
                                                                                const int32_t *__restrict__ ids,
                                                                                const float *__restrict__ weights,
@@ -99,27 +100,16 @@ __global__ __launch_bounds__(64 * EXPERTS_DOWN_WAVES) void experts_down_kernel(c
     }
 }
 
-// Rows a workgroup, in eights.  Two workgroups fit a CU, and one takes about as long as quantizing its slots' intermediates
-// (two eights' worth of time) and its eights one after the other: a few workgroups past a whole round would cost a
-// second one (2048 rows of Q6_K at 6 tokens top-6 of 1280 columns, the layer: 516 workgroups of 24 rows 52.4 us, 384 of 32 48.2).
-static inline int experts_down_rows_wg(size_t rows_e, size_t batch) {
-    int best = 1;
-    size_t least = SIZE_MAX;
-    for (int n = 1; n <= EXPERTS_DOWN_MAX_ROWS / EXPERTS_DOWN_ROWS; n++) {
-        const size_t wgs = (rows_e + EXPERTS_DOWN_ROWS * n - 1) / (EXPERTS_DOWN_ROWS * n) * batch, time = (wgs + 511) / 512 * (size_t)(n + 2);
-        if (time < least) least = time, best = n;
-    }
-    return EXPERTS_DOWN_ROWS * best;
-}
+int experts_down_rows_wg(size_t rows_e, size_t batch, int waves, int simd_waves);  // frk_gemv_direct.hip
 static_assert(EXPERTS_DOWN_ROWS * 8 == EXPERTS_DOWN_MAX_ROWS && EXPERTS_DOWN_MAX_ROWS <= 64, "a thread a row, one wavefront at least");
 
-template <class Unit, int LPR, int STEPS, int XB>
+template <class Unit, int LPR, int STEPS, int XB, int SIMD_WAVES>
 static int launch_experts_down_as(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids,
                                   const float *weights, size_t batch, int k, float *out, hipStream_t s) {
     const int nb = (int)(w->cols / QK_K), waves = k < EXPERTS_DOWN_WAVES ? k : EXPERTS_DOWN_WAVES;
-    const int rows_wg = experts_down_rows_wg(rows_e, batch);
+    const int rows_wg = experts_down_rows_wg(rows_e, batch, waves, SIMD_WAVES);
     const size_t lds = (size_t)waves * experts_down_act_bytes(nb) + (size_t)k * rows_wg * 4;
-    hipLaunchKernelGGL((experts_down_kernel<Unit, LPR, STEPS, XB>), dim3((unsigned)((rows_e + rows_wg - 1) / rows_wg), (unsigned)batch),
+    hipLaunchKernelGGL((experts_down_kernel<Unit, LPR, STEPS, XB, SIMD_WAVES>), dim3((unsigned)((rows_e + rows_wg - 1) / rows_wg), (unsigned)batch),
                        dim3(64 * waves), lds, s, w->dev, w->layout, (int)rows_e, rows_wg, nb, n_experts, k, ids, weights, act, out);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(FRK_ERR_HIP, "experts_down launch: %s", hipGetErrorString(e));

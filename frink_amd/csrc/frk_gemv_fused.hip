@@ -1176,9 +1176,9 @@ int launch_gemv_q4_k_experts(const frk_weights *w, const frk_weights *w2, int n_
 // out[token][rows_e] = sum over the slots of weights * (rows of expert ids) . act[token][slot]; rows of at most 8 blocks
 int launch_q4_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids, const float *weights,
                              size_t batch, int k, float *out, hipStream_t s) {
-    if (w->cols <= 4 * QK_K) return launch_experts_down_as<Q4ExpertsUnit, 8, 1, 4>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
-    if (w->cols <= 6 * QK_K) return launch_experts_down_as<Q4ExpertsUnit, 16, 2, 6>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
-    return launch_experts_down_as<Q4ExpertsUnit, 16, 2, 8>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
+    if (w->cols <= 4 * QK_K) return launch_experts_down_as<Q4ExpertsUnit, 8, 1, 4, 5>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
+    if (w->cols <= 6 * QK_K) return launch_experts_down_as<Q4ExpertsUnit, 16, 2, 6, 4>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
+    return launch_experts_down_as<Q4ExpertsUnit, 16, 2, 8, 4>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
 }
 // act[r] = silu(gate[r] . x) * (up[r] . x): both matrices Q4_K of one shape, fused_gemv_fits
 int launch_gemv_q4_k_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s) {

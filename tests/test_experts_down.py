@@ -15,3 +15,15 @@ from test_gpu_parity import _moe_case, fa  # noqa: F401 (fa: the module's fixtur
 def test_down_projection_with_the_weighted_sum(fa, n_experts, k, hidden, ffn, batch, down_kind):
     print("experts down", down_kind, n_experts, k, hidden, ffn, batch, flush=True)
     _moe_case(fa, n_experts, k, hidden, ffn, batch, seed=n_experts + 31 * batch, down_kind=down_kind)
+
+
+@pytest.mark.parametrize("rows_e,batch,waves,simd_waves,rows", [
+    (2048, 15, 1, 3, 16), (2048, 1, 8, 4, 8), (3840, 13, 6, 4, 56), (512, 5, 6, 3, 16), (5120, 10, 8, 3, 40), (1, 1, 1, 5, 8), (1 << 20, 16, 8, 3, 64),
+])
+def test_rows_of_a_workgroup_by_how_many_fit_a_cu(rows_e, batch, waves, simd_waves, rows):
+    import ctypes as C
+
+    import frink_amd
+    f = frink_amd.lib()._ZN3frk20experts_down_rows_wgEmmii  # frk::experts_down_rows_wg
+    f.restype, f.argtypes = C.c_int, [C.c_size_t] * 2 + [C.c_int] * 2
+    assert f(rows_e, batch, waves, simd_waves) == rows
