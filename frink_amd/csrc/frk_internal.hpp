@@ -373,6 +373,7 @@ int launch_gemv_q6_k_experts(const frk_weights *w, int n_experts, size_t rows_e,
                              const int32_t *ids, size_t jobs, float *y, hipStream_t s);
 // a token's (or a few tokens') down projection with the weighted sum of its experts; down rows of at most 8 blocks
 constexpr size_t EXPERTS_DOWN_MAX_COLS = 8 * QK_K;
+bool experts_down_takes(int down_kind, size_t rows_e, size_t ffn, size_t batch, size_t k);  // frk_moe.hip
 int launch_q6_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids, const float *weights,
                              size_t batch, int k, float *out, hipStream_t s);
 int launch_q4_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e, const float *act, const int32_t *ids, const float *weights,

@@ -719,6 +719,19 @@ bool moe_takes_per_token_path(size_t batch, size_t hidden, size_t ffn, int down_
     const bool down_ok = down_kind == FRK_KIND_Q4_K || (down_kind == FRK_KIND_Q6_K && ffn <= 4096);
     return down_ok && batch <= MOE_PER_TOKEN_MAX_BATCH && hidden <= FUSED_GEMV_MAX_COLS && ffn <= FUSED_GEMV_MAX_COLS;
 }
+// Whether the down projection's launch adds up a token's experts too (frk_experts_down.hpp).  A wavefront takes a slot: with five to
+// seven of them a CU's SIMDs have unequal shares, past eight a wavefront has its slots one after the other, and the longer the rows (and
+// the registers they take) the fewer workgroups hide that; the launches apart give every pair workgroups of its own.  Layer without / with it,
+// us: 16 tokens of 128 experts top-8 of 2048 / 768 75 / 64 (Q6_K) and 77 / 61 (Q4_K), 8 tokens of 60 top-4 of 2048 / 1280 33.1 / 29.2 (Q6_K);
+// rows of five and six Q6_K blocks over 52 drawn layers top-8 0.91 of the time, 64 top-6 0.94 below eight tokens and 1.02 from there; seven
+// and eight blocks top-5 .. 16 1.00 (0.93 .. 1.13; Q6_K top-8 0.95), top-1 .. 4 0.94; short rows of more than 16 slots only where they are many: 48 top-48 of
+// 2304 / 256 at one token 31.2 / 36.9, 64 top-64 of 512 / 256 20.9 / 26.7.
+bool experts_down_takes(int down_kind, size_t rows_e, size_t ffn, size_t batch, size_t k) {
+    if (ffn > EXPERTS_DOWN_MAX_COLS) return false;
+    if (ffn <= 4 * QK_K) return k <= 16 || rows_e * batch >= 112 * k;
+    if (k <= 4 || (k == 8 && down_kind == FRK_KIND_Q6_K)) return true;
+    return ffn <= 6 * QK_K && k <= 8 && (down_kind == FRK_KIND_Q4_K || batch < 8);
+}
 static int launch_moe_ffn_per_token(const frk_weights *gate, const frk_weights *up, const frk_weights *down,
                                     int n_experts, const float *x, size_t batch, const int32_t *ids,
                                     const float *weights, int k, float *out, const MoeScratch &m, hipStream_t s) {
@@ -726,13 +739,7 @@ static int launch_moe_ffn_per_token(const frk_weights *gate, const frk_weights *
     float *act = m.gate_out;  // [batch*k][ffn]
     int rc = launch_gemv_q4_k_experts(gate, up, n_experts, (size_t)ffn, x, (size_t)hidden, ids, batch, (size_t)k, act, s);
     if (rc) return rc;
-    // The weighted sum in the down projection's launch (frk_experts_down.hpp; offsets within an expert are 32 bits wide).
-    // Layer before / with it, us: one token of 128 experts top-8 of 2048 / 768 23.5 / 20.6 (bound by the host's calls), 16
-    // tokens 75 / 64 (Q6_K) and 77 / 61 (Q4_K), 8 tokens of 60 top-4 of 2048 / 1280 42 / 36.  Not for longer Q6_K rows of
-    // five to seven slots, whose wavefronts share a CU's SIMDs unevenly (top-6 of 2048 / 1536 at 3 tokens 34.0 / 34.4, of
-    // 2048 / 1280 at 6 46.4 / 48.2, at 12 78.3 / 79.3; top-8 at 3 tokens 40.8 / 39.6).
-    const bool uneven = down->kind == FRK_KIND_Q6_K && ffn > 4 * QK_K && k > 4 && k < 8 && batch > 2;
-    if (down->cols <= EXPERTS_DOWN_MAX_COLS && (size_t)hidden * down->layout.row_stride <= 0xffffffffu && !uneven)
+    if (experts_down_takes(down->kind, (size_t)hidden, (size_t)ffn, batch, (size_t)k) && (size_t)hidden * down->layout.row_stride <= 0xffffffffu)  // (32-bit offsets)
         return down->kind == FRK_KIND_Q6_K
                    ? launch_q6_k_experts_down(down, n_experts, (size_t)hidden, act, ids, weights, batch, k, out, s)
                    : launch_q4_k_experts_down(down, n_experts, (size_t)hidden, act, ids, weights, batch, k, out, s);

@@ -27,3 +27,18 @@ def test_rows_of_a_workgroup_by_how_many_fit_a_cu(rows_e, batch, waves, simd_wav
     f = frink_amd.lib()._ZN3frk20experts_down_rows_wgEmmii  # frk::experts_down_rows_wg
     f.restype, f.argtypes = C.c_int, [C.c_size_t] * 2 + [C.c_int] * 2
     assert f(rows_e, batch, waves, simd_waves) == rows
+
+
+@pytest.mark.parametrize("kind,rows,ffn,batch,k,takes", [
+    (fo.Q6_K, 512, 1024, 1, 16, True), (fo.Q6_K, 2304, 256, 1, 48, False), (fo.Q4_K, 2304, 256, 16, 48, True), (fo.Q4_K, 512, 256, 1, 64, False),
+    (fo.Q6_K, 2048, 1280, 16, 4, True), (fo.Q6_K, 2048, 1280, 7, 6, True), (fo.Q6_K, 2048, 1280, 8, 6, False), (fo.Q6_K, 2048, 1536, 16, 8, True),
+    (fo.Q4_K, 2048, 1536, 16, 7, True), (fo.Q4_K, 2048, 1536, 1, 9, False), (fo.Q6_K, 5120, 2048, 1, 5, False), (fo.Q6_K, 2816, 1792, 1, 8, True), (fo.Q4_K, 2816, 1792, 1, 8, False), (fo.Q6_K, 2816, 1792, 1, 9, False),
+    (fo.Q4_K, 512, 1792, 1, 9, False), (fo.Q4_K, 512, 2048, 1, 4, True), (fo.Q4_K, 512, 2304, 1, 1, False),
+])
+def test_where_the_sum_is_in_the_down_projection(kind, rows, ffn, batch, k, takes):
+    import ctypes as C
+
+    import frink_amd
+    f = frink_amd.lib()._ZN3frk18experts_down_takesEimmmm  # frk::experts_down_takes
+    f.restype, f.argtypes = C.c_bool, [C.c_int] + [C.c_size_t] * 4
+    assert f(kind, rows, ffn, batch, k) == takes
