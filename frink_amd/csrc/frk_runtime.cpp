@@ -630,8 +630,9 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
 // Whether a batch takes the matrix-core GEMM.  Its cost is flat up to 32 rows (64 x 32 tiles) and up to 64; below, the thin
 // kernels' groups of 16 (Q4_K, Q5_K) or 8 rows are ahead by what a group costs at the matrix's shape.  nb blocks a row, with
 // quantization (us; thin / GEMM), within 32768 columns:
-//   Q4_K  from 17 rows on always (of 71 drawn matrices the GEMM is ahead for all: 14336x4096 at 17 19.6 / 14.9; 3335x5120, the
-//         closest, 0.92 of the time).  From 9 on rows of 30 blocks and more (1861x7680 at 9 0.98, 4096x11008 19.9 / 16.6) and,
+//   Q4_K  from 17 rows on (14336x4096 at 17 19.6 / 14.9; 3335x5120 0.92 of the time), but for 8 and 12 blocks up to 4096 rows, where two thin
+//         launches take as long (1264x2048 at 23 9.5 / 9.9, 2375x3072 10.2 / 10.3, 4054x2048 at 19 9.8 / 9.8; at 17 and 18, whose second one is
+//         slower, 10.3 / 9.7) and activations quantized beforehand need no tiled copy (frk_hip_gemm_q8k_dev 7.3 / 9.2).  From 9 on rows of 30 blocks and more (1861x7680 at 9 0.98, 4096x11008 19.9 / 16.6) and,
 //         past one workgroup a CU, of 24: 4771x7168 0.72, but 1798x6144 1.07, 7986x5120 1.15.
 //   Q5_K  from 17 rows on (62 of 65 drawn ahead; 14257x2304 1.09, 4096x4096 at 17 20.4 / 13.4), and from 9 on rows of 32 blocks
 //         and more (4096x11008 25.3 / 19.3) and, past 4608 rows, of 24: 5230x6144 0.78, but 2491x6912 1.20.
@@ -647,6 +648,7 @@ static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     const bool measured = nb <= 128;
     if (w->kind == FRK_KIND_Q4_K) {
         const bool eights = thin_gemm_max_batch(w) < 16;  // rows of a thin launch
+        if ((nb == 8 || nb == 12) && w->rows <= 4096 && batch >= 19 && batch <= 32) return false;
         if (batch >= 17) return measured || batch >= 33 || n > 20 * M || eights;
         return measured && (nb >= 30 || (nb >= 24 && w->rows > 4096 && (eights || w->rows <= 8192)));
     }

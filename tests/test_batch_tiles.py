@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle as fo
-from test_gpu_parity import fa, to_dev  # noqa: F401 (fa: the module's fixture)
+from test_gpu_parity import fa, make_weights, to_dev  # noqa: F401 (fa: the module's fixture)
 
 
 @pytest.mark.gpu
@@ -193,3 +193,17 @@ def test_twelve_parts_are_added_in_pairs(fa, rows, batch, cols):
     print(error, want, flush=True)
     assert want["pairs"] < 0.92 * want["order"]
     assert error < (want["pairs"] * want["order"]) ** 0.5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,batch", [(1264, 2048, 19), (300, 2048, 32), (4096, 3072, 23)])
+def test_short_rows_stay_on_the_thin_kernels(fa, rows, cols, batch):
+    """Q4_K of 8 and 12 blocks: a row's results do not depend on the batch that it came in with, up to 32 rows."""
+    from frink_amd import synth
+    w = fa.Weights.from_host(fo.Q4_K, make_weights(fo.Q4_K, rows, cols, seed=rows), rows, cols)
+    x = to_dev(synth.activations(batch, batch, cols))
+    y, first = w.gemm(x).cpu().numpy(), w.gemm(x[:16].contiguous()).cpu().numpy()
+    assert np.array_equal(y[:16].view(np.uint32), first.view(np.uint32))
+    q8k = w.gemm_q8k(fa.quantize_q8_k(x.reshape(-1)), batch).cpu().numpy()
+    assert np.array_equal(q8k.view(np.uint32), y.view(np.uint32))
+    w.release()
