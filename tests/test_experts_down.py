@@ -18,7 +18,7 @@ def test_down_projection_with_the_weighted_sum(fa, n_experts, k, hidden, ffn, ba
 
 
 @pytest.mark.parametrize("rows_e,batch,waves,simd_waves,rows", [
-    (2048, 15, 1, 3, 16), (2048, 1, 8, 4, 8), (3840, 13, 6, 4, 56), (512, 5, 6, 3, 16), (5120, 10, 8, 3, 40), (1, 1, 1, 5, 8), (1 << 20, 16, 8, 3, 64),
+    (2048, 15, 1, 3, 16), (2048, 1, 8, 4, 8), (3840, 13, 6, 4, 56), (512, 5, 6, 3, 16), (5120, 10, 8, 3, 56), (2048, 4, 4, 4, 16), (1, 1, 1, 5, 8), (1 << 20, 16, 8, 3, 64),
 ])
 def test_rows_of_a_workgroup_by_how_many_fit_a_cu(rows_e, batch, waves, simd_waves, rows):
     import ctypes as C
