@@ -638,7 +638,8 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
 //         and more (4096x11008 25.3 / 19.3) and, past 4608 rows, of 24: 5230x6144 0.78, but 2491x6912 1.20.
 //   Q6_K  odd nb (not the streamed thin kernel's): from 9 on matrices of 18 M weights (4096x11008 at 13 28.9 / 19.7, 2631x7936
 //         0.67, but 1914x8960 at 16 1.08), at 17 of 8 M and more than 1280 rows (1822x5376 0.68, but 1144x8448 1.07), at 33 of 5 M.
-//         Even: from 9 on past 48 M and 4096 rows (4207x12288 0.81, but 4096x14336 20.1 / 22.2), at 17 past 23 M (6574x6144
+//         Even: from 9 on past 48 M and 4096 rows (4207x12288 0.81, but 4096x14336 20.1 / 22.2; over 250 drawn 0.86, five of them, 8200 .. 9200 rows of 28 .. 32
+//         blocks and one more, 1.05 .. 1.10), at 17 past 23 M (6574x6144
 //         0.79, 2015x12800 0.92, but 4788x4096 1.11), at 25 past 17 M (4788x4096 0.98, but 1897x6656 1.05).
 // (Below tiled_from(cols) none: a batch quantized without knowing its matrices has tiles from there on.)
 static size_t tiled_from(size_t cols) { return cols >= 24 * QK_K ? 9 : 17; }
