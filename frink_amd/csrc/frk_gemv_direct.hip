@@ -690,17 +690,18 @@ int launch_gemv_q6_k_experts(const frk_weights *w, int n_experts, size_t rows_e,
 
 // Rows a workgroup, in eights.  A workgroup takes about as long as quantizing its slots' intermediates (two eights' worth of
 // time) and its eights one after the other; as many fit a CU as its SIMDs have room for (a workgroup of five to eight wavefronts has two on
-// a SIMD), and a few workgroups past a whole round cost a second one.  What all wavefronts of a CU issue counts a fifth of that.  Over 940
+// a SIMD; of four wavefronts more than two workgroups gain nothing, 1.013 either way), and a few workgroups past a whole round cost a
+// second one.  What all wavefronts of a CU issue counts a fifth of that, which four wavefronts do not show.  Over 940
 // drawn layers of 1 .. 16 tokens and 1 .. 16 slots the layer takes 1.012 of the time of the best number of rows, 1.15 at worst; 1.038 and
 // 1.25 with two workgroups a CU assumed whatever their size (Q6_K's 159 registers for five and six blocks let one workgroup of six wavefronts fit:
 // 2304 rows of five blocks at two tokens top-6, 16 rows 27.8 us, 24 rows 22.7; one wavefront: 2048 rows at 15 tokens top-1 64 rows 22.4 us, 16 rows 18.7).
 int experts_down_rows_wg(size_t rows_e, size_t batch, int waves, int simd_waves) {
-    const int fit = waves > 4 ? simd_waves / 2 : 4 * simd_waves / waves;
+    const int fit = waves > 4 ? simd_waves / 2 : waves == 4 ? 2 : 4 * simd_waves / waves, issue = waves == 4 ? 0 : waves;
     int best = 1;
     size_t least = SIZE_MAX;
     for (int n = 1; n <= EXPERTS_DOWN_MAX_ROWS / EXPERTS_DOWN_ROWS; n++) {
         const size_t wgs = (rows_e + EXPERTS_DOWN_ROWS * n - 1) / (EXPERTS_DOWN_ROWS * n) * batch, round = 256 * (size_t)fit;
-        const size_t time = (wgs + round - 1) / round * (size_t)(n + 2) * 1280 + wgs * (size_t)(waves * (n + 1));
+        const size_t time = (wgs + round - 1) / round * (size_t)(n + 2) * 1280 + wgs * (size_t)(issue * (n + 1));
         if (time < least) least = time, best = n;
     }
     return EXPERTS_DOWN_ROWS * best;
