@@ -641,7 +641,7 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
 //         Even: from 9 on past 48 M and 4096 rows (4207x12288 0.81, but 4096x14336 20.1 / 22.2; over 250 drawn 0.86, five of them, 8200 .. 9200 rows of 28 .. 32
 //         blocks and one more, 1.05 .. 1.10), at 17 past 23 M (6574x6144
 //         0.79, 2015x12800 0.92, but 4788x4096 1.11), at 25 past 17 M (4788x4096 0.98, but 1897x6656 1.05).
-// (Below tiled_from(cols) none: a batch quantized without knowing its matrices has tiles from there on.)
+// Of what gemm_k_rows_kernel does not take (k_rows_take, which comes first).
 static size_t tiled_from(size_t cols) { return cols >= 24 * QK_K ? 9 : 17; }
 static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     if (batch < tiled_from(w->cols)) return false;
@@ -687,11 +687,64 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
     }
     return batch >= std::max(from, tiled_from(w->cols));
 }
+// Whether gemm_k_rows_kernel takes a batch (frk_gemm_rows.hip: sixteen rows a workgroup, no split, no second launch), ahead of both the
+// thin kernels and the 64 x 32 tiles of the pipelined GEMM.  It reads all tokens' tiles once for every sixteen rows, so what
+// is against it is many rows times many tokens (from 17 on twice the bytes) and rows so few and long that its workgroups'
+// chains are the launch.  nb blocks a row, with quantization, us before / now:
+//   Q4_K  in batches of up to 8 not the span kernel's rows of 4, 12, 16 .. 32 blocks (6181x3072 at 4 7.8 / 8.6; but 4096x11008 at 8
+//         14.8 / 11.9), nor at 3 and 4 past one round of the chip (7810x9984 16.1 / 17.1), nor where a second one is nearly full (0.95 at best, and
+//         slower from activations quantized beforehand).  9 .. 16 rows 14336x4096 19.5 / 14.1, 4096x14336 18.0 / 14.0.
+//         From 17 on rows of up to 19 blocks (4096x4096 at 32 12.3 / 9.1) and, in one round of the chip, of up to 32; but 14336x4096 16.3 / 18.9,
+//         4096x14336 19.2 / 19.8.
+//   Q5_K  4096x11008 at 8 and 16 16.0 / 12.7 and 19.1 / 12.8, 4096x4096 at 32 13.7 / 9.9, in one round of the chip at 32 whatever
+//         the length (4096x14336 22.8 / 20.9), but 12000x12032 38.4 / 42.3.
+//   Q6_K  odd nb always (4096x11008 at 8, 13 and 32 17.7 / 13.6, 19.8 / 13.8, 21.1 / 16.1); even up to 8 rows not the streamed thin
+//         kernel's longer or taller ones (4096x14336 14.3 / 16.0); 4096x14336 at 16 and 32 20.7 / 16.1, 23.4 / 19.3; but 1741x11776 at 10 13.1 / 14.1,
+//         13523x6144 at 31 25.9 / 31.0.
+// Over 1774 drawn batches of 2 .. 32 rows of 256 .. 14336 rows and 4 .. 56 blocks: 0.87 of the time before in the mean (the
+// better of both everywhere would be 0.2 % less), 1.12 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
+// From activations quantized beforehand (frk_hip_gemm_q8k_dev, frk_hip_gemm_acts_dev) 0.84 and 0.77, gemm_pair 0.78.
+static bool k_rows_take(const frk_weights *w, size_t batch) {
+    const size_t rows = w->rows, nb = w->cols / QK_K;
+    if (batch < 2 || batch > 32 || nb > 128) return false;
+    const bool one_round = rows > 2048 && rows <= 4096, few = rows < 1024;
+    if (w->kind == FRK_KIND_Q4_K) {
+        const bool span = nb % 4 == 0 && nb <= 32;
+        if (batch == 2) return false;
+        if (batch <= 8) return !(span && nb != 8) && (rows <= 4096 || (batch > 4 && !(rows > 6144 && rows <= 8192)));
+        if (batch <= 16) return !(few && nb >= 44) && !(span && rows < 2048 && (nb == 4 || nb == 16 || nb == 20));
+        return rows <= 8192 && (nb < 20 || (nb <= 32 && one_round));
+    }
+    if (w->kind == FRK_KIND_Q5_K) {
+        if (batch <= 4) return rows <= 10240 || nb < 20;
+        if (batch <= 16) return batch <= 8 || !(few && nb >= 44);
+        return nb < 20 || one_round || (nb < 28 && rows > 6144 && rows <= 8192);
+    }
+    if (w->kind != FRK_KIND_Q6_K || batch == 2) return false;
+    if (batch <= 8) return nb % 2 || nb < 16 || (nb <= 32 && rows <= 4096);
+    if (batch <= 16) return nb % 2 || nb < 40 || rows >= 2048;
+    return (nb % 2 || nb < 33 || rows >= 2048) && (rows <= 12288 || nb < 24);
+}
+// Q6_K batches of up to 8 rows it reads as plain Q8_K rows, whose quantization is the shorter launch (2.7 us, as tiles 3.6).  A
+// load then touches a line a row: over 290 drawn ones 0.96 of the time from tiles, but Q4_K and Q5_K, whose loads are twice as
+// many, 1.08 and 1.11 of it.
+static bool k_rows_plain(const frk_weights *w, size_t batch) { return w->kind == FRK_KIND_Q6_K && batch <= 8; }
+// A K-quant batch that is multiplied from its tiles: gemm_k_rows_kernel's, or the pipelined GEMM's.
+static bool takes_tiles(const frk_weights *w, size_t batch) {
+    return k_rows_take(w, batch) ? !k_rows_plain(w, batch) : k_quant_takes_the_matrix_cores(w, batch);
+}
+static size_t tiled_parts_bytes(const frk_weights *w, size_t batch) {
+    return k_rows_take(w, batch) ? 0 : pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows);
+}
+static int gemm_tiled(const frk_weights *w, const Q8KTiled &acts, size_t batch, float *y, void *parts, hipStream_t s) {
+    return k_rows_take(w, batch) ? launch_gemm_k_rows(w, (int)batch, acts, nullptr, y, s) : launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+}
+
 static size_t acts_plain_bytes(size_t batch, size_t cols) {
     const size_t n = batch * cols;
     return round_up(n, 256) + round_up(n / QK_K * 4, 256) + round_up(n / 16 * 2, 256);
 }
-// A batch between the two crossings needs more scratch memory on the matrix cores than the thin kernels do (none of their own, or
+// A batch below the higher crossing needs more scratch memory as tiles than the thin kernels do (none of their own, or
 // plain rows): on a stream that is being captured its buffer grows where it would have done for those.
 static size_t held_for_capture(const frk_weights *w, size_t batch) {
     return matrix_cores_only(w, batch) ? SIZE_MAX : acts_plain_bytes(batch, w->cols);
@@ -702,10 +755,11 @@ static bool thin_kernels_hold(const frk_weights *w, size_t batch) {
     return k_quant && batch >= 2 && !matrix_cores_only(w, batch) && thin_gemm_max_batch(w) >= 2;
 }
 
-// a thin batch over activations already in Q8_K: `thin` rows a launch (thin_gemm_max_batch), or one launch over a
+// a thin batch over activations already in Q8_K: gemm_k_rows_kernel's, `thin` rows a launch (thin_gemm_max_batch), or one launch over a
 // grid of such groups where the kernel has that form
 static int thin_gemm_acts(const frk_weights *w, const Q8KActs &a, size_t batch, int thin, float *y, hipStream_t s) {
     const size_t nb = w->cols / QK_K;
+    if (k_rows_take(w, batch) && k_rows_plain(w, batch)) return launch_gemm_k_rows(w, (int)batch, Q8KTiled{}, &a, y, s);
     if (batch > (size_t)thin && batch <= (size_t)thin_gemm_wide_rows(w)) return launch_thin_gemm_wide(w, (int)batch, a, y, s);
     for (size_t b0 = 0; b0 < batch; b0 += (size_t)thin) {
         const int n = (int)std::min<size_t>((size_t)thin, batch - b0);
@@ -791,16 +845,16 @@ static int gemm_units_int(const frk_weights *w, const float *x, size_t batch, fl
 static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *y, void *stream, Scratch &scratch) {
     // one row is the decode path, whatever the kind
     if (batch == 1) return gemv_impl(w, x, y, FRK_ACT_F32, (hipStream_t)stream, scratch);
-    if (k_quant_takes_the_matrix_cores(w, batch)) {  // (frk_hip_gemm_pair_dev: the same test)
+    if (takes_tiles(w, batch)) {  // (frk_hip_gemm_pair_dev: the same test)
         hipStream_t s = (hipStream_t)stream;
         void *ws = nullptr, *parts = nullptr;
-        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts,
+        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), tiled_parts_bytes(w, batch), s, &ws, &parts,
                              held_for_capture(w, batch));
         if (rc) return rc;
         const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
         rc = launch_quantize_q8_k_tiled(x, batch, w->cols, acts, s);
         if (rc) return rc;
-        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        return gemm_tiled(w, acts, batch, y, parts, s);
     }
     // Q8_0: a batch is the integer path, as in the reference (Q8_0 activation blocks and dot_q8_0_q8,
     // crates/frink-core/src/weight_matrix.rs:2701-2829); a single row keeps the f32 dot of its decode path
@@ -867,15 +921,19 @@ int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
                          "quantizes into a tiled form of its own): frk_hip_gemm_dev / frk_hip_gemm_pair_dev", batch);
     Q8KActs a{q, d, bsums};
     hipStream_t s = (hipStream_t)stream;
-    if (k_quant_takes_the_matrix_cores(w, batch)) {
+    // (for a small matrix, or a few rows, a launch to make tiles of them costs more than what the rows' lines do)
+    const bool small = w->rows * w->cols < (size_t)16 << 20 && batch <= (w->kind == FRK_KIND_Q6_K ? 32 : 16);
+    if (k_rows_take(w, batch) && (batch <= 4 || k_rows_plain(w, batch) || small))
+        return launch_gemm_k_rows(w, (int)batch, Q8KTiled{}, &a, y, s);
+    if (takes_tiles(w, batch)) {
         void *ws = nullptr, *parts = nullptr;
         Scratch scratch;
-        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows), s, &ws, &parts, 0);
+        int rc = scratch.get(q8k_tiled_bytes(batch, w->cols), tiled_parts_bytes(w, batch), s, &ws, &parts, 0);
         if (rc) return rc;
         const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
         rc = launch_tile_q8_k(a, batch, w->cols, acts, s);
         if (rc) return rc;
-        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        return gemm_tiled(w, acts, batch, y, parts, s);
     }
     return thin_gemm_acts(w, a, batch, thin_gemm_max_batch(w), y, s);
 }
@@ -889,11 +947,10 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
         return set_error(FRK_ERR_SHAPE, "the matrices have %zu and %zu columns: they share one batch of activations", w0->cols, w1->cols);
     hipStream_t s = (hipStream_t)stream;
     Scratch scratch;
-    if (k_quant_takes_the_matrix_cores(w0, batch) && k_quant_takes_the_matrix_cores(w1, batch)) {
+    if (takes_tiles(w0, batch) && takes_tiles(w1, batch)) {
         // one quantization into the tiled form, then the two GEMMs (each with its own room for a split's parts)
         const size_t acts_bytes = round_up(q8k_tiled_bytes(batch, w0->cols), 256);
-        const size_t part0 = round_up(pipe_gemm_parts_bytes(w0->kind, batch, w0->cols, w0->rows), 256);
-        const size_t part1 = pipe_gemm_parts_bytes(w1->kind, batch, w1->cols, w1->rows);
+        const size_t part0 = round_up(tiled_parts_bytes(w0, batch), 256), part1 = tiled_parts_bytes(w1, batch);
         // (one matrix beyond the higher crossing: what it needs on its own)
         auto alone = [&](const frk_weights *w, size_t parts) { return matrix_cores_only(w, batch) ? acts_bytes + parts : held_for_capture(w, batch); };
         const bool only = matrix_cores_only(w0, batch) && matrix_cores_only(w1, batch);
@@ -903,9 +960,9 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
         const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
         rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
         if (rc) return rc;
-        rc = launch_pipe_gemm_acts(w0, acts, batch, y0, parts, s);
+        rc = gemm_tiled(w0, acts, batch, y0, parts, s);
         if (rc) return rc;
-        return launch_pipe_gemm_acts(w1, acts, batch, y1, (char *)parts + part0, s);
+        return gemm_tiled(w1, acts, batch, y1, (char *)parts + part0, s);
     }
     // otherwise each matrix takes the path frk_hip_gemm_dev gives it (the same results, two quantizations)
     int rc = gemm_impl(w0, x, batch, y0, stream, scratch);
@@ -917,9 +974,9 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
 // The object owns room for both forms the K-quant kernels read: plain Q8_K rows (the decode and thin kernels)
 // and the tiled form (the matrix-core GEMMs).  Which of them a batch gets depends on its size alone, so that
 // the quantization does not need to know the matrices: plain rows up to ACTS_PLAIN_MAX_BATCH rows (the thin
-// kernels take at most 40), tiles from tiled_from(cols) rows on, both out of one launch where a
+// kernels take at most 40), tiles from two rows on (a single one is the decode kernels'), both out of one launch where a
 // batch has both.
-constexpr size_t ACTS_PLAIN_MAX_BATCH = 64;
+constexpr size_t ACTS_PLAIN_MAX_BATCH = 64, ACTS_TILED_MIN_BATCH = 2;
 }  // extern "C"
 struct frk_batch_acts {
     size_t max_batch = 0, cols = 0;
@@ -945,7 +1002,7 @@ int frk_hip_batch_acts_create(size_t max_batch, size_t cols, frk_batch_acts **ou
     a->max_batch = max_batch;
     a->cols = cols;
     a->tiled_off = round_up(acts_plain_bytes(std::min(max_batch, ACTS_PLAIN_MAX_BATCH), cols), 256);
-    const size_t bytes = a->tiled_off + (max_batch >= tiled_from(cols) ? round_up(q8k_tiled_bytes(max_batch, cols), 256) : 0);
+    const size_t bytes = a->tiled_off + (max_batch >= ACTS_TILED_MIN_BATCH ? round_up(q8k_tiled_bytes(max_batch, cols), 256) : 0);
     hipError_t e = hipMalloc(&a->base, bytes);
     if (e != hipSuccess) {
         delete a;
@@ -971,7 +1028,7 @@ int frk_hip_quantize_batch_acts_dev(frk_batch_acts *a, const float *x, size_t ba
         return set_error(FRK_ERR_SHAPE, "a batch of %zu rows in an object made for at most %zu", batch, a->max_batch);
     hipStream_t s = (hipStream_t)stream;
     a->batch = 0;
-    const bool tiled = batch >= tiled_from(a->cols);
+    const bool tiled = batch >= ACTS_TILED_MIN_BATCH;
     Q8KActsOut plain;
     if (batch <= ACTS_PLAIN_MAX_BATCH) {
         const size_t n = batch * a->cols;
@@ -998,9 +1055,9 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *a, float *
         return set_error(FRK_ERR_UNSUPPORTED, "Q8_K activations feed Q4_K, Q5_K and Q6_K weights only (kind %d): frk_hip_gemm_dev", w->kind);
     const size_t batch = a->batch;
     hipStream_t s = (hipStream_t)stream;
-    if (k_quant_takes_the_matrix_cores(w, batch)) {
+    if (takes_tiles(w, batch)) {
         const Q8KTiled acts = q8k_tiled_carve((char *)a->base + a->tiled_off, batch, a->cols);
-        const size_t parts_bytes = pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows);
+        const size_t parts_bytes = tiled_parts_bytes(w, batch);
         void *parts = nullptr;
         Scratch scratch;
         if (parts_bytes) {  // a split of the blocks between workgroups: room for the parts' sums
@@ -1008,7 +1065,7 @@ int frk_hip_gemm_acts_dev(const frk_weights *w, const frk_batch_acts *a, float *
             int rc = scratch.get(parts_bytes, 0, s, &parts, &none, matrix_cores_only(w, batch) ? SIZE_MAX : 0);
             if (rc) return rc;
         }
-        return launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+        return gemm_tiled(w, acts, batch, y, parts, s);
     }
     // (below the matrix-core GEMMs' batches the plain rows are there: ACTS_PLAIN_MAX_BATCH covers every such batch)
     if (batch > ACTS_PLAIN_MAX_BATCH)
