@@ -691,53 +691,54 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 // thin kernels and the 64 x 32 tiles of the pipelined GEMM.  It reads all tokens' tiles once for every sixteen rows, so what
 // is against it is many rows times many tokens (from 17 on twice the bytes) and rows so few and long that its workgroups'
 // chains are the launch.  nb blocks a row, with quantization, us before / now:
-//   Q4_K  in batches of up to 8 not the span kernel's rows of 4, 12, 16 .. 32 blocks (6181x3072 at 4 7.8 / 8.6; but 4096x11008 at 8
-//         14.8 / 11.9), nor at 3 and 4 past one round of the chip (7810x9984 16.1 / 17.1), nor where a second one is nearly full (0.95 at best, and
-//         slower from activations quantized beforehand).  9 .. 16 rows 14336x4096 19.5 / 14.1, 4096x14336 18.0 / 14.0.
-//         From 17 on rows of up to 19 blocks (4096x4096 at 32 12.3 / 9.1) and, in one round of the chip, of up to 32; but 14336x4096 16.3 / 18.9,
-//         4096x14336 19.2 / 19.8.
-//   Q5_K  4096x11008 at 8 and 16 16.0 / 12.7 and 19.1 / 12.8, 4096x4096 at 32 13.7 / 9.9, in one round of the chip at 32 whatever
-//         the length (4096x14336 22.8 / 20.9), but 12000x12032 38.4 / 42.3.
-//   Q6_K  odd nb always (4096x11008 at 8, 13 and 32 17.7 / 13.6, 19.8 / 13.8, 21.1 / 16.1); even up to 8 rows not the streamed thin
-//         kernel's longer or taller ones (4096x14336 14.3 / 16.0); 4096x14336 at 16 and 32 20.7 / 16.1, 23.4 / 19.3; but 1741x11776 at 10 13.1 / 14.1,
-//         13523x6144 at 31 25.9 / 31.0.
-// Over 1774 drawn batches of 2 .. 32 rows of 256 .. 14336 rows and 4 .. 56 blocks: 0.87 of the time before in the mean (the
-// better of both everywhere would be 0.2 % less), 1.12 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
-// From activations quantized beforehand (frk_hip_gemm_q8k_dev, frk_hip_gemm_acts_dev) 0.84 and 0.77, gemm_pair 0.78.
+//   Q4_K  two rows of short blocks (4 .. 19 blocks 0.92 of the time; past 33 blocks 1.01 and more).  Up to 8 not the span kernel's rows of 4,
+//         12 and 16 .. 32 blocks but tall ones (24 .. 32 blocks past 4096 rows 0.89; 14336x4096 at 8 12.0 / 12.6).  4096x11008 at 8 14.8 / 11.5; at
+//         3 and 4 long rows past one round of the chip 0.95 .. 1.1.  9 .. 16 rows 14336x4096 19.5 / 12.7, 4096x14336 18.0 / 13.5.  From 17 on rows of up to 19
+//         blocks (4096x4096 at 32 12.3 / 8.1) and, in one round of the chip, of up to 39; but 14336x4096 16.3 / 18.
+//   Q5_K  4096x11008 at 8 and 16 16.0 / 12.3 and 19.1 / 12.4, 4096x4096 at 32 13.7 / 8.6, in one round of the chip at 32 whatever
+//         the length (4096x14336 22.8 / 20.1), but 12000x12032 38.4 / 42.
+//   Q6_K  odd nb always (4096x11008 at 8, 13 and 32 17.7 / 12.7, 19.8 / 12.9, 21.1 / 15.2); even up to 8 rows not the streamed thin
+//         kernel's longer or taller ones (4096x14336 14.3 / 15.2); 4096x14336 at 16 and 32 20.7 / 15.1, 23.4 / 18.1; but 573x14336 at 32
+//         1.16 of the time, 13523x6144 at 31 25.9 / 30.
+// Over 2409 drawn batches of 2 .. 32 rows of 256 .. 14336 rows and 4 .. 56 blocks: 0.82 of the time before in the mean (the
+// better of both everywhere would be 0.2 % less), 1.1 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
+// From activations quantized beforehand (frk_hip_gemm_q8k_dev, which has tiles to make, and frk_hip_gemm_acts_dev) 0.84 and 0.75, gemm_pair
+// 0.73.
 static bool k_rows_take(const frk_weights *w, size_t batch) {
     const size_t rows = w->rows, nb = w->cols / QK_K;
     if (batch < 2 || batch > 32 || nb > 128) return false;
     const bool one_round = rows > 2048 && rows <= 4096, few = rows < 1024;
     if (w->kind == FRK_KIND_Q4_K) {
-        const bool span = nb % 4 == 0 && nb <= 32;
-        if (batch == 2) return false;
-        if (batch <= 8) return !(span && nb != 8) && (rows <= 4096 || (batch > 4 && !(rows > 6144 && rows <= 8192)));
-        if (batch <= 16) return !(few && nb >= 44) && !(span && rows < 2048 && (nb == 4 || nb == 16 || nb == 20));
-        return rows <= 8192 && (nb < 20 || (nb <= 32 && one_round));
+        if (batch == 2) return nb < 20 && rows <= 8192;
+        if (batch <= 8 && nb % 4 == 0 && nb <= 32 && nb != 8) return nb >= 20 && rows > 4096;  // (the span kernel's)
+        if (batch <= 4) return rows <= 6144 || (nb < 33 && rows <= 12288);
+        if (batch <= 16) return batch <= 8 || !(few && nb >= 48);
+        return nb < 20 ? rows <= 8192 : nb < 24 ? rows <= 6144 : nb < 40 && one_round;
     }
     if (w->kind == FRK_KIND_Q5_K) {
-        if (batch <= 4) return rows <= 10240 || nb < 20;
-        if (batch <= 16) return batch <= 8 || !(few && nb >= 44);
-        return nb < 20 || one_round || (nb < 28 && rows > 6144 && rows <= 8192);
+        if (batch <= 4) return rows <= 12288 || nb < 20;
+        if (batch <= 16) return batch <= 8 || !(few && nb >= 48);
+        return nb < 24 || one_round || (nb <= 32 && rows > 2048 && rows <= 12288);
     }
-    if (w->kind != FRK_KIND_Q6_K || batch == 2) return false;
-    if (batch <= 8) return nb % 2 || nb < 16 || (nb <= 32 && rows <= 4096);
-    if (batch <= 16) return nb % 2 || nb < 40 || rows >= 2048;
-    return (nb % 2 || nb < 33 || rows >= 2048) && (rows <= 12288 || nb < 24);
+    if (w->kind != FRK_KIND_Q6_K) return false;
+    if (batch == 2) return nb < 20 && rows <= 8192;
+    if (nb % 2) return true;
+    if (batch <= 8) return nb < 16 || (nb < 20 ? rows <= 10240 : nb < 48 && rows <= 4096);  // (else the streamed thin kernel's)
+    if (batch <= 16) return !(few && nb >= 48);
+    return !(few && nb >= 33) && !(rows > 12288 && nb >= 24);
 }
-// Q6_K batches of up to 8 rows it reads as plain Q8_K rows, whose quantization is the shorter launch (2.7 us, as tiles 3.6).  A
-// load then touches a line a row: over 290 drawn ones 0.96 of the time from tiles, but Q4_K and Q5_K, whose loads are twice as
-// many, 1.08 and 1.11 of it.
-static bool k_rows_plain(const frk_weights *w, size_t batch) { return w->kind == FRK_KIND_Q6_K && batch <= 8; }
 // A K-quant batch that is multiplied from its tiles: gemm_k_rows_kernel's, or the pipelined GEMM's.
-static bool takes_tiles(const frk_weights *w, size_t batch) {
-    return k_rows_take(w, batch) ? !k_rows_plain(w, batch) : k_quant_takes_the_matrix_cores(w, batch);
-}
+static bool takes_tiles(const frk_weights *w, size_t batch) { return k_rows_take(w, batch) || k_quant_takes_the_matrix_cores(w, batch); }
 static size_t tiled_parts_bytes(const frk_weights *w, size_t batch) {
     return k_rows_take(w, batch) ? 0 : pipe_gemm_parts_bytes(w->kind, batch, w->cols, w->rows);
 }
 static int gemm_tiled(const frk_weights *w, const Q8KTiled &acts, size_t batch, float *y, void *parts, hipStream_t s) {
     return k_rows_take(w, batch) ? launch_gemm_k_rows(w, (int)batch, acts, nullptr, y, s) : launch_pipe_gemm_acts(w, acts, batch, y, parts, s);
+}
+
+// (the pipelined GEMM wants the rows past a batch cleared)
+static int quantize_tiles(const float *x, size_t batch, size_t cols, bool rows_only, const Q8KTiled &acts, hipStream_t s) {
+    return rows_only ? launch_quantize_q8_k_one_tile(x, batch, cols, acts, s) : launch_quantize_q8_k_tiled(x, batch, cols, acts, s);
 }
 
 static size_t acts_plain_bytes(size_t batch, size_t cols) {
@@ -755,11 +756,10 @@ static bool thin_kernels_hold(const frk_weights *w, size_t batch) {
     return k_quant && batch >= 2 && !matrix_cores_only(w, batch) && thin_gemm_max_batch(w) >= 2;
 }
 
-// a thin batch over activations already in Q8_K: gemm_k_rows_kernel's, `thin` rows a launch (thin_gemm_max_batch), or one launch over a
+// a thin batch over activations already in Q8_K: `thin` rows a launch (thin_gemm_max_batch), or one launch over a
 // grid of such groups where the kernel has that form
 static int thin_gemm_acts(const frk_weights *w, const Q8KActs &a, size_t batch, int thin, float *y, hipStream_t s) {
     const size_t nb = w->cols / QK_K;
-    if (k_rows_take(w, batch) && k_rows_plain(w, batch)) return launch_gemm_k_rows(w, (int)batch, Q8KTiled{}, &a, y, s);
     if (batch > (size_t)thin && batch <= (size_t)thin_gemm_wide_rows(w)) return launch_thin_gemm_wide(w, (int)batch, a, y, s);
     for (size_t b0 = 0; b0 < batch; b0 += (size_t)thin) {
         const int n = (int)std::min<size_t>((size_t)thin, batch - b0);
@@ -852,7 +852,7 @@ static int gemm_impl(const frk_weights *w, const float *x, size_t batch, float *
                              held_for_capture(w, batch));
         if (rc) return rc;
         const Q8KTiled acts = q8k_tiled_carve(ws, batch, w->cols);
-        rc = launch_quantize_q8_k_tiled(x, batch, w->cols, acts, s);
+        rc = quantize_tiles(x, batch, w->cols, k_rows_take(w, batch), acts, s);
         if (rc) return rc;
         return gemm_tiled(w, acts, batch, y, parts, s);
     }
@@ -922,8 +922,8 @@ int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
     Q8KActs a{q, d, bsums};
     hipStream_t s = (hipStream_t)stream;
     // (for a small matrix, or a few rows, a launch to make tiles of them costs more than what the rows' lines do)
-    const bool small = w->rows * w->cols < (size_t)16 << 20 && batch <= (w->kind == FRK_KIND_Q6_K ? 32 : 16);
-    if (k_rows_take(w, batch) && (batch <= 4 || k_rows_plain(w, batch) || small))
+    const bool q6 = w->kind == FRK_KIND_Q6_K, small = w->rows * w->cols < (size_t)16 << 20 && batch <= (q6 ? 32 : 16);
+    if (k_rows_take(w, batch) && (batch <= (q6 ? 8 : 4) || small))
         return launch_gemm_k_rows(w, (int)batch, Q8KTiled{}, &a, y, s);
     if (takes_tiles(w, batch)) {
         void *ws = nullptr, *parts = nullptr;
@@ -958,7 +958,7 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
         int rc = scratch.get(acts_bytes, part0 + part1, s, &ws, &parts, only ? SIZE_MAX : std::max(alone(w0, part0), alone(w1, part1)));
         if (rc) return rc;
         const Q8KTiled acts = q8k_tiled_carve(ws, batch, w0->cols);
-        rc = launch_quantize_q8_k_tiled(x, batch, w0->cols, acts, s);
+        rc = quantize_tiles(x, batch, w0->cols, k_rows_take(w0, batch) && k_rows_take(w1, batch), acts, s);
         if (rc) return rc;
         rc = gemm_tiled(w0, acts, batch, y0, parts, s);
         if (rc) return rc;
@@ -1037,7 +1037,9 @@ int frk_hip_quantize_batch_acts_dev(frk_batch_acts *a, const float *x, size_t ba
         plain.bsums = (int16_t *)((char *)a->base + round_up(n, 256) + round_up(n / QK_K * 4, 256));
         a->plain = Q8KActs{plain.q, plain.d, plain.bsums};
     }
-    const int rc = tiled ? launch_quantize_q8_k_tiled(x, batch, a->cols, q8k_tiled_carve((char *)a->base + a->tiled_off, batch, a->cols), s, plain)
+    const Q8KTiled tiles = q8k_tiled_carve((char *)a->base + a->tiled_off, batch, a->cols);
+    const int rc = tiled ? (batch < tiled_from(a->cols) ? launch_quantize_q8_k_one_tile(x, batch, a->cols, tiles, s, plain)
+                                                        : launch_quantize_q8_k_tiled(x, batch, a->cols, tiles, s, plain))
                          : launch_quantize_q8_k(x, batch * a->cols, plain.q, plain.d, plain.bsums, s);
     if (rc) return rc;
     a->batch = batch;
