@@ -158,6 +158,9 @@ int launch_dequant_rows(const frk_weights *w, const int32_t *ids, size_t n_out, 
 int launch_repack(int kind, const uint8_t *src, uint8_t *dst, size_t rows, size_t cols, const Layout &l,
                   hipStream_t s);
 int launch_copy(const void *src, void *dst, size_t bytes, hipStream_t s);
+// `bytes` of device memory into page-locked host memory, chunk by chunk: flags[c] becomes `epoch` when chunk c is there
+constexpr size_t STAGE_CHUNK = 8192;
+int launch_stage_out(const void *src, void *host, uint32_t *flags, uint32_t epoch, size_t bytes, hipStream_t s);
 int launch_read(const void *src, size_t bytes, void *sink, hipStream_t s);
 // calibration of the matrix-core kernels' issue budget (frk_probe.hip): 16 floats, four per count of vector instructions
 int launch_issue_probe(float *out, hipStream_t s);

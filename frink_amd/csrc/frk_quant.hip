@@ -219,6 +219,17 @@ __global__ __launch_bounds__(256) void copy_kernel(const uint4 *__restrict__ src
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) dst[i] = src[i];
 }
 
+// The host-buffer entry points' results into page-locked memory: a workgroup a chunk of STAGE_CHUNK bytes, whose flag it raises behind its
+// last store, so that the host takes the first chunks while the others travel.
+__global__ __launch_bounds__(256) void stage_out_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ host, uint32_t *flags, uint32_t epoch, size_t n) {
+    constexpr size_t PIECES = STAGE_CHUNK / 16;
+    const size_t first = (size_t)blockIdx.x * PIECES, end = first + PIECES < n ? first + PIECES : n;
+    for (size_t i = first + threadIdx.x; i < end; i += 256) host[i] = src[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flags + blockIdx.x, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // (Two 16-byte loads a thread and round, up to 8192 workgroups: the fastest of the shapes tried for
 // 8 .. 280 MB -- four loads a thread over 2048 workgroups took 5 % longer at 33 MB.)
 __global__ __launch_bounds__(256) void read_kernel(const uint4 *__restrict__ src, size_t n, uint32_t *__restrict__ sink) {
@@ -337,6 +348,13 @@ int launch_copy(const void *src, void *dst, size_t bytes, hipStream_t s) {
     const unsigned g = (unsigned)std::min<size_t>(blocks_for(n, 256), 256 * 16);
     hipLaunchKernelGGL(copy_kernel, dim3(g), dim3(256), 0, s, (const uint4 *)src, (uint4 *)dst, n);
     FRK_LAUNCH_CHECK("copy");
+    return FRK_OK;
+}
+
+int launch_stage_out(const void *src, void *host, uint32_t *flags, uint32_t epoch, size_t bytes, hipStream_t s) {
+    hipLaunchKernelGGL(stage_out_kernel, dim3((unsigned)((bytes + STAGE_CHUNK - 1) / STAGE_CHUNK)), dim3(256), 0, s, (const uint4 *)src,
+                       (uint4 *)host, flags, epoch, (bytes + 15) / 16);
+    FRK_LAUNCH_CHECK("stage_out");
     return FRK_OK;
 }
 

@@ -1,6 +1,7 @@
 // Host runtime of libfrink_hip: error strings, device probe, the env switch, the resident
 // weight cache, the per-device workspace and the extern "C" entry points.
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -35,6 +36,8 @@ struct DeviceState {
     // host staging for the host-buffer entry points
     void *x_dev = nullptr, *y_dev = nullptr;
     size_t x_bytes = 0, y_bytes = 0;
+    char *pinned = nullptr;  // page-locked: STAGE_MAX bytes of inputs, as many of results, a flag for each of their chunks
+    uint32_t epoch = 0;
     std::map<std::pair<const void *, size_t>, frk_weights *> cache;
 };
 static DeviceState g_dev;
@@ -1337,6 +1340,87 @@ static int stage_buffers(size_t x_bytes, size_t y_bytes) {
 // (crates/frink-core/src/weight_matrix/gpu_backend.rs:722-725).
 static std::mutex g_launch_mu;
 
+// Inputs and results of up to STAGE_MAX bytes go through page-locked memory of the library's own: the input is copied there and
+// read from the device, the results are written there by a kernel whose chunks the host takes as their flags are raised.
+// hipMemcpyAsync of the caller's pageable memory, once each way, and the stream's wait took 28 us of a 50 us call (32000 x
+// 4096 in Q6_K; the matrix 22 of them): us before / now, 32000 x 4096 50.4 / 39.5, 1000 x 2048 29 / 18, 4096 x 4096 by 8 and 32 rows 48 / 31 and 82 / 70.
+// Past 1 MB each way the runtime's own pieces are as fast (64 rows 131 / 130, 128 223 / 224).
+constexpr size_t STAGE_MAX = 1 << 20;
+static char *pinned_locked() {  // g_launch_mu is held; null where there is none
+    if (!g_dev.pinned) {
+        const size_t flags = STAGE_MAX / STAGE_CHUNK * sizeof(uint32_t);
+        if (hipHostMalloc((void **)&g_dev.pinned, 2 * STAGE_MAX + flags, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess)
+            memset(g_dev.pinned + 2 * STAGE_MAX, 0, flags);
+        else
+            g_dev.pinned = nullptr, (void)hipGetLastError();
+    }
+    return g_dev.pinned;
+}
+static int stage_in(const void *src, size_t bytes) {
+    char *pinned = bytes <= STAGE_MAX ? pinned_locked() : nullptr;
+    if (pinned) {
+        memcpy(pinned, src, bytes);
+        return launch_copy(pinned, g_dev.x_dev, round_up(bytes, 16), g_dev.stream);
+    }
+    hipError_t e = hipMemcpyAsync(g_dev.x_dev, src, bytes, hipMemcpyHostToDevice, g_dev.stream);
+    return e == hipSuccess ? FRK_OK : set_error(FRK_ERR_HIP, "hipMemcpyAsync(input): %s", hipGetErrorString(e));
+}
+struct HostOut {
+    void *dst;
+    size_t bytes;
+};
+// The results, back to back in y_dev, to the caller's buffers; waits for them, and for the stream where the call has failed (rc).
+static int stage_out(int rc, const HostOut *outs, size_t n) {
+    hipStream_t s = g_dev.stream;
+    size_t total = 0;
+    for (size_t i = 0; i < n; i++) total += outs[i].bytes;
+    char *pinned = !rc && total <= STAGE_MAX ? pinned_locked() : nullptr;
+    if (!pinned) {
+        size_t at = 0;
+        for (size_t i = 0; i < n && !rc; at += outs[i++].bytes) {
+            hipError_t e = hipMemcpyAsync(outs[i].dst, (const char *)g_dev.y_dev + at, outs[i].bytes, hipMemcpyDeviceToHost, s);
+            if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(results): %s", hipGetErrorString(e));
+        }
+        hipError_t e = hipStreamSynchronize(s);
+        if (!rc && e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
+        return rc;
+    }
+    const char *y = pinned + STAGE_MAX;
+    uint32_t *flags = (uint32_t *)(pinned + 2 * STAGE_MAX);
+    const uint32_t epoch = ++g_dev.epoch;
+    rc = launch_stage_out(g_dev.y_dev, pinned + STAGE_MAX, flags, epoch, total, s);
+    if (rc) {
+        (void)hipStreamSynchronize(s);
+        return rc;
+    }
+    // a chunk's flag is watched for 2 ms at most, then the stream waited for: a launch that fails raises no flag
+    size_t ready = 0;  // bytes that are there
+    bool waited = false;
+    auto wait_for = [&](size_t end) {
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+        while (ready < end) {
+            if (waited || __atomic_load_n(flags + ready / STAGE_CHUNK, __ATOMIC_ACQUIRE) == epoch) {
+                ready += STAGE_CHUNK;
+            } else if (std::chrono::steady_clock::now() > until) {
+                hipError_t e = hipStreamSynchronize(s);
+                if (e != hipSuccess) return set_error(FRK_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
+                waited = true;
+            }
+        }
+        return (int)FRK_OK;
+    };
+    size_t at = 0;
+    for (size_t i = 0; i < n; i++)
+        for (size_t done = 0; done < outs[i].bytes;) {
+            const size_t part = std::min(outs[i].bytes - done, STAGE_CHUNK - at % STAGE_CHUNK);
+            rc = wait_for(at + part);
+            if (rc) return rc;
+            memcpy((char *)outs[i].dst + done, y + at, part);
+            done += part, at += part;
+        }
+    return FRK_OK;
+}
+
 static int host_launch(int kind, const uint8_t *weights, size_t weights_len, const float *x, size_t rows,
                        size_t cols, size_t batch, float *out) {
     frk_weights *w = nullptr;
@@ -1345,20 +1429,12 @@ static int host_launch(int kind, const uint8_t *weights, size_t weights_len, con
     std::lock_guard<std::mutex> lk(g_launch_mu);
     size_t xb = batch * cols * sizeof(float), yb = batch * rows * sizeof(float);
     rc = stage_buffers(xb, yb);
-    hipStream_t s = g_dev.stream;
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(g_dev.x_dev, x, xb, hipMemcpyHostToDevice, s);
-        if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(x): %s", hipGetErrorString(e));
-    }
+    if (!rc) rc = stage_in(x, xb);
     if (!rc)
-        rc = batch == 1 ? frk_hip_gemv_dev(w, (const float *)g_dev.x_dev, (float *)g_dev.y_dev, FRK_ACT_F32, s)
-                        : frk_hip_gemm_dev(w, (const float *)g_dev.x_dev, batch, (float *)g_dev.y_dev, s);
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(out, g_dev.y_dev, yb, hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(y): %s", hipGetErrorString(e));
-    }
-    hipError_t e = hipStreamSynchronize(s);
-    if (!rc && e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
+        rc = batch == 1 ? frk_hip_gemv_dev(w, (const float *)g_dev.x_dev, (float *)g_dev.y_dev, FRK_ACT_F32, g_dev.stream)
+                        : frk_hip_gemm_dev(w, (const float *)g_dev.x_dev, batch, (float *)g_dev.y_dev, g_dev.stream);
+    const HostOut y = {out, yb};
+    rc = stage_out(rc, &y, 1);
     char keep[sizeof g_err];
     memcpy(keep, g_err, sizeof keep);
     frk_hip_weights_release(w);
@@ -1376,19 +1452,10 @@ int frk_hip_get_rows(const frk_weights *w, const int32_t *ids, size_t n_ids, flo
     std::lock_guard<std::mutex> lk(g_launch_mu);
     const size_t ib = n_ids * sizeof(int32_t), ob = n_ids * w->cols * sizeof(float);
     int rc = stage_buffers(ib, ob);
-    hipStream_t s = g_dev.stream;
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(g_dev.x_dev, ids, ib, hipMemcpyHostToDevice, s);
-        if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(ids): %s", hipGetErrorString(e));
-    }
-    if (!rc) rc = launch_dequant_rows(w, (const int32_t *)g_dev.x_dev, n_ids, (float *)g_dev.y_dev, s);
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(out, g_dev.y_dev, ob, hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(rows): %s", hipGetErrorString(e));
-    }
-    hipError_t e = hipStreamSynchronize(s);
-    if (!rc && e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
-    return rc;
+    if (!rc) rc = stage_in(ids, ib);
+    if (!rc) rc = launch_dequant_rows(w, (const int32_t *)g_dev.x_dev, n_ids, (float *)g_dev.y_dev, g_dev.stream);
+    const HostOut rows = {out, ob};
+    return stage_out(rc, &rows, 1);
 }
 
 int frk_hip_launch_matvec(int kind, const uint8_t *weights, size_t weights_len, const float *x, size_t x_len,
@@ -1468,24 +1535,17 @@ int frk_hip_launch_matvec_multi(const float *x, size_t x_len, const frk_matvec_l
     if (!rc) {
         std::lock_guard<std::mutex> lk(g_launch_mu);
         rc = stage_buffers(x_len * sizeof(float), total_rows * sizeof(float));
-        hipStream_t s = g_dev.stream;
-        if (!rc) {
-            hipError_t e = hipMemcpyAsync(g_dev.x_dev, x, x_len * sizeof(float), hipMemcpyHostToDevice, s);
-            if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(x): %s", hipGetErrorString(e));
-        }
+        if (!rc) rc = stage_in(x, x_len * sizeof(float));
         std::vector<float *> ys(n);
+        std::vector<HostOut> results(n);
         size_t off = 0;
         for (size_t i = 0; i < n; i++) {
             ys[i] = (float *)g_dev.y_dev + off;
+            results[i] = {outs[i], launches[i].rows * sizeof(float)};
             off += launches[i].rows;
         }
-        if (!rc) rc = frk_hip_gemv_multi_dev(ws.data(), n, (const float *)g_dev.x_dev, ys.data(), s);
-        for (size_t i = 0; i < n && !rc; i++) {
-            hipError_t e = hipMemcpyAsync(outs[i], ys[i], launches[i].rows * sizeof(float), hipMemcpyDeviceToHost, s);
-            if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(y): %s", hipGetErrorString(e));
-        }
-        hipError_t e = hipStreamSynchronize(s);
-        if (!rc && e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
+        if (!rc) rc = frk_hip_gemv_multi_dev(ws.data(), n, (const float *)g_dev.x_dev, ys.data(), g_dev.stream);
+        rc = stage_out(rc, results.data(), n);
     }
     char keep[sizeof g_err];
     memcpy(keep, g_err, sizeof keep);
@@ -1513,18 +1573,10 @@ int frk_hip_launch_dense_ffn_swiglu(const frk_matvec_launch *gate, const frk_mat
     if (!rc) {
         std::lock_guard<std::mutex> lk(g_launch_mu);
         rc = stage_buffers(x_len * sizeof(float), down->rows * sizeof(float));
-        hipStream_t s = g_dev.stream;
-        if (!rc) {
-            hipError_t e = hipMemcpyAsync(g_dev.x_dev, x, x_len * sizeof(float), hipMemcpyHostToDevice, s);
-            if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(x): %s", hipGetErrorString(e));
-        }
-        if (!rc) rc = frk_hip_ffn_swiglu_dev(ws[0], ws[1], ws[2], (const float *)g_dev.x_dev, (float *)g_dev.y_dev, s);
-        if (!rc) {
-            hipError_t e = hipMemcpyAsync(out, g_dev.y_dev, down->rows * sizeof(float), hipMemcpyDeviceToHost, s);
-            if (e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipMemcpyAsync(y): %s", hipGetErrorString(e));
-        }
-        hipError_t e = hipStreamSynchronize(s);
-        if (!rc && e != hipSuccess) rc = set_error(FRK_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
+        if (!rc) rc = stage_in(x, x_len * sizeof(float));
+        if (!rc) rc = frk_hip_ffn_swiglu_dev(ws[0], ws[1], ws[2], (const float *)g_dev.x_dev, (float *)g_dev.y_dev, g_dev.stream);
+        const HostOut y = {out, down->rows * sizeof(float)};
+        rc = stage_out(rc, &y, 1);
     }
     char keep[sizeof g_err];
     memcpy(keep, g_err, sizeof keep);
