@@ -49,6 +49,6 @@ def test_compiled_kernels_keep_the_waits(tmp_path):
     asm = _assembly(tmp_path, "frk_gemm_rows.hip")
     assert isa_mfma_lint.violations(asm) == []
     names = isa_wait_lint.kernels(asm)
-    assert len(names) == 10, names
+    assert sum("gemm_k_rows" in k for k in names) == 10 and len(names) == 11, names  # (and the batch's quantizer)
     for k in names:
         assert isa_wait_lint.violations(asm, k) == [], k
