@@ -68,7 +68,7 @@ struct StreamArgs {
     Q8KTiled a;
     const int4 *tiles;  // {expert, first row of the grouped order, rows in use, first row of y}
     const int *n_tiles;
-    int row_tiles;  // ceil(rows / 256)
+    int row_tiles;  // ceil(rows / 128)
     // the gathering form: the activations are the source rows' Q8_K, quantized once each, and row r of the
     // grouped order is source row gather[r] (negative: a row not in use)
     Q8KRows src;
@@ -188,48 +188,53 @@ __global__ __launch_bounds__(512) void gemm_q5_k_pipe_kernel(GemmArgs g) {
 }
 
 // The grouped (per-expert) GEMM: with a few dozen activation rows per expert the work is a stream
-// over the experts' weights.  Persistent workgroups (one per CU, 8 wavefronts, 256 weight rows) walk
+// over the experts' weights.  Persistent workgroups (two per CU, 4 wavefronts, 128 weight rows) walk
 // a list of work items (tile, matrix, row group); one step = one 256-wide block of one item.  A
-// step's data travels into LDS three steps ahead, across item boundaries: the weights (a wavefront
-// fetches and reads only its own 32 rows, so that ring needs no barrier: two stages, each refilled as
-// soon as its block has left it for the registers) and the tile's activation record (shared, four
+// step's data travels into LDS ahead of it, across item boundaries: the weights two or three steps (a wavefront
+// fetches and reads only its own 32 rows, so that ring needs no barrier: two stages, Q6_K one, each refilled as
+// soon as its block has left it for the registers) and the tile's activation record one step (shared, two
 // stages, one barrier per step).  A tile is up to 64 activation rows, two 32-row halves that share
 // the unpacked weights; the second half is neither fetched nor multiplied when not in use.
+// (One workgroup of 8 wavefronts and 256 rows a CU, activations three steps ahead, had every wavefront of the CU wait for
+// the slowest at every step, and items half as many: where they did not fill the chip, 23.1 -> 17.6 us for gate and up of 16
+// experts of 1792 / 512 over 540 pairs, 29.7 -> 24.2 over 1494 of 2304 / 512; Q6_K down experts of 128 x 2048 x 768 over
+// 4096 pairs 63.9 -> 59, the layer's gate and up as before.  36 drawn layers of 32 to 1024 tokens 0.92 of the time in the
+// mean, 0.84 at best, 1.014 at most.)
 // The unpacked weights are double-buffered in registers: step s+1 is unpacked from inside the chain
-// of MFMAs of step s.  The two wavefronts of a SIMD (w and w+4) issue their loads at different
-// times, one before its MFMAs and one after: a wavefront is stalled while its loads wait for the
-// CU's address unit, and this way the other one has the matrix core meanwhile.
+// of MFMAs of step s.  Half of a workgroup's wavefronts ask for their weights before the MFMAs and half
+// after: a wavefront is stalled while its loads wait for the CU's address unit, and this way others have the
+// matrix cores meanwhile (all before: 1 % on the layer's time; all after: 0.5).
 // Items of a tile sit on one XCD (block id mod 8), whose L2 then serves the tile's activations.
 // GATHER: a tile's activation rows are fetched from where their source rows were quantized (plain rows,
 // each quantized once however many tiles it is part of) instead of from a record of the grouped order: a
 // lane's piece of a record is 16 bytes of one row in either form, so only the lane offsets differ -- the
 // source row times the row length, looked up per item from a table in LDS.
-// KIND: Q4_K or Q6_K.  A Q6_K block is half as large again (two stages: 106 KB), which leaves room for three stages of
-// activations: they travel two steps ahead, the weights three.  (Q6_K down experts of 128 x 2048 x 768, 4096 pairs: 63 us,
-// 165 MB of weights; the dense kernel by tile, one workgroup per tile and 256 rows with its three blocks, took 99.)
+// KIND: Q4_K or Q6_K.  A Q6_K block is half as large again: one stage of weights, two steps ahead.  (Q6_K down experts of
+// 128 x 2048 x 768, 4096 pairs, 165 MB of weights: the dense kernel by tile, one workgroup per tile and 256 rows with
+// its three blocks, took 99 us.)
 template <int KIND, bool GATHER>
 struct StreamLds {
     using Side = WeightSide<KIND>;
     static constexpr bool MINS = Side::MINS;
-    static constexpr int RG = 8;
+    static constexpr int RG = 4;
     static constexpr int W_WAVE = Side::SLOT;    // a wavefront's 32 rows of one block
     static constexpr int W_STAGE = RG * W_WAVE;
-    static constexpr int W_STAGES = 2;
+    static constexpr int W_STAGES = KIND == FRK_KIND_Q6_K ? 1 : 2;
     static constexpr int A_BS = 8192, A_DA = MINS ? 9216 : 8192;  // record of 32 rows: quants | sums (with mins) | scales
     static constexpr int A_HALF = A_DA + 256;  // (64 lanes fetch the 32 scales twice)
     static constexpr int A_STAGE = 2 * A_HALF;   // a tile is two records
-    static constexpr int A_STAGES = KIND == FRK_KIND_Q6_K ? 3 : 4;
+    static constexpr int A_STAGES = 2;
     static constexpr int OFF_A = W_STAGES * W_STAGE;
     // {expert, rows in use | matrix << 7 | row group << 8, first row of y, tile} of each of the workgroup's items, filled
     // once: looked up from LDS, an item change costs no global load (whose completion would count in vmcnt, in the
     // middle of the prefetch bookkeeping) and no division (a wavefront's end of step waits for it)
     static constexpr int OFF_ITEMS = OFF_A + A_STAGES * A_STAGE;
-    static constexpr int MAX_ITEMS = GATHER ? 64 : 128;
+    static constexpr int MAX_ITEMS = GATHER ? 28 : 128;
     // GATHER: the source rows of each item's tile, row r of the first half in the low 16 bits of word r and
     // row 32 + r in the high ones
     static constexpr int OFF_SRC = OFF_ITEMS + MAX_ITEMS * 16;
     static constexpr size_t BYTES = (size_t)OFF_SRC + (GATHER ? MAX_ITEMS * 128 : 0);
-    static_assert(BYTES <= 160 * 1024, "LDS of a CU");
+    static_assert(BYTES <= 80 * 1024, "two workgroups share the LDS of a CU");
 };
 
 template <int KIND, bool GATHER>
@@ -309,11 +314,10 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
     const uint8_t *f_x;
     const int8_t *f_q;
     const uint32_t lds_src = lds_address(lds + L::OFF_SRC);
-    constexpr bool ONE_CURSOR = L::A_STAGES == 4;  // (the activations of a step are fetched right before its weights)
     int w_last_row = -1;
-    int w_ord = 0, w_kb = 0, w_step = 0, a_ord = 0, a_kb = 0, a_stage = 0;
+    int w_ord = 0, w_kb = 0, w_step = 0, a_ord = 0, a_kb = 0, a_step = 0;
+    constexpr int SLICES = 8 / L::RG, SLICE_STEP = GATHER ? 32 * L::RG : 1024 * L::RG;  // quant slices of a wavefront, their distance
     bool f_two = false;  // the activations' cursor's tile has rows in its second half
-    int issued = 0;      // loads this wavefront made in the step
     auto weights_at = [&](const Item &it) {  // uniform
         const uint8_t *W = (it.mat ? g.W[1] : g.W[0]) + (size_t)it.expert * g.rows * g.row_stride;
         const int row_base = min(it.row_group * (32 * L::RG) + wave * 32, g.rows - 1), last_row = min(g.rows - 1 - row_base, 31);
@@ -348,23 +352,21 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
         }
     };
     auto fetch_acts = [&]() {  // of the cursor's step; moves the cursor on
-        const uint32_t st = lds_address(lds) + L::OFF_A + (uint32_t)(ONE_CURSOR ? w_step & 3 : a_stage) * L::A_STAGE;
-        dma16(st + wave * 1024, f_q, qa_off);
-        issued = 1;
+        const uint32_t st = lds_address(lds) + L::OFF_A + (uint32_t)(a_step & 1) * L::A_STAGE;
+#pragma unroll
+        for (int c = 0; c < SLICES; c++) dma16(st + (wave + c * L::RG) * 1024, f_q + c * SLICE_STEP, qa_off);
         if (f_two) {
-            dma16(st + L::A_HALF + wave * 1024, f_q, qb_off);
-            issued = 2;
+#pragma unroll
+            for (int c = 0; c < SLICES; c++) dma16(st + L::A_HALF + (wave + c * L::RG) * 1024, f_q + c * SLICE_STEP, qb_off);
         }
         if (x_small && (!x_second || f_two)) {
             const uint32_t half = st + (x_second ? L::A_HALF : 0);
             if (MINS && x_sums) dma16(half + L::A_BS, f_x, x_off);
             else dma4(half + L::A_DA, f_x, x_off);
-            issued++;
         }
         f_q += GATHER ? QK_K : 8192;
         f_x += GATHER ? (x_sums ? 32 : 4) : (x_sums ? 1024 : 128);
-        if (ONE_CURSOR) return;
-        a_stage = a_stage == L::A_STAGES - 1 ? 0 : a_stage + 1;
+        a_step++;
         if (++a_kb == nb) {
             a_kb = 0;
             if (++a_ord < my_items) acts_at(item(a_ord), a_ord);
@@ -372,21 +374,16 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
     };
     const uint32_t lds_w = lds_address(lds) + (uint32_t)wave * L::W_WAVE;
     auto fetch_weights = [&]() {  // of the cursor's step; moves the cursor on
-        wside.fetch(lds_w + (uint32_t)(w_step & 1) * L::W_STAGE, lane);
-        issued += Side::REQUESTS;
+        wside.fetch(lds_w + (uint32_t)(L::W_STAGES == 2 ? w_step & 1 : 0) * L::W_STAGE, lane);
         w_step++;
         if (++w_kb == nb) {
             w_kb = 0;
-            if (++w_ord < my_items) {
-                const Item it = item(w_ord);
-                weights_at(it);
-                if (ONE_CURSOR) acts_at(it, w_ord);
-            }
+            if (++w_ord < my_items) weights_at(item(w_ord));
         } else {
             wside.move_on(w_kb - 1);
         }
     };
-    // prologue: the weights of steps 0 and 1, the activations' stages but one or two
+    // prologue: the activations of step 0, as many steps' weights as there are stages
     {
         const Item it = item(0);
         weights_at(it);
@@ -394,10 +391,7 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
     }
     fetch_acts();
     fetch_weights();
-    if (total_steps > 1) {
-        if (L::A_STAGES > 3) fetch_acts();
-        fetch_weights();
-    }
+    if (total_steps > 1 && L::W_STAGES > 1) fetch_weights();
     wait_vm<0>();
     lds_barrier();
 
@@ -410,14 +404,14 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
     BPlanes B0, B1;
     v16f accF0 = v16f{0.0f}, accF1 = v16f{0.0f};  // the tile's two halves
     const bool fetch_late = wave >= L::RG / 2;
-    int c_ord = 0, c_kb = 0, c_stage = 0;
+    int c_ord = 0, c_kb = 0, c_step = 0;
     Item c_item = {0, 0, 0, 0, 0, 0};
     bool pending = false;  // `done` is an item whose results wait to be stored
     Item done = c_item;
     auto raw_of_step = [&](int s) {  // this lane's part of its row's block, read and arrived
         const int l = opaque_lane();
         typename Side::Raw R;
-        Side::read(R, lds_w + (uint32_t)(s & 1) * L::W_STAGE, l & 31, l >> 5);
+        Side::read(R, lds_w + (uint32_t)(L::W_STAGES == 2 ? s & 1 : 0) * L::W_STAGE, l & 31, l >> 5);
         return R;
     };
     auto multiply_half = [&](uint32_t st, v16f &accF, const BPlanes &B, auto between) {
@@ -437,8 +431,7 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
     };
     // (the next step's block R is unpacked into Bnext from inside the first half's chain of MFMAs)
     auto multiply_step = [&](const BPlanes &B, const typename Side::Raw &R, BPlanes &Bnext) {
-        const uint32_t st = lds0 + L::OFF_A + c_stage * L::A_STAGE;
-        c_stage = ONE_CURSOR ? (c_stage + 1) & 3 : c_stage == L::A_STAGES - 1 ? 0 : c_stage + 1;
+        const uint32_t st = lds0 + L::OFF_A + (uint32_t)(c_step++ & 1) * L::A_STAGE;
         if (c_kb == 0) c_item = item(c_ord++);
         const int lg_next = opaque_lane() >> 5;
         const typename Side::Scales sc = Side::scales(R, lg_next);
@@ -481,35 +474,30 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
         const typename Side::Scales sc = Side::scales(R, lg);
 #pragma unroll
         for (int i = 0; i < 9; i++) Side::unpack_piece(i, R, sc, lg, 0, B0);
-        if (total_steps > L::A_STAGES - 2) fetch_acts();
-        if (total_steps > 2) fetch_weights();
+        if (total_steps > L::W_STAGES) fetch_weights();
+        if (L::W_STAGES == 1) wait_vm<0>();  // (step 1's, which step 0 unpacks)
     }
     auto step = [&](int s, const BPlanes &Bcur, BPlanes &Bnext) {
         if (pending) {
             store_item();
             pending = false;
         }
-        // step s+1's raw weights leave LDS, which frees their stage for step s+3 (past the last step:
-        // whatever the stage holds, unpacked into a set nobody will use)
+        // step s+1's raw weights leave LDS, which frees their stage (past the last step: whatever the stage holds,
+        // unpacked into a set nobody will use)
         const typename Side::Raw R = raw_of_step(s + 1);
-        // A wavefront is stalled while its loads wait for the CU's one address unit (600 clocks for
-        // the first four wavefronts that ask, 1700 for the other four): so half of the wavefronts,
-        // one of every SIMD's two, fetch before they multiply and half after, and the unit serves
-        // the one half while the other half has the matrix cores.
-        const bool more = s + 3 < total_steps;
-        auto fetch = [&]() {
-            if (ONE_CURSOR ? more : s + L::A_STAGES - 1 < total_steps) fetch_acts();  // (into the stage last read in step s-1)
-            if (more) fetch_weights();
-        };
-        if (!fetch_late) fetch();
+        // A wavefront is stalled while its loads wait for the CU's one address unit: half of a workgroup's wavefronts
+        // fetch their weights before they multiply and half after, and the unit serves the one half while the other half
+        // has the matrix cores.  The activations of the step behind this one are wanted at its end and go out first (into
+        // the stage last read in step s-1).
+        const bool more = s + 1 + L::W_STAGES < total_steps;
+        if (s + 1 < total_steps) fetch_acts();
+        if (more && !fetch_late) fetch_weights();
         multiply_step(Bcur, R, Bnext);
-        if (fetch_late) fetch();
-        // the requests just made (the `issued` youngest loads; a finished item's stores are older) may stay in flight,
-        // everything older must have landed: the next step's activations and the weights of the one behind it
-        if (!more) wait_vm<0>();
-        else if (issued == Side::REQUESTS + 1) wait_vm<Side::REQUESTS + 1>();
-        else if (issued == Side::REQUESTS + 2) wait_vm<Side::REQUESTS + 2>();
-        else wait_vm<Side::REQUESTS + 3>();
+        if (more && fetch_late) fetch_weights();
+        // with two stages the weights just asked for (the youngest loads; a finished item's stores are older) may stay in
+        // flight, everything older must have landed: the next step's activations and the weights of the one behind it
+        if (more && L::W_STAGES > 1) wait_vm<Side::REQUESTS>();
+        else wait_vm<0>();
         lds_barrier();
     };
     for (int s = 0; s < total_steps; s += 2) {
@@ -520,10 +508,10 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
 }
 
 template <bool GATHER>
-__global__ __launch_bounds__(512) void gemm_q4_k_stream_kernel(StreamArgs g) {
+__global__ __launch_bounds__(256, 2) void gemm_q4_k_stream_kernel(StreamArgs g) {
     stream_gemm<FRK_KIND_Q4_K, GATHER>(g);
 }
-__global__ __launch_bounds__(512) void gemm_q6_k_stream_kernel(StreamArgs g) { stream_gemm<FRK_KIND_Q6_K, false>(g); }
+__global__ __launch_bounds__(256, 2) void gemm_q6_k_stream_kernel(StreamArgs g) { stream_gemm<FRK_KIND_Q6_K, false>(g); }
 
 // ------------------------------------------------------------------ launchers
 
@@ -715,7 +703,7 @@ static int launch_stream(void (*kernel)(StreamArgs), const StreamArgs &g, int ma
         if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::BYTES);
         if (e != hipSuccess) return set_error(FRK_ERR_HIP, "grouped GEMM setup: %s", hipGetErrorString(e));
-        grid = cus < 8 ? 8 : cus / 8 * 8;  // one workgroup per CU, a multiple of the 8 XCDs
+        grid = 2 * (cus < 8 ? 8 : cus / 8 * 8);  // two workgroups per CU, a multiple of the 8 XCDs
     }
     // more workgroups than CUs when a workgroup's share of the largest possible list would not fit
     // its item table
@@ -752,7 +740,7 @@ int launch_gemm_k_stream(const frk_weights *w0, const frk_weights *w1, size_t ro
     g.a = a;
     g.tiles = tiles;
     g.n_tiles = n_tiles;
-    g.row_tiles = (int)((rows_e + 255) / 256);
+    g.row_tiles = (int)((rows_e + 127) / 128);
     g.src = src ? *src : Q8KRows{nullptr, nullptr, nullptr};
     g.gather = gather;
     if (w0->kind == FRK_KIND_Q6_K) return launch_stream<FRK_KIND_Q6_K, false>(gemm_q6_k_stream_kernel, g, max_tiles, s);
