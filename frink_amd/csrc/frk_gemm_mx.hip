@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
     uint8_t *const lds = mx_lds;
     // The workgroups of a tile sit on one XCD (block id mod 8), whose L2 then serves the tile's digits.  One workgroup fits a
     // CU, so an XCD's jobs go in rounds of 32; where the last round is half empty, its jobs are cut in two: half the
-    // rows each, four wavefronts to the first tokens and four to the others of the same rows.
+    // rows each, four wavefronts to multiply them and the other four to help with the digits' requests.
     const int xcd = (int)blockIdx.x & 7, jobs = max(*g.n_tiles - xcd + 7, 0) / 8 * g.row_groups;
     int j = (int)blockIdx.x >> 3, part = -1;
     if (NW == 8) {
@@ -135,12 +135,6 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
     uint64_t *const expf_table = reinterpret_cast<uint64_t *>(lds + MX_STAGES * MX_STAGE + NW * MX_W_WAVE);
     if (GLU && threadIdx.x < 32) expf_table[threadIdx.x] = EXPF_TABLE[threadIdx.x];  // (read behind the first barrier)
     const int halves = (tile.z + 31) >> 5;  // of 32 rows, three at most
-    // this wavefront's: all of them; where a job's rows are cut in two, the first two (of two: one) or what is left
-    // (nothing left: the first again, not stored)
-    const int lower = halves > 2 ? 2 : 1;
-    const bool upper = part >= 0 && wave >= 4;
-    const int h_first = upper && halves > 1 ? lower : 0, h_count = part < 0 ? halves : upper ? max(halves - lower, 1) : lower;
-    const bool stores = !(upper && halves == 1);
 
     const uint32_t lds0 = lds_address(lds);
     // ---- weights: rows row0 + lane % 32 of the two groups.  Request c of a quad brings rows 16c .. 16c + 15 of the 64:
@@ -205,7 +199,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
 #pragma unroll
     for (int k = 0; k < 2; k++)
 #pragma unroll
-        for (int n = 0; n < 2; n++) piece_at[k][n] = (uint32_t)((32 * h_first + li) * MX_ROW + ((4 * n + 2 * lg + k) ^ ((li >> 1) & 7)) * 16);
+        for (int n = 0; n < 2; n++) piece_at[k][n] = (uint32_t)(li * MX_ROW + ((4 * n + 2 * lg + k) ^ ((li >> 1) & 7)) * 16);
 
     mx_v16f acc[3][2];  // [half][row group]
 #pragma unroll
@@ -233,7 +227,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
         return *reinterpret_cast<const mx_v4i *>(st + h * 32 * MX_ROW + (n >> 1) * 128 + piece_at[k][n & 1]);
     };
     auto act_scales = [&](const uint8_t *st, int h, int k) {
-        return *reinterpret_cast<const int *>(st + MX_STAGE_SCALES + (32 * (h_first + h) + li) * 16 + (2 * lg + k) * 4);
+        return *reinterpret_cast<const int *>(st + MX_STAGE_SCALES + (32 * h + li) * 16 + (2 * lg + k) * 4);
     };
     // A step's operands come in two parts, planes 0 and 1 (A: dwords 0..3 of each, then dwords 4 and 5 of both; with the
     // planes' scales) and planes 2 and 3 (B): one is read while the other is multiplied.
@@ -309,12 +303,20 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
         }
     };
     request_digits(-2);
+    if (part >= 0 && wave >= 4) {  // a helper: the same barriers
+        for (int i = -1; i < quads; i++) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            lds_barrier();
+            request_digits(i);
+        }
+        return;
+    }
     for (int c = 0; c < 4; c++) fetch_codes(0, c);
     fetch_weight_scales(0);
     request_codes(-1, 0);
     request_codes(-1, 2);
-    if (h_count > 2) all_quads(std::integral_constant<int, 3>());
-    else if (h_count > 1) all_quads(std::integral_constant<int, 2>());
+    if (halves > 2) all_quads(std::integral_constant<int, 3>());
+    else if (halves > 1) all_quads(std::integral_constant<int, 2>());
     else all_quads(std::integral_constant<int, 1>());
 #undef FRK_MX_READ_A
 #undef FRK_MX_READ_B
@@ -327,14 +329,14 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
     // (silu ahead of the stores and their conditions, so that several values' chains of operations run beside each other)
 #pragma unroll
     for (int h = 0; h < 3; h++) {
-        if (h >= h_count || !stores) break;
+        if (h >= halves) break;
         if (GLU) {
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[h][0][r] = silu_as_host(acc[h][0][r], expf_table) * acc[h][1][r];
         }
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const int tok = 32 * (h_first + h) + 8 * (r >> 2) + 4 * lg + (r & 3);
+            const int tok = 32 * h + 8 * (r >> 2) + 4 * lg + (r & 3);
             if (tok >= tile.z) continue;
             float *dst = g.y + (size_t)(tile.w + tok) * g.rows;
             if (row0 < g.rows) dst[row0] = acc[h][0][r];
@@ -347,8 +349,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_mx_grouped_kernel(MxGemmArgs 
     // the second.
     auto infinite_rows = [&](int first) {  // of 64 rows
         bool again = false;
-        const int half = (first + lane) >> 5;
-        if (stores && first + lane < tile.z && half >= h_first && half < h_first + h_count) {
+        if (first + lane < tile.z) {
             const int src = g.src_rows ? g.src_rows[tile.y + first + lane] : tile.y + first + lane;
             again = src >= 0 && g.acts.infinite[src] != 0;
         }
