@@ -362,6 +362,10 @@ int launch_gemv_units_int_jobs(const frk_weights *w, const frk_weights *w2, size
                                size_t n_jobs, int act_div, const int8_t *aq, const float *ad, float *y, float *y2, hipStream_t s);
 // the routed layer over experts of these kinds: every (token, slot) pair a job of the integer decode kernel
 size_t moe_units_workspace_bytes(size_t batch, int k, int hidden, int ffn);
+// a token or a few through MXFP4 experts in two launches (frk_mx_experts.hip); q, d: room for the pairs' quantized intermediate
+bool mx_experts_take(const frk_weights *gate, const frk_weights *up, const frk_weights *down, size_t batch, size_t k);
+int launch_mx_experts(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts, const float *x, size_t batch,
+                      const int32_t *ids, const float *weights, int k, int8_t *q, float *d, float *out, hipStream_t s);
 int launch_moe_ffn_units(const frk_weights *gate, const frk_weights *up, const frk_weights *down, int n_experts, const float *x,
                          size_t batch, const int32_t *ids, const float *weights, int k, float *out, void *ws, hipStream_t s);
 // Q5_0 / MXFP4 rows decoded into the Q8_0 planar form (signed bytes and f16 scales; `dst` rows dst_stride apart, the

@@ -5,6 +5,8 @@
 // with each token's experts added in the order the reference adds them (moe_combine_kernel).
 #include "frk_mx_quant.hpp"
 
+#include <cmath>
+
 namespace frk {
 
 // route_top_k_softmax (crates/frink-moe/src/lib.rs:567-589): one wavefront per token.  The
@@ -866,8 +868,8 @@ int launch_gemm_grouped(const frk_weights *w, size_t n_groups, const int32_t *gr
 // keeps its experts in MXFP4): every (token, slot) pair is a job of the integer decode kernel -- gate and up over the
 // token's quantized activation, silu(g) * u, that row quantized, down -- and the weighted sum in the reference's order
 // for the batch size.  Q8_0 activation blocks for Q5_0 and MXFP4 projections, Q8_K for IQ4_XS ones.  (A batch of
-// hundreds of tokens would read an expert's matrices once per pair here: from 32 tokens on, and MXFP4 experts from two
-// pairs an expert on, the layer takes the bucketed path below instead, where the kinds have a decoded form.)
+// hundreds of tokens would read an expert's matrices once per pair here: from 32 tokens on, and MXFP4 experts where
+// moe_units_takes_grouped_path says so, the layer takes the bucketed path below instead, where the kinds have a decoded form.)
 struct UnitsActs {
     int8_t *q;
     float *d;
@@ -905,9 +907,12 @@ int launch_moe_ffn_units(const frk_weights *gate, const frk_weights *up, const f
     const UnitsActs aa = units_acts_carve(p, pairs, ffn);
     p += units_acts_bytes(pairs, ffn);
     float *d_out = (float *)p;
+    // (its sum is in routing order, the order of batches below MOE_BUCKET_ORDER_FROM)
+    if (batch < MOE_BUCKET_ORDER_FROM && mx_experts_take(gate, up, down, batch, (size_t)k))
+        return launch_mx_experts(gate, up, down, n_experts, x, batch, ids, weights, k, aa.q, aa.d, out, s);
     int rc = quantize_for_units(gate->kind, x, batch * (size_t)hidden, xa, s);
     if (rc) return rc;
-    // five launches: the tokens quantized; gate and up of every pair; silu(g) * u quantized; down; the weighted sum
+    // (MXFP4 rows of up to 3072 columns are done.)  Five launches: the tokens quantized; gate and up of every pair; silu(g) * u quantized; down; the weighted sum
     rc = launch_gemv_units_int_jobs(gate, up, (size_t)ffn, n_experts, ids, pairs, k, xa.q, xa.d, g_out, u_out, s);
     if (rc) return rc;
     rc = down->kind == FRK_KIND_IQ4_XS ? launch_swiglu_quantize_q8_k(g_out, u_out, pairs * (size_t)ffn, aa.q, aa.d, aa.bsums, s)
@@ -953,12 +958,23 @@ bool moe_units_takes_grouped_path(const frk_weights *gate, const frk_weights *up
                                   int k) {
     if (!units_have_planar_form(gate) || !units_have_planar_form(up) || !units_have_planar_form(down)) return false;
     if (batch >= MOE_BUCKET_ORDER_FROM) return true;
-    // Below 32 tokens a job per pair reads an expert once for every pair, the grouped kernel once.  It pays from about two
-    // pairs an expert on, and from 32 pairs (per pair / grouped, us): 32 experts top-4 of 2880 / 2880 at 8, 12, 16 tokens
-    // 143 / 187, 207 / 196, 263 / 197; 16 top-4 of 1440 / 2880 at 6, 8 77 / 82, 97 / 83; 16 top-2 of 2048 / 1440 at 12, 16
-    // 56 / 58, 67 / 59; 8 top-2 of 1024 / 1024 at 12, 16, 24 39 / 42, 45 / 42, 59 / 43.
-    const size_t pairs = batch * (size_t)k, ffn = down->cols;
-    return pairs >= std::max<size_t>(2 * (size_t)n_experts, 32) && units_native(gate->kind, down->kind, batch, pairs, n_experts, gate->cols, ffn).down;
+    const size_t pairs = batch * (size_t)k, hidden = gate->cols, ffn = down->cols;
+    if (!units_native(gate->kind, down->kind, batch, pairs, n_experts, hidden, ffn).down) return false;
+    // Below 32 tokens a job per pair reads an expert once for every pair, the grouped kernels once.  The jobs' two launches
+    // take 7 us and a time per weight; the grouped ones a chain as long as the rows, or the bytes of the experts that
+    // random routing is expected to reach (per pair / grouped, us: 8 experts top-2 of 2880 / 2880 at 8, 16 tokens 49 / 62,
+    // 84 / 63; 16 top-4 of 1056 / 2176 at 8, 16 35 / 55, 58 / 56; 32 top-2 of 1024 / 1024 at 31 27 / 37; 32 top-4 of 2880 / 2880 at
+    // 8, 16 85 / 133, 158 / 151).  Over 240 layers of 8 to 32 experts the choice is 0.03 % behind the better one on
+    // average, 2.8 % at most.
+    if (mx_experts_take(gate, up, down, batch, (size_t)k)) {
+        const double weights = 3.0 * (double)hidden * (double)ffn, e = (double)n_experts;
+        const double reached = e * (1.0 - std::pow(1.0 - (double)k / e, (double)batch));
+        const double jobs_us = 7.0 + (double)pairs * weights / 10.5e6;
+        const double grouped_us = std::max(22.0 + 0.007 * (double)(hidden + ffn), 15.0 + reached * weights * (17.0 / 32.0) / 2.6e6);
+        return jobs_us > grouped_us;
+    }
+    // (rows too long for those two: a row a wavefront, from about two pairs an expert and 32 pairs on)
+    return pairs >= std::max<size_t>(2 * (size_t)n_experts, 32);
 }
 struct UnitsGroupedScratch {
     uint8_t *gate_w, *up_w, *down_w;  // decoded experts (not of projections in their own form)

@@ -283,8 +283,8 @@ int frk_hip_route_top_k_softmax_dev(const float *logits_dev, size_t batch, size_
  * crates/frink-moe/src/lib.rs:1246-1263).  gate/up/down hold the experts stacked row-wise
  * (expert e = rows [e*ffn, (e+1)*ffn) of gate and up, [e*hidden, (e+1)*hidden) of down); gate and up
  * are Q4_K, down is Q4_K or Q6_K; or all three of Q5_0 / IQ4_XS / MXFP4 (gate and up of one kind): below 32 tokens
- * every (token, slot) pair runs on the integer decode kernel of its kind (MXFP4: until there are two pairs an expert
- * and 32 pairs), from there on the pairs are bucketed by expert and the experts run on a grouped matrix-core kernel,
+ * every (token, slot) pair runs on the integer decode kernel of its kind (MXFP4: while that is estimated to be the
+ * faster one), from there on the pairs are bucketed by expert and the experts run on a grouped matrix-core kernel,
  * decoded to signed bytes in scratch memory or (MXFP4 rows of 384 columns and more) as they are stored; an MXFP4
  * stack with scale bytes outside 104..143 keeps the per-pair jobs.  Other combinations: FRK_ERR_UNSUPPORTED.
  * ids[batch][k] / weights[batch][k] are a RoutingDecision per token (lib.rs:112-115); an id outside
