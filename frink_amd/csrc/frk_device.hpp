@@ -299,4 +299,67 @@ __device__ __forceinline__ size_t q8k_tiled_index(int nb, int row, int kb, int k
     return rec * 8192 + (k >> 5) * 1024 + (((k >> 4) & 1) * 32 + (row & 31)) * 16 + (k & 15);
 }
 
+// The matrix of a GEMV's workgroup: the launch's one, or one of up to four of a kind and a row length that multiply the same
+// activation (q/k/v, gate and up: launch_matvec_multi, crates/frink-cuda/src/matvec_launch.rs:485-534), whose workgroups
+// follow each other.  A launch each cost what a launch costs: q/k/v of 4096 + 1024 + 1024 rows x 4096 in Q8_0 12.2 -> 7.4 us,
+// in Q6_K 10.3 -> 5.6, of 4864 + 608 + 608 x 4864 in Q6_K 17.8 -> 8.6.  (The one matrix in a type of its own: a hundred bytes
+// more of kernel arguments are 0.06 us.)
+struct GemvMatrix {
+    const uint8_t *W;
+    float *y;
+    int rows, block;  // the workgroup's number within the matrix
+};
+struct GemvOne {
+    const uint8_t *W;
+    float *y;
+    int rows;
+    __device__ __forceinline__ GemvMatrix pick() const { return {W, y, rows, (int)blockIdx.x}; }
+};
+struct GemvGroup {
+    const uint8_t *W[4];
+    float *y[4];
+    int rows[4], first[4];  // a matrix's first workgroup (no matrix: INT_MAX)
+    __device__ __forceinline__ GemvMatrix pick() const {
+        const int b = (int)blockIdx.x;
+#if defined(__HIP_DEVICE_COMPILE__)
+        // (a choice of values, global pointers: else the compiler chooses addresses, and keeps a copy of the arrays in
+        // scratch memory -- the Q6_K kernel with a row a wavefront took twice the time)
+        typedef const __attribute__((address_space(1))) uint8_t *weights_t;
+        typedef __attribute__((address_space(1))) float *out_t;
+        weights_t w = (weights_t)W[0];
+        out_t out = (out_t)y[0];
+        int n = rows[0], from = 0;
+#pragma unroll
+        for (int i = 1; i < 4; i++) {
+            weights_t wi = (weights_t)W[i];
+            out_t yi = (out_t)y[i];
+            int ni = rows[i], fi = first[i];
+            asm("" : "+s"(wi), "+s"(yi), "+s"(ni), "+s"(fi));
+            const bool here = b >= fi;
+            w = here ? wi : w, out = here ? yi : out, n = here ? ni : n, from = here ? fi : from;
+        }
+        return {(const uint8_t *)w, (float *)out, n, b - from};
+#else
+        return {W[0], y[0], rows[0], b};
+#endif
+    }
+};
+// workgroups of n matrices, rows_wg rows each
+inline size_t gemv_workgroups(const frk_weights *const *ws, size_t n, size_t rows_wg) {
+    size_t total = 0;
+    for (size_t i = 0; i < n; i++) total += (ws[i]->rows + rows_wg - 1) / rows_wg;
+    return total;
+}
+inline GemvGroup gemv_group(const frk_weights *const *ws, size_t n, float *const *ys, size_t rows_wg) {
+    GemvGroup g;
+    for (size_t i = 0; i < 4; i++) {
+        const size_t j = i < n ? i : 0;
+        g.W[i] = ws[j]->dev;
+        g.y[i] = ys[j];
+        g.rows[i] = (int)ws[j]->rows;
+        g.first[i] = i < n ? (int)gemv_workgroups(ws, i, rows_wg) : 0x7fffffff;
+    }
+    return g;
+}
+
 }  // namespace frk

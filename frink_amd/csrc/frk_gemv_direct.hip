@@ -23,16 +23,19 @@ namespace frk {
 // flight, and its 16 rows share that one copy (a row of this kind is shorter than the activation it
 // multiplies, so per-lane reads of the activation from L2 would double the traffic); otherwise the
 // quantized activation is read from global memory.
-template <int U, int XB, bool FUSED>
+template <int U, int XB, bool FUSED, class M>
 __global__ __launch_bounds__(FUSED ? 1024 : 256) void gemv_q6_k_direct_kernel(
-    const uint8_t *__restrict__ W, Layout lay, int rows, int nb, const float *__restrict__ x,
-    const int8_t *__restrict__ aq, const float *__restrict__ ad, const int16_t *__restrict__ absums,
-    float *__restrict__ y) {
+    M matrices, Layout lay, int nb, const float *__restrict__ x,
+    const int8_t *__restrict__ aq, const float *__restrict__ ad, const int16_t *__restrict__ absums) {
+    const GemvMatrix m = matrices.pick();
+    const uint8_t *__restrict__ const W = m.W;
+    float *__restrict__ const y = m.y;
+    const int rows = m.rows;
     constexpr int WAVES = FUSED ? 16 : 4;
     extern __shared__ uint4 smem_direct[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = min((int)blockIdx.x * WAVES + wave, rows - 1);  // a wavefront past the end repeats the last row
-    const bool store = (int)blockIdx.x * WAVES + wave < rows;
+    const int r = min(m.block * WAVES + wave, rows - 1);  // a wavefront past the end repeats the last row
+    const bool store = m.block * WAVES + wave < rows;
     const uint8_t *row = W + (size_t)r * lay.row_stride;
     const int units = nb * 4;
 
@@ -149,9 +152,12 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void gemv_q6_k_direct_kernel(
 // Round j of a wavefront covers rows 4j .. 4j+3 of the workgroup: lane = 16 * (row of the round) + unit,
 // unit = (block of the slice, half, 16-byte column) as above.
 constexpr int COLS_WAVE_LDS = 4 * (QK_K + 32 + 4);  // four blocks: quants, 16-wide sums, scale
-template <int U, bool NT = false>
-__global__ __launch_bounds__(1024) void gemv_q6_k_cols_kernel(const uint8_t *__restrict__ W, Layout lay, int rows, int nb,
-                                                             const float *__restrict__ x, float *__restrict__ y) {
+template <int U, bool NT, class M>
+__global__ __launch_bounds__(1024) void gemv_q6_k_cols_kernel(M matrices, Layout lay, int nb, const float *__restrict__ x) {
+    const GemvMatrix m = matrices.pick();
+    const uint8_t *__restrict__ const W = m.W;
+    float *__restrict__ const y = m.y;
+    const int rows = m.rows;
     typedef float xv_t __attribute__((ext_vector_type(4)));
     typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
     typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
@@ -160,7 +166,7 @@ __global__ __launch_bounds__(1024) void gemv_q6_k_cols_kernel(const uint8_t *__r
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     uint8_t *mine = reinterpret_cast<uint8_t *>(smem_cols) + wave * COLS_WAVE_LDS;
     float *parts = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(smem_cols) + waves * COLS_WAVE_LDS);
-    const int b0 = wave * 4, r0 = (int)blockIdx.x * 4 * U;
+    const int b0 = wave * 4, r0 = m.block * 4 * U;
 
     // the activation's loads first: a wavefront's loads return in issue order
     xv_t xv[4];
@@ -464,16 +470,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_q8_0_f32_shared_kernel(const 
 // columns in every row and keeps its 64 bytes of the activation in registers, read straight from global memory
 // -- no copy in LDS, hence no barrier between the requests and the arithmetic; the wavefronts' partial sums of a
 // row meet in LDS at the end and are added in the order of the columns.
-template <int R>
-__global__ __launch_bounds__(1024) void gemv_q8_0_f32_cols_kernel(const uint8_t *__restrict__ W, Layout lay, int rows, int nb,
-                                                                 const float *__restrict__ x, float *__restrict__ y) {
+template <int R, class M>
+__global__ __launch_bounds__(1024) void gemv_q8_0_f32_cols_kernel(M matrices, Layout lay, int nb, const float *__restrict__ x) {
+    const GemvMatrix m = matrices.pick();
+    const uint8_t *__restrict__ const W = m.W;
+    float *__restrict__ const y = m.y;
+    const int rows = m.rows;
     extern __shared__ uint4 smem_direct[];
     float *parts = reinterpret_cast<float *>(smem_direct);  // [wavefront][row]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int units = nb * 2;
     const bool live = wave * 64 + lane < units;
     const int u = min(wave * 64 + lane, units - 1);  // (a lane past the end: the last unit again, not added)
-    const int r0 = (int)blockIdx.x * R;
+    const int r0 = m.block * R;
     const float4 *xp = reinterpret_cast<const float4 *>(x + (size_t)u * 16);
     const float4 x0 = xp[0], x1 = xp[1], x2 = xp[2], x3 = xp[3];
     uint4 qv[R];
@@ -591,8 +600,8 @@ int launch_gemv_q6_k_direct(const frk_weights *w, Q8KActs a, float *y, hipStream
     const int u = (nb * 4 + 63) / 64;
     const dim3 grid((unsigned)((w->rows + 3) / 4)), block(256);
 #define FRK_GO(UU)                                                                                              \
-    hipLaunchKernelGGL((gemv_q6_k_direct_kernel<UU, 1, false>), grid, block, 0, s, w->dev, w->layout, (int)w->rows, \
-                       nb, (const float *)nullptr, a.q, a.d, a.bsums, y)
+    hipLaunchKernelGGL((gemv_q6_k_direct_kernel<UU, 1, false, GemvOne>), grid, block, 0, s, GemvOne{w->dev, y, (int)w->rows}, w->layout, \
+                       nb, (const float *)nullptr, a.q, a.d, a.bsums)
     if (u == 1) FRK_GO(1);
     else if (u == 2) FRK_GO(2);
     else if (u == 3) FRK_GO(3);
@@ -616,8 +625,9 @@ static int compute_units_direct() {
     }();
     return n;
 }
-// One launch: Q8_K quantization of x inside the kernel.  nb <= 64 (direct_gemv_fits).
-int launch_gemv_q6_k_fused(const frk_weights *w, const float *x, float *y, hipStream_t s) {
+// One launch for n <= 4 matrices of one row length: Q8_K quantization of x inside the kernel.  nb <= 64 (direct_gemv_fits).
+int launch_gemv_q6_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+    const frk_weights *const w = ws[0];
     const int nb = (int)(w->cols / QK_K);
     if (q6_k_cols_form(w)) {  // the wavefronts split the columns, not the rows
         const int waves = (nb + 3) / 4;
@@ -628,18 +638,20 @@ int launch_gemv_q6_k_fused(const frk_weights *w, const float *x, float *y, hipSt
         int best_u = 1;
         size_t best = SIZE_MAX;
         for (int u = 1; u <= (waves == 1 ? 2 : 6); u++) {
-            const size_t wgs = (w->rows + 4 * u - 1) / (4 * u);
+            const size_t wgs = gemv_workgroups(ws, n, 4 * u);
             const size_t cost = (wgs + cus - 1) / cus * (4 * u + 5);
             if (cost <= best) best = cost, best_u = u;
         }
         const size_t lds = (size_t)waves * (COLS_WAVE_LDS + 4 * best_u * 4);
-        const dim3 grid((unsigned)((w->rows + 4 * best_u - 1) / (4 * best_u))), block(64 * waves);
+        const dim3 grid((unsigned)gemv_workgroups(ws, n, 4 * best_u)), block(64 * waves);
+        const GemvOne one{w->dev, ys[0], (int)w->rows};
+        const GemvGroup group = gemv_group(ws, n, ys, 4 * best_u);
         const bool whole_lines = w->layout.row_stride % 128 == 0 && nb % 4 == 0;  // (every wavefront's four blocks of ql: 512 bytes)
 #define FRK_GO_COLS(UU)                                                                                                              \
-    if (whole_lines)                                                                                                                 \
-        hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true>), grid, block, lds, s, w->dev, w->layout, (int)w->rows, nb, x, y);      \
-    else                                                                                                                             \
-        hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, false>), grid, block, lds, s, w->dev, w->layout, (int)w->rows, nb, x, y)
+    if (n > 1 && whole_lines) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true, GemvGroup>), grid, block, lds, s, group, w->layout, nb, x); \
+    else if (n > 1) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, false, GemvGroup>), grid, block, lds, s, group, w->layout, nb, x);          \
+    else if (whole_lines) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true, GemvOne>), grid, block, lds, s, one, w->layout, nb, x);         \
+    else hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, false, GemvOne>), grid, block, lds, s, one, w->layout, nb, x)
         if (best_u == 1) FRK_GO_COLS(1);
         else if (best_u == 2) FRK_GO_COLS(2);
         else if (best_u == 3) FRK_GO_COLS(3);
@@ -651,11 +663,18 @@ int launch_gemv_q6_k_fused(const frk_weights *w, const float *x, float *y, hipSt
         return FRK_OK;
     }
     const int u = (nb * 4 + 63) / 64;
-    const dim3 grid((unsigned)((w->rows + 15) / 16)), block(1024);
+    const dim3 grid((unsigned)gemv_workgroups(ws, n, 16)), block(1024);
     const size_t shmem = (size_t)nb * (256 + 32 + 4);
-#define FRK_GO(UU, XX)                                                                                              \
-    hipLaunchKernelGGL((gemv_q6_k_direct_kernel<UU, XX, true>), grid, block, shmem, s, w->dev, w->layout, (int)w->rows, \
-                       nb, x, (const int8_t *)nullptr, (const float *)nullptr, (const int16_t *)nullptr, y)
+    const int8_t *const no_q = nullptr;
+    const float *const no_d = nullptr;
+    const int16_t *const no_sums = nullptr;
+#define FRK_GO(UU, XX)                                                                                                                   \
+    if (n > 1)                                                                                                                           \
+        hipLaunchKernelGGL((gemv_q6_k_direct_kernel<UU, XX, true, GemvGroup>), grid, block, shmem, s, gemv_group(ws, n, ys, 16), w->layout, \
+                           nb, x, no_q, no_d, no_sums);                                                                                  \
+    else                                                                                                                                 \
+        hipLaunchKernelGGL((gemv_q6_k_direct_kernel<UU, XX, true, GemvOne>), grid, block, shmem, s, GemvOne{w->dev, ys[0], (int)w->rows},   \
+                           w->layout, nb, x, no_q, no_d, no_sums)
     if (u == 1) FRK_GO(1, 1);       // nb <= 16
     else if (u == 2) FRK_GO(2, 2);  // nb <= 32
     else if (u == 3) FRK_GO(3, 3);  // nb <= 48
@@ -664,6 +683,7 @@ int launch_gemv_q6_k_fused(const frk_weights *w, const float *x, float *y, hipSt
     FRK_LAUNCH_CHECK("gemv_q6_k_fused");
     return FRK_OK;
 }
+int launch_gemv_q6_k_fused(const frk_weights *w, const float *x, float *y, hipStream_t s) { return launch_gemv_q6_k_group(&w, 1, x, &y, s); }
 
 // expert rows of at most 64 units (4096 columns), at most 16 blocks for the workgroup to quantize
 bool q6_k_experts_gemv_fits(const frk_weights *w) {
@@ -715,24 +735,36 @@ int launch_q6_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e,
     return launch_experts_down_as<Q6Unit, 32, 4, 8, 3>(w, n_experts, rows_e, act, ids, weights, batch, k, out, s);
 }
 
-int launch_gemv_q8_0_f32_direct(const frk_weights *w, const float *x, float *y, hipStream_t s) {
+// Q8_0 rows of 512 to 16384 columns (direct_gemv_fits): the wavefronts of a workgroup split the columns.  n <= 4 matrices.
+bool q8_0_cols_form(const frk_weights *w) { return w->kind == FRK_KIND_Q8_0 && direct_gemv_fits(w) && w->cols / Q8_0_ELEMS * 2 <= 1024; }
+int launch_gemv_q8_0_f32_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+    const frk_weights *const w = ws[0];
     const int nb = (int)(w->cols / Q8_0_ELEMS);
     const int u = (nb * 2 + 63) / 64;
-    if (u <= 16) {  // rows of up to 16384 columns: the wavefronts of a workgroup split the columns
-        // Eight rows to a workgroup; four where eight would leave a CU fewer than a dozen wavefronts.  (Measured
-        // against the kernel below, which shares the activation through LDS: 4096x4096 5.6 against 5.7 us,
-        // 14336x4096 13.2 / 14.0, 4096x8192 8.9 / 10.0, 4096x11008 11.3 / 12.9, 4096x14336 15.0 / 17.3; twelve and
-        // sixteen rows to a workgroup are slower everywhere.)
-        const bool four = (w->rows / 8) * (size_t)u < 12 * (size_t)compute_units_direct();
+    // Eight rows to a workgroup; four where eight would leave a CU fewer than a dozen wavefronts.  (Measured
+    // against the kernel below, which shares the activation through LDS: 4096x4096 5.6 against 5.7 us,
+    // 14336x4096 13.2 / 14.0, 4096x8192 8.9 / 10.0, 4096x11008 11.3 / 12.9, 4096x14336 15.0 / 17.3; twelve and
+    // sixteen rows to a workgroup are slower everywhere.)
+    size_t rows = 0;
+    for (size_t i = 0; i < n; i++) rows += ws[i]->rows;
+    const bool four = (rows / 8) * (size_t)u < 12 * (size_t)compute_units_direct();
 #define FRK_GO_COLS(RR)                                                                                                              \
-    hipLaunchKernelGGL((gemv_q8_0_f32_cols_kernel<RR>), dim3((unsigned)((w->rows + RR - 1) / RR)), dim3(64 * u), (size_t)u * RR * 4, s, \
-                       w->dev, w->layout, (int)w->rows, nb, x, y)
-        if (four) FRK_GO_COLS(4);
-        else FRK_GO_COLS(8);
+    if (n > 1)                                                                                                                           \
+        hipLaunchKernelGGL((gemv_q8_0_f32_cols_kernel<RR, GemvGroup>), dim3((unsigned)gemv_workgroups(ws, n, RR)), dim3(64 * u),           \
+                           (size_t)u * RR * 4, s, gemv_group(ws, n, ys, RR), w->layout, nb, x);                                           \
+    else                                                                                                                                 \
+        hipLaunchKernelGGL((gemv_q8_0_f32_cols_kernel<RR, GemvOne>), dim3((unsigned)gemv_workgroups(ws, n, RR)), dim3(64 * u),             \
+                           (size_t)u * RR * 4, s, GemvOne{w->dev, ys[0], (int)w->rows}, w->layout, nb, x)
+    if (four) FRK_GO_COLS(4);
+    else FRK_GO_COLS(8);
 #undef FRK_GO_COLS
-        FRK_LAUNCH_CHECK("gemv_q8_0_f32_cols");
-        return FRK_OK;
-    }
+    FRK_LAUNCH_CHECK("gemv_q8_0_f32_cols");
+    return FRK_OK;
+}
+int launch_gemv_q8_0_f32_direct(const frk_weights *w, const float *x, float *y, hipStream_t s) {
+    if (q8_0_cols_form(w)) return launch_gemv_q8_0_f32_group(&w, 1, x, &y, s);
+    const int nb = (int)(w->cols / Q8_0_ELEMS);
+    const int u = (nb * 2 + 63) / 64;
     // longer rows (direct_gemv_fits: up to 28672 columns, at least 1024 rows): a row to a wavefront, the activation
     // through LDS, one workgroup to a CU
     constexpr int WAVES = 8;

@@ -742,9 +742,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_q4_k_rows_kernel(const uint8_
 // Round j of a wavefront covers rows 8j .. 8j+7 of the workgroup: lane = 8 * (row of the round) + unit, a unit
 // being a half block as in gemv_q4_k_fused_kernel (the block's header and four of its eight 16-byte words).
 constexpr int COLS_WAVE_LDS = 4 * (QK_K + 32 + 4);  // four blocks: quants, 16-wide sums, scale
-template <int U, bool Q5 = false>
-__global__ __launch_bounds__(1024) void gemv_q4_k_cols_kernel(const uint8_t *__restrict__ W, size_t row_stride, int rows, int nb,
-                                                             const float *__restrict__ x, float *__restrict__ y) {
+template <int U, bool Q5, class M>
+__global__ __launch_bounds__(1024) void gemv_q4_k_cols_kernel(M matrices, size_t row_stride, int nb, const float *__restrict__ x) {
+    const GemvMatrix m = matrices.pick();
+    const uint8_t *__restrict__ const W = m.W;
+    float *__restrict__ const y = m.y;
+    const int rows = m.rows;
     typedef float xv_t __attribute__((ext_vector_type(4)));
     typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
     extern __shared__ uint4 smem[];
@@ -752,7 +755,7 @@ __global__ __launch_bounds__(1024) void gemv_q4_k_cols_kernel(const uint8_t *__r
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     uint8_t *mine = reinterpret_cast<uint8_t *>(smem) + wave * COLS_WAVE_LDS;
     float *parts = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(smem) + waves * COLS_WAVE_LDS);
-    const int b0 = wave * 4, r0 = (int)blockIdx.x * 8 * U;
+    const int b0 = wave * 4, r0 = m.block * 8 * U;
 
     // the activation's loads first: a wavefront's loads return in issue order
     xv_t xv[4];
@@ -1061,7 +1064,9 @@ int launch_gemv_rows_preq(const frk_weights *w, Q8KActs a, float *y, hipStream_t
 //   5120x5120 7.8 / 5.9 / 6.9    6144x6144 8.7 / 8.8 / 9.0    8192x3072 5.5 / 5.2 / 6.7    3072x3072 3.7 / 4.6 / 5.9
 //   2560x2560 3.4 / 4.5 / 5.8
 // Rows of 8, 16 and 32 blocks have the whole-cache-line kernel (14336x4096: 8.2 / 8.9 / 10.3).
-int launch_gemv_q4_k_cols(const frk_weights *w, const float *x, float *y, hipStream_t s) {
+// n <= 4 matrices of one kind and row length
+static int launch_cols_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+    const frk_weights *const w = ws[0];
     const int nb = (int)(w->cols / QK_K), waves = (nb + 3) / 4;
     const int cus = compute_units();
     int best_u = 1;
@@ -1070,16 +1075,20 @@ int launch_gemv_q4_k_cols(const frk_weights *w, const float *x, float *y, hipStr
     // of the activation, about seven rows' worth), the larger of equals
     const bool q5 = w->kind == FRK_KIND_Q5_K;
     for (int u = 1; u <= (q5 ? 2 : 3); u++) {
-        const size_t wgs = (w->rows + 8 * u - 1) / (8 * u);
+        const size_t wgs = gemv_workgroups(ws, n, 8 * u);
         const size_t cost = (wgs + cus - 1) / cus * (8 * u + 7);
         if (cost <= best) best = cost, best_u = u;
     }
     const size_t lds = (size_t)waves * (COLS_WAVE_LDS + 8 * best_u * 4);
-    const dim3 grid((unsigned)((w->rows + 8 * best_u - 1) / (8 * best_u))), block(64 * waves);
-#define FRK_GO_COLS(UU) \
-    hipLaunchKernelGGL((gemv_q4_k_cols_kernel<UU>), grid, block, lds, s, w->dev, w->layout.row_stride, (int)w->rows, nb, x, y)
-#define FRK_GO_COLS5(UU) \
-    hipLaunchKernelGGL((gemv_q4_k_cols_kernel<UU, true>), grid, block, lds, s, w->dev, w->layout.row_stride, (int)w->rows, nb, x, y)
+    const dim3 grid((unsigned)gemv_workgroups(ws, n, 8 * best_u)), block(64 * waves);
+    const GemvOne one{w->dev, ys[0], (int)w->rows};
+    const GemvGroup group = gemv_group(ws, n, ys, 8 * best_u);
+#define FRK_GO_COLS(UU)                                                                                                                    \
+    if (n > 1) hipLaunchKernelGGL((gemv_q4_k_cols_kernel<UU, false, GemvGroup>), grid, block, lds, s, group, w->layout.row_stride, nb, x); \
+    else hipLaunchKernelGGL((gemv_q4_k_cols_kernel<UU, false, GemvOne>), grid, block, lds, s, one, w->layout.row_stride, nb, x)
+#define FRK_GO_COLS5(UU)                                                                                                                  \
+    if (n > 1) hipLaunchKernelGGL((gemv_q4_k_cols_kernel<UU, true, GemvGroup>), grid, block, lds, s, group, w->layout.row_stride, nb, x); \
+    else hipLaunchKernelGGL((gemv_q4_k_cols_kernel<UU, true, GemvOne>), grid, block, lds, s, one, w->layout.row_stride, nb, x)
     if (q5 && best_u == 1) FRK_GO_COLS5(1);
     else if (q5) FRK_GO_COLS5(2);
     else if (best_u == 1) FRK_GO_COLS(1);
@@ -1090,6 +1099,7 @@ int launch_gemv_q4_k_cols(const frk_weights *w, const float *x, float *y, hipStr
     FRK_LAUNCH_CHECK("gemv_q4_k_cols");
     return FRK_OK;
 }
+int launch_gemv_q4_k_cols(const frk_weights *w, const float *x, float *y, hipStream_t s) { return launch_cols_group(&w, 1, x, &y, s); }
 
 // Which kernel a one-launch GEMV of Q4_K / Q5_K rows of other lengths than 8 and 16 blocks takes.
 int rows_gemv_form(const frk_weights *w) {
@@ -1103,10 +1113,22 @@ int rows_gemv_form(const frk_weights *w) {
         // 4096x8192 7.2 / 6.8; rows of 20 blocks 5120x5120 6.3 / 6.0, of 16 blocks 14336x4096 10.5 / 8.1.
         if (nb > 20 && nb != 32) return ROWS_FORM_COLUMNS;
         if (nb == 32 && (w->rows <= 2048 || w->rows >= 6144)) return ROWS_FORM_COLUMNS;
+        // Shorter rows, weights from memory (not from the 256 MB cache): 9 to 12 blocks 1024x3072 3.6 -> 3.2, 4096x3072 4.5 -> 3.7, 7168x3072 6.1 ->
+        // 5.8, 11008x2816 7.2 -> 6.8, but 14336x3072 7.6 / 8.4 (13 to 15: 0.86 to 1.18 of the time, but the experts' kernels have the other
+        // form's bits); 17 to 20 1024x5120 5.1 -> 4.1, 4096x5120 5.7 -> 5.5, 7168x5120 8.3 / 8.3,
+        // but 11008x5120 9.0 / 10.1.
+        if (nb > 8 && nb <= 12 && w->rows < 12288) return ROWS_FORM_COLUMNS;
+        if (nb > 16 && nb <= 20 && w->rows <= 8192) return ROWS_FORM_COLUMNS;
     }
     // Q5_K on the same kernel (two rounds at most): 4096x14336 12.8 / 14.8, 4096x11008 10.4 / 13.7, 8192x10240 17.5 / 22.5,
-    // 4096x16384 13.3 / 16.8, 2048x16384 8.3 / 9.1; up to 32 blocks it is behind (5120x5120 7.6 / 6.8, 4096x8192 8.3 / 7.3)
+    // 4096x16384 13.3 / 16.8, 2048x16384 8.3 / 9.1; at 32 blocks it is behind (4096x8192 8.3 / 7.3)
     if (w->kind == FRK_KIND_Q5_K && nb > 32) return ROWS_FORM_COLUMNS;
+    // Shorter rows, weights from memory: 9 to 15 blocks against a quantization launch and a GEMV 1024x3072 6.5 -> 3.5, 4096x3072 7.5 -> 5.0,
+    // 14336x3072 11.3 -> 11.0; 17 to 20 1024x5120 5.7 -> 4.6, 4096x5120 6.6 -> 6.5, 7168x5120 11.1 -> 9.7, but 11008x5120 12.3 / 12.9; 21 to
+    // 31 1024x6144 6.0 -> 4.7, 11008x6144 17.7 -> 14.3, but 4096x6144 7.2 / 7.4.
+    if (w->kind == FRK_KIND_Q5_K && nb > 8 && nb < 16) return ROWS_FORM_COLUMNS;
+    if (w->kind == FRK_KIND_Q5_K && nb > 16 && nb <= 20 && w->rows <= 8192) return ROWS_FORM_COLUMNS;
+    if (w->kind == FRK_KIND_Q5_K && nb > 20 && nb < 32 && (w->rows <= 2048 || w->rows >= 6144)) return ROWS_FORM_COLUMNS;
     if (nb > 16 && nb < 32) return ROWS_FORM_ONE_LAUNCH;
     if (rows_gemv_takes_quantized(w)) return ROWS_FORM_QUANTIZED;
     return ROWS_FORM_NONE;
@@ -1136,23 +1158,47 @@ int launch_gemv_q5_k_fused(const frk_weights *w, const float *x, float *y, hipSt
 int launch_gemv_q5_k_preq(const frk_weights *w, Q8KActs a, float *y, hipStream_t s) {
     return launch_q5_k_lines<MODE_PREQ_LDS>(w, nullptr, a, y, s);
 }
-// ys[i] = ws[i] . x for 2..4 Q4_K matrices of one row length (fused_gemv_fits), one launch
-int launch_gemv_q4_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+// n <= 4 matrices as one list of rows
+static MultiArgs multi_args(const frk_weights *const *ws, size_t n, float *const *ys, size_t *total) {
     MultiArgs ma;
-    size_t total = 0;
+    *total = 0;
     for (size_t i = 0; i < 4; i++) {
         const size_t j = i < n ? i : n - 1;
         ma.W[i] = ws[j]->dev;
         ma.y[i] = ys[j];
-        ma.first[i] = (int)total;
-        if (i < n) total += ws[i]->rows;
+        ma.first[i] = (int)*total;
+        if (i < n) *total += ws[i]->rows;
     }
-    for (size_t i = n; i < 4; i++) ma.first[i] = (int)total;
+    for (size_t i = n; i < 4; i++) ma.first[i] = (int)*total;
+    return ma;
+}
+// ys[i] = ws[i] . x for up to four Q5_K matrices of one row length (rows_gemv_fits), one launch.  The column form, but for rows of 8
+// and 16 blocks the whole-cache-line kernel (us, that / columns: 2048 + 256 + 256 rows x 2048 3.7 / 4.0, three times 2048 x 2048 4.1 / 4.5,
+// 4096 + 1024 + 1024 x 4096 5.8 / 5.8 -- a single 4096 x 4096 from memory, not from the 256 MB cache, 4.5 / 5.4 --; of 32 blocks
+// 8192 + 1024 + 1024 x 8192 17.4 / 13.9).  A shared quantization launch and one for every matrix: 9.8, 12.2, 12.1, 21.5.
+int launch_gemv_q5_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+    const size_t nb = ws[0]->cols / QK_K;
+    bool lines = n > 1 && (nb == 8 || nb == 16);
+    for (size_t i = 0; i < n; i++) lines = lines && lines_kernel_fits(ws[i]) && ws[i]->rows % (64 / nb) == 0;
+    if (!lines) return launch_cols_group(ws, n, x, ys, s);
+    size_t total = 0;
+    const MultiArgs ma = multi_args(ws, n, ys, &total);
+    const Q8KActs none{nullptr, nullptr, nullptr};
+    if (nb == 8) return launch_q4_k_lines_as<8, MODE_FUSED, 4, true, 0, true>(ws[0], x, none, ys[0], s, total, &ma);
+    return launch_q4_k_lines_as<16, MODE_FUSED, 4, true, 0, true>(ws[0], x, none, ys[0], s, total, &ma);
+}
+// ys[i] = ws[i] . x for 2..4 Q4_K matrices of one row length (fused_gemv_fits), one launch
+int launch_gemv_q4_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+    size_t total = 0;
+    const MultiArgs ma = multi_args(ws, n, ys, &total);
     // rows of 8 or 16 blocks, every matrix a whole number of spans: the whole-cache-line kernel over the list
     // (q/k/v of 4096 + 1024 + 1024 rows x 4096: 5.3 us against 6.3 on the per-lane kernel)
     const size_t nb = ws[0]->cols / QK_K;
     bool lines = nb == 8 || nb == 16;
     for (size_t i = 0; i < n; i++) lines = lines && lines_kernel_fits(ws[i]) && ws[i]->cols == ws[0]->cols && ws[i]->rows % (64 / nb) == 0;
+    // other lengths: the column form, but for short rows that are many (q/k/v of 4864 + 608 + 608 x 4864 8.2 -> 5.4 us, 3072 + 768 + 768 x 3072
+    // 5.2 -> 4.1, 6656 + 1664 + 1664 x 6656 11.1 -> 9.3; a single 14336 x 3072 from memory 7.6 here, 8.4 there)
+    if (!lines && rows_gemv_fits(ws[0]) && (nb > 16 || total < 12288)) return launch_cols_group(ws, n, x, ys, s);
     if (lines) {
         const Q8KActs none{nullptr, nullptr, nullptr};
         if (nb == 8) return launch_q4_k_lines_as<8, MODE_FUSED, 8, false, 0, true>(ws[0], x, none, ys[0], s, total, &ma);

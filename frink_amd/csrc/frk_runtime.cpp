@@ -562,7 +562,7 @@ static int gemv_impl(const frk_weights *w, const float *x, float *y, int act_mod
     switch (w->kind) {
     case FRK_KIND_Q4_K:
     case FRK_KIND_Q5_K: {
-        const int form = rows_gemv_form(w);  // rows of 17..31 and of 33..64 blocks: whole rows to a wavefront
+        const int form = rows_gemv_form(w);  // rows of other lengths than 8 and 16 blocks
         if (form == ROWS_FORM_COLUMNS) return launch_gemv_q4_k_cols(w, x, y, s);
         if (form == ROWS_FORM_ONE_LAUNCH) return launch_gemv_rows_fused(w, x, y, s);
         if (form == ROWS_FORM_QUANTIZED) {
@@ -1140,23 +1140,30 @@ int frk_hip_gemv_multi_dev(const frk_weights *const *ws, size_t n, const float *
     bool all_fused = true;
     for (size_t i = 0; i < n; i++) {
         const frk_weights *w = ws[i];
-        all_fused = all_fused && ((w->kind == FRK_KIND_Q4_K && fused_gemv_fits(w)) ||
+        all_fused = all_fused && ((w->kind == FRK_KIND_Q4_K && fused_gemv_fits(w)) || (w->kind == FRK_KIND_Q5_K && rows_gemv_fits(w)) ||
                                   (w->kind == FRK_KIND_Q6_K && (direct_gemv_fits(w) || q6_k_cols_form(w))) || w->kind == FRK_KIND_Q8_0 ||
                                   w->kind == FRK_KIND_Q4_0);
     }
     if (all_fused) {
-        // Q4_K neighbours go out in one launch, four at most: the kernel walks their rows as one list
+        // neighbours of a kind go out in one launch, four at most
+        auto grouped = [](const frk_weights *w) { return w->kind != FRK_KIND_Q4_0 && (w->kind != FRK_KIND_Q8_0 || q8_0_cols_form(w)); };
         size_t i = 0;
         while (i < n) {
             size_t m = 1;
             size_t rows = ws[i]->rows;
-            if (ws[i]->kind == FRK_KIND_Q4_K)
-                while (i + m < n && m < 4 && ws[i + m]->kind == FRK_KIND_Q4_K && rows + ws[i + m]->rows < (1u << 30)) {
+            const int kind = ws[i]->kind;
+            if (grouped(ws[i]))
+                while (i + m < n && m < 4 && ws[i + m]->kind == kind && grouped(ws[i + m]) && rows + ws[i + m]->rows < (1u << 30)) {
                     rows += ws[i + m]->rows;
                     m++;
                 }
-            int rc = m > 1 ? launch_gemv_q4_k_group(ws + i, m, x, ys + i, s)
-                           : frk_hip_gemv_dev(ws[i], x, ys[i], FRK_ACT_F32, stream);
+            const bool q5_alone = kind == FRK_KIND_Q5_K && !q5_k_lines_gemv_fits(ws[i]) && rows_gemv_form(ws[i]) == ROWS_FORM_NONE;
+            int rc;
+            if (m == 1 && !q5_alone) rc = frk_hip_gemv_dev(ws[i], x, ys[i], FRK_ACT_F32, stream);
+            else if (kind == FRK_KIND_Q4_K) rc = launch_gemv_q4_k_group(ws + i, m, x, ys + i, s);
+            else if (kind == FRK_KIND_Q5_K) rc = launch_gemv_q5_k_group(ws + i, m, x, ys + i, s);
+            else if (kind == FRK_KIND_Q6_K) rc = launch_gemv_q6_k_group(ws + i, m, x, ys + i, s);
+            else rc = launch_gemv_q8_0_f32_group(ws + i, m, x, ys + i, s);
             if (rc) return rc;
             i += m;
         }
