@@ -166,7 +166,7 @@ __global__ __launch_bounds__(1024) void gemv_q6_k_cols_kernel(M matrices, Layout
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     uint8_t *mine = reinterpret_cast<uint8_t *>(smem_cols) + wave * COLS_WAVE_LDS;
     float *parts = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(smem_cols) + waves * COLS_WAVE_LDS);
-    const int b0 = wave * 4, r0 = m.block * 4 * U;
+    const int b0 = wave * 4, r0 = m.block * (M::GLU ? 2 : 4) * U;
 
     // the activation's loads first: a wavefront's loads return in issue order
     xv_t xv[4];
@@ -182,8 +182,11 @@ __global__ __launch_bounds__(1024) void gemv_q6_k_cols_kernel(M matrices, Layout
     u2_t scv[U];
     uint32_t dbits[U];
     auto request = [&](int j) {
-        const int r = min(r0 + 4 * j + (lane >> 4), rows - 1);  // a row past the end: the last one again, not stored
-        const uint8_t *row = W + (size_t)r * lay.row_stride;
+        // (a row past the end: the last one again, not stored; gate and up: a round's rows 2 and 3 are up's)
+        const int r = min(M::GLU ? r0 + 2 * j + ((lane >> 4) & 1) : r0 + 4 * j + (lane >> 4), rows - 1);
+        const uint8_t *base = W;
+        if constexpr (M::GLU) base = lane & 32 ? matrices.up : W;
+        const uint8_t *row = base + (size_t)r * lay.row_stride;
         const uint8_t *p_l = row + (size_t)b * 128 + h * 64 + t * 16;
         const uint8_t *p_h = row + lay.off_a + (size_t)b * 64 + h * 32 + t * 16;
         const uint8_t *p_s = row + lay.off_b + (size_t)b * 16 + h * 8;
@@ -272,10 +275,18 @@ __global__ __launch_bounds__(1024) void gemv_q6_k_cols_kernel(M matrices, Layout
         if (ul == 0) parts[wave * (4 * U) + 4 * j + (lane >> 4)] = sums[j];
     lds_barrier();
     // a row's partial sums, in the order of the columns
-    if ((int)threadIdx.x < 4 * U && r0 + (int)threadIdx.x < rows) {
+    const int at = (int)threadIdx.x;
+    if constexpr (M::GLU) {
+        if (at < 2 * U && r0 + at < rows) {
+            const float *p = parts + (at >> 1) * 4 + (at & 1);
+            float g = 0.0f, u = 0.0f;
+            for (int w = 0; w < waves; w++) g += p[w * (4 * U)], u += p[w * (4 * U) + 2];
+            y[r0 + at] = silu_as_host(g) * u;
+        }
+    } else if (at < 4 * U && r0 + at < rows) {
         float v = 0.0f;
-        for (int w = 0; w < waves; w++) v += parts[w * (4 * U) + threadIdx.x];
-        y[r0 + threadIdx.x] = v;
+        for (int w = 0; w < waves; w++) v += parts[w * (4 * U) + at];
+        y[r0 + at] = v;
     }
 }
 
@@ -482,14 +493,17 @@ __global__ __launch_bounds__(1024) void gemv_q8_0_f32_cols_kernel(M matrices, La
     const int units = nb * 2;
     const bool live = wave * 64 + lane < units;
     const int u = min(wave * 64 + lane, units - 1);  // (a lane past the end: the last unit again, not added)
-    const int r0 = m.block * R;
+    const int r0 = m.block * (M::GLU ? R / 2 : R);
     const float4 *xp = reinterpret_cast<const float4 *>(x + (size_t)u * 16);
     const float4 x0 = xp[0], x1 = xp[1], x2 = xp[2], x3 = xp[3];
     uint4 qv[R];
     uint32_t dbits[R];
 #pragma unroll
     for (int k = 0; k < R; k++) {
-        const uint8_t *row = W + (size_t)min(r0 + k, rows - 1) * lay.row_stride;  // (a row past the end: the last again)
+        // (a row past the end: the last again; gate and up: the second half of the rows is up's)
+        const uint8_t *base = W;
+        if constexpr (M::GLU) base = k < R / 2 ? W : matrices.up;
+        const uint8_t *row = base + (size_t)min(r0 + (M::GLU ? k % (R / 2) : k), rows - 1) * lay.row_stride;
         qv[k] = stream_load16(row + (size_t)u * 16);
         dbits[k] = stream_load2(row + lay.off_a + (size_t)(u >> 1) * 2);
     }
@@ -510,10 +524,17 @@ __global__ __launch_bounds__(1024) void gemv_q8_0_f32_cols_kernel(M matrices, La
         if (lane == 0) parts[wave * R + k] = v;
     }
     __syncthreads();
-    if ((int)threadIdx.x < R && r0 + (int)threadIdx.x < rows) {
+    const int at = (int)threadIdx.x;
+    if constexpr (M::GLU) {
+        if (at < R / 2 && r0 + at < rows) {
+            float g = 0.0f, h = 0.0f;
+            for (int w = 0; w < waves; w++) g += parts[w * R + at], h += parts[w * R + R / 2 + at];
+            y[r0 + at] = silu_as_host(g) * h;
+        }
+    } else if (at < R && r0 + at < rows) {
         float v = 0.0f;
-        for (int w = 0; w < waves; w++) v += parts[w * R + threadIdx.x];
-        y[r0 + threadIdx.x] = v;
+        for (int w = 0; w < waves; w++) v += parts[w * R + at];
+        y[r0 + at] = v;
     }
 }
 
@@ -626,7 +647,8 @@ static int compute_units_direct() {
     return n;
 }
 // One launch for n <= 4 matrices of one row length: Q8_K quantization of x inside the kernel.  nb <= 64 (direct_gemv_fits).
-int launch_gemv_q6_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+// glu (q6_k_cols_form only): gate and up, ys[0] = silu(gate x) * (up x).
+static int launch_q6_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s, bool glu) {
     const frk_weights *const w = ws[0];
     const int nb = (int)(w->cols / QK_K);
     if (q6_k_cols_form(w)) {  // the wavefronts split the columns, not the rows
@@ -638,17 +660,20 @@ int launch_gemv_q6_k_group(const frk_weights *const *ws, size_t n, const float *
         int best_u = 1;
         size_t best = SIZE_MAX;
         for (int u = 1; u <= (waves == 1 ? 2 : 6); u++) {
-            const size_t wgs = gemv_workgroups(ws, n, 4 * u);
+            const size_t wgs = glu ? gemv_workgroups(ws, 1, 2 * u) : gemv_workgroups(ws, n, 4 * u);
             const size_t cost = (wgs + cus - 1) / cus * (4 * u + 5);
             if (cost <= best) best = cost, best_u = u;
         }
         const size_t lds = (size_t)waves * (COLS_WAVE_LDS + 4 * best_u * 4);
-        const dim3 grid((unsigned)gemv_workgroups(ws, n, 4 * best_u)), block(64 * waves);
+        const dim3 grid((unsigned)(glu ? gemv_workgroups(ws, 1, 2 * best_u) : gemv_workgroups(ws, n, 4 * best_u))), block(64 * waves);
+        const GemvGlu pair{w->dev, ws[n - 1]->dev, ys[0], (int)w->rows};
         const GemvOne one{w->dev, ys[0], (int)w->rows};
         const GemvGroup group = gemv_group(ws, n, ys, 4 * best_u);
         const bool whole_lines = w->layout.row_stride % 128 == 0 && nb % 4 == 0;  // (every wavefront's four blocks of ql: 512 bytes)
 #define FRK_GO_COLS(UU)                                                                                                              \
-    if (n > 1 && whole_lines) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true, GemvGroup>), grid, block, lds, s, group, w->layout, nb, x); \
+    if (glu && whole_lines) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true, GemvGlu>), grid, block, lds, s, pair, w->layout, nb, x);        \
+    else if (glu) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, false, GemvGlu>), grid, block, lds, s, pair, w->layout, nb, x);                 \
+    else if (n > 1 && whole_lines) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true, GemvGroup>), grid, block, lds, s, group, w->layout, nb, x); \
     else if (n > 1) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, false, GemvGroup>), grid, block, lds, s, group, w->layout, nb, x);          \
     else if (whole_lines) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true, GemvOne>), grid, block, lds, s, one, w->layout, nb, x);         \
     else hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, false, GemvOne>), grid, block, lds, s, one, w->layout, nb, x)
@@ -683,7 +708,15 @@ int launch_gemv_q6_k_group(const frk_weights *const *ws, size_t n, const float *
     FRK_LAUNCH_CHECK("gemv_q6_k_fused");
     return FRK_OK;
 }
+int launch_gemv_q6_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+    return launch_q6_k_group(ws, n, x, ys, s, false);
+}
 int launch_gemv_q6_k_fused(const frk_weights *w, const float *x, float *y, hipStream_t s) { return launch_gemv_q6_k_group(&w, 1, x, &y, s); }
+// act = silu(gate x) * (up x): one shape, q6_k_cols_form
+int launch_gemv_q6_k_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s) {
+    const frk_weights *const ws[2] = {gate, up};
+    return launch_q6_k_group(ws, 2, x, &act, s, true);
+}
 
 // expert rows of at most 64 units (4096 columns), at most 16 blocks for the workgroup to quantize
 bool q6_k_experts_gemv_fits(const frk_weights *w) {
@@ -737,7 +770,7 @@ int launch_q6_k_experts_down(const frk_weights *w, int n_experts, size_t rows_e,
 
 // Q8_0 rows of 512 to 16384 columns (direct_gemv_fits): the wavefronts of a workgroup split the columns.  n <= 4 matrices.
 bool q8_0_cols_form(const frk_weights *w) { return w->kind == FRK_KIND_Q8_0 && direct_gemv_fits(w) && w->cols / Q8_0_ELEMS * 2 <= 1024; }
-int launch_gemv_q8_0_f32_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+static int launch_q8_0_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s, bool glu) {
     const frk_weights *const w = ws[0];
     const int nb = (int)(w->cols / Q8_0_ELEMS);
     const int u = (nb * 2 + 63) / 64;
@@ -749,7 +782,10 @@ int launch_gemv_q8_0_f32_group(const frk_weights *const *ws, size_t n, const flo
     for (size_t i = 0; i < n; i++) rows += ws[i]->rows;
     const bool four = (rows / 8) * (size_t)u < 12 * (size_t)compute_units_direct();
 #define FRK_GO_COLS(RR)                                                                                                              \
-    if (n > 1)                                                                                                                           \
+    if (glu)                                                                                                                             \
+        hipLaunchKernelGGL((gemv_q8_0_f32_cols_kernel<RR, GemvGlu>), dim3((unsigned)gemv_workgroups(ws, 1, RR / 2)), dim3(64 * u),         \
+                           (size_t)u * RR * 4, s, GemvGlu{w->dev, ws[n - 1]->dev, ys[0], (int)w->rows}, w->layout, nb, x);                \
+    else if (n > 1)                                                                                                                      \
         hipLaunchKernelGGL((gemv_q8_0_f32_cols_kernel<RR, GemvGroup>), dim3((unsigned)gemv_workgroups(ws, n, RR)), dim3(64 * u),           \
                            (size_t)u * RR * 4, s, gemv_group(ws, n, ys, RR), w->layout, nb, x);                                           \
     else                                                                                                                                 \
@@ -760,6 +796,14 @@ int launch_gemv_q8_0_f32_group(const frk_weights *const *ws, size_t n, const flo
 #undef FRK_GO_COLS
     FRK_LAUNCH_CHECK("gemv_q8_0_f32_cols");
     return FRK_OK;
+}
+int launch_gemv_q8_0_f32_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+    return launch_q8_0_group(ws, n, x, ys, s, false);
+}
+// act = silu(gate x) * (up x): one shape, q8_0_cols_form
+int launch_gemv_q8_0_f32_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s) {
+    const frk_weights *const ws[2] = {gate, up};
+    return launch_q8_0_group(ws, 2, x, &act, s, true);
 }
 int launch_gemv_q8_0_f32_direct(const frk_weights *w, const float *x, float *y, hipStream_t s) {
     if (q8_0_cols_form(w)) return launch_gemv_q8_0_f32_group(&w, 1, x, &y, s);

@@ -755,7 +755,7 @@ __global__ __launch_bounds__(1024) void gemv_q4_k_cols_kernel(M matrices, size_t
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     uint8_t *mine = reinterpret_cast<uint8_t *>(smem) + wave * COLS_WAVE_LDS;
     float *parts = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(smem) + waves * COLS_WAVE_LDS);
-    const int b0 = wave * 4, r0 = m.block * 8 * U;
+    const int b0 = wave * 4, r0 = m.block * (M::GLU ? 4 : 8) * U;
 
     // the activation's loads first: a wavefront's loads return in issue order
     xv_t xv[4];
@@ -771,8 +771,11 @@ __global__ __launch_bounds__(1024) void gemv_q4_k_cols_kernel(M matrices, size_t
     constexpr int BB = Q5 ? Q5_K_BYTES : Q4_K_BYTES, LOADS = Q5 ? 7 : 5;
     u4_t wh[U], w0[U], w1[U], w2[U], w3[U], fa[Q5 ? U : 1], fb[Q5 ? U : 1];
     auto request = [&](int j) {
-        const int r = min(r0 + 8 * j + (lane >> 3), rows - 1);  // a row past the end: the last one again, not stored
-        const uint8_t *blk = W + (size_t)r * row_stride + (size_t)b * BB;
+        // (a row past the end: the last one again, not stored; gate and up: a round's rows 4 .. 7 are up's)
+        const int r = min(M::GLU ? r0 + 4 * j + ((lane >> 3) & 3) : r0 + 8 * j + (lane >> 3), rows - 1);
+        const uint8_t *base = W;
+        if constexpr (M::GLU) base = lane & 32 ? matrices.up : W;
+        const uint8_t *blk = base + (size_t)r * row_stride + (size_t)b * BB;
         const uint8_t *qs = blk + (BB - 128) + 32 * q;
         asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(wh[j]) : "v"(blk) : "memory");
         if constexpr (Q5) {
@@ -850,10 +853,18 @@ __global__ __launch_bounds__(1024) void gemv_q4_k_cols_kernel(M matrices, size_t
         if (ul == 0) parts[wave * (8 * U) + 8 * j + (lane >> 3)] = sums[j];
     lds_barrier();
     // a row's partial sums, in the order of the columns
-    if ((int)threadIdx.x < 8 * U && r0 + (int)threadIdx.x < rows) {
+    const int at = (int)threadIdx.x;
+    if constexpr (M::GLU) {
+        if (at < 4 * U && r0 + at < rows) {
+            const float *p = parts + (at >> 2) * 8 + (at & 3);
+            float g = 0.0f, u = 0.0f;
+            for (int w = 0; w < waves; w++) g += p[w * (8 * U)], u += p[w * (8 * U) + 4];
+            y[r0 + at] = silu_as_host(g) * u;
+        }
+    } else if (at < 8 * U && r0 + at < rows) {
         float v = 0.0f;
-        for (int w = 0; w < waves; w++) v += parts[w * (8 * U) + threadIdx.x];
-        y[r0 + threadIdx.x] = v;
+        for (int w = 0; w < waves; w++) v += parts[w * (8 * U) + at];
+        y[r0 + at] = v;
     }
 }
 
@@ -1064,8 +1075,8 @@ int launch_gemv_rows_preq(const frk_weights *w, Q8KActs a, float *y, hipStream_t
 //   5120x5120 7.8 / 5.9 / 6.9    6144x6144 8.7 / 8.8 / 9.0    8192x3072 5.5 / 5.2 / 6.7    3072x3072 3.7 / 4.6 / 5.9
 //   2560x2560 3.4 / 4.5 / 5.8
 // Rows of 8, 16 and 32 blocks have the whole-cache-line kernel (14336x4096: 8.2 / 8.9 / 10.3).
-// n <= 4 matrices of one kind and row length
-static int launch_cols_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {
+// n <= 4 matrices of one kind and row length, or (glu, Q5_K only) gate and up with ys[0] = silu(gate x) * (up x)
+static int launch_cols_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s, bool glu = false) {
     const frk_weights *const w = ws[0];
     const int nb = (int)(w->cols / QK_K), waves = (nb + 3) / 4;
     const int cus = compute_units();
@@ -1075,12 +1086,19 @@ static int launch_cols_group(const frk_weights *const *ws, size_t n, const float
     // of the activation, about seven rows' worth), the larger of equals
     const bool q5 = w->kind == FRK_KIND_Q5_K;
     for (int u = 1; u <= (q5 ? 2 : 3); u++) {
-        const size_t wgs = gemv_workgroups(ws, n, 8 * u);
+        const size_t wgs = glu ? gemv_workgroups(ws, 1, 4 * u) : gemv_workgroups(ws, n, 8 * u);
         const size_t cost = (wgs + cus - 1) / cus * (8 * u + 7);
         if (cost <= best) best = cost, best_u = u;
     }
     const size_t lds = (size_t)waves * (COLS_WAVE_LDS + 8 * best_u * 4);
-    const dim3 grid((unsigned)gemv_workgroups(ws, n, 8 * best_u)), block(64 * waves);
+    const dim3 grid((unsigned)(glu ? gemv_workgroups(ws, 1, 4 * best_u) : gemv_workgroups(ws, n, 8 * best_u))), block(64 * waves);
+    if (glu) {
+        const GemvGlu pair{w->dev, ws[1]->dev, ys[0], (int)w->rows};
+        if (best_u == 1) hipLaunchKernelGGL((gemv_q4_k_cols_kernel<1, true, GemvGlu>), grid, block, lds, s, pair, w->layout.row_stride, nb, x);
+        else hipLaunchKernelGGL((gemv_q4_k_cols_kernel<2, true, GemvGlu>), grid, block, lds, s, pair, w->layout.row_stride, nb, x);
+        FRK_LAUNCH_CHECK("gemv_q5_k_glu");
+        return FRK_OK;
+    }
     const GemvOne one{w->dev, ys[0], (int)w->rows};
     const GemvGroup group = gemv_group(ws, n, ys, 8 * best_u);
 #define FRK_GO_COLS(UU)                                                                                                                    \
@@ -1186,6 +1204,11 @@ int launch_gemv_q5_k_group(const frk_weights *const *ws, size_t n, const float *
     const Q8KActs none{nullptr, nullptr, nullptr};
     if (nb == 8) return launch_q4_k_lines_as<8, MODE_FUSED, 4, true, 0, true>(ws[0], x, none, ys[0], s, total, &ma);
     return launch_q4_k_lines_as<16, MODE_FUSED, 4, true, 0, true>(ws[0], x, none, ys[0], s, total, &ma);
+}
+// act = silu(gate x) * (up x): one shape, rows_gemv_fits
+int launch_gemv_q5_k_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s) {
+    const frk_weights *const ws[2] = {gate, up};
+    return launch_cols_group(ws, 2, x, &act, s, true);
 }
 // ys[i] = ws[i] . x for 2..4 Q4_K matrices of one row length (fused_gemv_fits), one launch
 int launch_gemv_q4_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s) {

@@ -201,6 +201,11 @@ int launch_gemv_q4_k_group(const frk_weights *const *ws, size_t n, const float *
 int launch_gemv_q5_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s);
 int launch_gemv_q6_k_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s);
 int launch_gemv_q8_0_f32_group(const frk_weights *const *ws, size_t n, const float *x, float *const *ys, hipStream_t s);
+// gate and up of one shape in one launch, act = silu(gate x) * (up x): Q5_K where rows_gemv_fits, Q6_K where q6_k_cols_form, Q8_0 where
+// q8_0_cols_form
+int launch_gemv_q5_k_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s);
+int launch_gemv_q6_k_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s);
+int launch_gemv_q8_0_f32_glu(const frk_weights *gate, const frk_weights *up, const float *x, float *act, hipStream_t s);
 bool q8_0_cols_form(const frk_weights *w);
 int launch_gemv_q4_k_experts(const frk_weights *w, const frk_weights *w2, int n_experts, size_t rows_e, const float *x,
                              size_t x_stride, const int32_t *ids, size_t jobs, size_t per_job, float *y, hipStream_t s);

@@ -1209,6 +1209,17 @@ int frk_hip_ffn_swiglu_dev(const frk_weights *gate, const frk_weights *up, const
         // gate, up and SwiGLU in one launch: row r of both matrices is computed by the same lanes
         rc = launch_gemv_q4_k_glu(gate, up, x, act, s);
         if (rc) return rc;
+    } else if (gate->kind == FRK_KIND_Q5_K && up->kind == FRK_KIND_Q5_K && rows_gemv_fits(gate)) {
+        // the column forms' gate and up: ahead of a group and a SwiGLU launch at every length (0.92 over 44 shapes; Q5_K rows of 8
+        // and 16 blocks too, whose group has the whole-cache-line kernel)
+        rc = launch_gemv_q5_k_glu(gate, up, x, act, s);
+        if (rc) return rc;
+    } else if (up->kind == FRK_KIND_Q6_K && q6_k_cols_form(gate)) {
+        rc = launch_gemv_q6_k_glu(gate, up, x, act, s);
+        if (rc) return rc;
+    } else if (up->kind == FRK_KIND_Q8_0 && q8_0_cols_form(gate)) {
+        rc = launch_gemv_q8_0_f32_glu(gate, up, x, act, s);
+        if (rc) return rc;
     } else {
         const frk_weights *pair[2] = {gate, up};
         float *outs[2] = {g_out, u_out};

@@ -61,3 +61,33 @@ def test_neighbours_of_a_kind_in_a_mixed_list(fa):
         assert_rows_close(y.cpu().numpy()[None], fo.gemv(k, d, 24 + i, cols, x, fo.F32_DOT if k == fo.Q8_0 else fo.INT_DOT)[None], "mixed, matrix %d" % i)
     for w in ws:
         w.release()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [fo.Q5_K, fo.Q6_K, fo.Q8_0])
+@pytest.mark.parametrize("blocks,ffn", [(2, 32), (4, 96), (5, 1568), (8, 2080), (9, 64), (15, 224), (16, 160), (17, 4128), (20, 32), (24, 2816), (28, 1120), (32, 96),
+                                        (40, 672), (63, 64), (64, 3104), (66, 32)])
+def test_gate_up_and_swiglu_in_one_launch(fa, kind, blocks, ffn):
+    """frk_hip_ffn_swiglu_dev's gate and up against the two matrices' own GEMVs and the oracle's SwiGLU; the down projection is a
+    Q8_0 diagonal, so that the result shows every intermediate (127 f16(1/127) times it, rounded twice)."""
+    from frink_amd import synth
+    print("glu", kind, blocks, ffn, flush=True)
+    cols = 256 * blocks
+    data = [make_weights(kind, ffn, cols, seed=11 * blocks + ffn + i) for i in range(2)]
+    x = synth.activations(cols + ffn, 1, cols, outlier_frac=0.01)[0]
+    scale = np.float16(1.0 / 127)
+    diagonal = np.zeros((ffn, ffn // 32, 34), np.uint8)
+    diagonal[:, :, :2] = np.frombuffer(scale.tobytes(), np.uint8)
+    for i in range(ffn):
+        diagonal[i, i // 32, 2 + i % 32] = 127
+    wg, wu = (fa.Weights.from_host(kind, d, ffn, cols) for d in data)
+    wd = fa.Weights.from_host(fo.Q8_0, diagonal.reshape(ffn, -1), ffn, ffn)
+    got = fa.ffn_swiglu(wg, wu, wd, to_dev(x)).cpu().numpy()
+    g, u = (w.gemv(to_dev(x)).cpu().numpy() for w in (wg, wu))
+    want = fo.swiglu(g, u) * np.float32(127) * np.float32(scale)
+    if kind == fo.Q5_K:  # (rows of 8 and 16 blocks alone: the whole-cache-line kernel, whose sums go in another order)
+        assert_rows_close(got[None], want[None], "glu kind %d %dx%d" % (kind, ffn, cols))
+    else:
+        assert np.array_equal(bits(got), bits(want))
+    for w in (wg, wu, wd):
+        w.release()
