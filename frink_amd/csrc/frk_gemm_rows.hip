@@ -1,4 +1,5 @@
-// Batches of 2 to 32 rows of the K-quants on the matrix cores (batched decoding): y[tok][row] is dot_q{4,5,6}_k_q8's
+// Batches of 2 to 32 rows of the K-quants on the matrix cores (batched decoding), and larger ones of small matrices, every 32 tokens by
+// workgroups of their own (blockIdx.y): y[tok][row] is dot_q{4,5,6}_k_q8's
 // (crates/frink-quant/src/lib.rs:822-869, 886-938, 1069-1110), the integers exact, the float step the thin kernels'.
 //
 // A workgroup is sixteen weight rows, its wavefronts shares of the columns.  A wavefront streams its share two blocks at a
@@ -269,14 +270,17 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) __attribute__((amdgpu_waves_per_eu
     const uint32_t slot_lds = lds_address(rows_lds) + (uint32_t)wave * Side::SLOT;
     const uint8_t *const first = g.W + (size_t)row0 * g.row_stride;
     const Side side(g, lane, min(g.rows - 1 - row0, 15));
-    auto buffer = [&](const void *tile, const void *rows, int bytes) {  // (bytes a block of a token)
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(PLAIN ? rows : tile), 0, (PLAIN ? g.M : 32) * g.nb * bytes, 0x00027000);
+    const int tile = (int)blockIdx.y, M = min(g.M - 32 * tile, 32);
+    const size_t tile_at = (size_t)tile * 32 * g.nb;
+    auto buffer = [&](const void *tiles, const void *rows, int bytes) {  // (bytes a block of a token)
+        const uint8_t *const at = PLAIN ? (const uint8_t *)rows : (const uint8_t *)tiles + tile_at * bytes;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(at), 0, (PLAIN ? M : 32) * g.nb * bytes, 0x00027000);
     };
-    const RowsActs<PLAIN> acts = {buffer(g.a.q, g.plain.q, 256), buffer(g.a.bs, g.plain.bsums, 32), buffer(g.a.d, g.plain.d, 4), g.nb, g.M};
+    const RowsActs<PLAIN> acts = {buffer(g.a.q, g.plain.q, 256), buffer(g.a.bs, g.plain.bsums, 32), buffer(g.a.d, g.plain.d, 4), g.nb, M};
     typename Side::Acts A[TT];
     auto load_acts = [&](int kb) {  // (tokens past the batch repeat the last one)
 #pragma unroll
-        for (int t = 0; t < TT; t++) Side::load_acts(A[t], acts, kb, t, min(16 * t + lr, g.M - 1), lq);
+        for (int t = 0; t < TT; t++) Side::load_acts(A[t], acts, kb, t, min(16 * t + lr, M - 1), lq);
     };
     v4f acc[TT];
 #pragma unroll
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int t = 0; t < TT; t++) *reinterpret_cast<v4f *>(slot + t * 1024 + lane * 16) = acc[t];
     __syncthreads();
-    for (int i = threadIdx.x; i < 16 * g.M; i += 64 * waves) {
+    for (int i = threadIdx.x; i < 16 * M; i += 64 * waves) {
         const int tok = i >> 4, r = i & 15;
         const uint32_t at = (uint32_t)((tok >> 4) * 1024 + ((tok >> 2 & 3) * 16 + r) * 16 + (tok & 3) * 4);
         float v[ROWS_WAVES];
@@ -319,12 +323,12 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) __attribute__((amdgpu_waves_per_eu
             v[w] = w < waves ? one : 0.0f;
         }
         const float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-        if (row0 + r < g.rows) g.y[(size_t)tok * g.rows + row0 + r] = sum;
+        if (row0 + r < g.rows) g.y[(size_t)(32 * tile + tok) * g.rows + row0 + r] = sum;
     }
 #endif
 }
 
-// One tile of up to 32 rows in the tiled form, straight from the lanes: a wavefront a (row, block), no LDS, no barrier, rows past the
+// Tiles of 32 rows in the tiled form, straight from the lanes: a wavefront a (row, block), no LDS, no barrier, the last tile's rows past the
 // batch left as they are (gemm_k_rows_kernel does not use them).  A workgroup a block, which puts its rows together in LDS and clears
 // the tile's others (quantize_q8_k_tiled_kernel), takes 3.6 us at 16 x 4096 where this takes 2.4; the batches of 2 .. 32 rows that
 // have it as their first launch, 0.95 of the time.  `plain`: the same quants as plain rows too.
@@ -337,9 +341,11 @@ __global__ __launch_bounds__(256) void quantize_q8_k_one_tile_kernel(const float
     int sum;  // of the 16-wide group
     const uint32_t packed = quantize_q8_k_lane(v, d, sum);
     // slice lane / 8, 16-byte half lane / 4 % 2; the sum of group lane / 4
-    reinterpret_cast<uint32_t *>(out.q + (size_t)kb * 8192)[(lane >> 3) * 256 + ((lane >> 2 & 1) * 32 + row) * 4 + (lane & 3)] = packed;
-    if ((lane & 3) == 0) out.bs[(size_t)kb * 512 + ((lane >> 5) * 32 + row) * 8 + (lane >> 2 & 7)] = (_Float16)sum;
-    if (lane == 0) out.d[(size_t)kb * 32 + row] = d;
+    const size_t rec = (size_t)(row >> 5) * nb + kb;
+    const int at32 = row & 31;
+    reinterpret_cast<uint32_t *>(out.q + rec * 8192)[(lane >> 3) * 256 + ((lane >> 2 & 1) * 32 + at32) * 4 + (lane & 3)] = packed;
+    if ((lane & 3) == 0) out.bs[rec * 512 + ((lane >> 5) * 32 + at32) * 8 + (lane >> 2 & 7)] = (_Float16)sum;
+    if (lane == 0) out.d[rec * 32 + at32] = d;
     if (!plain.q) return;
     reinterpret_cast<uint32_t *>(plain.q + (size_t)at * QK_K)[lane] = packed;
     if ((lane & 3) == 0) plain.bsums[(size_t)at * 16 + (lane >> 2)] = (int16_t)sum;
@@ -353,7 +359,7 @@ int launch_quantize_q8_k_one_tile(const float *x, size_t rows, size_t cols, Q8KT
     return FRK_OK;
 }
 
-// 2 <= batch <= 32 from one tile of the tiled form (plain null) or from plain rows (up to 16 of Q4_K and Q5_K): the same bits.
+// batch >= 2 from the tiled form (plain null), or up to 32 from plain rows (16 of Q4_K and Q5_K): the same bits.
 int launch_gemm_k_rows(const frk_weights *w, int batch, Q8KTiled a, const Q8KActs *plain, float *y, hipStream_t s) {
     RowsArgs g;
     g.W = w->dev;
@@ -370,13 +376,14 @@ int launch_gemm_k_rows(const frk_weights *w, int batch, Q8KTiled a, const Q8KAct
     const int pairs = (g.nb + 1) / 2;
     g.each = (pairs + ROWS_WAVES - 1) / ROWS_WAVES;
     const int waves = (pairs + g.each - 1) / g.each;
-    const dim3 grid((unsigned)((w->rows + 15) / 16)), block(64 * waves);
+    const dim3 grid((unsigned)((w->rows + 15) / 16), (unsigned)((batch + 31) / 32)), block(64 * waves);
 #define FRK_GO(KIND, TT, PLAIN) \
     hipLaunchKernelGGL((gemm_k_rows_kernel<KIND, TT, PLAIN>), grid, block, waves * RowsSide<KIND>::SLOT, s, g)
 #define FRK_GO_KIND(KIND)                         \
     if (plain) FRK_GO(KIND, 1, true);             \
     else if (batch <= 16) FRK_GO(KIND, 1, false); \
     else FRK_GO(KIND, 2, false)
+    if (plain && batch > 32) return set_error(FRK_ERR_UNSUPPORTED, "more than 32 plain rows");
     if (w->kind == FRK_KIND_Q6_K) {
         if (plain && batch > 16) FRK_GO(FRK_KIND_Q6_K, 2, true);
         else FRK_GO_KIND(FRK_KIND_Q6_K);

@@ -251,9 +251,9 @@ constexpr size_t SPLIT_PARTS_BYTES = (size_t)FRK_NOALLOC_PARTS_MIB << 20;
 // batched GEMM of the K-quants on the int8 matrix cores, over activations quantized into the tiled form; `parts` holds
 // pipe_gemm_parts_bytes(...) of the parts' sums where the blocks are split between workgroups (0: they are not)
 size_t pipe_gemm_parts_bytes(int kind, size_t M, size_t cols, size_t rows);
-// up to 32 rows as one tile, whose other rows are left as they are (for launch_gemm_k_rows)
+// the last tile's other rows left as they are (for launch_gemm_k_rows)
 int launch_quantize_q8_k_one_tile(const float *x, size_t rows, size_t cols, Q8KTiled out, hipStream_t s, Q8KActsOut plain = Q8KActsOut());
-// batches of 2 .. 32 rows from the tiled form, or (up to 16 of Q4_K and Q5_K) from plain rows
+// a batch from the tiled form, or (up to 32 rows, 16 of Q4_K and Q5_K) from plain rows
 int launch_gemm_k_rows(const frk_weights *w, int batch, Q8KTiled a, const Q8KActs *plain, float *y, hipStream_t s);
 int launch_pipe_gemm_acts(const frk_weights *w, Q8KTiled acts, size_t M, float *y, void *parts, hipStream_t s);
 // y[n] = partial[0][n] + partial[1][n] + ..., always in the same pairs (the split GEMMs' second step; frk_gemm_q6.hip)

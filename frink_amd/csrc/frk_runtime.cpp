@@ -691,7 +691,7 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
     return batch >= std::max(from, tiled_from(w->cols));
 }
 // Whether gemm_k_rows_kernel takes a batch (frk_gemm_rows.hip: sixteen rows a workgroup, no split, no second launch), ahead of both the
-// thin kernels and the 64 x 32 tiles of the pipelined GEMM.  It reads all tokens' tiles once for every sixteen rows, so what
+// thin kernels and the pipelined GEMM.  It reads all tokens' tiles once for every sixteen rows, so what
 // is against it is many rows times many tokens (from 17 on twice the bytes) and rows so few and long that its workgroups'
 // chains are the launch.  nb blocks a row, with quantization, us before / now:
 //   Q4_K  two rows of short blocks (4 .. 19 blocks 0.92 of the time; past 33 blocks 1.01 and more).  Up to 8 not the span kernel's rows of 4,
@@ -707,9 +707,21 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 // better of both everywhere would be 0.2 % less), 1.1 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
 // From activations quantized beforehand (frk_hip_gemm_q8k_dev, which has tiles to make, and frk_hip_gemm_acts_dev) 0.84 and 0.75, gemm_pair
 // 0.73.
+//   33 to 512 rows of small matrices, every 32 tokens by workgroups of their own, where the pipelined GEMM takes 15 us and more however little there
+//         is to do: Q5_K 2146x3328 at 70 16.5 / 10.2, Q6_K 3856x3584 at 52 17.2 / 9.9, Q4_K 1101x2048 at 103 12.6 / 7.7; past the
+//         line Q4_K 4704x9984 at 53 21.2 / 29.4, Q6_K 3459x5632 at 99 22.3 / 29.2.  A few hundred rows of many blocks are few workgroups
+//         for their chains (Q5_K 513x11520 at 226 23.5 / 28.2).  Over 700 drawn sizes with up to 420000 blocks times tiles 0.77 of the time
+//         (the better of both everywhere would be 0.5 % less), 1.09 at worst; the 2-norm error against 64 bits of 60 that changed 0.98, 1.04 at most.
 static bool k_rows_take(const frk_weights *w, size_t batch) {
     const size_t rows = w->rows, nb = w->cols / QK_K;
-    if (batch < 2 || batch > 32 || nb > 128) return false;
+    if (batch < 2 || batch > 512 || nb > 128) return false;
+    if (batch > 32) {
+        const size_t work = (batch + 31) / 32 * rows * nb;  // blocks times tiles of 32 tokens
+        if (w->kind == FRK_KIND_Q4_K) return work <= (nb >= 36 || (nb >= 28 && rows < 1100) ? 130000 : 190000);
+        if (w->kind != FRK_KIND_Q5_K && w->kind != FRK_KIND_Q6_K) return false;
+        if (nb >= 28 && rows < 1100) return work <= 130000;
+        return work <= (nb <= 16 && rows < 4096 ? 320000 : w->kind == FRK_KIND_Q5_K && nb >= 36 ? 190000 : 230000);
+    }
     const bool one_round = rows > 2048 && rows <= 4096, few = rows < 1024;
     if (w->kind == FRK_KIND_Q4_K) {
         if (batch == 2) return nb < 20 && rows <= 8192;

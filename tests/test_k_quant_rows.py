@@ -1,4 +1,4 @@
-"""K-quant batches of 2 to 32 rows on sixteen-row workgroups (gemm_k_rows_kernel, frk_gemm_rows.hip): rows that fill no
+"""K-quant batches of 2 to 32 rows, and more of small matrices, on sixteen-row workgroups (gemm_k_rows_kernel, frk_gemm_rows.hip): rows that fill no
 workgroup, odd numbers of blocks and of pairs a wavefront, one and two tiles of tokens; every entry point the same bits."""
 import numpy as np
 import pytest
@@ -18,6 +18,18 @@ SHAPES = [(fo.Q4_K, 15, 2304, 3), (fo.Q4_K, 17, 256, 16), (fo.Q4_K, 33, 1280, 17
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,rows,cols,batch", SHAPES)
 def test_batches_match_exact_arithmetic(fa, kind, rows, cols, batch):
+    _check(fa, kind, rows, cols, batch)
+
+
+# (several tiles of tokens: one and sixteen rows of the last, whole ones; both sides of the line to the pipelined GEMM)
+TILES = [(fo.Q4_K, 17, 256, 33), (fo.Q4_K, 1101, 2048, 103), (fo.Q4_K, 47, 9216, 64), (fo.Q4_K, 1319, 9216, 63), (fo.Q4_K, 1318, 9216, 128), (fo.Q5_K, 15, 1280, 48),
+         (fo.Q5_K, 1782, 3072, 65), (fo.Q5_K, 33, 17152, 40), (fo.Q5_K, 4100, 512, 81), (fo.Q6_K, 1, 768, 34), (fo.Q6_K, 600, 3584, 511), (fo.Q6_K, 601, 3584, 512),
+         (fo.Q6_K, 31, 8448, 96)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,cols,batch", TILES)
+def test_several_tiles_match_exact_arithmetic(fa, kind, rows, cols, batch):
     _check(fa, kind, rows, cols, batch)
 
 
@@ -52,3 +64,30 @@ def test_compiled_kernels_keep_the_waits(tmp_path):
     assert sum("gemm_k_rows" in k for k in names) == 10 and len(names) == 11, names  # (and the batch's quantizer)
     for k in names:
         assert isa_wait_lint.violations(asm, k) == [], k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,cols,batch", [TILES[i] for i in (0, 1, 6, 7, 12)])
+def test_every_entry_point_has_the_same_bits_over_several_tiles(fa, kind, rows, cols, batch):
+    import torch
+    from frink_amd import synth
+    print("k-quant rows, tiles", kind, rows, cols, batch, flush=True)
+    w = fa.Weights.from_host(kind, make_weights(kind, rows, cols, seed=rows), rows, cols)
+    x = to_dev(synth.activations(batch, batch, cols))
+    room = torch.full((batch * rows + 128,), 7.0, device="cuda")
+    y = room[64:-64].view(batch, rows)
+    w.gemm(x, out=y)
+    want = bits(y.cpu().numpy())
+    assert (room[:64] == 7.0).all() and (room[-64:] == 7.0).all()
+    acts = fa.BatchActs(batch, cols)
+    acts.quantize(x)
+    assert np.array_equal(bits(w.gemm_acts(acts).cpu().numpy()), want)
+    for y in fa.gemm_pair(w, w, x):
+        assert np.array_equal(bits(y.cpu().numpy()), want)
+    y = torch.full((batch, rows), float("nan"), device="cuda")
+    w.gemm_noalloc(x, y)
+    assert np.array_equal(bits(y.cpu().numpy()), want)
+    for t in range(0, batch, 32):  # (a tile of its own: the tokens of a batch of 2 to 32 where those are this kernel's too)
+        if min(batch - t, 32) > 1 and rows <= 2048 and cols < 19 * 256:
+            assert np.array_equal(bits(w.gemm(x[t:t + 32].contiguous()).cpu().numpy()), want[t:t + 32])
+    w.release()
