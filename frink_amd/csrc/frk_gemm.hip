@@ -57,6 +57,30 @@ __global__ __launch_bounds__(64 * WAVES) void quantize_q8_k_tiled_kernel(const f
     });
 }
 
+// The same without `gather`, straight from the lanes: a wavefront a (row, block), no LDS, no barrier.  A workgroup is eight rows of a block, whose
+// sixteen-byte pieces and sums are whole lines of 128 bytes (with four blocks of one row a workgroup, lines are put together from
+// eight CUs' stores: 512 x 14336 11.7 us where this takes 8.9).
+__global__ __launch_bounds__(512) void quantize_q8_k_octets_kernel(const float *__restrict__ x, int rows, int nb, Q8KTiled out, Q8KActsOut plain) {
+    const int lane = threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    const int octet = (int)blockIdx.x / nb, kb = (int)blockIdx.x - octet * nb, row = octet * 8 + wave;
+    const size_t at = (size_t)row * nb + kb;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row < rows) v = reinterpret_cast<const float4 *>(x + at * QK_K)[lane];
+    float d;
+    int sum;  // of the 16-wide group
+    const uint32_t packed = quantize_q8_k_lane(v, d, sum);
+    // slice lane / 8, 16-byte half lane / 4 % 2; the sum of group lane / 4
+    const size_t rec = (size_t)(row >> 5) * nb + kb;
+    const int at32 = row & 31;
+    reinterpret_cast<uint32_t *>(out.q + rec * 8192)[(lane >> 3) * 256 + ((lane >> 2 & 1) * 32 + at32) * 4 + (lane & 3)] = packed;
+    if ((lane & 3) == 0) out.bs[rec * 512 + ((lane >> 5) * 32 + at32) * 8 + (lane >> 2 & 7)] = (_Float16)sum;
+    if (lane == 0) out.d[rec * 32 + at32] = d;
+    if (!plain.q || row >= rows) return;
+    reinterpret_cast<uint32_t *>(plain.q + at * QK_K)[lane] = packed;
+    if ((lane & 3) == 0) plain.bsums[at * 16 + (lane >> 2)] = (int16_t)sum;
+    if (lane == 0) plain.d[at] = d;
+}
+
 // The grouped form: work items (tile, matrix, row group of 256 rows) streamed by persistent workgroups.
 struct StreamArgs {
     const uint8_t *W[2];
@@ -546,6 +570,15 @@ static int launch_quantize_records(const float *x, size_t rows, size_t nb, const
 int launch_quantize_q8_k_tiled(const float *x, size_t rows, size_t cols, Q8KTiled out, hipStream_t s, Q8KActsOut plain) {
     const size_t nb = cols / QK_K, n_rec = (rows + 31) / 32 * nb;
     if (n_rec == 0) return FRK_OK;
+    // Up to 400 records without LDS: a launch of 2.5 to 5 us is its chain of dependent steps, and a record's barrier and copies are the longer one;
+    // past that both are bound by the stores, which a record's are the wider of.  us, launch after launch, a record / eight rows a workgroup: 48 x 4096
+    // 3.08 / 2.49, 64 x 8192 3.12 / 2.41, 197 x 4096 3.22 / 2.54, 200 x 14336 5.27 / 4.92, 512 x 4096 3.75 / 3.72, but 512 x 14336
+    // 8.79 / 8.92, 2000 x 8192 16.7 / 19.4, 2048 x 14336 28.5 / 33.6.
+    if (n_rec <= 400) {
+        hipLaunchKernelGGL(quantize_q8_k_octets_kernel, dim3((unsigned)(n_rec * 4)), dim3(512), 0, s, x, (int)rows, (int)nb, out, plain);
+        FRK_LAUNCH_CHECK("quantize_q8_k_octets");
+        return FRK_OK;
+    }
     // (sixteen wavefronts a record, two rows each, at every size, us under the profiler, sixteen / eight / four: 512x4096 5.9 / 7.1 /
     // 10.2, 512x14336 10.4 / 12.0 / 14.0, 700x12288 10.6 / 12.0 / 13.5, 2000x8192 16.8 / 18.6 / 22.0)
     return launch_quantize_records<16>(x, rows, nb, nullptr, n_rec, out, s, plain);

@@ -91,3 +91,32 @@ def test_every_entry_point_has_the_same_bits_over_several_tiles(fa, kind, rows, 
         if min(batch - t, 32) > 1 and rows <= 2048 and cols < 19 * 256:
             assert np.array_equal(bits(w.gemm(x[t:t + 32].contiguous()).cpu().numpy()), want[t:t + 32])
     w.release()
+
+
+# (the pipelined GEMM's batches whose tiles come from the same quantizer, rows past the batch cleared: one row of an octet and all of it, and both
+# sides of the 400 records from where a record is a workgroup's)
+CLEARED = [(fo.Q4_K, 2000, 9216, 33), (fo.Q4_K, 2000, 9216, 40), (fo.Q5_K, 3000, 9216, 41), (fo.Q6_K, 3300, 9216, 63), (fo.Q4_K, 400, 9216, 352),
+           (fo.Q4_K, 400, 9216, 353)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,cols,batch", CLEARED)
+def test_pipelined_batches_from_the_lanes_match_exact_arithmetic(fa, kind, rows, cols, batch):
+    _check(fa, kind, rows, cols, batch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,cols,batch", CLEARED)
+def test_rows_of_an_earlier_batch_leave_the_tiles(fa, kind, rows, cols, batch):
+    from frink_amd import synth
+    print("octets after a larger batch", kind, rows, cols, batch, flush=True)
+    w = fa.Weights.from_host(kind, make_weights(kind, rows, cols, seed=rows), rows, cols)
+    x = to_dev(synth.activations(batch, batch, cols))
+    want = bits(w.gemm(x).cpu().numpy())
+    acts = fa.BatchActs(batch + 31, cols)
+    large = to_dev(synth.activations(batch, batch + 31, cols))
+    large[batch:] = float("inf")  # (scales that are not finite in the rows that the next batch does not have)
+    acts.quantize(large)
+    acts.quantize(x)
+    assert np.array_equal(bits(w.gemm_acts(acts).cpu().numpy()), want)
+    w.release()
