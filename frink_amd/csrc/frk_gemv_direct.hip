@@ -668,7 +668,7 @@ static int launch_q6_k_group(const frk_weights *const *ws, size_t n, const float
         const dim3 grid((unsigned)(glu ? gemv_workgroups(ws, 1, 2 * best_u) : gemv_workgroups(ws, n, 4 * best_u))), block(64 * waves);
         const GemvGlu pair{w->dev, ws[n - 1]->dev, ys[0], (int)w->rows};
         const GemvOne one{w->dev, ys[0], (int)w->rows};
-        const GemvGroup group = gemv_group(ws, n, ys, 4 * best_u);
+        const GemvGroup group = glu ? GemvGroup{} : gemv_group(ws, n, ys, 4 * best_u);  // (gate and up have one output)
         const bool whole_lines = w->layout.row_stride % 128 == 0 && nb % 4 == 0;  // (every wavefront's four blocks of ql: 512 bytes)
 #define FRK_GO_COLS(UU)                                                                                                              \
     if (glu && whole_lines) hipLaunchKernelGGL((gemv_q6_k_cols_kernel<UU, true, GemvGlu>), grid, block, lds, s, pair, w->layout, nb, x);        \
