@@ -86,7 +86,8 @@ template <int S>
 __global__ __launch_bounds__(512, 4) void mx_experts_gate_up_kernel(MxeGateUpArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ uint4 sq[2 * MXE_MAX_UNITS];
-    __shared__ float sd[MXE_MAX_UNITS], gates[32], ups[32];
+    __shared__ __align__(16) float gates[32];  // (read as float4 too)
+    __shared__ float sd[MXE_MAX_UNITS], ups[32];
     __shared__ uint64_t table[32];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l = lane % MXE_LANES, part = lane / MXE_LANES;
     const int pair = blockIdx.y, id = g.ids[pair];
