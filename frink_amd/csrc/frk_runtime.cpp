@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "frk_internal.hpp"
+#include "frk_stage.hpp"
 
 namespace frk {
 
@@ -37,7 +38,7 @@ struct DeviceState {
     void *x_dev = nullptr, *y_dev = nullptr;
     size_t x_bytes = 0, y_bytes = 0;
     char *pinned = nullptr;  // page-locked: STAGE_MAX bytes of inputs, as many of results, a flag for each of their chunks
-    uint32_t epoch = 0;
+    uint32_t epoch = 0;      // the last call's number in the flags (next_epoch)
     std::map<std::pair<const void *, size_t>, frk_weights *> cache;
 };
 static DeviceState g_dev;
@@ -1418,7 +1419,7 @@ static int stage_out(int rc, const HostOut *outs, size_t n) {
     }
     const char *y = pinned + STAGE_MAX;
     uint32_t *flags = (uint32_t *)(pinned + 2 * STAGE_MAX);
-    const uint32_t epoch = ++g_dev.epoch;
+    const uint32_t epoch = g_dev.epoch = next_epoch(g_dev.epoch, flags, STAGE_MAX / STAGE_CHUNK);
     rc = launch_stage_out(g_dev.y_dev, pinned + STAGE_MAX, flags, epoch, total, s);
     if (rc) {
         (void)hipStreamSynchronize(s);
