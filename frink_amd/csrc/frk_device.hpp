@@ -258,8 +258,8 @@ __device__ __forceinline__ uint32_t quantize_q8_k_lane(float4 v, float &d_out, i
 // -- quantizing straight into the tiled form would write it in 4-byte pieces.  These kernels are
 // bound by latency: few records want many wavefronts each, many records small workgroups.
 struct Q8KRecordLds {
-    uint32_t q[2048];
-    _Float16 bs[512];
+    alignas(16) uint32_t q[2048];
+    alignas(16) _Float16 bs[512];
     float d[32];
 };
 // (`keep(r, quants, d, sum)` sees a lane's four values of row r as well, `sum` in every fourth lane)

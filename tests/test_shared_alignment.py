@@ -30,6 +30,16 @@ def test_vector_accesses_of_shared_arrays(path):
     assert misaligned(open(path).read()) == []
 
 
+def test_vector_accesses_of_the_quantizers_record():
+    """Q8KRecordLds, a shared structure: the members that its users read as wider vectors."""
+    text = open(os.path.join(fb.CSRC, "frk_device.hpp")).read()
+    members = re.findall(r"(?:alignas\((\d+)\) )?(\w+) (\w+)\[\d+\];", re.search(r"struct Q8KRecordLds \{(.*?)\};", text, re.S).group(1))
+    aligned = {name: max(int(align or 1), SIZES[kind]) for align, kind, name in members}
+    read = re.findall(r"reinterpret_cast<const (\w+) \*>\(L\.(\w+)\)", text)
+    assert len(aligned) == 3 and read
+    assert [(name, aligned[name], kind) for kind, name in read if SIZES[kind] > aligned[name]] == []
+
+
 def test_the_check_sees_a_float_array_read_as_float4():
     kernel = "__shared__ %sfloat a[3], b[32], c[8];\n f = reinterpret_cast<const float4 *>(b)[t];"
     assert misaligned(kernel % "") == [("b", 4, "float4")]
