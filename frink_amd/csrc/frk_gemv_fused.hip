@@ -1119,6 +1119,9 @@ static int launch_cols_group(const frk_weights *const *ws, size_t n, const float
 }
 int launch_gemv_q4_k_cols(const frk_weights *w, const float *x, float *y, hipStream_t s) { return launch_cols_group(&w, 1, x, &y, s); }
 
+// The whole-rows kernel's workgroups of 8 x 3 rows (17 to 21 blocks) in one round of 256 CUs, where the column form's of sixteen are more than
+// a round and those of 24 take longer.
+static bool threes_fill_the_chip(size_t rows) { return rows > 4096 && rows <= 6144; }
 // Which kernel a one-launch GEMV of Q4_K / Q5_K rows of other lengths than 8 and 16 blocks takes.
 int rows_gemv_form(const frk_weights *w) {
     if (!rows_gemv_fits(w)) return ROWS_FORM_NONE;
@@ -1133,20 +1136,23 @@ int rows_gemv_form(const frk_weights *w) {
         if (nb == 32 && (w->rows <= 2048 || w->rows >= 6144)) return ROWS_FORM_COLUMNS;
         // Shorter rows, weights from memory (not from the 256 MB cache): 9 to 12 blocks 1024x3072 3.6 -> 3.2, 4096x3072 4.5 -> 3.7, 7168x3072 6.1 ->
         // 5.8, 11008x2816 7.2 -> 6.8, but 14336x3072 7.6 / 8.4 (13 to 15: 0.86 to 1.18 of the time, but the experts' kernels have the other
-        // form's bits); 17 to 20 1024x5120 5.1 -> 4.1, 4096x5120 5.7 -> 5.5, 7168x5120 8.3 / 8.3,
-        // but 11008x5120 9.0 / 10.1.
+        // form's bits); 17 to 20 1024x5120 5.1 -> 4.1, 4096x5120 5.8 -> 5.3, 6285x4352 6.9 -> 6.2, 7168x5120 8.3 / 8.3,
+        // but 11008x5120 9.0 / 10.1; and 4284x5120 5.8 / 6.4 (threes_fill_the_chip).
         if (nb > 8 && nb <= 12 && w->rows < 12288) return ROWS_FORM_COLUMNS;
-        if (nb > 16 && nb <= 20 && w->rows <= 8192) return ROWS_FORM_COLUMNS;
+        if (nb > 16 && nb <= 20 && w->rows <= 8192 && !threes_fill_the_chip(w->rows)) return ROWS_FORM_COLUMNS;
     }
     // Q5_K on the same kernel (two rounds at most): 4096x14336 12.8 / 14.8, 4096x11008 10.4 / 13.7, 8192x10240 17.5 / 22.5,
     // 4096x16384 13.3 / 16.8, 2048x16384 8.3 / 9.1; at 32 blocks it is behind (4096x8192 8.3 / 7.3)
     if (w->kind == FRK_KIND_Q5_K && nb > 32) return ROWS_FORM_COLUMNS;
     // Shorter rows, weights from memory: 9 to 15 blocks against a quantization launch and a GEMV 1024x3072 6.5 -> 3.5, 4096x3072 7.5 -> 5.0,
-    // 14336x3072 11.3 -> 11.0; 17 to 20 1024x5120 5.7 -> 4.6, 4096x5120 6.6 -> 6.5, 7168x5120 11.1 -> 9.7, but 11008x5120 12.3 / 12.9; 21 to
-    // 31 1024x6144 6.0 -> 4.7, 11008x6144 17.7 -> 14.3, but 4096x6144 7.2 / 7.4.
-    if (w->kind == FRK_KIND_Q5_K && nb > 8 && nb < 16) return ROWS_FORM_COLUMNS;
-    if (w->kind == FRK_KIND_Q5_K && nb > 16 && nb <= 20 && w->rows <= 8192) return ROWS_FORM_COLUMNS;
-    if (w->kind == FRK_KIND_Q5_K && nb > 20 && nb < 32 && (w->rows <= 2048 || w->rows >= 6144)) return ROWS_FORM_COLUMNS;
+    // 14336x3072 11.3 -> 11.0, 36784x3072 22.0 -> 21.3, but 88059x3072 39.0 / 41.9, 58054x3840 31.3 / 33.7 (9 and 10 blocks at 140000 rows 0.83 and
+    // 0.93 of the time); 17 to 20 1024x5120 5.7 -> 4.6, 4096x5120 6.6 -> 6.5, 6285x4352 10.9 -> 9.1, 7168x5120 11.1 -> 9.7, but 11008x5120 12.3 / 12.9
+    // and 4439x5120 6.9 / 7.7; 21 to 31 1024x6144 6.0 -> 4.7, 11008x6144 17.7 -> 14.3, but 4096x6144 7.2 / 7.4, and of 21, three rows a wavefront of
+    // the other kernel still, 9980x5376 12.8 / 13.2, 17631x5376 19.1 / 21.0.
+    if (w->kind == FRK_KIND_Q5_K && nb > 8 && nb < 16 && (nb <= 10 || w->rows <= 40960)) return ROWS_FORM_COLUMNS;
+    if (w->kind == FRK_KIND_Q5_K && nb > 16 && nb <= 20 && w->rows <= 8192 && !threes_fill_the_chip(w->rows)) return ROWS_FORM_COLUMNS;
+    if (w->kind == FRK_KIND_Q5_K && nb > 20 && nb < 32 && (w->rows <= 2048 || w->rows > 6144) && !(nb == 21 && w->rows > 8192 && w->rows <= 18432))
+        return ROWS_FORM_COLUMNS;
     if (nb > 16 && nb < 32) return ROWS_FORM_ONE_LAUNCH;
     if (rows_gemv_takes_quantized(w)) return ROWS_FORM_QUANTIZED;
     return ROWS_FORM_NONE;

@@ -1,40 +1,17 @@
 """The decode launchers' host code under the address sanitizer, on the CPU: every kind, length and number of matrices that the
-grouped launches take, each with an array of outputs no longer than it has matrices.  The HIP runtime is a stub that counts launches
-(nothing reaches a device; the kernels' code is not compiled)."""
-import os
-import subprocess
+grouped launches take, each with an array of outputs no longer than it has matrices."""
+import host_library
 
-from frink_amd import build as fb
-
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-SOURCE = r"""
+DRIVER = r"""
 #include <cstdio>
-#include <vector>
 #include "frink_amd/csrc/frk_internal.hpp"
-static int launches;
-extern "C" {
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
-hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s) { *g = *b = dim3(1), *lds = 0, *s = nullptr; return hipSuccess; }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { launches++; return hipSuccess; }
-hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
-hipError_t hipGetDevice(int *dev) { *dev = 0; return hipSuccess; }
-hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
-const char *hipGetErrorString(hipError_t) { return ""; }
-void **__hipRegisterFatBinary(const void *) { static void *handle; return &handle; }
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *, int *) {}
-void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
-void __hipUnregisterFatBinary(void **) {}
-}
-namespace frk {
-int set_error(int code, const char *, ...) { return code; }
-}
 using namespace frk;
 static int failed, calls;
 static void took(int rc, const char *what, size_t nb, size_t rows, size_t n) {
     calls++;
-    if (rc != FRK_OK || launches != 1) printf("%s: %zu blocks, %zu rows, %zu matrices: status %d, %d launches\n", what, nb, rows, n, rc, launches), failed = 1;
-    launches = 0;
+    const size_t launches = HipStub::get().launched.size();
+    if (rc != FRK_OK || launches != 1) printf("%s: %zu blocks, %zu rows, %zu matrices: status %d, %zu launches\n", what, nb, rows, n, rc, launches), failed = 1;
+    HipStub::get().launched.clear();
 }
 int main() {
     const int kinds[] = {FRK_KIND_Q4_K, FRK_KIND_Q5_K, FRK_KIND_Q6_K, FRK_KIND_Q8_0};
@@ -75,16 +52,5 @@ int main() {
 
 
 def test_grouped_and_paired_launches_stay_inside_their_arrays(tmp_path):
-    # (unoptimized: a read past a parameter is otherwise undefined before the sanitizer sees it)
-    flags = ["-x", "hip", "--offload-arch=gfx950", "--offload-host-only", "-O0", "-g1", "-std=c++17", "-w", "-I", ROOT, "-Xarch_host", "-fsanitize=address"]
-    (tmp_path / "launches.cpp").write_text(SOURCE)
-    objs = []
-    for src in (str(tmp_path / "launches.cpp"), os.path.join(fb.CSRC, "frk_gemv_direct.hip"), os.path.join(fb.CSRC, "frk_gemv_fused.hip")):
-        objs.append(str(tmp_path / (os.path.basename(src) + ".o")))
-        subprocess.check_call([fb.hipcc()] + flags + ["-c", src, "-o", objs[-1]])
-    clang = "/opt/rocm/llvm/bin/clang++"
-    binary = str(tmp_path / "launches")
-    # (the kernels' image has no symbol in a host-only object)
-    subprocess.check_call([clang, "-fsanitize=address", "-no-pie", "-Wl,--unresolved-symbols=ignore-all"] + objs + ["-o", binary])
-    run = subprocess.run([binary], capture_output=True, text=True, timeout=120)
-    assert run.returncode == 0, (run.stdout + run.stderr)[-3000:]
+    calls = int(host_library.run(host_library.build(tmp_path, DRIVER)).split()[0])
+    assert calls == 5 * (64 * 3 + 64 * 4 + 64 * 4 + 62 * 4 + 64 + 64 + 53 + 62)

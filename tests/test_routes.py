@@ -1,0 +1,64 @@
+"""Which kernels a call goes to, on the CPU (host_library.py): shapes that were timed on both of the kernels a rule chooses from, each
+with the kernel that was the faster one, around the lines that the rules draw and beyond the sizes they were first fitted to."""
+import pytest
+
+import host_library
+import oracle as fo
+
+DRIVER = r"""
+#include <cstdio>
+#include "frink_amd/csrc/frk_internal.hpp"
+#include "include/frink_hip.h"
+int main() {  // a call a line: its name, kind, rows, blocks of 256 columns, tokens; the kernels it launches
+    char call[16];
+    int kind;
+    size_t rows, nb, batch;
+    static float room[64];
+    while (scanf("%15s %d %zu %zu %zu", call, &kind, &rows, &nb, &batch) == 5) {
+        frk_weights w;
+        w.kind = kind, w.rows = rows, w.cols = nb * 256, w.layout = frk::layout_for(kind, w.cols), w.dev = (uint8_t *)room;
+        const std::string name = call;
+        int rc = -99;
+        if (name == "gemv") rc = frk_hip_gemv_dev(&w, room, room, FRK_ACT_F32, nullptr);
+        if (name == "gemm") rc = frk_hip_gemm_dev(&w, room, batch, room, nullptr);
+        if (name == "q8k") rc = frk_hip_gemm_q8k_dev(&w, (int8_t *)room, room, (int16_t *)room, batch, room, nullptr);
+        printf("%d %s\n", rc, HipStub::get().take().c_str());
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    binary = host_library.build(tmp_path_factory.mktemp("routes"), DRIVER)
+
+    def of(calls):
+        lines = host_library.run(binary, "".join("%s %d %d %d %d\n" % c for c in calls)).splitlines()
+        assert len(lines) == len(calls)
+        return [(int(line.split()[0]), line.split(None, 1)[1]) for line in lines]
+
+    return of
+
+
+def check(kernels, call, kind, shapes, kernel, taken):
+    """shapes: (rows, blocks, tokens)"""
+    got = kernels([(call, kind, r, nb, m) for r, nb, m in shapes])
+    for shape, (rc, names) in zip(shapes, got):
+        assert rc == 0, (shape, rc)
+        assert (kernel in names) == taken, (call, kind, shape, names)
+
+
+# us, a quantization launch and a GEMV / columns: 36784 x 12 blocks 22.0 / 21.3, 88059 x 12 39.0 / 41.9, 58054 x 15 31.3 / 33.7, 141333 x 9 55.3 / 46.0
+def test_one_q5_k_row_of_9_to_15_blocks(kernels):
+    check(kernels, "gemv", fo.Q5_K, [(512, 9, 1), (14336, 12, 1), (36784, 12, 1), (141333, 9, 1), (138618, 10, 1)], "gemv_q4_k_cols_kernel", True)
+    check(kernels, "gemv", fo.Q5_K, [(88059, 12, 1), (58054, 15, 1), (68476, 12, 1)], "gemv_q4_k_cols_kernel", False)
+
+
+# us, whole rows a wavefront / columns: Q4_K 4284 x 20 blocks 5.8 / 6.4, 4096 x 20 5.8 / 5.3, 6285 x 17 6.9 / 6.2; Q5_K 4439 x 20 6.9 / 7.7,
+# 3948 x 20 6.6 / 6.5, 6285 x 17 10.9 / 9.1, 9980 x 21 12.8 / 13.2, 8192 x 21 12.4 / 11.5, 10128 x 22 17.3 / 13.5
+def test_one_row_of_17_to_21_blocks(kernels):
+    for kind, columns, rows in ((fo.Q4_K, [(512, 17), (4096, 20), (6285, 17), (8192, 20), (9980, 21)], [(4284, 20), (4710, 20), (5827, 19), (6144, 18), (8208, 20)]),
+                                (fo.Q5_K, [(512, 17), (4096, 20), (6285, 17), (8192, 20), (2048, 21), (6285, 21), (8192, 21), (10128, 22), (16475, 23)],
+                                 [(4439, 20), (5029, 19), (6144, 18), (8208, 20), (9980, 21), (12286, 21), (17631, 21)])):
+        check(kernels, "gemv", kind, [s + (1,) for s in columns], "gemv_q4_k_cols_kernel", True)
+        check(kernels, "gemv", kind, [s + (1,) for s in rows], "gemv_q4_k_cols_kernel", False)
