@@ -4,6 +4,7 @@
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <string>
@@ -694,18 +695,27 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 // Whether gemm_k_rows_kernel takes a batch (frk_gemm_rows.hip: sixteen rows a workgroup, no split, no second launch), ahead of both the
 // thin kernels and the pipelined GEMM.  It reads all tokens' tiles once for every sixteen rows, so what
 // is against it is many rows times many tokens (from 17 on twice the bytes) and rows so few and long that its workgroups'
-// chains are the launch.  nb blocks a row, with quantization, us before / now:
-//   Q4_K  two rows of short blocks (4 .. 19 blocks 0.92 of the time; past 33 blocks 1.01 and more).  Up to 8 not the span kernel's rows of 4,
-//         12 and 16 .. 32 blocks but tall ones (24 .. 32 blocks past 4096 rows 0.89; 14336x4096 at 8 12.0 / 12.6).  4096x11008 at 8 14.8 / 11.5; at
-//         3 and 4 long rows past one round of the chip 0.95 .. 1.1.  9 .. 16 rows 14336x4096 19.5 / 12.7, 4096x14336 18.0 / 13.5.  From 17 on rows of up to 19
-//         blocks (4096x4096 at 32 12.3 / 8.1) and, in one round of the chip, of up to 39; but 14336x4096 16.3 / 18.
-//   Q5_K  4096x11008 at 8 and 16 16.0 / 12.3 and 19.1 / 12.4, 4096x4096 at 32 13.7 / 8.6, in one round of the chip at 32 whatever
-//         the length (4096x14336 22.8 / 20.1), but 12000x12032 38.4 / 42.
-//   Q6_K  odd nb always (4096x11008 at 8, 13 and 32 17.7 / 12.7, 19.8 / 12.9, 21.1 / 15.2); even up to 8 rows not the streamed thin
-//         kernel's longer or taller ones (4096x14336 14.3 / 15.2); 4096x14336 at 16 and 32 20.7 / 15.1, 23.4 / 18.1; but 573x14336 at 32
-//         1.16 of the time, 13523x6144 at 31 25.9 / 30.
-// Over 2409 drawn batches of 2 .. 32 rows of 256 .. 14336 rows and 4 .. 56 blocks: 0.82 of the time before in the mean (the
-// better of both everywhere would be 0.2 % less), 1.1 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
+// chains are the launch.  It is one workgroup a CU up to 4096 rows and two up to 8192, and behind where the kernel that has a batch otherwise
+// fills its rounds of the chip and it does not: the lines below are by that kernel.  nb blocks a row, with quantization, us before / now:
+//   The pipelined GEMM's 64 x 32 tiles (k_quant_takes_the_matrix_cores), whose split fills the chip at any size: the longest rows that
+//         are ahead, by kind, tokens and rows.  9 .. 16 tokens Q4_K 14336x4096 19.5 / 12.7, 4096x14336 18.0 / 13.5, Q6_K 4096x11008 at 13 19.8 /
+//         12.9, but Q4_K 4193x12288 19.2 / 20.2, 4689x31488 34.7 / 45.8, 63220x7424 66.9 / 76.8, Q5_K 4532x29440 38.8 / 47.3, Q6_K 661x29952 at 13 18.4 /
+//         26.1.  17 .. 32 Q4_K 4096x4096 12.3 / 8.1 but 4956x5888 15.2 / 16.9, Q5_K 4096x4096 13.7 / 8.6 but 10256x6144 25.1 / 30.3, 2108x30720 26.3 / 38.5,
+//         Q6_K 4096x11008 at 32 21.1 / 15.2 but 13840x5120 26.2 / 31.1, 4233x12544 27.5 / 30.0, 921x30976 19.8 / 32.1.  (Q6_K of 13 to 16 blocks,
+//         a pair of blocks a wavefront here and a fourth step there, at 12289 .. 16384 rows too: 13840x3584 22.3 / 19.4, but 14336x3072 20.7 / 22.2.)
+//   The thin kernels that take fewer rows than the batch has, a launch for each group: always (Q4_K of 57 blocks and more at 5 .. 8 rows, Q5_K 0.2 to 0.6 of
+//         the time).
+//   The thin kernels of eight wavefronts (Q4_K, Q5_K), one workgroup of 16, 32, 64 or 128 rows a CU: Q4_K 4096x11008 at 8 14.8 / 11.5, Q5_K 4096x11008
+//         16.0 / 12.3, but where they fill a round (thin_rounds_are_full) with rows of 33 blocks and more Q4_K 7659x13056 at 6 22.3 / 24.1,
+//         14336x11008 27.7 / 31.6, 30394x10240 43.8 / 59.0, Q5_K 7432x12800 at 3 22.0 / 25.8; at 3 and 4 rows of Q4_K, which they stage in half the
+//         LDS, all past 4096 rows (5961x13056 20.7 / 22.9); lists of more than 40960 rows, where they are past two rounds: 61849x3584 at 7 33.7 / 39.3.
+//   The span kernel (Q4_K rows of 4, 8 .. 32 blocks): up to 8 tokens its rows of 4, 12 and 16 .. 32 blocks but tall ones (24 .. 32 blocks past 4096 rows 0.89;
+//         14336x4096 at 8 12.0 / 12.6; 14336x2048 8.9 / 9.5; 5120x8192 at 3 1.05), from 9 on short of 57088 rows of 24 blocks and more (97913x6144 84.8 / 101).
+//   Two tokens of Q4_K and Q6_K, the dot-product kernel: short rows (4 .. 19 blocks up to 4096 rows 0.9; 6785x4096 9.1 / 9.95, Q6_K 7398x4096 11.1 / 12.1).
+//   Q6_K of odd nb otherwise always (0.2 .. 0.95); the streamed thin kernel's even ones up to 8 tokens not the longer or taller (4096x14336 14.3 / 15.2),
+//         4096x14336 at 16 20.7 / 15.1, but 1069x13312 at 11 13.8 / 15.0, 1024x10240 at 28 1.13 of the time, 1064x13312 at 23 14.9 / 17.7.
+// Over 6200 drawn batches of 2 .. 32 rows of 64 .. 160000 rows and 1 .. 128 blocks: 0.79 of the time before in the mean of the 3911 it takes, six of
+// them past 1.03 and 1.05 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
 // From activations quantized beforehand (frk_hip_gemm_q8k_dev, which has tiles to make, and frk_hip_gemm_acts_dev) 0.84 and 0.75, gemm_pair
 // 0.73.
 //   33 to 512 rows of small matrices, every 32 tokens by workgroups of their own, where the pipelined GEMM takes 15 us and more however little there
@@ -713,35 +723,63 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 //         line Q4_K 4704x9984 at 53 21.2 / 29.4, Q6_K 3459x5632 at 99 22.3 / 29.2.  A few hundred rows of many blocks are few workgroups
 //         for their chains (Q5_K 513x11520 at 226 23.5 / 28.2).  Over 700 drawn sizes with up to 420000 blocks times tiles 0.77 of the time
 //         (the better of both everywhere would be 0.5 % less), 1.09 at worst; the 2-norm error against 64 bits of 60 that changed 0.98, 1.04 at most.
+static bool k_rows_beside_tiles(const frk_weights *w, size_t batch) {
+    static constexpr size_t ROWS[] = {1024, 2048, 2560, 4096, 5376, 8192, 12288, 16384, 24576, 28544, 32768, 40960};
+    static constexpr uint8_t LONGEST[3][2][13] = {  // blocks: Q4_K, Q5_K, Q6_K; up to 16 tokens, more
+        {{47, 64, 79, 104, 40, 56, 56, 28, 56, 43, 30, 56, 30}, {23, 23, 33, 39, 19, 19, 0, 0, 0, 0, 0, 0, 0}},
+        {{47, 60, 104, 128, 50, 128, 128, 56, 56, 56, 50, 56, 56}, {23, 23, 35, 56, 23, 32, 19, 11, 22, 15, 15, 15, 15}},
+        {{56, 72, 112, 128, 56, 128, 128, 128, 128, 128, 128, 128, 128}, {43, 48, 72, 96, 33, 80, 80, 10, 56, 56, 41, 56, 31}}};
+    const size_t rows = w->rows, nb = w->cols / QK_K, at = (size_t)(std::lower_bound(std::begin(ROWS), std::end(ROWS), rows) - std::begin(ROWS));
+    const int kind = w->kind == FRK_KIND_Q4_K ? 0 : w->kind == FRK_KIND_Q5_K ? 1 : 2;
+    if (kind == 2 && batch > 16 && rows > 12288 && nb >= 24 && nb % 2 == 0) return false;
+    return nb <= LONGEST[kind][batch > 16][at] || (kind == 2 && at == 7 && nb > 12 && nb <= 16);
+}
+// launch_thin_mfma_rg's workgroups, of 2, 4 or 8 groups of sixteen rows, are nearly a whole round of the 256 CUs, or several rounds
+static bool thin_rounds_are_full(size_t rows) {
+    for (size_t groups = 2; groups <= 8; groups *= 2)
+        if (rows > 223 * 16 * groups && rows <= 256 * 16 * groups) return true;
+    return rows > 223 * 16 * 16;
+}
+static bool k_rows_beside_thin(const frk_weights *w, size_t batch) {
+    const size_t rows = w->rows, nb = w->cols / QK_K;
+    if (w->kind == FRK_KIND_Q6_K) {
+        if (batch == 2) return nb < 20 && rows <= 4096;
+        if (nb % 2) return true;
+        if (batch <= 8) return nb < 16 ? nb == 8 || rows <= (nb < 12 ? 16384u : 12288u) : nb < 20 ? rows <= 8192 : nb < 48 && rows <= 4096;
+        if (rows > 2048 || (rows >= 1024 && !thin_gemm_wide_rows(w)) || (batch <= 16 && nb < 48)) return true;
+        return batch > 16 && nb >= 4 && (nb < 33 || (rows > 1024 && nb <= 36) || (rows > 1408 && nb <= 52));
+    }
+    const bool q4 = w->kind == FRK_KIND_Q4_K;
+    if (q4 && batch == 2) return nb < 20 && (rows <= 4096 || (rows <= 8192 && (nb < 12 || nb > 16)));
+    if (q4 && nb % 4 == 0 && nb <= 32 && batch <= 16) {  // (the span kernel's)
+        if (batch > 8) return nb < 24 || rows <= (nb < 28 ? 28544u : 14272u);
+        return nb == 8 ? rows <= 8192 : nb >= 20 && rows > (nb == 32 ? 8192u : 4096u);
+    }
+    if ((size_t)thin_gemm_max_batch(w) < batch) return batch > 4 || rows <= 12288;
+    const bool full = thin_rounds_are_full(rows), between = rows <= 24576 || (rows > 32768 && rows <= 40960);  // a round and a half, two and a half
+    if (nb < (q4 ? 8 : 10)) return !q4 || batch > 4 || rows <= 12288;
+    if (batch <= 4) {
+        if (nb < 20) return rows <= 12288 || (!q4 && between);
+        if (rows <= 4096) return nb < 80 || rows <= 512;
+        if (rows > 12288) return false;
+        if (full && nb >= 28) return false;
+        return q4 ? nb < 33 && !full : (nb < 41 || nb == 46 || nb > 48) && nb <= 104;
+    }
+    if (batch <= 8) {
+        if (nb < 20) return between || rows <= 28544;
+        return nb < 28 ? rows <= 14272 || (rows > 16384 && between) : between && !full;
+    }
+    return (rows <= 14272 || nb < 16 || !full) && (between || rows <= 28544 || (nb < 16 && rows > 32768 && rows <= 49152));
+}
 static bool k_rows_take(const frk_weights *w, size_t batch) {
     const size_t rows = w->rows, nb = w->cols / QK_K;
+    if (w->kind != FRK_KIND_Q4_K && w->kind != FRK_KIND_Q5_K && w->kind != FRK_KIND_Q6_K) return false;
     if (batch < 2 || batch > 512 || nb > 128) return false;
-    if (batch > 32) {
-        const size_t work = (batch + 31) / 32 * rows * nb;  // blocks times tiles of 32 tokens
-        if (w->kind == FRK_KIND_Q4_K) return work <= (nb >= 36 || (nb >= 28 && rows < 1100) ? 130000 : 190000);
-        if (w->kind != FRK_KIND_Q5_K && w->kind != FRK_KIND_Q6_K) return false;
-        if (nb >= 28 && rows < 1100) return work <= 130000;
-        return work <= (nb <= 16 && rows < 4096 ? 320000 : w->kind == FRK_KIND_Q5_K && nb >= 36 ? 190000 : 230000);
-    }
-    const bool one_round = rows > 2048 && rows <= 4096, few = rows < 1024;
-    if (w->kind == FRK_KIND_Q4_K) {
-        if (batch == 2) return nb < 20 && rows <= 8192;
-        if (batch <= 8 && nb % 4 == 0 && nb <= 32 && nb != 8) return nb >= 20 && rows > 4096;  // (the span kernel's)
-        if (batch <= 4) return rows <= 6144 || (nb < 33 && rows <= 12288);
-        if (batch <= 16) return batch <= 8 || !(few && nb >= 48);
-        return nb < 20 ? rows <= 8192 : nb < 24 ? rows <= 6144 : nb < 40 && one_round;
-    }
-    if (w->kind == FRK_KIND_Q5_K) {
-        if (batch <= 4) return rows <= 12288 || nb < 20;
-        if (batch <= 16) return batch <= 8 || !(few && nb >= 48);
-        return nb < 24 || one_round || (nb <= 32 && rows > 2048 && rows <= 12288);
-    }
-    if (w->kind != FRK_KIND_Q6_K) return false;
-    if (batch == 2) return nb < 20 && rows <= 8192;
-    if (nb % 2) return true;
-    if (batch <= 8) return nb < 16 || (nb < 20 ? rows <= 10240 : nb < 48 && rows <= 4096);  // (else the streamed thin kernel's)
-    if (batch <= 16) return !(few && nb >= 48);
-    return !(few && nb >= 33) && !(rows > 12288 && nb >= 24);
+    if (batch <= 32) return k_quant_takes_the_matrix_cores(w, batch) ? k_rows_beside_tiles(w, batch) : k_rows_beside_thin(w, batch);
+    const size_t work = (batch + 31) / 32 * rows * nb;  // blocks times tiles of 32 tokens
+    if (w->kind == FRK_KIND_Q4_K) return work <= (nb >= 36 || (nb >= 28 && rows < 1100) ? 130000 : 190000);
+    if (nb >= 28 && rows < 1100) return work <= 130000;
+    return work <= (nb <= 16 && rows < 4096 ? 320000 : w->kind == FRK_KIND_Q5_K && nb >= 36 ? 190000 : 230000);
 }
 // A K-quant batch that is multiplied from its tiles: gemm_k_rows_kernel's, or the pipelined GEMM's.
 static bool takes_tiles(const frk_weights *w, size_t batch) { return k_rows_take(w, batch) || k_quant_takes_the_matrix_cores(w, batch); }

@@ -12,7 +12,7 @@ from test_gpu_parity import bits, fa, make_weights, to_dev  # noqa: F401 (fa: th
 SHAPES = [(fo.Q4_K, 15, 2304, 3), (fo.Q4_K, 17, 256, 16), (fo.Q4_K, 33, 1280, 17), (fo.Q4_K, 1, 4864, 32), (fo.Q4_K, 1030, 11008, 8),
           (fo.Q4_K, 2100, 8192, 31), (fo.Q4_K, 100, 8448, 9), (fo.Q5_K, 1, 256, 2), (fo.Q5_K, 31, 512, 15), (fo.Q5_K, 16, 4864, 17), (fo.Q5_K, 50, 17152, 5),
           (fo.Q5_K, 2070, 14336, 32), (fo.Q6_K, 1, 256, 3), (fo.Q6_K, 18, 768, 17), (fo.Q6_K, 47, 4096, 16), (fo.Q6_K, 16, 4352, 32), (fo.Q6_K, 35, 17152, 9),
-          (fo.Q6_K, 2062, 9984, 30)]
+          (fo.Q6_K, 2062, 9984, 30), (fo.Q5_K, 2570, 14336, 32)]
 
 
 @pytest.mark.gpu

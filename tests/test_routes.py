@@ -62,3 +62,29 @@ def test_one_row_of_17_to_21_blocks(kernels):
                                  [(4439, 20), (5029, 19), (6144, 18), (8208, 20), (9980, 21), (12286, 21), (17631, 21)])):
         check(kernels, "gemv", kind, [s + (1,) for s in columns], "gemv_q4_k_cols_kernel", True)
         check(kernels, "gemv", kind, [s + (1,) for s in rows], "gemv_q4_k_cols_kernel", False)
+
+
+# (us, what was there / sixteen-row workgroups; rows, blocks, tokens)
+SIXTEEN_ROWS = {
+    fo.Q4_K: [(4096, 16, 2), (4096, 43, 8), (14336, 16, 16), (4096, 56, 16), (4096, 16, 32), (5120, 56, 7), (12068, 44, 7), (17240, 31, 7), (7426, 64, 6), (16671, 38, 11), (135580, 16, 13),
+              (7, 2, 32)],
+    fo.Q5_K: [(4096, 43, 8), (4096, 43, 16), (4096, 16, 32), (9030, 49, 3), (7914, 125, 7), (33961, 31, 5), (3926, 92, 9), (16495, 18, 22), (154414, 4, 2)],
+    fo.Q6_K: [(4096, 43, 8), (4096, 43, 32), (4096, 56, 32), (411, 127, 15), (421, 127, 27), (13840, 14, 23), (5537, 91, 10), (88582, 8, 8), (1376, 47, 19)],
+}
+OTHERS = {
+    # thin kernels that fill a round: 22.3 / 24.1, 27.7 / 31.6, 43.8 / 59.0, 33.7 / 39.3, 73.1 / 92.3
+    # their four tokens' form: 20.7 / 22.9; span: 8.9 / 9.5, 84.8 / 101
+    # tiles: 19.2 / 20.2, 34.7 / 45.8, 18.5 / 24.3, 56.8 / 60.7, 54.2 / 62.4, 15.2 / 16.9
+    fo.Q4_K: [(7659, 51, 6), (14336, 43, 6), (30394, 40, 6), (61849, 14, 7), (58326, 37, 5), (5961, 51, 3), (14336, 8, 5), (97913, 24, 15),
+              (4193, 48, 13), (4689, 123, 16), (1322, 126, 11), (14889, 83, 12), (58128, 23, 10), (4956, 23, 17), (6785, 16, 2)],
+    # 22.0 / 25.8, 28.9 / 31.9, 71.5 / 81.9; 38.8 / 47.3, 25.1 / 30.3, 26.3 / 38.5, 19.9 / 31.0
+    fo.Q5_K: [(7432, 50, 3), (14755, 36, 7), (130371, 14, 3), (4532, 115, 10), (10256, 24, 27), (2108, 120, 21), (14559, 23, 19), (2084, 62, 24)],
+    # 18.4 / 26.1, 19.8 / 32.1, 26.2 / 31.1, 27.5 / 30.0, 14.9 / 17.7, 13.8 / 15.0, 1.13 of the time
+    fo.Q6_K: [(661, 117, 13), (921, 121, 18), (13840, 20, 22), (4233, 49, 28), (1064, 52, 23), (1069, 52, 11), (1024, 40, 28), (7398, 16, 2), (143833, 12, 8)],
+}
+
+
+@pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K, fo.Q6_K])
+def test_two_to_thirty_two_tokens(kernels, kind):
+    check(kernels, "gemm", kind, SIXTEEN_ROWS[kind], "gemm_k_rows_kernel", True)
+    check(kernels, "gemm", kind, OTHERS[kind], "gemm_k_rows_kernel", False)
