@@ -706,11 +706,12 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 //   The thin kernels that take fewer rows than the batch has, a launch for each group: always (Q4_K of 57 blocks and more at 5 .. 8 rows, Q5_K 0.2 to 0.6 of
 //         the time).
 //   The thin kernels of eight wavefronts (Q4_K, Q5_K), one workgroup of 16, 32, 64 or 128 rows a CU: Q4_K 4096x11008 at 8 14.8 / 11.5, Q5_K 4096x11008
-//         16.0 / 12.3, but where they fill a round (thin_rounds_are_full) with rows of 33 blocks and more Q4_K 7659x13056 at 6 22.3 / 24.1,
+//         16.0 / 12.3, but where they fill a round (thin_rounds_are_full) with rows of 28 blocks and more Q4_K 7659x13056 at 6 22.3 / 24.1,
 //         14336x11008 27.7 / 31.6, 30394x10240 43.8 / 59.0, Q5_K 7432x12800 at 3 22.0 / 25.8; at 3 and 4 rows of Q4_K, which they stage in half the
 //         LDS, all past 4096 rows (5961x13056 20.7 / 22.9); lists of more than 40960 rows, where they are past two rounds: 61849x3584 at 7 33.7 / 39.3.
 //   The span kernel (Q4_K rows of 4, 8 .. 32 blocks): up to 8 tokens its rows of 4, 12 and 16 .. 32 blocks but tall ones (24 .. 32 blocks past 4096 rows 0.89;
-//         14336x4096 at 8 12.0 / 12.6; 14336x2048 8.9 / 9.5; 5120x8192 at 3 1.05), from 9 on short of 57088 rows of 24 blocks and more (97913x6144 84.8 / 101).
+//         14336x4096 at 8 12.0 / 12.6; 14336x2048 8.9 / 9.5; 5120x8192 at 3 1.05), from 9 on all but long lists of 24 and 28 blocks, which the kernel above has
+//         (97913x6144 84.8 / 101).
 //   Two tokens of Q4_K and Q6_K, the dot-product kernel: short rows (4 .. 19 blocks up to 4096 rows 0.9; 6785x4096 9.1 / 9.95, Q6_K 7398x4096 11.1 / 12.1).
 //   Q6_K of odd nb otherwise always (0.2 .. 0.95); the streamed thin kernel's even ones up to 8 tokens not the longer or taller (4096x14336 14.3 / 15.2),
 //         4096x14336 at 16 20.7 / 15.1, but 1069x13312 at 11 13.8 / 15.0, 1024x10240 at 28 1.13 of the time, 1064x13312 at 23 14.9 / 17.7.
@@ -718,11 +719,6 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 // them past 1.03 and 1.05 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
 // From activations quantized beforehand (frk_hip_gemm_q8k_dev, which has tiles to make, and frk_hip_gemm_acts_dev) 0.84 and 0.75, gemm_pair
 // 0.73.
-//   33 to 512 rows of small matrices, every 32 tokens by workgroups of their own, where the pipelined GEMM takes 15 us and more however little there
-//         is to do: Q5_K 2146x3328 at 70 16.5 / 10.2, Q6_K 3856x3584 at 52 17.2 / 9.9, Q4_K 1101x2048 at 103 12.6 / 7.7; past the
-//         line Q4_K 4704x9984 at 53 21.2 / 29.4, Q6_K 3459x5632 at 99 22.3 / 29.2.  A few hundred rows of many blocks are few workgroups
-//         for their chains (Q5_K 513x11520 at 226 23.5 / 28.2).  Over 700 drawn sizes with up to 420000 blocks times tiles 0.77 of the time
-//         (the better of both everywhere would be 0.5 % less), 1.09 at worst; the 2-norm error against 64 bits of 60 that changed 0.98, 1.04 at most.
 static bool k_rows_beside_tiles(const frk_weights *w, size_t batch) {
     static constexpr size_t ROWS[] = {1024, 2048, 2560, 4096, 5376, 8192, 12288, 16384, 24576, 28544, 32768, 40960};
     static constexpr uint8_t LONGEST[3][2][13] = {  // blocks: Q4_K, Q5_K, Q6_K; up to 16 tokens, more
@@ -771,15 +767,37 @@ static bool k_rows_beside_thin(const frk_weights *w, size_t batch) {
     }
     return (rows <= 14272 || nb < 16 || !full) && (between || rows <= 28544 || (nb < 16 && rows > 32768 && rows <= 49152));
 }
+// 33 to 512 rows of small matrices, every 32 tokens by workgroups of their own, where the pipelined GEMM takes 15 us and more however little
+// there is to do: Q5_K 2146x3328 at 70 16.5 / 10.2, Q6_K 3856x3584 at 52 17.2 / 9.9, Q4_K 1101x2048 at 103 12.6 / 7.7; past the line Q4_K
+// 4704x9984 at 53 21.2 / 29.4, Q6_K 3459x5632 at 99 22.3 / 29.2. A few hundred rows of many blocks are few workgroups for their chains (Q5_K
+// 513x11520 at 226 23.5 / 28.2). Q4_K and Q5_K rows of 24 blocks and more: as many workgroups as CUs, or (Q5_K) nearly two on each; in
+// between, and (Q5_K of 20 and more) past two, some CUs have twice the others' (Q4_K 308x7424 at 401 18.5 / 21.3, 2443x7936 at 34 17.0 / 18.9,
+// 1193x6912 at 136 17.6 / 19.0, Q5_K 2087x11008 at 42 22.3 / 24.8, 1025x5632 at 248 20.3 / 23.2). Past 39 blocks (56 up to 64 tokens) Q4_K
+// 107x13568 at 243 20.6 / 21.9, 144x27392 at 63 24.9 / 30.3, past 72 Q5_K 42x32000 at 115 35.5 / 39.1; more than eight workgroups a CU (Q6_K
+// of one or three blocks: sixteen) 31622x512 in Q4_K at 63 12.3 / 15.4, 3304x1536 in Q6_K at 508 1.18 of the time. Q6_K at 33 to 40 tokens is
+// the streamed thin kernel's where its rows are few and long (284x9728 at 34 11.7 / 13.3) or of two blocks. Over 2490 drawn sizes 0.73 of the
+// time in the mean of the 1686 it takes, two of them past 1.03 and 1.04 at worst; the 2-norm error against 64 bits of 60 that changed 0.98,
+// 1.04 at most.
+static bool k_rows_of_small_matrices(const frk_weights *w, size_t batch) {
+    const size_t rows = w->rows, nb = w->cols / QK_K, tiles = (batch + 31) / 32;
+    const size_t work = tiles * rows * nb, workgroups = tiles * ((rows + 15) / 16);  // work: blocks times tiles of 32 tokens
+    const bool few = nb >= 28 && rows < 1100;
+    if (workgroups > (w->kind == FRK_KIND_Q6_K && (nb == 1 || nb == 3) ? 4096u : 2048u)) return false;
+    if (w->kind == FRK_KIND_Q4_K) {
+        if (nb > (batch <= 64 ? 56u : 39u) || work > (nb < 24 ? 160000u : nb >= 36 || few ? 130000u : 190000u)) return false;
+        return nb < 24 || workgroups <= 256;
+    }
+    const bool q5 = w->kind == FRK_KIND_Q5_K;
+    if (work > (few ? 130000u : !q5 && nb <= 16 && rows < 4096 ? 320000u : (q5 && nb >= 36) || nb >= 48 ? 190000u : 230000u)) return false;
+    if (q5) return nb < 20 || (nb <= 72 && (workgroups <= 256 || ((nb < 24 || workgroups > 384) && workgroups <= 512)));
+    return batch > 40 || nb % 2 || (nb >= 4 && nb < 33) || rows > (nb < 4 ? 2048u : 768u) || !thin_gemm_wide_rows(w);
+}
 static bool k_rows_take(const frk_weights *w, size_t batch) {
     const size_t rows = w->rows, nb = w->cols / QK_K;
     if (w->kind != FRK_KIND_Q4_K && w->kind != FRK_KIND_Q5_K && w->kind != FRK_KIND_Q6_K) return false;
     if (batch < 2 || batch > 512 || nb > 128) return false;
     if (batch <= 32) return k_quant_takes_the_matrix_cores(w, batch) ? k_rows_beside_tiles(w, batch) : k_rows_beside_thin(w, batch);
-    const size_t work = (batch + 31) / 32 * rows * nb;  // blocks times tiles of 32 tokens
-    if (w->kind == FRK_KIND_Q4_K) return work <= (nb >= 36 || (nb >= 28 && rows < 1100) ? 130000 : 190000);
-    if (nb >= 28 && rows < 1100) return work <= 130000;
-    return work <= (nb <= 16 && rows < 4096 ? 320000 : w->kind == FRK_KIND_Q5_K && nb >= 36 ? 190000 : 230000);
+    return k_rows_of_small_matrices(w, batch);
 }
 // A K-quant batch that is multiplied from its tiles: gemm_k_rows_kernel's, or the pipelined GEMM's.
 static bool takes_tiles(const frk_weights *w, size_t batch) { return k_rows_take(w, batch) || k_quant_takes_the_matrix_cores(w, batch); }

@@ -88,3 +88,18 @@ OTHERS = {
 def test_two_to_thirty_two_tokens(kernels, kind):
     check(kernels, "gemm", kind, SIXTEEN_ROWS[kind], "gemm_k_rows_kernel", True)
     check(kernels, "gemm", kind, OTHERS[kind], "gemm_k_rows_kernel", False)
+
+
+# (us, the pipelined GEMM / every 32 tokens by workgroups of their own)
+SMALL = {fo.Q4_K: [(1101, 8, 103), (1115, 33, 90), (854, 32, 102), (369, 31, 295), (19, 2, 63)], fo.Q5_K: [(2146, 13, 70), (272, 71, 54), (385, 27, 298), (20, 2, 34)],
+         fo.Q6_K: [(3856, 14, 52), (129, 75, 259), (63, 110, 33), (857, 42, 40), (18163, 3, 67)]}
+# 18.5 / 21.3, 17.0 / 18.9, 17.6 / 19.0, 24.9 / 30.3, 12.3 / 15.4, 21.2 / 29.4; 22.3 / 24.8, 23.7 / 25.7, 35.5 / 39.1, 15.7 / 17.2; 11.7 / 13.3, 12.8 / 15.8, 22.3 / 29.2,
+# 12.8 / 13.8, 1.18 of the time
+LARGER = {fo.Q4_K: [(308, 29, 401), (2443, 31, 34), (1193, 27, 136), (144, 107, 63), (31622, 2, 63), (4704, 39, 53)], fo.Q5_K: [(2087, 43, 42), (1028, 27, 242), (42, 125, 115), (8551, 2, 248)],
+          fo.Q6_K: [(284, 38, 34), (261, 52, 36), (3459, 22, 99), (12202, 2, 111), (3304, 6, 508)]}
+
+
+@pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K, fo.Q6_K])
+def test_more_tokens_of_small_matrices(kernels, kind):
+    check(kernels, "gemm", kind, SMALL[kind], "gemm_k_rows_kernel", True)
+    check(kernels, "gemm", kind, LARGER[kind], "gemm_k_rows_kernel", False)
