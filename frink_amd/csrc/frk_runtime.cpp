@@ -632,21 +632,17 @@ int frk_hip_gemv_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
     return set_error(FRK_ERR_UNSUPPORTED, "Q8_K activations feed Q4_K, Q5_K and Q6_K weights only (kind %d)", w->kind);
 }
 
-// Whether a batch takes the matrix-core GEMM.  Its cost is flat up to 32 rows (64 x 32 tiles) and up to 64; below, the thin
-// kernels' groups of 16 (Q4_K, Q5_K) or 8 rows are ahead by what a group costs at the matrix's shape.  nb blocks a row, with
-// quantization (us; thin / GEMM), within 32768 columns:
-//   Q4_K  from 17 rows on (14336x4096 at 17 19.6 / 14.9; 3335x5120 0.92 of the time), but for 8 and 12 blocks up to 4096 rows, where two thin
-//         launches take as long (1264x2048 at 23 9.5 / 9.9, 2375x3072 10.2 / 10.3, 4054x2048 at 19 9.8 / 9.8; at 17 and 18, whose second one is
-//         slower, 10.3 / 9.7) and activations quantized beforehand need no tiled copy (frk_hip_gemm_q8k_dev 7.3 / 9.2).  From 9 on rows of 30 blocks and more (1861x7680 at 9 0.98, 4096x11008 19.9 / 16.6) and,
-//         past one workgroup a CU, of 24: 4771x7168 0.72, but 1798x6144 1.07, 7986x5120 1.15.
-//   Q5_K  from 17 rows on (62 of 65 drawn ahead; 14257x2304 1.09, 4096x4096 at 17 20.4 / 13.4), and from 9 on rows of 32 blocks
-//         and more (4096x11008 25.3 / 19.3) and, past 4608 rows, of 24: 5230x6144 0.78, but 2491x6912 1.20.
-//   Q6_K  odd nb (not the streamed thin kernel's): from 9 on matrices of 18 M weights (4096x11008 at 13 28.9 / 19.7, 2631x7936
-//         0.67, but 1914x8960 at 16 1.08), at 17 of 8 M and more than 1280 rows (1822x5376 0.68, but 1144x8448 1.07), at 33 of 5 M.
-//         Even: from 9 on past 48 M and 4096 rows (4207x12288 0.81, but 4096x14336 20.1 / 22.2; over 250 drawn 0.86, five of them, 8200 .. 9200 rows of 28 .. 32
-//         blocks and one more, 1.05 .. 1.10), at 17 past 23 M (6574x6144
-//         0.79, 2015x12800 0.92, but 4788x4096 1.11), at 25 past 17 M (4788x4096 0.98, but 1897x6656 1.05).
-// Of what gemm_k_rows_kernel does not take (k_rows_take, which comes first).
+// Which kernel has a batch that gemm_k_rows_kernel does not take: the pipelined matrix-core GEMM, or the thin kernels.  k_rows_take asks it which of
+// its own lines holds, and matrix_cores_only beyond which batches there is nothing but the GEMM.  The GEMM's cost is flat up to 32 rows (64 x 32 tiles)
+// and up to 64; below, the thin kernels' groups of 16 (Q4_K, Q5_K) or 8 rows are ahead by what a group costs at the matrix's shape.  nb blocks a row,
+// with quantization (us; thin / GEMM), within 32768 columns:
+//   Q4_K  from 17 rows on (14336x4096 at 17 19.6 / 14.9; 3335x5120 0.92 of the time).  From 9 on rows of 30 blocks and more (1861x7680 at 9 0.98,
+//         4096x11008 19.9 / 16.6) and, past one workgroup a CU, of 24: 4771x7168 0.72, but 1798x6144 1.07, 7986x5120 1.15.
+//   Q5_K  from 17 rows on (14257x2304 1.09, 4096x4096 at 17 20.4 / 13.4), and from 9 on rows of 24 blocks and more (4096x11008 25.3 / 19.3, 5230x6144
+//         0.78).
+//   Q6_K  odd nb: from 9 on matrices of 18 M weights (4096x11008 at 13 28.9 / 19.7, 2631x7936 0.67), at 17 of 8 M and more than 1280 rows (1822x5376
+//         0.68): gemm_k_rows_kernel takes what is below them.  Even: from 9 on past 48 M and 4096 rows (4207x12288 0.81, but 4096x14336 20.1 / 22.2), at
+//         17 past 23 M (6574x6144 0.79, 2015x12800 0.92, but 4788x4096 1.11), at 25 past 17 M (4788x4096 0.98, but 1897x6656 1.05).
 static size_t tiled_from(size_t cols) { return cols >= 24 * QK_K ? 9 : 17; }
 static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     if (batch < tiled_from(w->cols)) return false;
@@ -654,19 +650,16 @@ static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     const bool measured = nb <= 128;
     if (w->kind == FRK_KIND_Q4_K) {
         const bool eights = thin_gemm_max_batch(w) < 16;  // rows of a thin launch
-        if ((nb == 8 || nb == 12) && w->rows <= 4096 && batch >= 19 && batch <= 32) return false;
-        if (batch >= 17) return measured || batch >= 33 || n > 20 * M || eights;
+        if (batch >= 17) return true;
         return measured && (nb >= 30 || (nb >= 24 && w->rows > 4096 && (eights || w->rows <= 8192)));
     }
     if (w->kind == FRK_KIND_Q5_K) {
-        if (batch >= 17) return batch >= 33 || (measured && (nb >= 10 || w->rows <= 8192));
-        return measured && (nb >= 32 || (nb >= 24 && w->rows > 4608));
+        return batch >= 33 || (measured && (batch >= 17 || nb >= 24));
     }
     if (w->kind != FRK_KIND_Q6_K) return false;
     if (batch >= 41) return true;
     if (measured && nb % 2) {
-        if (batch >= 33) return n > 5 * M;
-        return n > 18 * M || (batch >= 17 && n > 8 * M && w->rows > 1280);
+        return batch >= 33 || n > 18 * M || (batch >= 17 && n > 8 * M && w->rows > 1280);
     }
     if (batch >= 25) return n > 32 * M || (measured && n > (batch >= 33 ? 23 : 17) * M);
     if (batch >= 17) return measured && n > 23 * M;
