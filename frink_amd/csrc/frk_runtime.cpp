@@ -983,8 +983,8 @@ int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
     if (!k_quant) return set_error(FRK_ERR_UNSUPPORTED, "Q8_K activations feed Q4_K, Q5_K and Q6_K weights only (kind %d)", w->kind);
     if (!thin_kernels_hold(w, batch))
         return set_error(FRK_ERR_UNSUPPORTED,
-                         "a batch of %zu rows of this matrix does not multiply on the thin kernels (the matrix-core GEMM "
-                         "quantizes into a tiled form of its own): frk_hip_gemm_dev / frk_hip_gemm_pair_dev", batch);
+                         "a batch of %zu rows of this matrix is more than this call takes (a batch like this is quantized into tiles at once): "
+                         "frk_hip_gemm_dev / frk_hip_gemm_pair_dev, or frk_hip_quantize_batch_acts_dev", batch);
     Q8KActs a{q, d, bsums};
     hipStream_t s = (hipStream_t)stream;
     // (for a small matrix, or a few rows, a launch to make tiles of them costs more than what the rows' lines do)

@@ -220,9 +220,10 @@ int frk_hip_gemm_dev(const frk_weights *w, const float *x_dev, size_t batch, flo
  * call over the same batch) has already quantized to Q8_K: q [batch][cols] i8, d [batch][cols/256] f32,
  * bsums [batch][cols/16] i16, the layout frk_hip_quantize_q8_k_dev writes (BatchActs::Q8K,
  * crates/frink-core/src/weight_matrix.rs:757-768, handed to apply_batch_with_acts, :2481-2487).  Bit for bit
- * frk_hip_gemm_dev's result (one row: frk_hip_gemv_q8k_dev).  K-quants; the batches that the thin kernels hold (up to 16
- * or 32 rows for Q4_K and up to 24 or 40 for Q6_K by the matrix's size, 32 for Q5_K; those that frk_hip_gemm_dev multiplies on the
- * matrix cores are put into their tiled form in scratch memory first): FRK_ERR_UNSUPPORTED beyond, where the matrix-core GEMM quantizes for itself. */
+ * frk_hip_gemm_dev's result (one row: frk_hip_gemv_q8k_dev).  K-quants, batches of up to 16 or 32 rows for Q4_K, 24 or 40 for
+ * Q6_K and 32 for Q5_K, by the matrix's size; FRK_ERR_UNSUPPORTED beyond.  The kernels of those batches read the rows as they
+ * are, or in the tiled form that the call makes of them in scratch memory first, whichever has frk_hip_gemm_dev's bits
+ * sooner.  (A larger batch costs less quantized into tiles at once: frk_hip_quantize_batch_acts_dev.) */
 int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q_dev, const float *d_dev, const int16_t *bsums_dev,
                          size_t batch, float *y_dev, void *stream);
 
@@ -238,12 +239,13 @@ int frk_hip_gemm_pair_dev(const frk_weights *w0, const frk_weights *w1, const fl
  * gate and up of a prefill, or activations a caller keeps.  The object owns its device memory
  * (frk_hip_batch_acts_create allocates for up to max_batch rows of cols columns, _release frees; neither
  * belongs in a hot loop) and holds the batch in whichever form the kernels of that batch size read: plain
- * Q8_K rows (the decode and thin kernels), the tiled form of the matrix-core GEMMs, or both.
+ * Q8_K rows (up to 64: the decode and thin kernels), the tiled form of the matrix-core kernels (from two rows
+ * on, whole tiles of 32), or both: which the matrices read is not known yet when the batch is quantized.
  * frk_hip_quantize_batch_acts_dev and frk_hip_gemm_acts_dev allocate nothing themselves (a GEMM whose
  * blocks are split between workgroups takes room for the parts from the stream's scratch buffer, like
  * frk_hip_gemm_dev); y is bit for bit frk_hip_gemm_dev's for two rows and more, and frk_hip_gemv_q8k_dev's for
- * one (which is frk_hip_gemv_dev's wherever both forms of the decode step are one kernel, and the same integers
- * added in another order for rows of more than 20 blocks).  K-quant matrices (Q4_K, Q5_K, Q6_K) of `cols`
+ * one (which is frk_hip_gemv_dev's for Q4_K rows of up to 16 blocks of 256 columns, Q5_K of up to 8 and of 16 and 32, Q6_K of up
+ * to 19 and all of more than 64; for other lengths it may be the same integers added in another order).  K-quant matrices (Q4_K, Q5_K, Q6_K) of `cols`
  * columns; other kinds return FRK_ERR_UNSUPPORTED.  A quantization and the GEMMs that read it are ordered
  * by the stream they are enqueued on; the object is not to be re-quantized while a GEMM that reads it is
  * still in flight on another stream. */
