@@ -700,10 +700,8 @@ static int launch_q6_k_group(const frk_weights *const *ws, size_t n, const float
     else                                                                                                                                 \
         hipLaunchKernelGGL((gemv_q6_k_direct_kernel<UU, XX, true, GemvOne>), grid, block, shmem, s, GemvOne{w->dev, ys[0], (int)w->rows},   \
                            w->layout, nb, x, no_q, no_d, no_sums)
-    if (u == 1) FRK_GO(1, 1);       // nb <= 16
-    else if (u == 2) FRK_GO(2, 2);  // nb <= 32
-    else if (u == 3) FRK_GO(3, 3);  // nb <= 48
-    else FRK_GO(4, 4);              // nb <= 64
+    if (u == 1) FRK_GO(1, 1);  // 9 to 16 blocks
+    else FRK_GO(2, 2);         // 17 to 19 (q6_k_cols_form has the longer and the shorter)
 #undef FRK_GO
     FRK_LAUNCH_CHECK("gemv_q6_k_fused");
     return FRK_OK;

@@ -710,8 +710,9 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 //         4096x14336 at 16 20.7 / 15.1, but 1069x13312 at 11 13.8 / 15.0, 1024x10240 at 28 1.13 of the time, 1064x13312 at 23 14.9 / 17.7.
 // Over 6200 drawn batches of 2 .. 32 rows of 64 .. 160000 rows and 1 .. 128 blocks: 0.79 of the time before in the mean of the 3911 it takes, six of
 // them past 1.03 and 1.05 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
-// From activations quantized beforehand (frk_hip_gemm_q8k_dev, which has tiles to make, and frk_hip_gemm_acts_dev) 0.84 and 0.75, gemm_pair
-// 0.73.
+// From activations quantized beforehand over the same draws: frk_hip_gemm_acts_dev 0.84 in the mean of 400, 1.02 at worst.  frk_hip_gemm_q8k_dev
+// 0.86 in the mean of 460, but 33 of them past 1.03 and 1.12 at worst (Q5_K 2132x13056 at 3 12.6 / 14.1, 3945x4608 at 8 8.5 / 9.3): it has
+// frk_hip_gemm_dev's bits, and so its kernel, also where that one is ahead by its quantization alone.
 static bool k_rows_beside_tiles(const frk_weights *w, size_t batch) {
     static constexpr size_t ROWS[] = {1024, 2048, 2560, 4096, 5376, 8192, 12288, 16384, 24576, 28544, 32768, 40960};
     static constexpr uint8_t LONGEST[3][2][13] = {  // blocks: Q4_K, Q5_K, Q6_K; up to 16 tokens, more

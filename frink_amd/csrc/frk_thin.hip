@@ -1,6 +1,8 @@
-// Thin batched GEMM (2..8 activation rows, batched decode): y[b][r] = sum_k W[r][k] * x[b][k].
+// Thin batched GEMM (up to 16 activation rows of Q4_K and Q5_K, groups of 8 of Q6_K), of the batches that gemm_k_rows_kernel is
+// not ahead at: y[b][r] = sum_k W[r][k] * x[b][k].
 //
-// Still bandwidth-bound: the weights are read from HBM once for the whole batch, unpacked once per
+// The first two kernels (two activation rows; four of Q4_K rows of 105 to 131 blocks) are
+// still bandwidth-bound: the weights are read from HBM once for the whole batch, unpacked once per
 // 64-weight unit, and multiplied against each of the NB quantized activation rows, which live in
 // LDS (NB * cols bytes of quants plus their sums and scales).  Arithmetic per (row, activation) is
 // exactly the decode GEMV's (dot_q4_k_q8 / dot_q6_k_q8, crates/frink-quant/src/lib.rs:822-869,
@@ -361,13 +363,6 @@ __global__ __launch_bounds__(64 * TM_WAVES) __attribute__((amdgpu_waves_per_eu(2
                                                                         const int16_t *__restrict__ absums,
                                                                         float *__restrict__ y) {
     constexpr int KS = TM_WAVES / RG;
-    // a batch wider than ACTS is a grid of groups of ACTS activation rows: blockIdx.y picks the group
-    // (every group streams the weights again, out of L2 after the first)
-    aq += (size_t)blockIdx.y * ACTS * nb * QK_K;
-    ad += (size_t)blockIdx.y * ACTS * nb;
-    absums += (size_t)blockIdx.y * ACTS * nb * 16;
-    y += (size_t)blockIdx.y * ACTS * rows;
-    batch = min(ACTS, batch - (int)blockIdx.y * ACTS);
     constexpr int BB = Q5 ? Q5_K_BYTES : Q4_K_BYTES;  // bytes of a block
     constexpr int PR = BB / 16, NP = 16 * PR;         // 16-byte pieces of a row's block, of 16 rows' blocks
     constexpr int QS = Q5 ? 48 : 16;                  // where the nibbles start
@@ -562,203 +557,6 @@ __global__ __launch_bounds__(64 * TM_WAVES) __attribute__((amdgpu_waves_per_eu(2
     }
 }
 
-// ------------------------------------------------------------------ thin GEMM on the matrix cores (Q6_K)
-//
-// Same plan as the Q4_K kernel above, for up to 8 activation rows.  Q6_K scales sixteen weights at
-// a time, and a K=32 MFMA would add up two such groups.  So the 16 rows of the MFMA's activation
-// operand hold the (at most 8) activation rows twice: rows 0..7 with only the first sixteen k of
-// every 32 (the rest zero), rows 8..15 with only the second sixteen.  One MFMA then returns, for
-// each (activation, weight row), the two 16-wide dots side by side -- in the lanes of k-groups 0..1
-// and 2..3, which multiply them by their own group's int8 scale; the two halves of a result meet
-// once, at the end.  The 6-bit codes go in as signed bytes q - 32 (one add and one xor per four
-// codes), so there is no "-32 * sum of the activations" term to carry: the integers are
-// dot_q6_k_q8's (crates/frink-quant/src/lib.rs:1069-1110), split in two partial sums per block.
-// Weights are the resident planar form (ql | qh | sc | d per row); in LDS a row of a block is
-// [ql 128 | qh 64 | sc 16 | d 2], 240 bytes apart so that the 16 rows of a read fall in
-// different banks.
-constexpr int T6_ROW = 240;
-constexpr int T6_WBLOCK = 16 * T6_ROW;  // 3840
-__host__ __device__ inline size_t t6_lds_bytes(int acts, int cols) {
-    return (size_t)acts * tm_q_stride(cols) + (size_t)(cols / QK_K) * 32 + (size_t)TM_WAVES * T6_WBLOCK;
-}
-
-template <int RG, int ACTS>
-__global__ __launch_bounds__(64 * TM_WAVES) __attribute__((amdgpu_waves_per_eu(2, 4))) void thin_mfma_q6_k_kernel(
-    const uint8_t *__restrict__ W, Layout lay, int rows, int nb, int batch, const int8_t *__restrict__ aq,
-    const float *__restrict__ ad, float *__restrict__ y) {
-    constexpr int KS = TM_WAVES / RG;
-    extern __shared__ uint4 smem[];
-    uint8_t *lds = reinterpret_cast<uint8_t *>(smem);
-    const int cols = nb * QK_K;
-    // a batch wider than ACTS is a grid of groups of ACTS activation rows: blockIdx.y picks the group
-    // (every group streams the matrix again; the groups after the first find it in the caches)
-    aq += (size_t)blockIdx.y * ACTS * cols;
-    ad += (size_t)blockIdx.y * ACTS * nb;
-    y += (size_t)blockIdx.y * ACTS * rows;
-    batch = min(ACTS, batch - (int)blockIdx.y * ACTS);
-    const int q_stride = tm_q_stride(cols);
-    uint8_t *lds_q = lds;                                                         // [ACTS][q_stride]
-    float *lds_d = reinterpret_cast<float *>(lds_q + (size_t)ACTS * q_stride);    // [nb][8]
-    uint8_t *lds_w = reinterpret_cast<uint8_t *>(lds_d + (size_t)nb * 8);         // [wave][3840]
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int j = lane & 15, g = lane >> 4;
-    const int rgrp = wave % RG, ksp = wave / RG;
-    const int row0 = (blockIdx.x * RG + rgrp) * 16;
-    const int my_blocks = nb > ksp ? (nb - ksp + KS - 1) / KS : 0;
-
-    // ---- this wavefront's weight stream: the four planes of its 16 rows, 16-byte pieces ----
-    // ql: piece p = 64*c + lane (c = 0, 1) is row p/8, piece p%8; qh: piece lane is row lane/4, piece
-    // lane%4; sc: lanes 0..15, one piece per row; d: lanes 0..15, two bytes per row
-    auto row_ptr = [&](int r) { return W + (size_t)min(row0 + r, rows - 1) * lay.row_stride; };
-    const uint8_t *src_ql0 = row_ptr(lane >> 3) + (lane & 7) * 16 + (size_t)ksp * 128;
-    const uint8_t *src_ql1 = row_ptr(8 + (lane >> 3)) + (lane & 7) * 16 + (size_t)ksp * 128;
-    const uint8_t *src_qh = row_ptr(lane >> 2) + lay.off_a + (lane & 3) * 16 + (size_t)ksp * 64;
-    const uint8_t *src_sc = row_ptr(lane & 15) + lay.off_b + (size_t)ksp * 16;
-    const uint8_t *src_d = row_ptr(lane & 15) + lay.off_c + (size_t)ksp * 2;
-    struct Raw {
-        uint4 ql0, ql1, qh, sc;
-        uint32_t d;
-    };
-    auto fetch_block = [&](int i) {  // (past the last block: the last one again, never used)
-        const size_t k = (size_t)KS * max(min(i, my_blocks - 1), 0);
-        Raw R;
-        R.ql0 = *reinterpret_cast<const uint4 *>(src_ql0 + k * 128);
-        R.ql1 = *reinterpret_cast<const uint4 *>(src_ql1 + k * 128);
-        R.qh = *reinterpret_cast<const uint4 *>(src_qh + k * 64);
-        R.sc = *reinterpret_cast<const uint4 *>(src_sc + k * 16);  // lanes 16.. repeat rows 0..15
-        R.d = *reinterpret_cast<const uint16_t *>(src_d + k * 2);
-        return R;
-    };
-    static_assert(TM_AHEAD == 4, "the ring is four named buffers");
-    Raw R0, R1, R2, R3;
-
-    // ---- the activations, once per workgroup: staging loads first, the weight ring behind them ----
-    {
-        constexpr int T = 64 * TM_WAVES;
-        const int row_g = cols / 16;  // 16-byte granules of quants per row
-        auto load_q = [&](int base, int u) {  // (past the end: a valid address, the value is not written)
-            const int idx = min(base + u * T + tid, ACTS * row_g - 1);
-            const int a = idx / row_g, i = idx - a * row_g;
-            return reinterpret_cast<const uint4 *>(aq + (size_t)min(a, batch - 1) * cols)[i];
-        };
-        auto store_q = [&](int base, int u, uint4 v) {
-            const int idx = base + u * T + tid;
-            if (idx < ACTS * row_g) {
-                const int a = idx / row_g, i = idx - a * row_g;
-                *reinterpret_cast<uint4 *>(lds_q + (size_t)a * q_stride + i * 16) = v;
-            }
-        };
-        auto load_d = [&](int idx) {
-            idx = min(idx, nb * 8 - 1);
-            return ad[(size_t)min(idx & 7, batch - 1) * nb + (idx >> 3)];
-        };
-        const uint4 q0 = load_q(0, 0), q1 = load_q(0, 1), q2 = load_q(0, 2), q3 = load_q(0, 3);
-        const float d0 = load_d(tid);
-        R0 = fetch_block(0);
-        R1 = fetch_block(1);
-        R2 = fetch_block(2);
-        R3 = fetch_block(3);
-        store_q(0, 0, q0);
-        store_q(0, 1, q1);
-        store_q(0, 2, q2);
-        store_q(0, 3, q3);
-        if (tid < nb * 8) lds_d[tid] = d0;
-        // what one round does not cover (long rows): behind the ring, at the ring's pace
-        for (int base = 4 * T; base < ACTS * row_g; base += 4 * T)
-#pragma unroll
-            for (int u = 0; u < 4; u++) store_q(base, u, load_q(base, u));
-        for (int idx = T + tid; idx < nb * 8; idx += T) lds_d[idx] = load_d(idx);
-    }
-    __syncthreads();
-
-    // ---- the loop ----
-    // activation operand row j: activation j % 8, and only the k-groups of its half are real
-    const bool real = (j < 8) == (g < 2);
-    const uint8_t *a_q = lds_q + (size_t)min(j & 7, ACTS - 1) * q_stride + 8 * g;
-    const float *a_d = lds_d + 4 * (g & 1);
-    uint8_t *area = lds_w + (size_t)wave * T6_WBLOCK;
-    const uint8_t *a_w = area + j * T6_ROW;
-    auto as_long = [](uint2 v) { return (long)(((unsigned long)v.y << 32) | v.x); };
-    v4f_t acc = {0.f, 0.f, 0.f, 0.f};
-    auto multiply_block = [&](int i, Raw R) {  // returns the block that takes this one's place in the ring
-        const int kb = ksp + KS * i;
-        *reinterpret_cast<uint4 *>(area + (lane >> 3) * T6_ROW + (lane & 7) * 16) = R.ql0;
-        *reinterpret_cast<uint4 *>(area + (8 + (lane >> 3)) * T6_ROW + (lane & 7) * 16) = R.ql1;
-        *reinterpret_cast<uint4 *>(area + (lane >> 2) * T6_ROW + 128 + (lane & 3) * 16) = R.qh;
-        if (lane < 16) {
-            *reinterpret_cast<uint4 *>(area + lane * T6_ROW + 192) = R.sc;
-            *reinterpret_cast<uint32_t *>(area + lane * T6_ROW + 208) = R.d;
-        }
-        R = fetch_block(i + TM_AHEAD);  // the registers are free again
-        const uint4 scv = *reinterpret_cast<const uint4 *>(a_w + 192);
-        const uint32_t scw[4] = {scv.x, scv.y, scv.z, scv.w};
-        const float d = h2f(*reinterpret_cast<const uint32_t *>(a_w + 208) & 0xffffu);
-        const v4i_t zero = {0, 0, 0, 0};
-        v4i_t isum = {0, 0, 0, 0};
-        const uint8_t *aq_k = a_q + (size_t)kb * QK_K;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint2 qla = *reinterpret_cast<const uint2 *>(a_w + h * 64 + 8 * g);
-            const uint2 qlb = *reinterpret_cast<const uint2 *>(a_w + h * 64 + 32 + 8 * g);
-            const uint2 qh = *reinterpret_cast<const uint2 *>(a_w + 128 + h * 32 + 8 * g);
-#pragma unroll
-            for (int v = 0; v < 4; v++) {  // weights h*128 + 32*v + l, l = 8g .. 8g+7
-                const uint2 ql = (v & 1) ? qlb : qla;
-                auto code = [&](uint32_t lo, uint32_t hi) {  // four 6-bit codes, as signed bytes q - 32
-                    const uint32_t nib = (v >= 2 ? lo >> 4 : lo) & 0x0f0f0f0fu;
-                    const uint32_t top = ((hi >> (2 * v)) & 0x03030303u) << 4;
-                    return ((nib | top) + 0x60606060u) ^ 0x80808080u;
-                };
-                const uint2 wq = make_uint2(code(ql.x, qh.x), code(ql.y, qh.y));
-                uint2 a = *reinterpret_cast<const uint2 *>(aq_k + h * 128 + 32 * v);
-                if (!real) a = make_uint2(0u, 0u);
-                const v4i_t t = __builtin_amdgcn_mfma_i32_16x16x32_i8(as_long(a), as_long(wq), zero, 0, 0, 0);
-                // the scale of this lane's 16-wide group: sc[h*8 + 2*v + g/2]
-                const int si = h * 8 + 2 * v + (g >> 1);
-                const int sc = (int)(int8_t)((scw[si >> 2] >> (8 * (si & 3))) & 0xff);
-#pragma unroll
-                for (int r = 0; r < 4; r++) isum[r] += __mul24(sc, t[r]);
-            }
-        }
-        const v4f_t da = *reinterpret_cast<const v4f_t *>(a_d + (size_t)kb * 8);
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[r] += (d * da[r]) * (float)isum[r];
-        return R;
-    };
-    for (int i = 0; i < my_blocks; i += TM_AHEAD) {
-        R0 = multiply_block(i, R0);
-        if (i + 1 < my_blocks) R1 = multiply_block(i + 1, R1);
-        if (i + 2 < my_blocks) R2 = multiply_block(i + 2, R2);
-        if (i + 3 < my_blocks) R3 = multiply_block(i + 3, R3);
-    }
-    // the two 16-wide halves of every result sit 32 lanes apart
-#pragma unroll
-    for (int r = 0; r < 4; r++) acc[r] += __shfl_xor(acc[r], 32);
-
-    if (KS > 1) {  // add the splits up in order, through the (now idle) activation area
-        __syncthreads();
-        float *red = reinterpret_cast<float *>(lds);
-        if (ksp > 0) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) red[(((ksp - 1) * RG + rgrp) * 4 + r) * 64 + lane] = acc[r];
-        }
-        __syncthreads();
-        if (ksp > 0) return;
-#pragma unroll
-        for (int k = 0; k < KS - 1; k++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[r] += red[((k * RG + rgrp) * 4 + r) * 64 + lane];
-    }
-    if (g < 2) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int b = 4 * g + r;
-            if (b < batch && row0 + j < rows) y[(size_t)b * rows + row0 + j] = acc[r];
-        }
-    }
-}
-
 // ------------------------------------------------------------------ thin GEMM over whole spans (Q4_K)
 //
 // The kernel above walks a row group's blocks one after the other, four in flight: at 14336x4096 a
@@ -930,19 +728,27 @@ __global__ __launch_bounds__(512) void thin_span_q4_k_kernel(const uint8_t *__re
 
 // ------------------------------------------------------------------ thin GEMM streamed in chunks (Q6_K)
 //
-// The Q6_K kernel above loads a block's planes into registers with five gather-like loads per lane (sixteen
-// rows an instruction) and walks a row group's blocks as a chain of round trips.  Here a workgroup is ONE row
-// group of 16 rows and its wavefronts split the row's blocks; a wavefront moves a chunk -- S6_CB blocks of its 16
+// The same products as the Q4_K kernels', for groups of up to 8 activation rows.  Q6_K scales sixteen weights at
+// a time, and a K=32 MFMA would add up two such groups.  So the 16 rows of the MFMA's activation
+// operand hold the (at most 8) activation rows twice: rows 0..7 with only the first sixteen k of
+// every 32 (the rest zero), rows 8..15 with only the second sixteen.  One MFMA then returns, for
+// each (activation, weight row), the two 16-wide dots side by side -- in the lanes of k-groups 0..1
+// and 2..3, which multiply them by their own group's int8 scale; the two halves of a result meet
+// once, at the end.  The 6-bit codes go in as signed bytes q - 32 (one add and one xor per four
+// codes), so there is no "-32 * sum of the activations" term to carry: the integers are
+// dot_q6_k_q8's (crates/frink-quant/src/lib.rs:1069-1110), split in two partial sums per block.
+//
+// A workgroup is ONE row group of 16 rows and its wavefronts split the row's blocks; a wavefront moves a chunk -- S6_CB blocks of its 16
 // rows, and the same blocks of the (at most 8) quantized activation rows -- into an LDS buffer of its own with
 // global_load_lds (a lane names its own 16-byte piece: the LDS image is the rows back to back,
 // [ql CB x 128 | qh CB x 64 | sc CB x 16 | the 16 bytes around the chunk's d] a row; the activations CB x 16 pieces a
 // row and one of padding, so that the rows of a read fall in different banks), and multiplies the chunk when it
 // has landed; with two buffers the next chunk travels meanwhile.  Nothing is shared before the sums: no barrier in
-// the loop.  The arithmetic is the kernel's above.  (The longer a chunk, the longer the contiguous runs the
+// the loop.  (The longer a chunk, the longer the contiguous runs the
 // planar rows give the memory system: a block's run is 128 bytes.)
 // Measured at 4096 x 14336, 8 rows, from quantized activations (us): chunks of 2 blocks, one buffer, 14 wavefronts 16.3;
 // 2 blocks, two buffers, 7 wavefronts 16.7 - 17.1; one block, two to four buffers, 6 to 13 wavefronts 17.8 - 20.0; chunks of 4
-// blocks 23 and more; the kernel above 19.7.  More wavefronts beat deeper buffers: a wavefront issues one instruction
+// blocks 23 and more; a block's planes staged through registers, eight wavefronts a workgroup, 19.7.  More wavefronts beat deeper buffers: a wavefront issues one instruction
 // in five clocks or so, and a chunk is some 600 of them.
 constexpr int S6_CB = 2;                                // blocks of a chunk (2 or 4: the chunk's d sit in one aligned 16 bytes)
 constexpr int S6_BUFS = 1;                              // 1 or 2
@@ -1112,8 +918,8 @@ __global__ __launch_bounds__(64 * S6_MAX_WAVES) void thin_stream_q6_k_kernel(con
 
 static int thin_lanes_per_row(int units) { return units > 32 ? 64 : units > 16 ? 32 : 16; }
 
-static unsigned thin_grid(size_t rows, int lpr, int r) {
-    const size_t rows_per_wg = (THIN_THREADS / 64) * (size_t)(64 / lpr) * (size_t)r;
+static unsigned thin_grid(size_t rows, int lpr) {
+    const size_t rows_per_wg = (THIN_THREADS / 64) * (size_t)(64 / lpr);
     size_t g = (rows + rows_per_wg - 1) / rows_per_wg;
     if (g > 256) g = 256;  // a workgroup per CU; wavefronts loop over rows, so the activations are staged once
     return (unsigned)(g < 1 ? 1 : g);
@@ -1122,41 +928,43 @@ static unsigned thin_grid(size_t rows, int lpr, int r) {
 constexpr size_t THIN_LDS_LIMIT = 150 * 1024;
 
 template <int LPR, int NB>
-static int launch_thin_one(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
+static int launch_thin_q4(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
     const int nb = (int)(w->cols / QK_K);
-    const bool q4 = w->kind == FRK_KIND_Q4_K;
-    const size_t shmem = (size_t)NB * nb * (256 + (q4 ? 8 : 16) * 4 + 4);
-    constexpr int R4 = 1, R6 = 1;  // more rows per lane spill at 128 registers and were measured slower  // weight rows per lane and unit
-    const unsigned grid = thin_grid(w->rows, LPR, q4 ? R4 : R6);
-    if (q4) {
-        static bool sized = false;
-        if (shmem > 65536 && !sized) {
-            FRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&thin_q4_k_kernel<LPR, NB>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)THIN_LDS_LIMIT));
-            sized = true;
-        }
-        hipLaunchKernelGGL((thin_q4_k_kernel<LPR, NB>), dim3(grid), dim3(THIN_THREADS), shmem, s, w->dev,
-                           w->layout.row_stride, (int)w->rows, nb, batch, a.q, a.d, a.bsums, y);
-    } else {
-        static bool sized = false;
-        if (shmem > 65536 && !sized) {
-            FRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&thin_q6_k_kernel<LPR, NB, R6>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)THIN_LDS_LIMIT));
-            sized = true;
-        }
-        hipLaunchKernelGGL((thin_q6_k_kernel<LPR, NB, R6>), dim3(grid), dim3(THIN_THREADS), shmem, s, w->dev, w->layout,
-                           (int)w->rows, nb, batch, a.q, a.d, a.bsums, y);
+    const size_t shmem = (size_t)NB * nb * (256 + 8 * 4 + 4);
+    static bool sized = false;
+    if (shmem > 65536 && !sized) {
+        FRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&thin_q4_k_kernel<LPR, NB>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)THIN_LDS_LIMIT));
+        sized = true;
     }
-    FRK_LAUNCH_CHECK("thin gemm");
+    hipLaunchKernelGGL((thin_q4_k_kernel<LPR, NB>), dim3(thin_grid(w->rows, LPR)), dim3(THIN_THREADS), shmem, s, w->dev,
+                       w->layout.row_stride, (int)w->rows, nb, batch, a.q, a.d, a.bsums, y);
+    FRK_LAUNCH_CHECK("thin gemm (Q4_K)");
     return FRK_OK;
 }
-
-template <int NB>
-static int launch_thin_nb(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
+template <int LPR>
+static int launch_thin_q6(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
+    constexpr int NB = 2, R = 1;  // (more rows per lane spill at 128 registers and were measured slower)
+    const int nb = (int)(w->cols / QK_K);
+    const size_t shmem = (size_t)NB * nb * (256 + 16 * 4 + 4);
+    static bool sized = false;
+    if (shmem > 65536 && !sized) {
+        FRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&thin_q6_k_kernel<LPR, NB, R>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)THIN_LDS_LIMIT));
+        sized = true;
+    }
+    hipLaunchKernelGGL((thin_q6_k_kernel<LPR, NB, R>), dim3(thin_grid(w->rows, LPR)), dim3(THIN_THREADS), shmem, s, w->dev, w->layout,
+                       (int)w->rows, nb, batch, a.q, a.d, a.bsums, y);
+    FRK_LAUNCH_CHECK("thin gemm (Q6_K)");
+    return FRK_OK;
+}
+// one or two rows
+static int launch_thin_two(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
+    const bool q4 = w->kind == FRK_KIND_Q4_K;
     const int lpr = thin_lanes_per_row((int)(w->cols / QK_K) * 4);
-    if (lpr == 64) return launch_thin_one<64, NB>(w, batch, a, y, s);
-    if (lpr == 32) return launch_thin_one<32, NB>(w, batch, a, y, s);
-    return launch_thin_one<16, NB>(w, batch, a, y, s);
+    if (lpr == 64) return q4 ? launch_thin_q4<64, 2>(w, batch, a, y, s) : launch_thin_q6<64>(w, batch, a, y, s);
+    if (lpr == 32) return q4 ? launch_thin_q4<32, 2>(w, batch, a, y, s) : launch_thin_q6<32>(w, batch, a, y, s);
+    return q4 ? launch_thin_q4<16, 2>(w, batch, a, y, s) : launch_thin_q6<16>(w, batch, a, y, s);
 }
 
 constexpr size_t TM_LDS_LIMIT = 160 * 1024;
@@ -1172,8 +980,7 @@ static int launch_thin_mfma_kind(const frk_weights *w, int batch, Q8KActs a, flo
         sized = true;
     }
     const size_t groups = (w->rows + 15) / 16;
-    hipLaunchKernelGGL((thin_mfma_q4_k_kernel<RG, ACTS, Q5>), dim3((unsigned)((groups + RG - 1) / RG), (unsigned)((batch + ACTS - 1) / ACTS)),
-                       dim3(64 * TM_WAVES),
+    hipLaunchKernelGGL((thin_mfma_q4_k_kernel<RG, ACTS, Q5>), dim3((unsigned)((groups + RG - 1) / RG)), dim3(64 * TM_WAVES),
                        shmem, s, w->dev, w->layout.row_stride, (int)w->rows, (int)(w->cols / QK_K), batch, a.q, a.d,
                        a.bsums, y);
     FRK_LAUNCH_CHECK("thin mfma gemm");
@@ -1195,49 +1002,16 @@ static int launch_thin_mfma_rg(const frk_weights *w, int batch, Q8KActs a, float
     // row groups per workgroup: as many as still give (nearly) every CU a workgroup -- one per CU was
     // measured faster than two, the activations being staged half as often; the rest of the 8
     // wavefronts split the blocks, four or more each
+    // (Of more than 4 activation rows the smaller matrices are gemm_k_rows_kernel's.)
+    constexpr int LEAST = ACTS == 4 ? 1 : ACTS == 8 ? 2 : 4;
     const size_t groups = (w->rows + 15) / 16, nb = w->cols / QK_K;
     int rg = 8;
-    while (rg > 1 && ((groups + rg - 1) / rg < 224 && (size_t)(TM_WAVES / rg) * 4 <= nb)) rg /= 2;
-    switch (rg) {
-        case 8: return launch_thin_mfma<8, ACTS>(w, batch, a, y, s);
-        case 4: return launch_thin_mfma<4, ACTS>(w, batch, a, y, s);
-        case 2: return launch_thin_mfma<2, ACTS>(w, batch, a, y, s);
-        default: return launch_thin_mfma<1, ACTS>(w, batch, a, y, s);
-    }
-}
-
-template <int RG, int ACTS>
-static int launch_thin_mfma6(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
-    const size_t shmem = t6_lds_bytes(ACTS, (int)w->cols);
-    static bool sized = false;
-    if (!sized) {
-        FRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&thin_mfma_q6_k_kernel<RG, ACTS>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)TM_LDS_LIMIT));
-        sized = true;
-    }
-    const size_t groups = (w->rows + 15) / 16;
-    hipLaunchKernelGGL((thin_mfma_q6_k_kernel<RG, ACTS>), dim3((unsigned)((groups + RG - 1) / RG), (unsigned)((batch + ACTS - 1) / ACTS)),
-                       dim3(64 * TM_WAVES), shmem, s, w->dev, w->layout, (int)w->rows, (int)(w->cols / QK_K), batch, a.q, a.d, y);
-    FRK_LAUNCH_CHECK("thin mfma gemm");
-    return FRK_OK;
-}
-// rows of activations the Q6_K matrix-core kernel can stage for this matrix (8, 4 or 0)
-static int thin_mfma6_acts(const frk_weights *w) {
-    for (int acts = 8; acts >= 4; acts /= 2)
-        if (t6_lds_bytes(acts, (int)w->cols) <= TM_LDS_LIMIT) return acts;
-    return 0;
-}
-template <int ACTS>
-static int launch_thin_mfma6_rg(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
-    const size_t groups = (w->rows + 15) / 16, nb = w->cols / QK_K;
-    int rg = 8;
-    while (rg > 1 && ((groups + rg - 1) / rg < 224 && (size_t)(TM_WAVES / rg) * 4 <= nb)) rg /= 2;
-    switch (rg) {
-        case 8: return launch_thin_mfma6<8, ACTS>(w, batch, a, y, s);
-        case 4: return launch_thin_mfma6<4, ACTS>(w, batch, a, y, s);
-        case 2: return launch_thin_mfma6<2, ACTS>(w, batch, a, y, s);
-        default: return launch_thin_mfma6<1, ACTS>(w, batch, a, y, s);
-    }
+    while (rg > LEAST && ((groups + rg - 1) / rg < 224 && (size_t)(TM_WAVES / rg) * 4 <= nb)) rg /= 2;
+    if (rg == 8) return launch_thin_mfma<8, ACTS>(w, batch, a, y, s);
+    if (rg == 4) return launch_thin_mfma<4, ACTS>(w, batch, a, y, s);
+    if constexpr (LEAST <= 2)
+        if (rg == 2) return launch_thin_mfma<2, ACTS>(w, batch, a, y, s);
+    return launch_thin_mfma<LEAST, ACTS>(w, batch, a, y, s);
 }
 
 // ---- the streamed Q6_K kernel: rows of whole chunks of blocks, groups of 8 activation rows ----
@@ -1263,13 +1037,12 @@ static int launch_thin_stream6(const frk_weights *w, int batch, Q8KActs a, float
     return FRK_OK;
 }
 
-// ---- the span kernel: Q4_K rows of 4, 8, .. 32 blocks (a wavefront per four), up to 16 activation rows ----
+// ---- the span kernel: Q4_K rows of 4, 8, .. 32 blocks (a wavefront per four), up to 8 activation rows ----
 static bool thin_span_fits(const frk_weights *w, int batch) {
     const size_t nb = w->cols / QK_K, n_kg = nb / 4;
-    if (w->kind != FRK_KIND_Q4_K || nb % 4 || n_kg > 8 || batch < 1 || batch > 16) return false;
+    if (w->kind != FRK_KIND_Q4_K || nb % 4 || n_kg > 8 || batch < 1 || batch > 8) return false;
     if (nb * Q4_K_BYTES > w->layout.row_stride) return false;
-    const size_t lds = batch > 8 ? SpanLds<16>::bytes((int)n_kg, (int)n_kg) : SpanLds<8>::bytes((int)n_kg, (int)n_kg);
-    return lds <= TM_LDS_LIMIT;
+    return SpanLds<8>::bytes((int)n_kg, (int)n_kg) <= TM_LDS_LIMIT;
 }
 template <int ACTS>
 static int launch_thin_span(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
@@ -1299,23 +1072,14 @@ int thin_gemm_max_batch(const frk_weights *w) {
     return 0;
 }
 
-// A batch of any width in one launch, where the kind has a kernel that takes one (Q6_K and Q5_K on the
-// matrix cores: a grid of 8- and 16-row groups); 0 rows = no such kernel for this matrix.
-int thin_gemm_wide_rows(const frk_weights *w) {
-    if (w->kind == FRK_KIND_Q5_K && thin_mfma_acts(w) >= 16) return 65535 * 16;  // (groups of 16 rows)
-    return (w->kind == FRK_KIND_Q6_K && thin_mfma6_acts(w) >= 8) ? 65535 * 8 : 0;
-}
-int launch_thin_gemm_wide(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
-    // Q5_K: many groups of activation rows fill the chip whatever the matrix, so a workgroup takes eight row groups
-    if (w->kind == FRK_KIND_Q5_K) return launch_thin_mfma<8, 16>(w, batch, a, y, s);
-    if (thin_stream6_fits(w)) return launch_thin_stream6(w, batch, a, y, s);
-    return launch_thin_mfma6_rg<8>(w, batch, a, y, s);
-}
+// Rows of a batch that go in one launch (the streamed Q6_K kernel: a grid of groups of 8); 0 = no such kernel for this matrix.
+// (Rows of 64 blocks and more go eight or four activation rows a launch, where a whole batch has not been measured.)
+int thin_gemm_wide_rows(const frk_weights *w) { return thin_stream6_fits(w) && w->cols / QK_K <= 63 ? 65535 * 8 : 0; }
+int launch_thin_gemm_wide(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) { return launch_thin_stream6(w, batch, a, y, s); }
 
 // y[batch][rows] for 1 <= batch <= thin_gemm_max_batch(w) quantized activation rows (K-quants).
 int launch_thin_gemm(const frk_weights *w, int batch, Q8KActs a, float *y, hipStream_t s) {
-    if (batch > 2 && thin_span_fits(w, batch))
-        return batch > 8 ? launch_thin_span<16>(w, batch, a, y, s) : launch_thin_span<8>(w, batch, a, y, s);
+    if (batch > 2 && thin_span_fits(w, batch)) return launch_thin_span<8>(w, batch, a, y, s);
     // (two rows of Q4_K: the dot4 kernel is still ahead)
     if ((w->kind == FRK_KIND_Q4_K && thin_mfma_acts(w) > 0 && batch > 2) || w->kind == FRK_KIND_Q5_K) {
         // the fewest staged rows that hold the batch
@@ -1324,11 +1088,13 @@ int launch_thin_gemm(const frk_weights *w, int batch, Q8KActs a, float *y, hipSt
         return launch_thin_mfma_rg<16>(w, batch, a, y, s);
     }
     if (w->kind == FRK_KIND_Q6_K && batch > 2 && thin_stream6_fits(w)) return launch_thin_stream6(w, batch, a, y, s);
-    if (w->kind == FRK_KIND_Q6_K && batch > 2 && thin_mfma6_acts(w) >= (batch > 4 ? 8 : 4))
-        return batch > 4 ? launch_thin_mfma6_rg<8>(w, batch, a, y, s) : launch_thin_mfma6_rg<4>(w, batch, a, y, s);
-    if (batch > 4) return launch_thin_nb<8>(w, batch, a, y, s);
-    if (batch > 2) return launch_thin_nb<4>(w, batch, a, y, s);
-    return launch_thin_nb<2>(w, batch, a, y, s);
+    if (w->kind == FRK_KIND_Q4_K && batch > 2 && batch <= 4) return launch_thin_q4<64, 4>(w, batch, a, y, s);  // (rows of 105 to 131 blocks)
+    const size_t nb = w->cols / QK_K;
+    for (int b = 0; b < batch; b += 2) {
+        int rc = launch_thin_two(w, std::min(2, batch - b), Q8KActs{a.q + b * w->cols, a.d + b * nb, a.bsums + b * nb * 16}, y + b * w->rows, s);
+        if (rc) return rc;
+    }
+    return FRK_OK;
 }
 
 }  // namespace frk

@@ -40,7 +40,8 @@ def test_larger_q6_k_gate_and_up(fa, blocks, ffn):
 
 
 # Blocks at which one kernel's order of a row's sums is the other's, and lengths on either side
-@pytest.mark.parametrize("kind,equal,others", [(fo.Q4_K, (1, 8, 9, 12, 15, 16), (17, 20, 21)), (fo.Q5_K, (1, 7, 8, 16, 32), (9, 12, 15, 17)), (fo.Q6_K, (1, 8, 9, 12, 15, 17, 19), (20, 24))])
+@pytest.mark.parametrize("kind,equal,others", [(fo.Q4_K, (1, 8, 9, 12, 15, 16, 65, 72), (17, 20, 21)), (fo.Q5_K, (1, 7, 8, 16, 32, 65, 72), (9, 12, 15, 17)),
+                                               (fo.Q6_K, (1, 8, 9, 12, 15, 17, 19, 65, 72), (20, 24))])
 def test_one_row_from_quantized_activations(fa, kind, equal, others):
     """frk_hip_gemv_q8k_dev and a one-row frk_hip_gemm_acts_dev against frk_hip_gemv_dev: the same bits, or the same integers in another
     order (a chain of at most nb + 6 additions of f32 terms no larger than the row's magnitudes in either)."""
