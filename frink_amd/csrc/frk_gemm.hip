@@ -81,7 +81,7 @@ __global__ __launch_bounds__(512) void quantize_q8_k_octets_kernel(const float *
     if (lane == 0) plain.d[at] = d;
 }
 
-// The grouped form: work items (tile, matrix, row group of 256 rows) streamed by persistent workgroups.
+// The grouped form: work items (tile, matrix, row group of 128 rows) streamed by persistent workgroups.
 struct StreamArgs {
     const uint8_t *W[2];
     float *y[2];  // row (tile's first row of y + r) x [rows]: tile row r
@@ -311,18 +311,19 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
                     __builtin_amdgcn_readfirstlane(v.z)};
     };
 
-    // ---- the fetch side: a cursor (item, block) three steps ahead of the arithmetic; where the activations travel two
-    // steps ahead (A_STAGES) they have a cursor of their own.  weights of a step: this wavefront's 32 rows (WeightSide); activations: quant slice
-    // `wave`, plus the sums (wavefront 0) or the scales (wavefront 1).  Addresses are a uniform base that moves with
-    // the cursor plus a lane offset: the activations' is fixed per item, the weights' for the kernel (recomputing the
-    // offsets from the lane number cost ~60 vector instructions per step, and per item still 2 % of a layer).
+    // ---- the fetch side: two cursors (item, block).  While step s is multiplied the activations' asks for step s + 1
+    // (A_STAGES is 2: the stage that step s - 1 was read from, which the barrier at its end has freed) and the weights' for
+    // step s + 1 + W_STAGES, into the stage that step s + 1's block has just left for the registers: three steps ahead, Q6_K two.
+    // weights of a step: this wavefront's 32 rows (WeightSide), which no other wavefront reads.  Addresses are a uniform base
+    // that moves with the cursor plus a lane offset: the activations' is fixed per item, the weights' for the kernel (recomputing
+    // the offsets from the lane number cost ~60 vector instructions per step, and per item still 2 % of a layer).
     Side wside;
     auto opaque_lane = [&]() {  // the lane number as a value the compiler cannot hoist expressions of
         int l = lane;
         asm volatile("" : "+v"(l));
         return l;
     };
-    // activations: quant slice `wave` of each half in use, plus one of the four small pieces: sums
+    // activations: quant slices `wave` and `wave` + 4 of each half in use, plus one of the four small pieces: sums
     // (wavefronts 0, 2; only with mins) and scales (1, 3) of the first (0, 1) and second half (2, 3)
     const bool x_sums = (wave & 1) == 0;
     const bool x_small = wave < 4 && (MINS || !x_sums), x_second = wave >= 2;  // fetches a small piece at all; the second half's
@@ -356,7 +357,7 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
         const int t = it.tile;
         f_two = it.count > 32;
         if (GATHER) {
-            // piece (row, 16-byte half hk) of quant slice `wave`: bytes 32 * wave + 16 * hk of the row's block;
+            // piece (row, 16-byte half hk) of quant slice `wave`: bytes 32 * wave + 16 * hk of the row's block (SLICE_STEP on: the other slice's);
             // of the sums: 16 * hk of the block's 32 bytes; the scale: the block's 4 bytes
             uint32_t src;  // this lane's source rows of the tile (row lane % 32 of either half)
             asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(src) : "v"(lds_src + ord * 128 + (lane & 31) * 4));
@@ -518,8 +519,11 @@ __device__ __forceinline__ void stream_gemm(const StreamArgs &g) {
         if (more && !fetch_late) fetch_weights();
         multiply_step(Bcur, R, Bnext);
         if (more && fetch_late) fetch_weights();
-        // with two stages the weights just asked for (the youngest loads; a finished item's stores are older) may stay in
-        // flight, everything older must have landed: the next step's activations and the weights of the one behind it
+        // What may be in flight past this wait: with two stages the weights of step s + 3, asked for in this step (the youngest loads
+        // on either side of the products: the activations and a finished item's stores went out before them); step s + 1's activations
+        // and step s + 2's weights, which step s + 1 unpacks, have landed.  With one stage (step s + 2's weights are the ones
+        // just asked for), or where this step asked for none: nothing.  The barrier then makes the activations, fetched by four
+        // wavefronts, everybody's, and the stage that this step read free.
         if (more && L::W_STAGES > 1) wait_vm<Side::REQUESTS>();
         else wait_vm<0>();
         lds_barrier();
@@ -738,8 +742,8 @@ static int launch_stream(void (*kernel)(StreamArgs), const StreamArgs &g, int ma
         if (e != hipSuccess) return set_error(FRK_ERR_HIP, "grouped GEMM setup: %s", hipGetErrorString(e));
         grid = 2 * (cus < 8 ? 8 : cus / 8 * 8);  // two workgroups per CU, a multiple of the 8 XCDs
     }
-    // more workgroups than CUs when a workgroup's share of the largest possible list would not fit
-    // its item table
+    // more than two workgroups a CU (which then follow one another) when a workgroup's share of the largest possible list
+    // would not fit its item table
     const size_t most_items = ((size_t)max_tiles + 7) / 8 * g.n_mat * g.row_tiles;
     const unsigned rounds = (unsigned)((most_items + (size_t)(grid / 8) * L::MAX_ITEMS - 1) /
                                        ((size_t)(grid / 8) * L::MAX_ITEMS));
