@@ -1,6 +1,6 @@
-"""The pipelined K-quant GEMM where its tiles are not filled.  Batches of 9 to 32 rows on the 64 x 32 tiles: rows past the last whole
-tile, blocks that do not divide by a step's four shares, parts of few blocks, and the sizes on both sides of the rule that
-sends a batch there.  Larger ones whose last token tile has few rows in use."""
+"""The pipelined K-quant GEMM where its tiles are not filled.  Batches of 9 to 32 rows at the sizes of the 64 x 32 tiles: rows past the
+last whole tile, blocks that do not divide by a step's four shares, parts of few blocks (most of them are gemm_k_rows_kernel's by
+now; sizes that still go to the tiles are in test_thin_kernels.py).  Larger ones whose last token tile has few rows in use."""
 import ctypes as C
 
 import numpy as np
@@ -198,7 +198,8 @@ def test_twelve_parts_are_added_in_pairs(fa, rows, batch, cols):
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols,batch", [(1264, 2048, 19), (300, 2048, 32), (4096, 3072, 23)])
 def test_short_rows_stay_on_the_thin_kernels(fa, rows, cols, batch):
-    """Q4_K of 8 and 12 blocks: a row's results do not depend on the batch that it came in with, up to 32 rows."""
+    """Q4_K of 8 and 12 blocks: a row's results do not depend on the batch that it came in with, up to 32 rows (on gemm_k_rows_kernel,
+    as on the thin kernels before)."""
     from frink_amd import synth
     w = fa.Weights.from_host(fo.Q4_K, make_weights(fo.Q4_K, rows, cols, seed=rows), rows, cols)
     x = to_dev(synth.activations(batch, batch, cols))

@@ -42,6 +42,8 @@ def test_pipelined_gemm_at_the_edges_of_its_tiles(fa, kind, rows, cols, batch):
     (fo.Q5_K, 264, 4096),    # 16 blocks of few rows: from 17
     (fo.Q6_K, 4104, 8448),   # large, an odd number of blocks: from 9
     (fo.Q6_K, 8200, 4352),   # the same with 17 blocks, whose batches have no tiles below 17 rows: from 17
+    # (gemm_k_rows_kernel has those above on both sides of 9, the third and the last two of 17; on the tiles from 9, 9 and 17 on:)
+    (fo.Q4_K, 72, 12288), (fo.Q5_K, 72, 12288), (fo.Q6_K, 1300, 12544),
 ])
 def test_batches_around_the_step_from_thin_to_tiled(fa, kind, rows, cols):
     """Both sides of the batch size at which a matrix changes kernels, against 64-bit sums of the same quantized
@@ -66,9 +68,11 @@ def test_batches_around_the_step_from_thin_to_tiled(fa, kind, rows, cols):
     w.release()
 
 
-@pytest.mark.parametrize("kind,rows,cols", [(fo.Q4_K, 640, 9728), (fo.Q5_K, 640, 8192), (fo.Q6_K, 4104, 8448)])
+@pytest.mark.parametrize("kind,rows,cols", [(fo.Q4_K, 640, 9728), (fo.Q5_K, 640, 8192), (fo.Q6_K, 4104, 8448), (fo.Q4_K, 640, 12288), (fo.Q5_K, 640, 12288),
+                                            (fo.Q6_K, 1000, 20224)])
 def test_a_batch_past_the_thin_kernels_is_no_further_from_64_bit_sums(fa, kind, rows, cols):
-    """Eight rows run on the thin kernels and nine on the matrix cores: the larger batch must not be less precise.  The
+    """Eight rows run on sixteen-row workgroups and nine (of the last three sizes) on tiles whose parts are added by a second launch:
+    the larger batch must not be less precise.  The
     2-norms of thousands of independent errors are within a few percent of their expectation, hence the tenth."""
     from frink_amd import synth
     # (encoded rows, whose offsets and scaled codes nearly cancel as a checkpoint's do)

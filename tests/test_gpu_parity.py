@@ -320,7 +320,7 @@ def test_q4_k_gemv_over_whole_cache_lines(fa, kind, rows, cols):
 def test_thin_gemm_from_activations_quantized_beforehand(fa, kind, rows, cols, batches):
     """frk_hip_gemm_q8k_dev (apply_batch_with_acts with BatchActs::Q8K, weight_matrix.rs:2481-2487, 757-768): a thin
     batch over Q8_K activations that frk_hip_quantize_q8_k_dev (or the producing kernel) wrote -- bit for bit
-    frk_hip_gemm_dev's result (one row: frk_hip_gemv_q8k_dev's); a batch beyond the thin kernels' is refused with a
+    frk_hip_gemm_dev's result (one row: frk_hip_gemv_q8k_dev's); a batch beyond those is refused with a
     message that names the entry to call."""
     from frink_amd import synth
     data = make_weights(kind, rows, cols, seed=rows + cols)
@@ -346,13 +346,11 @@ def test_thin_gemm_from_activations_quantized_beforehand(fa, kind, rows, cols, b
                                        (2, 7936), (63, 7680), (33, 16384), (10, 3072), (9, 2560)])
 @pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K])
 def test_gemv_at_rows_between_the_line_lengths(fa, kind, rows, cols):
-    """Rows whose block count is not 8, 16 or 32.  From 17 blocks on (4352 columns) a wavefront takes the whole
-    rows that fit its 64 lanes -- 3 rows of 20 blocks, one of 56 -- and adds a row's blocks with a segmented
-    shuffle: in one launch up to 31 blocks (Q4_K: up to 20; longer rows take the kernel whose wavefronts split the
-    columns), behind a quantization launch from 33 on (Q5_K, and Q4_K from quantized activations); shorter rows keep
-    the per-lane kernel.  Row counts that fill spans, fall short of one and leave a short last span, for
-    frk_hip_gemv_dev and frk_hip_gemv_q8k_dev (whose staging once stopped at 256 pairs of 16-wide sums: wrong
-    results at 14336 columns)."""
+    """Rows whose block count is not 8, 16 or 32, few of them.  frk_hip_gemv_dev gives them to the kernel whose wavefronts
+    split the columns.  From quantized activations (frk_hip_gemv_q8k_dev) a wavefront takes the whole rows that fit its
+    64 lanes from 33 blocks on -- one row of 56 -- and adds a row's blocks with a segmented shuffle (its staging once stopped at
+    256 pairs of 16-wide sums: wrong results at 14336 columns); shorter rows have the per-lane kernel.  Row counts
+    that fill spans, fall short of one and leave a short last span.  (The whole-rows kernel in one launch: test_gemv_forms.py.)"""
     from frink_amd import synth
     data = make_weights(kind, rows, cols, seed=rows + cols)
     x = synth.activations(rows + cols, 1, cols, outlier_frac=0.01)[0]
@@ -372,8 +370,8 @@ def test_gemv_at_rows_between_the_line_lengths(fa, kind, rows, cols):
                                        (17, 11008), (24, 13824), (40, 16128), (100, 9472)])
 @pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K])
 def test_q4_k_gemv_with_the_columns_split_between_wavefronts(fa, kind, rows, cols):
-    """Q4_K rows of more than 20 blocks (of 32 blocks: few or many rows) and Q5_K rows of more than 32, one launch (the
-    other shapes in the list run on the kernels they had): a wavefront takes four blocks of
+    """Q4_K rows of more than 20 blocks (of 32 blocks: few or many rows), Q5_K rows of more than 32 and of 21 to 31 (few or
+    many rows), one launch (the other shapes in the list run on the kernels they had): a wavefront takes four blocks of
     columns of the workgroup's 8, 16 or 24 rows and quantizes exactly those blocks itself.  Row counts that fill a
     workgroup, fall short and leave a short last one, at every number of rows to a workgroup the launch picks (the
     large row counts: random block bytes); block counts that fill the last wavefront's four and do not."""
@@ -423,10 +421,9 @@ def test_host_buffer_launch_matvec_is_the_drop_in(fa, kind):
 def test_q5_k_decode_and_batches_at_full_size(fa):
     """Q5_K (Q4_K's scale packing, a fifth bit per code from a separate plane): the FFN shape with
     arbitrary block bytes (every bit pattern of the fifth-bit plane) against the oracle on slices of
-    rows, for one row (the decode kernel), 3, 16, 17 and 32 rows (the thin matrix-core kernel: 16 rows
-    a workgroup, wider batches as a grid of 16-row groups in one launch), 33, 70 and 512 rows (the tiled
-    matrix-core kernel, a scaled code's two bytes as its int8 planes, its blocks split between workgroups for
-    the small batches), and the whole output of a row against dequantized weights in float64."""
+    rows, for one row (the decode kernel), 3 rows (sixteen-row workgroups), 16 (the thin matrix-core kernel), 17, 32,
+    33, 70 and 512 rows (the tiled matrix-core kernel, a scaled code's two bytes as its int8 planes, its blocks split
+    between workgroups for the small batches), and the whole output of a row against dequantized weights in float64."""
     from frink_amd import synth
     rows, cols = 14336, 4096
     data = _random_q5_k(rows, cols, 41)
@@ -1488,9 +1485,10 @@ def test_thin_gemm_matches_the_oracle_and_the_gemv(fa, kind, rows, cols, batch):
 
 @pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K, fo.Q6_K, fo.Q8_0])
 def test_gemm_at_every_batch_size_where_the_kernel_changes(fa, kind):
-    """frk_hip_gemm_dev picks a kernel by the batch size (one row: the GEMV; 2: dot4; 3..16: thin on
-    the matrix cores; wider: 8-row groups, or the MFMA GEMM from 33 rows (Q4_K) or from 25 or 41 (Q6_K, by the matrix's size); Q8_0:
-    the MFMA GEMM from two rows, its token tile growing at 33 and 65): every size on either side of a threshold, on a ragged matrix, against the oracle."""
+    """frk_hip_gemm_dev picks a kernel by the batch size and the matrix (one row: the GEMV; K-quants of this size: sixteen-row workgroups,
+    a tile of 16 or 32 rows each and every 32 from 33 on, Q6_K of two blocks the streamed thin kernel's 8-row groups in between;
+    Q8_0: the MFMA GEMM from two rows, its token tile growing at 33 and 65): every size on either side of a threshold, on a ragged
+    matrix, against the oracle."""
     from frink_amd import synth
     rows, cols = 72, 512
     data = make_weights(kind, rows, cols, seed=900 + kind)
