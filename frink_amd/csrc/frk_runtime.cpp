@@ -665,9 +665,9 @@ static bool k_quant_takes_the_matrix_cores(const frk_weights *w, size_t batch) {
     if (batch >= 17) return measured && n > 23 * M;
     return measured && n > 48 * M && w->rows > 4096;
 }
-// The crossings against the 128 x 64 tiles, higher than those above: below them the thin kernels hold a batch, and
-// frk_hip_gemm_q8k_dev takes it (one between the two is put into the tiled form first, so that it has frk_hip_gemm_dev's bits).
-// (The first test holds for every batch beyond them today; a batch that stays on the thin kernels is held by them in any case.)
+// What frk_hip_gemm_q8k_dev refuses, and where a call's scratch buffer may grow during a capture: no question of speed any more, but of what the
+// entry point has always taken.  These were the crossings against the 128 x 64 tiles, higher than those above: below them the thin kernels hold
+// a batch, and frk_hip_gemm_q8k_dev takes it (with frk_hip_gemm_dev's kernel, so that it has its bits: from tiles that it makes first, or plain rows).
 static bool matrix_cores_only(const frk_weights *w, size_t batch) {
     if (!k_quant_takes_the_matrix_cores(w, batch)) return false;
     const size_t n = w->rows * w->cols, nb = w->cols / QK_K, M = (size_t)1 << 20;
