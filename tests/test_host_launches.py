@@ -2,7 +2,7 @@
 grouped launches take, each with an array of outputs no longer than it has matrices."""
 import host_library
 
-DRIVER = r"""
+PROGRAM = r"""
 #include <cstdio>
 #include "frink_amd/csrc/frk_internal.hpp"
 using namespace frk;
@@ -52,5 +52,5 @@ int main() {
 
 
 def test_grouped_and_paired_launches_stay_inside_their_arrays(tmp_path):
-    calls = int(host_library.run(host_library.build(tmp_path, DRIVER)).split()[0])
+    calls = int(host_library.run(host_library.build(tmp_path, PROGRAM)).split()[0])
     assert calls == 5 * (64 * 3 + 64 * 4 + 64 * 4 + 62 * 4 + 64 + 64 + 53 + 62)

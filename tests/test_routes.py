@@ -5,7 +5,7 @@ import pytest
 import host_library
 import oracle as fo
 
-DRIVER = r"""
+PROGRAM = r"""
 #include <cstdio>
 #include "frink_amd/csrc/frk_internal.hpp"
 #include "include/frink_hip.h"
@@ -30,7 +30,7 @@ int main() {  // a call a line: its name, kind, rows, blocks of 256 columns, tok
 
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
-    binary = host_library.build(tmp_path_factory.mktemp("routes"), DRIVER)
+    binary = host_library.build(tmp_path_factory.mktemp("routes"), PROGRAM)
 
     def of(calls):
         lines = host_library.run(binary, "".join("%s %d %d %d %d\n" % c for c in calls)).splitlines()
