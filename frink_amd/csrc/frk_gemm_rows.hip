@@ -30,7 +30,7 @@ constexpr int ROWS_WAVES = 8;
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // The activations behind buffer descriptors: a load's address is a lane offset and a scalar one.  As plain rows, not
-// tiles, a load touches a line for every token.
+// tiles, a load touches a line for every token (Q4_K and Q5_K: the quants come through LDS, see stage).
 template <bool PLAIN>
 struct RowsActs {
     __amdgpu_buffer_rsrc_t q, sums, d;
@@ -99,19 +99,40 @@ struct RowsSide {
         v4h sums;  // of the groups of sixteen 4g .. 4g + 3
         v4f d;     // of tokens 4g .. 4g + 3
     };
-    template <bool PLAIN>
-    static __device__ __forceinline__ void load_acts(Acts &A, const RowsActs<PLAIN> &a, int kb, int t, int tok, int g) {
-        const int at = PLAIN ? tok * a.nb * QK_K + 8 * g : (g >> 1) * 512 + tok * 16 + (g & 1) * 8;
+    static __device__ __forceinline__ void load_acts(Acts &A, const RowsActs<false> &a, int kb, int t, int tok, int g) {
+        const int at = (g >> 1) * 512 + tok * 16 + (g & 1) * 8;
 #pragma unroll
-        for (int s = 0; s < 8; s++)
-            A.q[s] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(a.q, at, PLAIN ? kb * QK_K + 32 * s : kb * 8192 + 1024 * s, 0));
-        if constexpr (PLAIN) {
-            const v2i four = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(a.sums, tok * a.nb * 32 + 8 * g, kb * 32, 0));
-            A.sums = v4h{(_Float16)(short)four.x, (_Float16)(short)(four.x >> 16), (_Float16)(short)four.y, (_Float16)(short)(four.y >> 16)};
-        } else {
-            A.sums = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(a.sums, at, kb * 1024, 0));
-        }
+        for (int s = 0; s < 8; s++) A.q[s] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(a.q, at, kb * 8192 + 1024 * s, 0));
+        A.sums = __builtin_bit_cast(v4h, __builtin_amdgcn_raw_buffer_load_b64(a.sums, at, kb * 1024, 0));
         A.d = a.scales(kb, t, g);
+    }
+    // Of plain rows a load of eight bytes a lane touches a line for every token, twice.  So their quants come through LDS, sixteen tokens
+    // of a block as four requests of whole rows' 256 bytes, piece p of token t in place p ^ t (a read's sixteen tokens then fall in different
+    // banks), and the next block's are asked for in front of the products and not behind them: 16 tokens of 525 x 4096 in Q4_K 6.7 -> 4.1 us, 3 of
+    // 2132 x 13056 in Q5_K 14.0 -> 10.8 (the thin kernels: 4.7 and 12.6).
+    struct Small {  // a block's sums as they are, and its scales
+        v2i sums;
+        v4f d;
+    };
+    static __device__ __forceinline__ void stage(uint32_t lds, const int8_t *q, const uint32_t (&from)[4], int kb) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) dma16(lds + c * 1024, q + (size_t)kb * QK_K, from[c]);
+    }
+    static __device__ __forceinline__ void load_small(Small &S, const RowsActs<true> &a, int kb, int tok, int g) {
+        S.sums = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(a.sums, tok * a.nb * 32 + 8 * g, kb * 32, 0));
+        S.d = a.scales(kb, 0, g);
+    }
+    static __device__ __forceinline__ void take(Acts &A, const Small &S, const uint8_t *staged, int lane) {
+        const int tok = lane & 15, g = lane >> 4;
+        const uint8_t *const mine = staged + tok * QK_K + (g & 1) * 8;
+        const int place = (tok ^ (g >> 1)) << 4;
+#pragma unroll
+        for (int s = 0; s < 8; s++) A.q[s] = *reinterpret_cast<const v2i *>(mine + (place ^ (s << 5)));
+        A.sums = v4h{(_Float16)(short)S.sums.x, (_Float16)(short)(S.sums.x >> 16), (_Float16)(short)S.sums.y, (_Float16)(short)(S.sums.y >> 16)};
+        A.d = S.d;
+#pragma unroll
+        for (int s = 0; s < 8; s++) asm volatile("" : "+v"(A.q[s]));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     // sum[t][r] += weight row lane % 16 times token 16t + 4g + r
     template <int TT>
@@ -253,6 +274,11 @@ struct RowsSide {  // (the host side needs the slot's size only)
     static constexpr int SLOT = KIND == FRK_KIND_Q4_K ? 16 * 19 * 16 : KIND == FRK_KIND_Q5_K ? 16 * 23 * 16 : 6912;
 };
 #endif
+// Whether the plain rows' quants go through LDS (of Q6_K a lane loads sixteen bytes, in half as many loads), and a wavefront's part of it
+template <int KIND, bool PLAIN>
+constexpr bool rows_staged() { return PLAIN && KIND != FRK_KIND_Q6_K; }
+template <int KIND, bool PLAIN>
+constexpr int rows_wave_lds() { return RowsSide<KIND>::SLOT + (rows_staged<KIND, PLAIN>() ? 16 * QK_K : 0); }
 
 // TT tiles of sixteen tokens.  At most 128 registers: two workgroups to a CU (with 180 two tiles took 1.3 to 1.5 times as long).
 template <int KIND, int TT, bool PLAIN>
@@ -265,9 +291,12 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) __attribute__((amdgpu_waves_per_eu
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
     const int lr = lane & 15, lq = lane >> 4;
     const int row0 = (int)blockIdx.x * 16;
+    constexpr bool STAGED = rows_staged<KIND, PLAIN>();
+    static_assert(!STAGED || TT == 1, "sixteen tokens are staged");
+    constexpr int WAVE_LDS = rows_wave_lds<KIND, PLAIN>();
     const int pairs = (g.nb + 1) >> 1, p0 = min(wave * g.each, pairs), p1 = min(p0 + g.each, pairs);
-    uint8_t *const slot = rows_lds + (size_t)wave * Side::SLOT;
-    const uint32_t slot_lds = lds_address(rows_lds) + (uint32_t)wave * Side::SLOT;
+    uint8_t *const slot = rows_lds + (size_t)wave * WAVE_LDS;
+    const uint32_t slot_lds = lds_address(rows_lds) + (uint32_t)wave * WAVE_LDS;
     const uint8_t *const first = g.W + (size_t)row0 * g.row_stride;
     const Side side(g, lane, min(g.rows - 1 - row0, 15));
     const int tile = (int)blockIdx.y, M = min(g.M - 32 * tile, 32);
@@ -278,35 +307,72 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) __attribute__((amdgpu_waves_per_eu
     };
     const RowsActs<PLAIN> acts = {buffer(g.a.q, g.plain.q, 256), buffer(g.a.bs, g.plain.bsums, 32), buffer(g.a.d, g.plain.d, 4), g.nb, M};
     typename Side::Acts A[TT];
-    auto load_acts = [&](int kb) {  // (tokens past the batch repeat the last one)
-#pragma unroll
-        for (int t = 0; t < TT; t++) Side::load_acts(A[t], acts, kb, t, min(16 * t + lr, M - 1), lq);
-    };
     v4f acc[TT];
 #pragma unroll
     for (int t = 0; t < TT; t++) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    if (p0 < p1) {
-        side.fetch(g, slot_lds, first, 2 * p0, lane);
-        load_acts(2 * p0);
-    }
-    for (int p = p0; p < p1; p++) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (STAGED) {
+        const uint8_t *const staged = slot + Side::SLOT;
+        const uint32_t staged_lds = slot_lds + Side::SLOT;
+        uint32_t from[4];  // (tokens past the batch repeat the last one)
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const int kb = 2 * p + b;
-            if (kb >= g.nb) break;
-            typename Side::Raw R;
-            side.read(R, slot, b, 2 * p, lane);
-            if (b && p + 1 < p1) {
-                // the pair is in registers: the next one travels beside its arithmetic
+        for (int c = 0; c < 4; c++) from[c] = (uint32_t)min(4 * c + lq, M - 1) * (uint32_t)(g.nb * QK_K) + (uint32_t)((lr ^ (4 * c + lq)) * 16);
+        typename Side::Small next;
+        const int end = min(2 * p1, g.nb);
+        auto request = [&](int kb) {
+            if (kb < end) Side::stage(staged_lds, g.plain.q, from, kb);
+            // (past the share the last block's again: loaded under a condition they would be waited for at its end)
+            Side::load_small(next, acts, min(kb, end - 1), min(lr, M - 1), lq);
+        };
+        if (p0 < p1) {
+            side.fetch(g, slot_lds, first, 2 * p0, lane);
+            request(2 * p0);
+        }
+        for (int p = p0; p < p1; p++) {
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                const int kb = 2 * p + b;
+                if (kb >= g.nb) break;
+                // everything asked for so far: this block's quants, sums and scales, at a pair's first block its weights too
+                asm volatile("s_waitcnt vmcnt(0)" : "+v"(next.sums), "+v"(next.d)::"memory");
+                typename Side::Raw R;
+                side.read(R, slot, b, 2 * p, lane);
+                Side::take(A[0], next, staged, lane);
                 Side::arrived(R);
-                side.fetch(g, slot_lds, first, 2 * p + 2, lane);
+                // what was read is in registers: the next pair, and the next block's tokens, travel beside the arithmetic
+                if (b && p + 1 < p1) side.fetch(g, slot_lds, first, 2 * p + 2, lane);
+                request(kb + 1);
+                Side::multiply(R, lq, A, acc);
+                asm volatile("" : "+v"(acc[0]));  // (in front of the branch, see below)
             }
-            Side::multiply(R, lq, A, acc);
-            // (in front of the branch: hipcc counts an MFMA's wait states within a basic block only)
+        }
+    } else {
+        auto load_acts = [&](int kb) {  // (tokens past the batch repeat the last one)
 #pragma unroll
-            for (int t = 0; t < TT; t++) asm volatile("" : "+v"(acc[t]));
-            if (kb + 1 < min(2 * p1, g.nb)) load_acts(kb + 1);
+            for (int t = 0; t < TT; t++) Side::load_acts(A[t], acts, kb, t, min(16 * t + lr, M - 1), lq);
+        };
+        if (p0 < p1) {
+            side.fetch(g, slot_lds, first, 2 * p0, lane);
+            load_acts(2 * p0);
+        }
+        for (int p = p0; p < p1; p++) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                const int kb = 2 * p + b;
+                if (kb >= g.nb) break;
+                typename Side::Raw R;
+                side.read(R, slot, b, 2 * p, lane);
+                if (b && p + 1 < p1) {
+                    // the pair is in registers: the next one travels beside its arithmetic
+                    Side::arrived(R);
+                    side.fetch(g, slot_lds, first, 2 * p + 2, lane);
+                }
+                Side::multiply(R, lq, A, acc);
+                // (in front of the branch: hipcc counts an MFMA's wait states within a basic block only)
+#pragma unroll
+                for (int t = 0; t < TT; t++) asm volatile("" : "+v"(acc[t]));
+                if (kb + 1 < min(2 * p1, g.nb)) load_acts(kb + 1);
+            }
         }
     }
     // register r of lane (row, g): token 4 * g + r
@@ -319,7 +385,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) __attribute__((amdgpu_waves_per_eu
         float v[ROWS_WAVES];
 #pragma unroll
         for (int w = 0; w < ROWS_WAVES; w++) {
-            const float one = *reinterpret_cast<const float *>(rows_lds + (size_t)min(w, waves - 1) * Side::SLOT + at);
+            const float one = *reinterpret_cast<const float *>(rows_lds + (size_t)min(w, waves - 1) * WAVE_LDS + at);
             v[w] = w < waves ? one : 0.0f;
         }
         const float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
@@ -359,6 +425,23 @@ int launch_quantize_q8_k_one_tile(const float *x, size_t rows, size_t cols, Q8KT
     return FRK_OK;
 }
 
+template <int KIND, int TT, bool PLAIN>
+static int launch_rows(const RowsArgs &g, dim3 grid, int waves, hipStream_t s) {
+    const int lds = waves * rows_wave_lds<KIND, PLAIN>();
+    if constexpr (ROWS_WAVES * rows_wave_lds<KIND, PLAIN>() > 65536) {
+        static bool sized = false;
+        if (!sized) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_k_rows_kernel<KIND, TT, PLAIN>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, ROWS_WAVES * rows_wave_lds<KIND, PLAIN>());
+            if (e != hipSuccess) return set_error(FRK_ERR_HIP, "gemm_k_rows setup: %s", hipGetErrorString(e));
+            sized = true;
+        }
+    }
+    hipLaunchKernelGGL((gemm_k_rows_kernel<KIND, TT, PLAIN>), grid, dim3(64 * waves), lds, s, g);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(FRK_ERR_HIP, "gemm_k_rows launch: %s", hipGetErrorString(e));
+    return FRK_OK;
+}
 // batch >= 2 from the tiled form (plain null), or up to 32 from plain rows (16 of Q4_K and Q5_K): the same bits.
 int launch_gemm_k_rows(const frk_weights *w, int batch, Q8KTiled a, const Q8KActs *plain, float *y, hipStream_t s) {
     RowsArgs g;
@@ -376,9 +459,8 @@ int launch_gemm_k_rows(const frk_weights *w, int batch, Q8KTiled a, const Q8KAct
     const int pairs = (g.nb + 1) / 2;
     g.each = (pairs + ROWS_WAVES - 1) / ROWS_WAVES;
     const int waves = (pairs + g.each - 1) / g.each;
-    const dim3 grid((unsigned)((w->rows + 15) / 16), (unsigned)((batch + 31) / 32)), block(64 * waves);
-#define FRK_GO(KIND, TT, PLAIN) \
-    hipLaunchKernelGGL((gemm_k_rows_kernel<KIND, TT, PLAIN>), grid, block, waves * RowsSide<KIND>::SLOT, s, g)
+    const dim3 grid((unsigned)((w->rows + 15) / 16), (unsigned)((batch + 31) / 32));
+#define FRK_GO(KIND, TT, PLAIN) return launch_rows<KIND, TT, PLAIN>(g, grid, waves, s)
 #define FRK_GO_KIND(KIND)                         \
     if (plain) FRK_GO(KIND, 1, true);             \
     else if (batch <= 16) FRK_GO(KIND, 1, false); \
@@ -396,9 +478,6 @@ int launch_gemm_k_rows(const frk_weights *w, int batch, Q8KTiled a, const Q8KAct
     }
 #undef FRK_GO_KIND
 #undef FRK_GO
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return set_error(FRK_ERR_HIP, "gemm_k_rows launch: %s", hipGetErrorString(e));
-    return FRK_OK;
 }
 
 }  // namespace frk

@@ -710,8 +710,8 @@ static bool matrix_cores_only(const frk_weights *w, size_t batch) {
 //         4096x14336 at 16 20.7 / 15.1, but 1069x13312 at 11 13.8 / 15.0, 1024x10240 at 28 1.13 of the time, 1064x13312 at 23 14.9 / 17.7.
 // Over 6200 drawn batches of 2 .. 32 rows of 64 .. 160000 rows and 1 .. 128 blocks: 0.79 of the time before in the mean of the 3911 it takes, six of
 // them past 1.03 and 1.05 at worst; the 2-norm error against 64 bits of 108 that changed 0.92, 1.03 at most.
-// From activations quantized beforehand over the same draws: frk_hip_gemm_acts_dev 0.84 in the mean of 400, 1.02 at worst.  frk_hip_gemm_q8k_dev
-// 0.86 in the mean of 460, but 33 of them past 1.03 and 1.12 at worst (Q5_K 2132x13056 at 3 12.6 / 14.1, 3945x4608 at 8 8.5 / 9.3): it has
+// From activations quantized beforehand over the same draws: frk_hip_gemm_acts_dev 0.84 in the mean of 400, 1.02 at worst; frk_hip_gemm_q8k_dev
+// 0.77 in the mean of 2915, 18 of them past 1.03 and 1.17 at worst (Q6_K of 25 to 32 tokens, 585x8192 at 30 9.5 / 11.1): it has
 // frk_hip_gemm_dev's bits, and so its kernel, also where that one is ahead by its quantization alone.
 static bool k_rows_beside_tiles(const frk_weights *w, size_t batch) {
     static constexpr size_t ROWS[] = {1024, 2048, 2560, 4096, 5376, 8192, 12288, 16384, 24576, 28544, 32768, 40960};
@@ -988,10 +988,12 @@ int frk_hip_gemm_q8k_dev(const frk_weights *w, const int8_t *q, const float *d, 
                          "frk_hip_gemm_dev / frk_hip_gemm_pair_dev, or frk_hip_quantize_batch_acts_dev", batch);
     Q8KActs a{q, d, bsums};
     hipStream_t s = (hipStream_t)stream;
-    // (for a small matrix, or a few rows, a launch to make tiles of them costs more than what the rows' lines do)
-    const bool q6 = w->kind == FRK_KIND_Q6_K, small = w->rows * w->cols < (size_t)16 << 20 && batch <= (q6 ? 32 : 16);
-    if (k_rows_take(w, batch) && (batch <= (q6 ? 8 : 4) || small))
-        return launch_gemm_k_rows(w, (int)batch, Q8KTiled{}, &a, y, s);
+    // Plain rows, whose quants go through LDS, cost nothing over tiles that a launch of 2 us has to make (us, tiles / plain: Q4_K 5525x6144 at 8
+    // 13.4 / 10.4, Q5_K 7518x5888 at 14 15.9 / 13.0; sixteen tokens is what the kernel stages, in whole pieces of sixteen bytes).  Q6_K's are loaded from
+    // where they are, a line for each token of every sixteen weight rows, so by tokens times weights: tiles 1.10 to 1.24 of the time at 9 to 16 tokens up
+    // to 64 M weights (6368x3072 at 10 11.3 / 8.7), 25 to 28 of 26 to 36 M 1.10, 13 to 16 past 64 M 1.02, 21 to 24 of 36 to 64 M 1.003.
+    const bool plain = w->kind == FRK_KIND_Q6_K ? batch <= 8 || batch * w->rows * w->cols <= (size_t)900 << 20 : batch <= 16 && (uintptr_t)q % 16 == 0;
+    if (plain && k_rows_take(w, batch)) return launch_gemm_k_rows(w, (int)batch, Q8KTiled{}, &a, y, s);
     if (takes_tiles(w, batch)) {
         void *ws = nullptr, *parts = nullptr;
         Scratch scratch;

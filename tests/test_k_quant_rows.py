@@ -120,3 +120,19 @@ def test_rows_of_an_earlier_batch_leave_the_tiles(fa, kind, rows, cols, batch):
     acts.quantize(x)
     assert np.array_equal(bits(w.gemm_acts(acts).cpu().numpy()), want)
     w.release()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K])
+@pytest.mark.parametrize("blocks", [1, 2, 3, 15, 16, 17, 31])  # (one block, a pair, a half pair at the end; shares of one and two pairs; more are refused from 9 rows on)
+def test_plain_rows_through_lds(fa, kind, blocks):
+    """From Q8_K rows as they are the same bits as from tiles, whatever tokens of the sixteen are in use."""
+    from frink_amd import synth
+    rows, cols = 35, 256 * blocks
+    w = fa.Weights.from_host(kind, make_weights(kind, rows, cols, seed=blocks), rows, cols)
+    for batch in (3, 5, 8, 11, 13, 16):
+        print("plain rows", kind, blocks, batch, flush=True)
+        x = to_dev(synth.activations(batch, batch, cols, outlier_frac=0.01))
+        got = w.gemm_q8k(fa.quantize_q8_k(x.reshape(-1)), batch)
+        assert np.array_equal(bits(got.cpu().numpy()), bits(w.gemm(x).cpu().numpy())), batch
+    w.release()

@@ -103,3 +103,13 @@ LARGER = {fo.Q4_K: [(308, 29, 401), (2443, 31, 34), (1193, 27, 136), (144, 107, 
 def test_more_tokens_of_small_matrices(kernels, kind):
     check(kernels, "gemm", kind, SMALL[kind], "gemm_k_rows_kernel", True)
     check(kernels, "gemm", kind, LARGER[kind], "gemm_k_rows_kernel", False)
+
+
+# (us, the tiled form made first / plain rows, the same bits: 22.4 / 18.8, 13.4 / 10.4; 9.2 / 6.9, 15.5 / 12.2, 15.9 / 13.0; 11.3 / 8.7, 19.9 / 17.5)
+PLAIN = {fo.Q4_K: [(13455, 26, 5), (5525, 24, 8)], fo.Q5_K: [(3945, 18, 8), (6956, 24, 8), (7518, 23, 14)], fo.Q6_K: [(6368, 12, 10), (14336, 16, 12)]}
+
+
+@pytest.mark.parametrize("kind", [fo.Q4_K, fo.Q5_K, fo.Q6_K])
+def test_a_batch_quantized_before_needs_no_tiles(kernels, kind):
+    check(kernels, "q8k", kind, PLAIN[kind], "gemm_k_rows_kernel<%d,1,true>" % kind, True)
+    check(kernels, "q8k", kind, PLAIN[kind], "tile_q8_k_kernel", False)
